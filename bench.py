@@ -34,11 +34,6 @@ ALGO_BYTES = {
                  "interval pair 8 B per point; rank, lower and upper interval ends 24 B per edge read "
                  "or written once; triangle rank 4 B)",
         "bytes": lambda st, T, n: 8.0 * n + 24.0 * st["nEdges"] + 4.0 * st["nTris"]},
-    "k_frame_remove": {
-        "model": "12 B per frame vertex examined (state 4 + priority 8) + 88 B per fan triangle of a "
-                 "removed frame vertex (triangle record 32 read, chain position 16 read, fill or dead "
-                 "slot 32 written, anchor and back-link 8 written)",
-        "bytes": lambda st, T, n: 12.0 * st["frameSeen"] + 88.0 * st["frameChain"]},
     "k_flip_test": {
         "model": "32 B per listed triangle: the flipping stage's 24F + 16V per pass over F triangles "
                  "and V = F / 2 vertices (24 B vertex + neighbour record, 16 B position); the "

@@ -107,10 +107,10 @@ struct galpha_ctx {
     DevBuf perm, xys, pcell, ccount, ccursor;   // spatial numbering of the real points
     DevBuf cls;                                  // alpha-complex classes (host queries)
     DevBuf tv, tn, remap, stamp, claim, modA, modB, cand, pos, vt, vstate, pix, deg, off, fill, fan,
-        moved, decide, mx, mlist, loc, lt, scratch, hnext, hedge, keys, keys2, vals, vals2, rot, newid,
+        moved, decide, mx, mlist, loc, lt, scratch, keys, keys2, vals, vals2, rot, newid,
         out9, counters, status, xy, scanTmp, sortTmp, tileCnt, tileOff, dellist, dbg;
     // batch plan on the device
-    DevBuf setsD, bmD, vset, hullCnt, hullOff, hullStart, setFirst, offsD, bboxTmp, lmark, ffan, modF, badset, bnd;
+    DevBuf setsD, bmD, vset, setFirst, offsD, bboxTmp, lmark;
     // constrained DT: input pairs, vertex-id pairs, inverse numbering, flags, walk counts, region
     // sizes and offsets, cavity regions, constraint key set
     DevBuf kin, kv, kinv, kdone, kcnt, krs, kroff, kwork, khash;
@@ -620,9 +620,6 @@ static void ensure_pba(galpha_ctx *c, const BatchPlan &b)
     c->setsD.ensure(sizeof(SetDesc) * b.sets.size());
     c->bmD.ensure(sizeof(int) * b.bm.size());
     int ns = b.nsets();
-    c->hullCnt.ensure(4 * (size_t)ns + 16);
-    c->hullOff.ensure(4 * (size_t)ns + 16);
-    c->hullStart.ensure(4 * (size_t)ns + 16);
     c->setFirst.ensure(4 * (size_t)ns + 16);
 }
 
@@ -709,89 +706,34 @@ static void bbox_host(const double *xy, int n, double *bb5)
 void bbox_device(const double *d_xy, int n, double *out5, void *tmp, hipStream_t st);
 void bbox_sets_device(const double *d_xy, const int *d_offs, int nsets, double *out5, void *tmp, hipStream_t st);
 
-// Bulk frame removal: when the real region of every set is bounded by one simple cycle through all
-// of its meshed points, drop all frame triangles and convexify each cycle by parallel ear rounds.
-// Returns false (mesh untouched) when some set does not qualify.
-// On success *ear_rounds = the rounds run (-1: read later) and *frame_list = the length of the
-// list of triangles it created (-1: not read).
-static bool bulk_frame_removal(galpha_ctx *c, MeshDev &m, int nsets, hipStream_t st, int *ear_rounds,
-                               long long *frame_list)
+// Frame removal: drops every triangle with a frame vertex and fills what they covered with the
+// Delaunay triangles of the real points (see mesh.hip).  Returns the counters after it.
+static Snap remove_frame(galpha_ctx *c, MeshDev &m, hipStream_t st)
 {
-    *frame_list = -1;
-    int V = m.V, n = m.n;
-    int *outdeg = m.decide, *cover = m.deg, *bidx = c->fill.as<int>(), *blist = c->mlist.as<int>();
-    c->badset.ensure(4 * (size_t)nsets + 16);
-    int *badset = c->badset.as<int>(), *hcnt = c->hullCnt.as<int>(), *hstart = c->hullStart.as<int>();
+    // buffers that are free after the flips, for B <= n boundary vertices: at most 3 B edges (the
+    // table takes 6 B entries of 16 bytes or the whole fan buffer, 4.5 V and more)
+    HullDev h{};
+    h.ftri = m.modA;
+    h.mark = m.decide;
+    h.bidx = c->off.as<int>();
+    h.blist = c->mlist.as<int>();
+    h.bpos = c->scratch.as<double2>();
+    h.bbox = (HullBox *)(h.bpos + m.n);
+    h.table = c->fan.as<unsigned long long>();
+    h.list = (int2 *)m.cand;
+    h.next = (int *)m.remap;
+    h.pool = m.modB;
+    h.share = m.dellist;
+    h.room = (int)std::min<size_t>({c->fan.bytes / 16, c->remap.bytes / 8, (size_t)1 << 30});
     {
         IntFills f;
-        f.add(m.hnext, (size_t)V, -1);
-        f.add(outdeg, (size_t)V, 0);
-        f.add(cover, (size_t)V, 0);
-        f.add(bidx, (size_t)V, -1);
-        f.add(hcnt, (size_t)nsets, 0);
-        f.add(badset, (size_t)nsets, 0);
-        f.add(hstart, (size_t)nsets, 0x7fffffff);
-        f.add(c->counters.as<int>() + C_BND, 1, 0);
+        f.add(h.mark, (size_t)m.n + 1, 0);
+        f.add(h.share, HULL_SHARES * HULL_SHARE_INTS, 0);
+        f.add(c->counters.as<int>() + C_FTRI, 3, 0);
         launch_fill_multi(f, st);
     }
-    launch_bnd_detect(m, outdeg, cover, hcnt, hstart, badset, blist, bidx, st);
-    std::vector<int> rd(2 * (size_t)nsets + 1);
-    ctx_read_segments(c, {{badset, nsets}, {hcnt, nsets}, {c->counters.as<int>() + C_BND, 1}}, rd.data());
-    std::vector<int> bad(rd.begin(), rd.begin() + nsets), cnt(rd.begin() + nsets, rd.begin() + 2 * nsets);
-    int B = rd[2 * (size_t)nsets];
-    long long tot = 0;
-    int maxh = 0;
-    std::vector<int> off(nsets);
-    for (int s = 0; s < nsets; s++) {
-        // a set needs a cycle of at least 3 vertices; very long cycles make the ear test's
-        // per-candidate scan too long, so those sets keep the round-by-round removal
-        if (bad[s] || cnt[s] < 3 || cnt[s] > 65536) return false;
-        off[s] = (int)tot;
-        tot += cnt[s];
-        maxh = std::max(maxh, cnt[s]);
-    }
-    if (tot != B) return false;
-    (void)n;
-    // cycle arrays, the cycle's positions, 5 doubles of grid parameters per set, then two arrays of
-    // claim keys
-    c->bnd.ensure(4 * (size_t)((11 * (size_t)B + 3) & ~(size_t)3) + 32 * (size_t)B + 40 * (size_t)nsets + 64);
-    HIPCHK(hipMemcpyAsync(c->hullOff.p, off.data(), 4 * (size_t)nsets, hipMemcpyHostToDevice, st));
-    int rounds = 1;
-    while ((1 << rounds) < maxh) rounds++;
-    rounds += 1;
-    launch_bnd_rank(m, B, rounds, blist, bidx, hstart, hcnt, c->hullOff.as<int>(), badset, c->bnd.as<int>(), st);
-    ctx_read_segments(c, {{badset, nsets}}, rd.data());
-    for (int s = 0; s < nsets; s++)
-        if (rd[s]) return false;
-    // from here on the mesh changes
-    launch_kill_frame(m, st);
-    int *bnd = c->bnd.as<int>(), *hoff = c->hullOff.as<int>();
-    if (nsets >= 32) {
-        // many sets: every set's rounds in one workgroup, one launch (the most rounds a set ran is
-        // read with the next snapshot)
-        launch_reset_counters(c->counters.as<int>(), C_EAR, -1, -1, -1, st);
-        launch_ear_sets(m, B, bnd, hcnt, hoff, nsets, c->modF.as<int>(), C_FRAME_LIST, c->op++, st);
-        *ear_rounds = -1;
-        return true;
-    }
-    // few sets: grid-wide rounds, eight per host read (a round after one without candidates
-    // returns at once).  Sets of 256K points and more take 20-24 rounds (1M uniform points,
-    // the 2M lattice + cluster set), so their first read comes after sixteen.
-    launch_ear_grid(m, B, bnd, hcnt, hoff, nsets, st);   // also zeroes counters[C_EAR]
-    int round = 0, per_read = m.n >= (1 << 18) ? 16 : 8;
-    for (;; round += per_read, per_read = 8) {
-        if (round > 200000) throw GalphaError("hull convexification did not finish");
-        launch_ear_rounds(m, B, bnd, hcnt, hoff, nsets, round, per_read, c->modF.as<int>(), C_FRAME_LIST, c->op++,
-                          st);
-        int cv[C_EAR_PREV - C_FRAME_LIST + 1];
-        ctx_counters_read(c, cv, C_FRAME_LIST, C_EAR_PREV - C_FRAME_LIST + 1);
-        if (cv[(((round + per_read - 1) & 1) ? C_EAR_PREV : C_EAR) - C_FRAME_LIST] == 0) {
-            *frame_list = cv[0];
-            break;
-        }
-    }
-    *ear_rounds = round + per_read;
-    return true;
+    launch_hull(m, h, c->op++, c->scanTmp.p, st);
+    return ctx_snapshot(c);
 }
 
 // Real points are renumbered in spatial order (set, then 16 x 16-pixel cells in Morton order;
@@ -871,12 +813,8 @@ static int run_batch(galpha_ctx *c, const double *d_xy, const BatchPlan &plan)
     c->lt.ensure(4 * (size_t)n);
     size_t scap = std::max((size_t)4 * 8192 + 64, (size_t)(8 * V) + 4096);
     c->scratch.ensure(4 * scap);
-    c->hnext.ensure(4 * (size_t)V);
-    c->hedge.ensure(4 * (size_t)V);
     c->dellist.ensure(4 * (size_t)cap);
     c->lmark.ensure(4 * (size_t)cap);
-    c->ffan.ensure(8 * (size_t)(V - n) + 16);
-    c->modF.ensure(4 * (size_t)cap);
     // Slot tags (stamp, claim keys, list marks) carry the context's op number, and the removal
     // rounds (deletion, frame) tag their per-vertex priority maxima with a round number; both
     // only grow, across runs too, so values left by earlier runs never match or beat later ones.
@@ -926,10 +864,7 @@ static int run_batch(galpha_ctx *c, const double *d_xy, const BatchPlan &plan)
     m.decide = c->decide.as<int>();
     m.dellist = c->dellist.as<int>();
     m.lt = c->lt.as<int>();
-    m.hnext = c->hnext.as<int>();
-    m.hedge = c->hedge.as<int>();
     m.lmark = c->lmark.as<int>();
-    m.ffan = c->ffan.as<int>();
 
     // ---- reconstruction + adjacency
     launch_recon(c->vor.as<int>(), c->pix.as<int>(), bd, m, c->tileCnt.as<int>(), c->tileOff.as<int>(),
@@ -1142,33 +1077,12 @@ static int run_batch(galpha_ctx *c, const double *d_xy, const BatchPlan &plan)
     ev_mark(c, 5, st);
     const Snap after_main = last;   // per-stage statistics: shifting, insertion and these flips
 
-    // ---- frame removal + hull convexification
-    // Triangles created by frame removal and convexification go to one list (each slot once);
-    // the mesh was Delaunay before, so only their edges can need flips afterwards.
-    m.list_op = c->op++;
-    launch_reset_counters(c->counters.as<int>(), C_FRAME_LIST, -1, -1, -1, st);
-    long long frame_list = -1;   // triangles listed by frame removal, when known
-    if (bulk_frame_removal(c, m, nsets, st, &S.earRounds, &frame_list)) {
-        S.frameBulk = 1;
-    } else {
-    for (int r = 0;; r += 2) {
-        if (r > 100000) throw GalphaError("frame removal did not finish");
-        for (int k = 0; k < 2; k++) {
-            launch_reset_counters(c->counters.as<int>(), C_SCR, -1, -1, -1, st);
-            launch_frame_round(m, c->mx.as<unsigned int>(), next_prio_round(), c->modF.as<int>(), C_FRAME_LIST,
-                               c->op++, st);
-        }
-        int left = (V - n) - ctx_stat(c, C_FRAME_DONE);
-        if (left <= 0) break;
-    }
-    launch_convexify(m, c->modF.as<int>(), C_FRAME_LIST, c->op++, c->hullCnt.as<int>(), c->hullOff.as<int>(),
-                     c->hullStart.as<int>(), c->scanTmp.p, st);
-    }
+    // ---- frame removal
+    last = remove_frame(c, m, st);
+    S.frameBulk = 1;
+    S.earRounds = 1;
     ev_mark(c, 6, st);
-    flip_until_done(c->modF.as<int>(), C_FRAME_LIST, m.modB, C_MODN2, m.list_op, frame_list);
-    ev_mark(c, 7, st);
-    const Snap after_frame = last;   // per-stage statistics: frame removal and the final flips
-    if (S.frameBulk && S.earRounds < 0) S.earRounds = after_frame.v[C_EAR];
+    const Snap after_frame = last;   // per-stage statistics: frame removal
     if (last.status()) throw GalphaError("device pipeline error (status " + std::to_string(last.status()) + ")");
 
     // ---- constraint edges (single-set runs): cavity insertion rounds, then constrained flips
@@ -1280,8 +1194,6 @@ static int run_batch(galpha_ctx *c, const double *d_xy, const BatchPlan &plan)
     c->last_F = F;
     S.nTris = F;
     S.flips = fin.stat(C_FLIPS_TOTAL);
-    S.frameSeen = fin.stat(C_FRAME_SEEN);
-    S.frameChain = fin.stat(C_FRAME_CHAIN);
     S.flipListed = fin.v[C_FLIP_LISTED];
     S.flipTailListed = fin.v[C_TAIL_LISTED];
     S.incircleTests = fin.stat(C_TESTS_INCIRCLE);
@@ -1292,7 +1204,7 @@ static int run_batch(galpha_ctx *c, const double *d_xy, const BatchPlan &plan)
     S.ms_shift = ev_ms(c, 2, 3);
     S.ms_missing = ev_ms(c, 3, 4);
     S.ms_boundary = ev_ms(c, 5, 6);
-    S.ms_flip = ev_ms(c, 4, 5) + ev_ms(c, 6, 7);
+    S.ms_flip = ev_ms(c, 4, 5);
     {
         const Snap *cut[4] = {nullptr, &after_main, &after_frame, &fin};
         for (int k = 0; k < 3; k++) {
@@ -1307,7 +1219,7 @@ static int run_batch(galpha_ctx *c, const double *d_xy, const BatchPlan &plan)
             S.stageOrientExact[k] = d(true, C_EXACT_ORIENT);
         }
     }
-    S.ms_constraints = ev_ms(c, 7, 9);
+    S.ms_constraints = ev_ms(c, 6, 9);
     S.ms_canon = ev_ms(c, 9, 8);
     S.constraintRounds = c->cons_rounds;
     S.ms_total = ev_ms(c, 0, 8);
@@ -1458,11 +1370,11 @@ static void release_all(galpha_ctx *c)
     DevBuf *bufs[] = {&c->smap, &c->g, &c->S, &c->cnt, &c->E, &c->ecnt, &c->vor, &c->bad, &c->fpix, &c->tv,
                       &c->tn, &c->remap, &c->stamp, &c->claim, &c->modA, &c->modB, &c->cand, &c->pos, &c->vt,
                       &c->vstate, &c->pix, &c->deg, &c->off, &c->fill, &c->fan, &c->moved, &c->decide, &c->mx,
-                      &c->mlist, &c->loc, &c->lt, &c->scratch, &c->hnext, &c->hedge, &c->keys, &c->keys2,
+                      &c->mlist, &c->loc, &c->lt, &c->scratch, &c->keys, &c->keys2,
                       &c->vals, &c->vals2, &c->rot, &c->newid, &c->out9, &c->counters, &c->status, &c->xy,
                       &c->scanTmp, &c->sortTmp, &c->tileCnt, &c->tileOff, &c->dellist, &c->dbg,
-                      &c->setsD, &c->bmD, &c->vset, &c->hullCnt, &c->hullOff, &c->hullStart, &c->setFirst,
-                      &c->offsD, &c->bboxTmp, &c->lmark, &c->ffan, &c->modF, &c->badset, &c->bnd, &c->plo,
+                      &c->setsD, &c->bmD, &c->vset, &c->setFirst,
+                      &c->offsD, &c->bboxTmp, &c->lmark, &c->plo,
                       &c->perm, &c->xys, &c->pcell, &c->ccount, &c->ccursor, &c->cls,
                       &c->kin, &c->kv, &c->kinv, &c->kdone, &c->kcnt, &c->krs, &c->kroff, &c->kwork, &c->khash, &c->rdbuf};
     for (DevBuf *b : bufs) b->release();
@@ -1477,11 +1389,11 @@ size_t galpha_ctx_device_bytes(galpha_ctx *c)
     DevBuf *bufs[] = {&c->smap, &c->g, &c->S, &c->cnt, &c->E, &c->ecnt, &c->vor, &c->bad, &c->fpix, &c->tv,
                       &c->tn, &c->remap, &c->stamp, &c->claim, &c->modA, &c->modB, &c->cand, &c->pos, &c->vt,
                       &c->vstate, &c->pix, &c->deg, &c->off, &c->fill, &c->fan, &c->moved, &c->decide, &c->mx,
-                      &c->mlist, &c->loc, &c->lt, &c->scratch, &c->hnext, &c->hedge, &c->keys, &c->keys2,
+                      &c->mlist, &c->loc, &c->lt, &c->scratch, &c->keys, &c->keys2,
                       &c->vals, &c->vals2, &c->rot, &c->newid, &c->out9, &c->counters, &c->status, &c->xy,
                       &c->scanTmp, &c->sortTmp, &c->tileCnt, &c->tileOff, &c->dellist, &c->dbg,
-                      &c->setsD, &c->bmD, &c->vset, &c->hullCnt, &c->hullOff, &c->hullStart, &c->setFirst,
-                      &c->offsD, &c->bboxTmp, &c->lmark, &c->ffan, &c->modF, &c->badset, &c->bnd, &c->plo,
+                      &c->setsD, &c->bmD, &c->vset, &c->setFirst,
+                      &c->offsD, &c->bboxTmp, &c->lmark, &c->plo,
                       &c->perm, &c->xys, &c->pcell, &c->ccount, &c->ccursor, &c->cls,
                       &c->kin, &c->kv, &c->kinv, &c->kdone, &c->kcnt, &c->krs, &c->kroff, &c->kwork, &c->khash, &c->rdbuf};
     size_t t = 0;
@@ -1513,8 +1425,9 @@ __attribute__((visibility("hidden"))) galpha_ctx *galpha_noalloc_ctx_new(int dev
 }
 
 // Upper bound of the bytes a single-set DT run of n points on a T x T texture carves: every
-// buffer the run ensures, at its largest size (slots at the capacity 3 V + 8192, boundary cycle
-// at V vertices), the scan and sort temporaries as rocPRIM reports them, and 256-byte rounding.
+// buffer the run ensures, at its largest size (slots at the capacity 3 V + 8192), the scan and sort
+// temporaries as rocPRIM reports them, and 256-byte rounding.  About 100 V bytes of it are room that
+// no buffer takes: the sizes that fit the scratch are part of the interface.
 __attribute__((visibility("hidden"))) size_t galpha_noalloc_need(int n, int T)
 {
     if (n < 3) return 4096;

@@ -102,15 +102,34 @@ struct MeshDev {
     int *decide;         // [V] greedy shifting decisions
     int *dellist;        // [cap] triangles created by a deletion round
     int *lt;             // [n] located type of every missing site
-    int *hnext, *hedge;  // [V] hull successor and hull edge of every hull vertex
     int *lmark;          // [cap] operation that last put the slot in a flip list (one entry per pass)
-    int *ffan;           // [2 * (V - n)] per frame vertex: first fan triangle (enc) and fan length
-    int list_op;         // lmark tag of the list that frame removal and convexification fill
     // constraint edges (set of (min << 32 | max) + 1 keys, open addressing, 0 = empty); NULL when
     // the run has no constraints.  k_flip_test never flips an edge in this set.
     const unsigned long long *chash;
     int chmask;
 };
+
+// Frame removal (see mesh.hip): the boundary vertices (real vertices of frame triangles, B of them)
+// and the table of the edges to fill from.  All in buffers that are free after the flips.
+struct HullBox {
+    double lx, ly, hx, hy;
+};
+struct HullDev {
+    int *ftri;                  // frame triangles (counters[C_FTRI])
+    int *mark;                  // [n + 1] 1 for a boundary vertex, 3 when it has an edge to another
+    int *bidx;                  // [n + 1] number of boundary vertices before v (bidx[n] = B)
+    int *blist;                 // [B] boundary vertices in vertex order
+    double2 *bpos;              // [B] their positions
+    HullBox *bbox;              // [B / 64 + 1] boxes of 64 consecutive ones
+    unsigned long long *table;  // [2 H] keys of the edges (0: free entry), then what is left of them
+    int2 *list;                 // first demands and the slots of their frame triangles (counters[C_HULL])
+    int *pool;                  // slots of the other frame triangles (counters[C_HULL_POOL])
+    int *share;                 // HULL_SHARES counters: slots taken from each share of the pool
+    int *next;                  // [2 H] links of the waves' stacks
+    int room;                   // most table entries
+};
+#define HULL_SHARES 32
+#define HULL_SHARE_INTS 32      // ints between the counters
 
 // vertex states
 #define VS_IN_MESH 1       // in the mesh, position final
@@ -142,16 +161,12 @@ struct MeshDev {
 #define C_ISLAND_SITES 19
 #define C_HSTART 20
 #define C_FLIPS_TOTAL 21
-#define C_FRAME_SEEN 22       // frame vertices examined by k_frame_remove (all launches)
-#define C_FRAME_CHAIN 23      // sum of the fan lengths of removed frame vertices
 #define C_FLIP_LISTED 24      // triangles listed for k_flip_test (all launches)
-#define C_FRAME_LIST 25       // triangles created by frame removal and convexification
-#define C_BND 26              // boundary vertices of the real region (bulk frame removal)
-#define C_EAR 27              // ear candidates of the current round
+#define C_FTRI 25             // frame triangles listed by k_hull_scan
+#define C_HULL 26             // first demands of frame removal
+#define C_HULL_POOL 27        // other frame triangles (free slots)
 #define C_MOVED 28            // vertices moved by greedy shifting rounds (statistic)
-#define C_FRAME_DONE 29       // frame vertices removed round by round (statistic)
 #define C_PLIST 30            // entries of the pending-vertex list (MeshDev::plist)
-#define C_EAR_PREV 31         // ear candidates of the previous round
 #define C_STATUS 32           // device status word (GA_ERR_* bits); MeshDev::status points here
 #define C_CONS_PEND 33        // constraints still to insert (the current insertion round's walk)
 #define C_CONS_MOD 34         // slots rewritten by the current insertion round
@@ -172,8 +187,7 @@ struct MeshDev {
 #endif
 #define C_FOLD 64             // counters[C_FOLD + k] = stripe sum of statistic k after a fold
 // Counters C_PEND, C_EXACT_*, C_INSERTED, C_DUPS, C_TESTS_INCIRCLE, C_RECON_TRIS, C_DELETED,
-// C_FLIPS_TOTAL, C_FRAME_SEEN, C_FRAME_CHAIN, C_MOVED and C_FRAME_DONE are striped statistics
-// (MeshDev::stats); the others are single words.
+// C_FLIPS_TOTAL and C_MOVED are striped statistics (MeshDev::stats); the others are single words.
 #define C_DBG 48          // 48..63: first failure dump
 #define C_NCOUNTERS 64
 
@@ -265,25 +279,8 @@ void launch_cons_setup(MeshDev &m, const int2 *cin, int nc, int *inv, int2 *cv, 
 void launch_cons_count(MeshDev &m, const int2 *cv, int nc, int *done, int *cnt, int *rsize, hipStream_t st);
 void launch_cons_insert(MeshDev &m, const int2 *cv, int nc, int *done, const int *cnt, const int *roff,
                         int *work, int *modlist, int op, hipStream_t st);
-void launch_frame_round(MeshDev &m, unsigned int *mx, int round, int *list_out, int cnt_out_slot, int op,
-                        hipStream_t st);
-// bulk frame removal (see mesh.hip); bnd = 11 * B ints (rounded up to 4) + B double2 cycle positions of
-// work space once B is known
-void launch_bnd_detect(MeshDev &m, int *outdeg, int *cover, int *hull_cnt, int *hull_start, int *badset,
-                       int *blist, int *bidx, hipStream_t st);
-void launch_bnd_rank(MeshDev &m, int B, int rounds, const int *blist, const int *bidx, const int *hull_start,
-                     const int *hull_cnt, const int *hull_off, int *badset, int *bnd, hipStream_t st);
-void launch_kill_frame(MeshDev &m, hipStream_t st);
-// bulk frame removal's ear rounds: the per-set grids, then rounds [r0, r0 + k) as grid-wide kernels
-// (counters[C_EAR] / [C_EAR_PREV] count the candidates of even / odd rounds)
-void launch_ear_grid(MeshDev &m, int B, int *bnd, const int *hull_cnt, const int *hull_off, int nsets, hipStream_t st);
-void launch_ear_rounds(MeshDev &m, int B, int *bnd, const int *hull_cnt, const int *hull_off, int nsets, int r0,
-                       int k, int *list_out, int cnt_out_slot, int op, hipStream_t st);
-// every set's ear rounds in one workgroup per set (bulk frame removal); counters[C_EAR] = most rounds
-void launch_ear_sets(MeshDev &m, int B, int *bnd, const int *hull_cnt, const int *hull_off, int nsets,
-                     int *list_out, int cnt_out_slot, int op, hipStream_t st);
-void launch_convexify(MeshDev &m, int *list_out, int cnt_out_slot, int op, int *hull_cnt, int *hull_off,
-                      int *hull_start, void *scan_tmp, hipStream_t st);
+// frame removal (see mesh.hip); mark, share and the counters C_FTRI .. C_HULL_POOL zero on entry
+void launch_hull(MeshDev &m, const HullDev &h, int op, void *scan_tmp, hipStream_t st);
 // canonical order: key (v0 << B) | v1 of input indices below 2^B, sorted on its low 2B bits
 void launch_canon_keys(MeshDev &m, unsigned long long *keys, int *vals, int *rot, int B, hipStream_t st);
 // canonical keys of 32 bits up to input indices below 2^CANON_KEY32_BITS (ties within 256 triangles)

@@ -15,8 +15,8 @@
 //   flipping            Cuda/cudaFlipping.cu:227-685: Lawson flips with an FP64 filter and an
 //                       exact integer fallback on the device (no CPU pass), lifted-perturbation
 //                       tie-break for co-circular quadruples.
-//   boundary removal    Cuda/cudaBoundary.cu:106-608: distance-2 independent frame-vertex
-//                       deletions with a ccw-stack fill, then a hull convexification pass.
+//   boundary removal    Cuda/cudaBoundary.cu:106-608: the frame triangles are dropped at once and
+//                       what they covered is filled by parallel gift wrapping.
 // Links after a modification are repaired by one generic pass: a modified triangle keeps the
 // old external link of each outer edge (stored as -(e+2)); if that neighbour was modified in
 // the same operation the new location is read from its remap[] entry, otherwise the link is
@@ -1281,258 +1281,6 @@ void launch_flip_pass(MeshDev &m, const int *list_in, int cnt_in_slot, int *list
     GA_LAUNCH(k_relink, dim3(grid), dim3(256), 0, st, m, (const int *)list_out, cnt_out_slot, op, C_CAND);
 }
 
-// ---- frame removal ---------------------------------------------------------------------------
-// fan of a hull vertex f: first triangle whose cw side (edge (f, l0)) is a hull edge
-GA_INLINE int fan_first(const MeshDev &m, int f, int *slot)
-{
-    int t = m.vt[f], i = slot_of(m.tv[t], f), guard = 0;
-    while (true) {
-        int e = ic(m.tn[t], m1(i));
-        if (e < 0) break;
-        t = enc_t(e);
-        i = slot_of(m.tv[t], f);
-        if (++guard > 1000000) { atomicOr(m.status, GA_ERR_WALK); break; }
-    }
-    *slot = i;
-    return t;
-}
-
-// Every remaining frame vertex marks its closed neighbourhood with its priority and records its
-// first fan triangle and fan length in ffan[] for k_frame_remove of the same round.
-__global__ void k_frame_prio(MeshDev m, unsigned long long *mx, int round)
-{
-    int nf = m.V - m.n;
-    GRID_STRIDE(k, nf) {
-        int f = m.n + k;
-        if (m.vstate[f] != VS_IN_MESH) continue;
-        unsigned long long p = prio64(f, round);
-        atomicMax(&mx[f], p);
-        int i, t = fan_first(m, f, &i);
-        m.ffan[2 * k] = enc(t, i);
-        atomicMax(&mx[ic(m.tv[t], p1(i))], p);
-        int kf = 0;
-        for (int guard = 0; guard < 1000000; guard++) {
-            kf++;
-            atomicMax(&mx[ic(m.tv[t], m1(i))], p);
-            int e = ic(m.tn[t], p1(i));
-            if (e < 0) break;
-            t = enc_t(e);
-            i = slot_of(m.tv[t], f);
-        }
-        m.ffan[2 * k + 1] = kf;
-    }
-}
-
-// Read-only: a frame vertex wins when every vertex of its closed neighbourhood holds its
-// priority; ffan[2k + 1] keeps the fan length of a winner and -1 otherwise.
-__global__ void k_frame_decide(MeshDev m, const unsigned long long *mx, int round)
-{
-    int nf = m.V - m.n;
-    GRID_STRIDE(k, nf) {
-        int f = m.n + k;
-        if (m.vstate[f] != VS_IN_MESH) continue;
-        unsigned long long p = prio64(f, round);
-        int kf = m.ffan[2 * k + 1];
-        bool win = mx[f] == p;
-        int t = enc_t(m.ffan[2 * k]), i = enc_j(m.ffan[2 * k]);
-        if (win) win = mx[ic(m.tv[t], p1(i))] == p;
-        for (int q = 0; q < kf && win; q++) {
-            int4 tt = m.tv[t];
-            if (mx[ic(tt, m1(i))] != p) win = false;
-            else if (q + 1 < kf) {
-                int e = ic(m.tn[t], p1(i));
-                if (e < 0) { win = false; atomicOr(m.status, GA_ERR_WALK); break; }
-                t = enc_t(e);
-                i = slot_of(m.tv[t], f);
-            }
-        }
-        if (!win) m.ffan[2 * k + 1] = -1;
-    }
-}
-
-__global__ void k_frame_remove(MeshDev m, const unsigned long long *mx, int round, int op, int *list_out,
-                               int cnt_out_slot)
-{
-    int nf = m.V - m.n;
-    int seen = 0, chainsum = 0;
-    for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < ((nf + 63) & ~63); k += gridDim.x * blockDim.x) {
-        // (full-wave loop so the work counters can be summed per wave at the end)
-        if (k >= nf) continue;
-        int f = m.n + k;
-        if (m.vstate[f] != VS_IN_MESH) continue;
-        seen++;
-        // winner decided by k_frame_decide this round; its fan is untouched by other winners
-        // (distance-2 independence), so the chain is read without races
-        int kf = m.ffan[2 * k + 1];
-        if (kf < 0) continue;
-        int t0 = enc_t(m.ffan[2 * k]), i0 = enc_j(m.ffan[2 * k]);
-        // chain l_0..l_kf, outer links o_0..o_{kf-1}, fan slots
-        int need = 4 * (kf + 1);
-        int base = atomicAdd(&m.counters[C_SCR], need);
-        if ((size_t)(base + need) > m.scratch_cap) { atomicOr(m.status, GA_ERR_SCRATCH); continue; }
-        int *chain = m.scratch + base, *olink = chain + (kf + 1), *slots = olink + (kf + 1), *st = slots + (kf + 1);
-        int t = t0, i = i0;
-        chain[0] = ic(m.tv[t0], p1(i0));
-        for (int q = 0; q < kf; q++) {
-            int4 tt = m.tv[t], nn = m.tn[t];
-            chain[q + 1] = ic(tt, m1(i));
-            olink[q] = ic(nn, i);
-            slots[q] = t;
-            int e = ic(nn, p1(i));
-            if (q + 1 < kf) {
-                if (e < 0) { atomicOr(m.status, GA_ERR_WALK); break; }
-                t = enc_t(e);
-                i = slot_of(m.tv[t], f);
-            }
-        }
-        // chain vertices keep an incident triangle: the outer one
-        for (int q = 0; q <= kf; q++) {
-            int o = q < kf ? olink[q] : -1;
-            if (o < 0 && q > 0) o = olink[q - 1];
-            if (o >= 0) m.vt[chain[q]] = enc_t(o);
-        }
-        // ccw-stack fill: stack st[], slink = olink reused as stack-edge links
-        int *slink = olink;   // slink[s] = outer side of stack edge (st[s], st[s+1]); olink[q] read before overwrite
-        int top = 0, used = 0;
-        st[0] = chain[0];
-        for (int q = 1; q <= kf; q++) {
-            int c = chain[q];
-            int cur = olink[q - 1];
-            while (top >= 1 && orient_dev(m, m.pos[st[top - 1]], m.pos[st[top]], m.pos[c]) > 0) {
-                int A = st[top - 1], B = st[top];
-                int T = slots[used++];
-                m.tv[T] = make_int4(A, B, c, 0);
-                m.tn[T] = make_int4(-1, -1, -1, 0);
-                bond(m, T, 2, slink[top - 1]);   // edge (A, B)
-                bond(m, T, 0, cur);              // edge (B, c)
-                m.vt[A] = T; m.vt[B] = T; m.vt[c] = T;
-                m.stamp[T] = op;
-                if (atomicExch(&m.lmark[T], m.list_op) != m.list_op)
-                    list_out[atomicAdd(&m.counters[cnt_out_slot], 1)] = T;
-                cur = enc(T, 1);                 // edge (c, A) seen from T
-                top--;
-            }
-            slink[top] = cur;
-            st[++top] = c;
-        }
-        // remaining stack edges become hull edges
-        for (int s = 0; s < top; s++) {
-            int X = slink[s];
-            if (X >= 0) set_link(m, enc_t(X), enc_j(X), -1);
-        }
-        for (int q = used; q < kf; q++) m.tv[slots[q]] = make_int4(GA_DEAD, GA_DEAD, GA_DEAD, 0);
-        m.vstate[f] = VS_REMOVED;
-        m.vt[f] = -1;
-        stat_inc(m.stats, C_FRAME_DONE, true);
-        chainsum += kf;
-    }
-    stat_add_full(m.stats, C_FRAME_SEEN, seen);
-    stat_add_full(m.stats, C_FRAME_CHAIN, chainsum);
-}
-
-void launch_frame_round(MeshDev &m, unsigned int *mxraw, int round, int *list_out, int cnt_out_slot, int op,
-                        hipStream_t st)
-{
-    unsigned long long *mx = (unsigned long long *)mxraw;
-    GA_LAUNCH(k_frame_prio, dim3(FIXED_GRID), dim3(256), 0, st, m, mx, round);
-    GA_LAUNCH(k_frame_decide, dim3(FIXED_GRID), dim3(256), 0, st, m, (const unsigned long long *)mx, round);
-    GA_LAUNCH(k_frame_remove, dim3(FIXED_GRID), dim3(256), 0, st, m, (const unsigned long long *)mx, round, op,
-                       list_out, cnt_out_slot);
-}
-
-// ---- hull convexification (one workgroup per set) --------------------------------------------
-// Hull cycle of set `blockIdx.x` in the scratch arena at 4 * hull_off[set]: verts[], owner[] (enc
-// of the triangle side of hull edge (verts[k] -> verts[k+1])), nxt[], prv[]; hull_cnt[set] is the
-// number of hull edges, so the cycle fits exactly.
-__global__ __launch_bounds__(256) void k_convexify(MeshDev m, const int *hnext, const int *hedge,
-                                                   const int *hull_cnt, const int *hull_off,
-                                                   const int *hull_start, int *list_out, int cnt_out_slot,
-                                                   int op)
-{
-    __shared__ int s_flag, s_start, s_h, s_cur, s_block;
-    int set = blockIdx.x;
-    int hcap = hull_cnt[set];
-    int *verts = m.scratch + 4 * (size_t)hull_off[set], *owner = verts + hcap, *nxt = owner + hcap,
-        *prv = nxt + hcap;
-    if (threadIdx.x == 0) {
-        int start = hull_start[set];
-        if (start == 0x7fffffff) start = -1;
-        int h = 0, v = start;
-        if (start >= 0) {
-            do {
-                if (h >= hcap) { atomicOr(m.status, GA_ERR_SCRATCH); h = -1; break; }
-                verts[h] = v;
-                owner[h] = hedge[v];
-                h++;
-                v = hnext[v];
-            } while (v != start && v >= 0);
-        }
-        if (h > 0) for (int k = 0; k < h; k++) { nxt[k] = (k + 1) % h; prv[k] = (k + h - 1) % h; }
-        s_h = h;
-        s_start = 0;
-    }
-    __syncthreads();
-    int h = s_h;
-    if (h < 3) return;
-    for (int pass = 0; pass < h + 2; pass++) {
-        if (threadIdx.x == 0) s_flag = 0;
-        __syncthreads();
-        int cur = s_start;
-        // one sweep around the cycle
-        for (int it = 0; it < 4 * h + 4; it++) {
-            __syncthreads();
-            if (threadIdx.x == 0) {
-                s_cur = cur;
-                s_block = 0;
-            }
-            __syncthreads();
-            int kc = s_cur, kp = prv[kc], kn = nxt[kc];
-            double2 Pp = m.pos[verts[kp]], C = m.pos[verts[kc]], N = m.pos[verts[kn]];
-            bool reflex = orient_dev(m, Pp, C, N) < 0;
-            if (reflex) {
-                // blocked if any other live hull vertex lies in the closed notch (P, N, C) minus P, N, C
-                for (int q = threadIdx.x; q < h; q += blockDim.x) {
-                    if (q == kc || q == kp || q == kn || nxt[q] < 0) continue;
-                    double2 Q = m.pos[verts[q]];
-                    if (orient_dev(m, Pp, N, Q) >= 0 && orient_dev(m, N, C, Q) >= 0 && orient_dev(m, C, Pp, Q) >= 0)
-                        s_block = 1;
-                }
-            }
-            __syncthreads();
-            if (threadIdx.x == 0) {
-                if (reflex && !s_block) {
-                    int T = atomicAdd(m.ntri, 1);
-                    if (T >= m.cap) { atomicOr(m.status, GA_ERR_CAPACITY); }
-                    else {
-                        int vp = verts[kp], vc = verts[kc], vn = verts[kn];
-                        m.tv[T] = make_int4(vp, vn, vc, 0);
-                        m.tn[T] = make_int4(-1, -1, -1, 0);
-                        bond(m, T, 0, owner[kc]);   // edge (vn, vc) = reverse of hull edge (vc -> vn)
-                        bond(m, T, 1, owner[kp]);   // edge (vc, vp) = reverse of hull edge (vp -> vc)
-                        m.stamp[T] = op;
-                        if (atomicExch(&m.lmark[T], m.list_op) != m.list_op)
-                            list_out[atomicAdd(&m.counters[cnt_out_slot], 1)] = T;
-                        owner[kp] = enc(T, 2);       // new hull edge (vp -> vn)
-                        nxt[kp] = kn; prv[kn] = kp;
-                        nxt[kc] = -1;
-                        if (s_start == kc) s_start = kp;
-                        s_flag = 1;
-                        cur = kp;
-                    }
-                } else {
-                    cur = kn;
-                }
-                s_cur = cur;
-            }
-            __syncthreads();
-            cur = s_cur;
-            if (cur == s_start && it > 0) break;
-        }
-        __syncthreads();
-        if (!s_flag) break;
-    }
-}
-
 // zero up to four counter slots in one launch (negative slot: unused)
 __global__ void k_reset_counters(int *c, int a, int b, int d, int e)
 {
@@ -1587,851 +1335,419 @@ void launch_counters_to_host(int *counters, int slot, int n, int fold, int *host
     GA_LAUNCH(k_counters_to_host, dim3(1), dim3(256), 0, st, counters, slot, n, fold, host);
 }
 
-__global__ void k_hull_edges(MeshDev m, int *hnext, int *hedge, int *hull_cnt, int *hull_start)
-{
-    int n = ntri_used(m);
-    GRID_STRIDE(t, n) {
-        int4 v = m.tv[t];
-        if (v.x == GA_DEAD) continue;
-        int4 nb = m.tn[t];
-        for (int i = 0; i < 3; i++)
-            if (ic(nb, i) < 0) {
-                int a = ic(v, p1(i)), b = ic(v, m1(i));
-                hnext[a] = b;
-                hedge[a] = enc(t, i);
-                int s = m.vset[a];
-                atomicMin(&hull_start[s], a);
-                atomicAdd(&hull_cnt[s], 1);
-            }
-    }
-}
-
-void launch_convexify(MeshDev &m, int *list_out, int cnt_out_slot, int op, int *hull_cnt, int *hull_off,
-                      int *hull_start, void *scan_tmp, hipStream_t st)
-{
-    IntFills f;
-    f.add(m.hnext, (size_t)m.V, -1);
-    f.add(hull_cnt, (size_t)m.nsets, 0);
-    f.add(hull_start, (size_t)m.nsets, 0x7fffffff);
-    launch_fill_multi(f, st);
-    GA_LAUNCH(k_hull_edges, dim3(FIXED_GRID), dim3(256), 0, st, m, m.hnext, m.hedge, hull_cnt, hull_start);
-    launch_exclusive_scan(hull_cnt, hull_off, m.nsets, scan_tmp, st);
-    GA_LAUNCH(k_convexify, dim3(m.nsets), dim3(256), 0, st, m, (const int *)m.hnext, (const int *)m.hedge,
-              (const int *)hull_cnt, (const int *)hull_off, (const int *)hull_start, list_out, cnt_out_slot, op);
-}
-
-// ---- bulk frame removal ------------------------------------------------------------------------
-// Every triangle of the current mesh whose vertices are all real is a triangle of the final
-// triangulation (its circumcircle holds no point at all).  When the region R of those triangles
-// has, in every set, a boundary that is one simple cycle through every meshed real point, all
-// frame triangles are dropped at once and R is made convex by parallel ear rounds on that cycle.
-// The checks below run before anything is modified; if one fails, the caller removes the frame
-// vertices round by round instead.
+// ---- frame removal -----------------------------------------------------------------------------
+// The mesh is the Delaunay triangulation of the real points and the frame.  Its triangles without
+// frame vertices belong to the triangulation of the real points (their circumcircles hold no
+// point); what the frame triangles cover has to be triangulated again without the frame.  Every
+// triangle there has its three vertices among the real vertices that touch a frame triangle (the
+// boundary vertices, B of them), so the triangle left of a directed edge p -> q is found on its own:
+// its apex is the boundary vertex left of the edge whose circle through p and q holds no other (the
+// minimum of a strict order, ties broken as everywhere).  That is parallel gift wrapping:
+//   demand   a directed edge whose left triangle is not known; at first the real edges of the
+//            frame triangles, later the far sides of new triangles;
+//   apex     one wave looks for it; none: a hull edge;
+//   create   one of the demands that found the same triangle claims it, links the sides whose
+//            other triangle is known, and its wave goes on with the others.
+// Most triangles have a side among the first demands, so the waves' chains are short whatever the
+// region's shape: pinches, dangling edges, several components and long straight sides need no
+// special case, and one launch does all sets.
+// The two demands of an undirected edge {u, v} share an entry e of an open-addressing table.  The
+// word own[e] holds, in its low half for u -> v (u < v) and its high half for v -> u, what is left
+// of that direction: bit 0 once it is a demand, above it 0 (unknown), 1 + 3 t + k for side k of triangle
+// t, or HULL_EDGE.  One atomic OR therefore records a side, lists the other direction and tells what
+// was known of it, and no fence orders anything: every link of a new triangle is written by
+// whichever of its two sides comes second (or by both, with one value).
+// Triangles and demands are those of a planar graph on B vertices: at most 3 B edges.
+// What bounds it is latency: the dependent reads of an apex and five device-scope atomics of a
+// triangle, 5 to 8 us a step.  The boundary stage, against cutting ears of the boundary cycle in
+// 16-32 rounds (which needed one simple cycle per set, and left flips to do; sets without one lost
+// their frame vertices in 18-58 rounds): 1M uniform points 0.57 -> 0.11 ms, 65,537 0.40 -> 0.08 ms,
+// 1,000 (no simple cycle) 0.87 -> 0.06 ms, a batch of 1,024 sets 11.5 -> 1.7 ms.
 GA_INLINE bool is_frame_tri(const MeshDev &m, int4 v) { return v.x >= m.n || v.y >= m.n || v.z >= m.n; }
-
-// boundary edges of R (a -> b with R on the left), their count and smallest tail per set; a vertex
-// with two outgoing boundary edges (a pinch) or a meshed real point in no R triangle marks its set
-// Each set's boundary-edge count and smallest boundary vertex are accumulated per thread (while
-// the set stays the same) and added once per wave when the wave's edges share one set: atomics
-// of every boundary edge on the set's two words would serialise.
-__global__ void k_bnd_edges(MeshDev m, int *outdeg, int *cover, int *hull_cnt, int *hull_start, int *badset)
+GA_INLINE int frame_vertices(const MeshDev &m, int4 v) { return (v.x >= m.n) + (v.y >= m.n) + (v.z >= m.n); }
+GA_INLINE int hull_b(const MeshDev &m, const HullDev &h) { return h.bidx[m.n]; }
+// entries of the table for B boundary vertices
+GA_INLINE int hull_table(const MeshDev &m, const HullDev &h)
 {
-    int n = ntri_used(m);
-    int cs = -1, cc = 0, cmin = 0x7fffffff;   // pending count and minimum of set cs
-    GRID_STRIDE(t, n) {
-        int4 v = m.tv[t];
-        if (v.x == GA_DEAD || is_frame_tri(m, v)) continue;
-        cover[v.x] = 1; cover[v.y] = 1; cover[v.z] = 1;
-        int4 nb = m.tn[t];
+    const long long want = 6ll * hull_b(m, h) + 64;
+    return (int)(want < h.room ? want : h.room);
+}
+typedef unsigned long long u64;
+#define HULL_LISTED 1u
+#define HULL_EDGE 0x7fffffffu
+GA_INLINE unsigned hull_value(int t, int k) { return 1u + 3u * (unsigned)t + (unsigned)k; }
+GA_INLINE unsigned hull_half(u64 w, int d) { return (unsigned)(w >> (32 * d)); }
+
+// table entry of edge {a, b}, added when it is not there
+GA_INLINE int hull_entry(const MeshDev &m, const HullDev &h, int H, int a, int b)
+{
+    const u64 k = cons_key(a, b);
+    unsigned e = (unsigned)(((cons_mix(k) & 0xffffffffull) * (u64)H) >> 32);
+    for (int probe = 0; probe < H; probe++) {
+        const u64 s = atomicCAS(&h.table[e], 0ull, k);
+        if (s == 0 || s == k) return (int)e;
+        e = e + 1 == (unsigned)H ? 0u : e + 1;
+    }
+    atomicOr(m.status, GA_ERR_SCRATCH);   // never: the table holds more entries than there are edges
+    return 0;
+}
+
+// the frame triangles listed and stamped, their real vertices marked (mark[] zero on entry)
+__global__ __launch_bounds__(256) void k_hull_scan(MeshDev m, HullDev h, int op)
+{
+    const int n = ntri_used(m);
+    for (int b0 = xcd_block() * 1024; b0 < n; b0 += gridDim.x * 1024) {
+        unsigned bits = 0;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const int t = b0 + j * 256 + (int)threadIdx.x;
+            if (t >= n) continue;
+            const int4 v = m.tv[t];
+            if (v.x == GA_DEAD || !is_frame_tri(m, v)) continue;
+            bits |= 1u << j;
+            m.stamp[t] = op;
+            for (int i = 0; i < 3; i++)
+                if (ic(v, i) < m.n) h.mark[ic(v, i)] = 1;
+        }
+        int k = block_reserve(&m.counters[C_FTRI], __popc(bits));
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+            if ((bits >> j) & 1) h.ftri[k++] = b0 + j * 256 + (int)threadIdx.x;
+    }
+}
+
+// bidx (the exclusive scan of the marks) numbers the boundary vertices in vertex order, so those of
+// a set are consecutive and in spatial order.  Clears the table, places the boundary vertices,
+// marks those with a real edge (mark 3).
+__global__ void k_hull_place(MeshDev m, HullDev h)
+{
+    const int H = hull_table(m, h), nt = m.counters[C_FTRI];
+    GRID_STRIDE(q, nt) {
+        const int4 v = m.tv[h.ftri[q]];
+        const int one = frame_vertices(m, v) == 1;
+#pragma unroll
         for (int i = 0; i < 3; i++) {
-            int e = ic(nb, i);
-            bool bnd = e < 0 || is_frame_tri(m, m.tv[enc_t(e)]);
-            if (!bnd) continue;
-            int a = ic(v, p1(i)), b = ic(v, m1(i));
-            m.hnext[a] = b;
-            m.hedge[a] = enc(t, i);
-            int s = m.vset[a];
-            if (atomicAdd(&outdeg[a], 1) != 0) badset[s] = 1;
-            if (s != cs) {
-                if (cc) {
-                    atomicMin(&hull_start[cs], cmin);
-                    atomicAdd(&hull_cnt[cs], cc);
-                }
-                cs = s;
-                cc = 0;
-                cmin = 0x7fffffff;
-            }
-            cc++;
-            cmin = min(cmin, a);
+            const int a = ic(v, i);
+            if (a >= m.n) continue;
+            const int k = h.bidx[a];
+            h.blist[k] = a;
+            h.bpos[k] = m.pos[a];
+            if (one) h.mark[a] = 3;
         }
     }
-    // every lane of the wave is here
-    const bool has = cc > 0;
-    const unsigned long long bal = __ballot(has);
-    if (!bal) return;
-    const int lane = threadIdx.x & 63, leader = __ffsll((long long)bal) - 1;
-    const int s0 = __shfl(cs, leader, 64);
-    if (__all(!has || cs == s0)) {
-        int sum = has ? cc : 0, mn = has ? cmin : 0x7fffffff;
+    GRID_STRIDE(e, 2 * H) h.table[e] = 0;   // own follows the keys
+}
+
+// The first demands: the real edge of every frame triangle with two real vertices (list: the demand
+// and the triangle's slot), with the real triangle across it.  The other frame triangles die here,
+// their slots go to the pool.  Also the boxes of 64 consecutive boundary vertices each, one wave
+// per box.
+__global__ __launch_bounds__(256) void k_hull_edges(MeshDev m, HullDev h, int op)
+{
+    const int H = hull_table(m, h), nt = m.counters[C_FTRI], B = hull_b(m, h);
+    u64 *own = h.table + H;
+    GRID_STRIDE(qq, nt) {
+        const int t = h.ftri[qq];
+        const int4 v = m.tv[t];
+        const bool one = frame_vertices(m, v) == 1;
+        const int k = wave_reserve(&m.counters[C_HULL], one);
+        const int kp = wave_reserve(&m.counters[C_HULL_POOL], !one);
+        if (!one) {
+            h.pool[kp] = t;
+            m.tv[t] = make_int4(GA_DEAD, GA_DEAD, GA_DEAD, 0);
+            continue;
+        }
+        const int i = v.x >= m.n ? 0 : (v.y >= m.n ? 1 : 2);
+        const int p = ic(v, p1(i)), q = ic(v, m1(i)), nb = ic(m.tn[t], i);
+        const int e = hull_entry(m, h, H, p, q), d = p < q ? 0 : 1;
+        u64 w = (u64)HULL_LISTED << (32 * d);
+        if (nb >= 0 && m.stamp[enc_t(nb)] != op) w |= (u64)(hull_value(enc_t(nb), enc_j(nb)) << 1) << (32 * (1 - d));
+        atomicOr(&own[e], w);
+        h.list[k] = make_int2(2 * e + d, t);
+    }
+    const int lane = threadIdx.x & 63, nw = (gridDim.x * blockDim.x) >> 6;
+    for (int g = (blockIdx.x * blockDim.x + threadIdx.x) >> 6; 64 * g < B; g += nw) {
+        const double2 X = h.bpos[min(64 * g + lane, B - 1)];
+        double lx = X.x, ly = X.y, hx = X.x, hy = X.y;
         for (int d = 32; d > 0; d >>= 1) {
-            sum += __shfl_xor(sum, d, 64);
-            mn = min(mn, __shfl_xor(mn, d, 64));
+            lx = fmin(lx, __shfl_xor(lx, d, 64)); ly = fmin(ly, __shfl_xor(ly, d, 64));
+            hx = fmax(hx, __shfl_xor(hx, d, 64)); hy = fmax(hy, __shfl_xor(hy, d, 64));
         }
-        if (lane == leader) {
-            atomicMin(&hull_start[s0], mn);
-            atomicAdd(&hull_cnt[s0], sum);
-        }
-    } else if (has) {
-        atomicMin(&hull_start[cs], cmin);
-        atomicAdd(&hull_cnt[cs], cc);
+        if (lane == 0) h.bbox[g] = HullBox{lx, ly, hx, hy};
     }
 }
 
-__global__ void k_bnd_cover(MeshDev m, const int *cover, int *badset, int *blist, int *bidx, int *bcount)
+// squared distances to v: true when a is nearer than b
+__device__ __noinline__ bool hull_nearer(double2 v, double2 a, double2 b, int *status)
 {
-    GRID_STRIDE(v, m.n) {
-        if (m.vstate[v] == VS_IN_MESH && !cover[v]) badset[m.vset[v]] = 1;
-        bool b = m.hnext[v] >= 0;
-        int k = wave_reserve(bcount, b);
-        if (b) { blist[k] = v; bidx[v] = k; }
+    const double ax = a.x - v.x, ay = a.y - v.y, bx = b.x - v.x, by = b.y - v.y;
+    const double da = ax * ax + ay * ay, db = bx * bx + by * by, eb = 8.0 * GA_EPS * (da + db);
+    if (da - db < -eb) return true;
+    if (da - db > eb) return false;
+    // |a - v|^2 - |b - v|^2 exactly
+    int ovf = 0;
+    const double c[6] = {v.x, v.y, a.x, a.y, b.x, b.y};
+    const int s = min_ulp_exp(c, 6);
+    BigInt<12> V, A, B, x, sum;
+    bi_zero(sum);
+    for (int k = 0; k < 2; k++) {
+        bi_from_double(V, c[k], s, &ovf);
+        bi_from_double(A, c[2 + k], s, &ovf);
+        bi_from_double(B, c[4 + k], s, &ovf);
+        bi_sub(A, A, V, &ovf);
+        bi_sub(B, B, V, &ovf);
+        bi_mul(x, A, A, &ovf);
+        bi_add(sum, sum, x, &ovf);
+        bi_mul(x, B, B, &ovf);
+        bi_sub(sum, sum, x, &ovf);
     }
+    if (ovf) atomicOr(status, GA_ERR_EXACT_OVERFLOW);
+    return bi_sign(sum) < 0;
 }
 
-// list ranking along each cycle, cut before its start vertex: d = steps to the cut
-__global__ void k_bnd_rank_init(MeshDev m, int B, const int *blist, const int *bidx, const int *hull_start,
-                                int *succ, int *d, int *badset)
+// the boundary vertex of the set [b0, b1) nearest to its position k (one wave; -1: there is no other)
+GA_INLINE int hull_nearest(const MeshDev &m, const HullDev &h, int k, int b0, int b1, int lane)
 {
-    GRID_STRIDE(k, B) {
-        int a = blist[k];
-        int nx = m.hnext[a];
-        bool last = nx == hull_start[m.vset[a]];
-        int si = last ? -1 : bidx[nx];
-        if (!last && (si < 0 || si >= B)) {   // successor without an outgoing boundary edge
-            badset[m.vset[a]] = 1;
-            si = -1;
-            last = true;
-        }
-        succ[k] = si;
-        d[k] = last ? 0 : 1;
-    }
-}
-
-__global__ void k_bnd_rank_step(int B, const int *succ, const int *d, int *succ2, int *d2)
-{
-    GRID_STRIDE(k, B) {
-        int s = succ[k];
-        if (s < 0) { succ2[k] = -1; d2[k] = d[k]; }
-        else { succ2[k] = succ[s]; d2[k] = d[k] + d[s]; }
-    }
-}
-
-// the same rounds in one workgroup, in place (each round reads every entry's successor into
-// registers, then writes), for cycles of up to RANK_BLOCK * RANK_PER positions: one launch instead
-// of one per round
-#define RANK_BLOCK 1024
-#define RANK_PER 16
-__global__ __launch_bounds__(RANK_BLOCK) void k_bnd_rank_block(int B, int rounds, int *succ, int *d)
-{
-    int sn[RANK_PER], dn[RANK_PER];
-    for (int r = 0; r < rounds; r++) {
-#pragma unroll
-        for (int j = 0; j < RANK_PER; j++) {
-            int k = threadIdx.x + j * RANK_BLOCK;
-            if (k >= B) continue;
-            int sk = succ[k], dk = d[k];
-            sn[j] = sk < 0 ? -1 : succ[sk];
-            dn[j] = sk < 0 ? dk : dk + d[sk];
-        }
-        __syncthreads();
-#pragma unroll
-        for (int j = 0; j < RANK_PER; j++) {
-            int k = threadIdx.x + j * RANK_BLOCK;
-            if (k >= B) continue;
-            succ[k] = sn[j];
-            d[k] = dn[j];
-        }
-        __syncthreads();
-    }
-}
-
-// a cycle that does not return to its start within the rounds (a second cycle in the set), or two
-// vertices ranked to one position, marks the set; verts[] starts at -1, so a position of a marked
-// set may stay unwritten (verts -1, nxt/prv unset) and later kernels skip it
-__global__ void k_bnd_place(MeshDev m, int B, const int *blist, const int *succ, const int *d, const int *hull_cnt,
-                            const int *hull_off, int *badset, int *verts, int *owner, int *nxt, int *prv,
-                            int *alive, int *pset, double2 *bpos)
-{
-    GRID_STRIDE(k, B) {
-        int a = blist[k];
-        int s = m.vset[a];
-        int h = hull_cnt[s];
-        if (succ[k] >= 0 || d[k] >= h) { badset[s] = 1; continue; }
-        int pos = h - 1 - d[k];
-        int p = hull_off[s] + pos;
-        if (atomicExch(&verts[p], a) != -1) badset[s] = 1;
-        bpos[p] = m.pos[a];
-        owner[p] = m.hedge[a];
-        nxt[p] = hull_off[s] + (pos + 1 == h ? 0 : pos + 1);
-        prv[p] = hull_off[s] + (pos == 0 ? h - 1 : pos - 1);
-        alive[p] = 1;
-        pset[p] = s;
-    }
-}
-
-// drop every frame triangle; R's triangles across a dropped edge get a hull link; frame vertices
-// leave the mesh; boundary vertices take their outgoing boundary triangle as anchor
-__global__ void k_kill_frame(MeshDev m)
-{
-    int n = ntri_used(m);
-    GRID_STRIDE(t, n) {
-        int4 v = m.tv[t];
-        if (v.x == GA_DEAD || !is_frame_tri(m, v)) continue;
-        int4 nb = m.tn[t];
-        for (int i = 0; i < 3; i++) {
-            int e = ic(nb, i);
-            if (e < 0) continue;
-            int u = enc_t(e);
-            if (!is_frame_tri(m, m.tv[u])) set_link(m, u, enc_j(e), -1);
-        }
-        m.tv[t] = make_int4(GA_DEAD, GA_DEAD, GA_DEAD, 0);
-    }
-    GRID_STRIDE(k, m.V - m.n) {
-        int f = m.n + k;
-        if (m.vstate[f] == VS_IN_MESH) m.vstate[f] = VS_REMOVED;
-        m.vt[f] = -1;
-    }
-    GRID_STRIDE(v, m.n) {
-        if (m.hnext[v] >= 0) m.vt[v] = enc_t(m.hedge[v]);
-    }
-}
-
-// bnd layout: succ[2][B], d[2][B], verts, owner, nxt, prv, alive, pset, cand (win reuses d[0]), then
-// the positions of the cycle (double2[B]) from int offset bnd_pos_off(B), 16-byte aligned
-GA_INLINE_HOST_DEVICE int bnd_pos_off(int B) { return (11 * B + 3) & ~3; }
-
-// Ear rounds.  A cycle position p (vertex C between P = prev and N = next) is a candidate when C
-// is reflex (P, C, N clockwise) and no other live vertex of its cycle lies in the closed triangle
-// (P, N, C); winners are candidates above every candidate within cycle distance 2 (so two winners
-// share no vertex), and each winner cuts its ear.  Rounds repeat until one has no candidate: the
-// cycle is then convex.  The emptiness test looks only at the vertices in the grid cells the ear's
-// bounding box covers: a uniform grid over each set's cycle, about two vertices per cell, built by
-// a counting sort before the first round.  Few large sets run their rounds as grid-wide kernels
-// (two per round, with fan ears over straight runs of the cycle, below); many small sets run all
-// their rounds in one launch, one workgroup per set.
-GA_INLINE uint32_t ear_prio(int p, int round) { return hash32((uint32_t)p * 0x9E3779B1u ^ (uint32_t)round); }
-GA_INLINE bool ear_beats(int p, int q, int round)
-{
-    uint32_t a = ear_prio(p, round), b = ear_prio(q, round);
-    return a > b || (a == b && p > q);
-}
-
-GA_INLINE int ear_cell(double v, double lo, double sc, int G)
-{
-    int c = (int)((v - lo) * sc);
-    return c < 0 ? 0 : (c >= G ? G - 1 : c);
-}
-
-// The cycle arrays of bulk frame removal (bnd layout: succ[2][B], d[2][B], verts, owner, nxt, prv,
-// alive, pset, cand, positions) and the grid of set s: cell ends in succ (2 h ints from 2 off; the
-// ranking is done), positions by cell in d[1], and (lx, ly, sx, sy, G) after the positions.
-struct EarCycle {
-    const int *verts;
-    int *owner, *nxt, *prv, *alive, *pset, *cand, *win;
-    const double2 *bpos;
-    double *param;
-    int *cells;
-    int B;
-};
-GA_INLINE EarCycle ear_cycle(int *bnd, int B)
-{
-    EarCycle e;
-    e.verts = bnd + 4 * B; e.owner = bnd + 5 * B; e.nxt = bnd + 6 * B; e.prv = bnd + 7 * B;
-    e.alive = bnd + 8 * B; e.pset = bnd + 9 * B; e.cand = bnd + 10 * B; e.win = bnd + 2 * B;
-    e.bpos = (const double2 *)(bnd + bnd_pos_off(B));
-    e.param = (double *)(bnd + bnd_pos_off(B) + 4 * B);
-    e.cells = bnd;
-    e.B = B;
-    return e;
-}
-GA_INLINE int *ear_cend(const EarCycle &e, int off) { return e.cells + 2 * (size_t)off; }
-GA_INLINE int *ear_citem(const EarCycle &e, int off) { return e.cells + 3 * (size_t)e.B + off; }
-
-#define EAR_THREADS 1024
-#define EAR_LDS_CELLS 16384   // grid cells k_ear_grid counts in LDS (64 KB); larger grids count in memory
-// The grid of the set of this workgroup (h positions from off): bounding box, counting sort of the
-// positions by cell (counts, exclusive starts, then a fill that counts each start up to its cell's
-// end: cell c holds [c ? cend[c - 1] : 0, cend[c])), parameters stored for other kernels.
-// lcells: LDS cells of the calling kernel (NULL: none); the counting sort runs there when the
-// grid fits in lcap cells, and its result is copied out
-GA_INLINE void ear_build_grid(const EarCycle &e, int s, int h, int off, int *lcells = nullptr, int lcap = 0)
-{
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    __shared__ double red[4][EAR_THREADS / 64];
-    __shared__ int s_total[EAR_THREADS / 64];
-    int *cend = ear_cend(e, off), *citem = ear_citem(e, off);
-    double lx = INFINITY, ly = INFINITY, hx = -INFINITY, hy = -INFINITY;
-    for (int k = tid; k < h; k += EAR_THREADS) {
-        double2 q = e.bpos[off + k];
-        lx = fmin(lx, q.x); ly = fmin(ly, q.y); hx = fmax(hx, q.x); hy = fmax(hy, q.y);
-    }
+    const double2 P = h.bpos[k];
+    int best = -1;
+    for (int j = b0 + lane; j < b1; j += 64)
+        if (j != k && (best < 0 || hull_nearer(P, h.bpos[j], h.bpos[best], m.status))) best = j;
     for (int d = 32; d > 0; d >>= 1) {
-        lx = fmin(lx, __shfl_xor(lx, d, 64)); ly = fmin(ly, __shfl_xor(ly, d, 64));
-        hx = fmax(hx, __shfl_xor(hx, d, 64)); hy = fmax(hy, __shfl_xor(hy, d, 64));
+        const int o = __shfl_xor(best, d, 64);
+        if (o >= 0 && (best < 0 || hull_nearer(P, h.bpos[o], h.bpos[best], m.status))) best = o;
     }
-    if (lane == 0) { red[0][wv] = lx; red[1][wv] = ly; red[2][wv] = hx; red[3][wv] = hy; }
-    __syncthreads();
-    lx = red[0][0]; ly = red[1][0]; hx = red[2][0]; hy = red[3][0];
-    for (int w = 1; w < EAR_THREADS / 64; w++) {
-        lx = fmin(lx, red[0][w]); ly = fmin(ly, red[1][w]); hx = fmax(hx, red[2][w]); hy = fmax(hy, red[3][w]);
-    }
-    int G = 1;
-    while (2 * G * G < h) G++;   // about two vertices per cell; G * G <= 2 h for h >= 3
-    const int ncell = G * G;
-    const double sx = hx > lx ? G / (hx - lx) : 0.0, sy = hy > ly ? G / (hy - ly) : 0.0;
-    if (tid == 0) {
-        double *pr = e.param + 5 * (size_t)s;
-        pr[0] = lx; pr[1] = ly; pr[2] = sx; pr[3] = sy; pr[4] = (double)G;
-    }
-    int *cnt = (lcells && ncell <= lcap) ? lcells : cend;
-    for (int c = tid; c < ncell; c += EAR_THREADS) cnt[c] = 0;
-    __syncthreads();
-    for (int k = tid; k < h; k += EAR_THREADS) {
-        double2 q = e.bpos[off + k];
-        atomicAdd(&cnt[ear_cell(q.y, ly, sy, G) * G + ear_cell(q.x, lx, sx, G)], 1);
-    }
-    __syncthreads();
-    {
-        int per = (ncell + EAR_THREADS - 1) / EAR_THREADS, c0 = tid * per, c1 = min(ncell, c0 + per);
-        int sum = 0;
-        for (int c = c0; c < c1; c++) sum += cnt[c];
-        int inc = sum;
-        for (int d = 1; d < 64; d <<= 1) {
-            int t = __shfl_up(inc, d, 64);
-            if (lane >= d) inc += t;
-        }
-        if (lane == 63) s_total[wv] = inc;
-        __syncthreads();
-        int base = inc - sum;
-        for (int w = 0; w < wv; w++) base += s_total[w];
-        for (int c = c0; c < c1; c++) {
-            int v = cnt[c];
-            cnt[c] = base;
-            base += v;
-        }
-    }
-    __syncthreads();
-    for (int k = tid; k < h; k += EAR_THREADS) {
-        double2 q = e.bpos[off + k];
-        int c = ear_cell(q.y, ly, sy, G) * G + ear_cell(q.x, lx, sx, G);
-        citem[atomicAdd(&cnt[c], 1)] = off + k;
-    }
-    __syncthreads();
-    if (cnt != cend)
-        for (int c = tid; c < ncell; c += EAR_THREADS) cend[c] = cnt[c];
+    return best < 0 ? -1 : h.blist[best];
 }
 
-// 1 when live position p of set s is reflex and its ear is empty
-GA_INLINE int ear_candidate(const MeshDev &m, const EarCycle &e, int p, int off)
-{
-    if (!e.alive[p]) return 0;
-    int kp = e.prv[p], kn = e.nxt[p];
-    if (kp == kn) return 0;
-    double2 P = e.bpos[kp], C = e.bpos[p], N = e.bpos[kn];
-    if (orient_dev(m, P, C, N) >= 0) return 0;
-    const double *pr = e.param + 5 * (size_t)e.pset[p];
-    const double lx = pr[0], ly = pr[1], sx = pr[2], sy = pr[3];
-    const int G = (int)pr[4];
-    const int *cend = ear_cend(e, off), *citem = ear_citem(e, off);
-    double bx0 = fmin(P.x, fmin(C.x, N.x)), bx1 = fmax(P.x, fmax(C.x, N.x));
-    double by0 = fmin(P.y, fmin(C.y, N.y)), by1 = fmax(P.y, fmax(C.y, N.y));
-    int cx0 = ear_cell(bx0, lx, sx, G), cx1 = ear_cell(bx1, lx, sx, G);
-    int cy0 = ear_cell(by0, ly, sy, G), cy1 = ear_cell(by1, ly, sy, G);
-    for (int cy = cy0; cy <= cy1; cy++)
-        for (int cx = cx0; cx <= cx1; cx++) {
-            int cc = cy * G + cx;
-            for (int j = cc ? cend[cc - 1] : 0, j1 = cend[cc]; j < j1; j++) {
-                int q = citem[j];
-                if (q == p || q == kp || q == kn || !e.alive[q]) continue;
-                double2 Q = e.bpos[q];
-                if (Q.x < bx0 || Q.x > bx1 || Q.y < by0 || Q.y > by1) continue;
-                if (orient_dev(m, P, N, Q) >= 0 && orient_dev(m, N, C, Q) >= 0 && orient_dev(m, C, P, Q) >= 0)
-                    return 0;
-            }
-        }
-    return 1;
-}
+// a candidate apex of p -> q
+struct HullBest {
+    int v;        // -1: none
+    double2 X;
+};
 
-// winner: a candidate above every candidate within cycle distance 2
-GA_INLINE int ear_winner(const EarCycle &e, int p, int round)
+// The wave's best c (the same in all lanes) against the boundary positions 64 g + lane of the set
+// [b0, b1): replaced by a vertex left of p -> q and inside its circle until no lane has one.  The
+// next to try is the one that sees the edge under the largest angle (in floating point: it only
+// decides how often the loop runs, mostly once).
+GA_INLINE void hull_chunk(const MeshDev &m, const HullDev &h, double2 P, double2 Q, int p, int q, int g, int b0,
+                          int b1, int lane, HullBest &c)
 {
-    if (!e.cand[p]) return 0;
-    int a = e.prv[p], b = e.nxt[p];
-    int q[4] = {a, b, e.prv[a], e.nxt[b]};
-    for (int j = 0; j < 4; j++)
-        if (q[j] != p && e.cand[q[j]] && !ear_beats(p, q[j], round)) return 0;
-    return 1;
-}
-
-// cut the ear of winner p: triangle (prev, next, p), new boundary edge prev -> next; false when the
-// triangle slots are exhausted (status set)
-GA_INLINE bool ear_cut(const MeshDev &m, const EarCycle &e, int p, int *list_out, int cnt_out_slot, int op)
-{
-    int kp = e.prv[p], kn = e.nxt[p];
-    int T = atomicAdd(m.ntri, 1);
-    if (T >= m.cap) {
-        atomicOr(m.status, GA_ERR_CAPACITY);
-        return false;
+    const int j = 64 * g + lane;
+    const bool in = j >= b0 && j < b1;
+    const double2 X = in ? h.bpos[j] : P;
+    const int x = in ? h.blist[j] : p;
+    int o = orient_filter(P, Q, X);
+    // p, q themselves and points on one axis-parallel line with them are exactly collinear
+    if (o == 0 && x != p && x != q && !(P.x == Q.x && Q.x == X.x) && !(P.y == Q.y && Q.y == X.y))
+        o = orient_dev(m, P, Q, X);
+    bool better = o > 0 && x != p && x != q;
+    double t = INFINITY;
+    if (better) {
+        const double ax = P.x - X.x, ay = P.y - X.y, bx = Q.x - X.x, by = Q.y - X.y;
+        const double cr = ax * by - ay * bx, dot = ax * bx + ay * by;
+        t = cr > 0.0 ? dot / cr : (dot < 0.0 ? -INFINITY : INFINITY);
+        if (c.v >= 0) better = x != c.v && incircle_at(m, P, Q, c.X, X, p, q, c.v, x) > 0;
     }
-    int vp = e.verts[kp], vc = e.verts[p], vn = e.verts[kn];
-    m.tv[T] = make_int4(vp, vn, vc, 0);
-    m.tn[T] = make_int4(-1, -1, -1, 0);
-    bond(m, T, 0, e.owner[p]);    // edge (vn, vc) = reverse of boundary edge (vc -> vn)
-    bond(m, T, 1, e.owner[kp]);   // edge (vc, vp) = reverse of boundary edge (vp -> vc)
-    m.stamp[T] = op;
-    if (atomicExch(&m.lmark[T], m.list_op) != m.list_op)
-        list_out[atomicAdd(&m.counters[cnt_out_slot], 1)] = T;
-    e.owner[kp] = enc(T, 2);      // new boundary edge (vp -> vn)
-    e.nxt[kp] = kn;
-    e.prv[kn] = kp;
-    e.alive[p] = 0;
-    m.vt[vp] = T; m.vt[vc] = T; m.vt[vn] = T;
-    return true;
-}
-
-// one workgroup per set: the grid
-__global__ __launch_bounds__(EAR_THREADS) void k_ear_grid(MeshDev m, int B, int *bnd, const int *hull_cnt,
-                                                          const int *hull_off)
-{
-    __shared__ int s_cells[EAR_LDS_CELLS];
-    int s = blockIdx.x, h = hull_cnt[s];
-    if (h < 3) return;
-    ear_build_grid(ear_cycle(bnd, B), s, h, hull_off[s], s_cells, EAR_LDS_CELLS);
-}
-
-// Grid-wide rounds: round r counts its candidates in counters[C_EAR + ...] by parity; a round
-// after one without candidates returns at once (so several run per host read), and the apply of
-// round r clears the counter round r + 1 will use.
-GA_INLINE int *ear_count(const MeshDev &m, int round) { return m.counters + ((round & 1) ? C_EAR_PREV : C_EAR); }
-
-// Fan ears.  Where the cycle runs straight (C, N, N2, ... collinear) only one of the run's vertices
-// is reflex at a time, and plain ears would take the run one vertex per round (a long thin pocket
-// between a straight side of lattice points and a hull edge takes hundreds).  A candidate C whose
-// neighbour N starts such a run instead cuts the fan (P, N, C), (P, N2, N), ... up to the farthest
-// run vertex E for which the closed triangle (P, E, C) holds no live vertex of the cycle outside
-// the positions P .. E (the run lies on its edge C E) and no fan triangle has P's other
-// neighbour in its circumcircle; the triangles nest, so E is found by binary search.  Mirrored for a run through P, with apex N.  A candidate's span is the positions from its
-// first to its last vertex; a winner holds the largest claim key (plain ear before fan, priority,
-// position) at every position of its span, so the spans of two winners never meet.  Plain ears
-// first: the apex of a pocket's fan is then its last reflex vertex left, not the first one met
-// (a fan from a shallow apex is far from Delaunay, and the flips that repair it run one
-// triangle per pass along the fan).
-#define FAN_CAP 1024    // most run vertices one fan takes (a longer run takes more rounds)
-#define EAR_WAVES 4     // waves per workgroup of the wave-per-position round kernels
-
-GA_INLINE unsigned long long ear_key(int p, int round, bool fan)
-{
-    return ((unsigned long long)!fan << 63) | ((unsigned long long)(ear_prio(p, round) >> 1) << 32) |
-           (unsigned)(p + 1);
-}
-// position k of the set's cyclic range [off, off + h), k within one turn of it
-GA_INLINE int ear_wrap(int k, int off, int h) { return k >= off + h ? k - h : (k < off ? k + h : k); }
-// positions from lo forward to hi in the cyclic range (both included)
-GA_INLINE int ear_span(int lo, int hi, int h) { return (hi >= lo ? hi - lo : hi - lo + h) + 1; }
-
-// wave-uniform: no live vertex of the set at a position outside [lo, hi] lies in the closed
-// triangle (A, Bq, C), clockwise order A, C, Bq
-GA_INLINE bool ear_empty_wave(const MeshDev &m, const EarCycle &e, int off, int h, const double *pr, double2 A,
-                              double2 Bq, double2 C, int lo, int hi)
-{
-    const int lane = threadIdx.x & 63;
-    const double lx = pr[0], ly = pr[1], sx = pr[2], sy = pr[3];
-    const int G = (int)pr[4];
-    const int *cend = ear_cend(e, off), *citem = ear_citem(e, off);
-    const int last = ear_span(lo, hi, h) - 1;
-    double bx0 = fmin(A.x, fmin(C.x, Bq.x)), bx1 = fmax(A.x, fmax(C.x, Bq.x));
-    double by0 = fmin(A.y, fmin(C.y, Bq.y)), by1 = fmax(A.y, fmax(C.y, Bq.y));
-    int cx0 = ear_cell(bx0, lx, sx, G), cx1 = ear_cell(bx1, lx, sx, G);
-    int cy0 = ear_cell(by0, ly, sy, G), cy1 = ear_cell(by1, ly, sy, G);
-    bool blocked = false;
-    for (int cy = cy0; cy <= cy1 && !__any(blocked); cy++) {
-        int c0 = cy * G + cx0, c1 = cy * G + cx1;
-        int j0 = c0 ? cend[c0 - 1] : 0, j1 = cend[c1];
-        for (int j = j0 + lane; j < j1; j += 64) {
-            int q = citem[j];
-            int dq = q - lo;
-            if (dq < 0) dq += h;
-            if (dq <= last || !e.alive[q]) continue;
-            double2 Q = e.bpos[q];
-            if (Q.x < bx0 || Q.x > bx1 || Q.y < by0 || Q.y > by1) continue;
-            if (orient_dev(m, A, Bq, Q) >= 0 && orient_dev(m, Bq, C, Q) >= 0 && orient_dev(m, C, A, Q) >= 0)
-                blocked = true;
-        }
+    while (__any(better)) {
+        double mt = better ? t : INFINITY;
+        for (int d = 32; d > 0; d >>= 1) mt = fmin(mt, __shfl_xor(mt, d, 64));
+        const int k = __ffsll((long long)__ballot(better && t <= mt)) - 1;
+        c = HullBest{__shfl(x, k, 64), make_double2(__shfl(X.x, k, 64), __shfl(X.y, k, 64))};
+        if (better) better = x != c.v && incircle_at(m, P, Q, c.X, X, p, q, c.v, x) > 0;
     }
-    return !__any(blocked);
 }
 
-// The run beyond X on the line (C, X): the live positions after x in direction d (+1 forward)
-// while they lie on the line beyond X; written to run[] in order (at most FAN_CAP).  Returns
-// their count (wave-uniform).  The scan ends at the latest at the candidate's other neighbour,
-// which is off the line.
-GA_INLINE int ear_run_wave(const MeshDev &m, const EarCycle &e, int off, int h, int x, int d, double2 C, double2 X,
-                           int *run)
+// The apex of p -> q among the boundary vertices [b0, b1) of its set (one wave; -1: none).  First
+// the vertices numbered next to p and q, which gives a circle near the final one; then the
+// boxes, 64 at a time: a box can hold a better apex only if it reaches left of the edge and into
+// the circle, which leaves one to three of B / 64.  (Every vertex tested, in steps of 64, took
+// 51 us per launch at B = 2,500, one dependent read after another.)  Both box tests keep a margin
+// far above their rounding; a circle too flat for that is not used.
+__device__ int hull_apex(const MeshDev &m, const HullDev &h, int p, int q, int b0, int b1, int lane)
 {
-    const int lane = threadIdx.x & 63;
-    const double dx = X.x - C.x, dy = X.y - C.y;
-    int R = 0;
-    for (int base = 1; base < h && R < FAN_CAP; base += 64) {
-        int k = base + lane, q = -1;
-        bool live = false, brk = false;
-        if (k < h) {
-            q = ear_wrap(x + d * k, off, h);
-            live = e.alive[q] != 0;
-            if (live) {
-                double2 Q = e.bpos[q];
-                brk = orient_dev(m, C, X, Q) != 0 || (Q.x - X.x) * dx + (Q.y - X.y) * dy <= 0.0;
-            }
-        }
-        unsigned long long bm = __ballot(brk), lm = __ballot(live);
-        if (bm) lm &= (1ull << (__ffsll((long long)bm) - 1)) - 1;   // live lanes before the first break
-        int idx = R + __popcll(lm & ((1ull << lane) - 1));
-        if (((lm >> lane) & 1) && idx < FAN_CAP) run[idx] = q;
-        R += __popcll(lm);
-        if (bm) break;
-    }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    return min(R, FAN_CAP);
-}
-
-// The usable part of a run: the fan's triangles up to run[k] keep the apex's other neighbour W
-// outside their circumcircles (exact, with the mesh's symbolic tie-break).  Going on past that
-// point would give the apex run edges that belong to W or to vertices beyond it in the final
-// mesh, and the flips that hand them over run one triangle per pass along the fan; stopped
-// there, the next rounds cut the apex and continue the run with W as apex.  d = +1: triangle
-// (apex, run[k], run[k - 1]); d = -1: (run[k], apex, run[k - 1]); run[-1] = x.
-GA_INLINE int ear_fan_delaunay(const MeshDev &m, const EarCycle &e, const int *run, int R, int d, int apex, int w,
-                               int x)
-{
-    const int lane = threadIdx.x & 63;
-    const double2 A = e.bpos[apex], W = e.bpos[w];
-    const int ia = e.verts[apex], iw = e.verts[w];
-    for (int b = 0; b < R; b += 64) {
-        int k = b + lane;
-        bool bad = false;
-        if (k < R) {
-            int qa = run[k], qb = k ? run[k - 1] : x;
-            double2 Qa = e.bpos[qa], Qb = e.bpos[qb];
-            int ja = e.verts[qa], jb = e.verts[qb];
-            bad = d > 0 ? incircle_at(m, A, Qa, Qb, W, ia, ja, jb, iw) > 0
-                        : incircle_at(m, Qa, A, Qb, W, ja, ia, jb, iw) > 0;
-        }
-        unsigned long long bm = __ballot(bad);
-        if (bm) return b + __ffsll((long long)bm) - 1;
-    }
-    return R;
-}
-
-// Largest k < R whose fan (end run[k]) is empty; -1 when even run[0]'s is not.  d = +1: apex P,
-// triangle (P, E, C), span kp .. E; d = -1: apex N, triangle (E, N, C), span E .. kn.
-GA_INLINE int ear_fan_end(const MeshDev &m, const EarCycle &e, int off, int h, const double *pr, const int *run,
-                          int R, int d, double2 P, double2 C, double2 N, int kp, int kn)
-{
-    auto empty = [&](int k) {
-        int q = run[k];
-        double2 E = e.bpos[q];
-        return d > 0 ? ear_empty_wave(m, e, off, h, pr, P, E, C, kp, q)
-                     : ear_empty_wave(m, e, off, h, pr, E, N, C, q, kn);
-    };
-    if (empty(R - 1)) return R - 1;
-    int lo = -1, hi = R - 1;   // run[lo] empty (-1: N or P itself), run[hi] blocked
-    while (hi - lo > 1) {
-        int mid = (lo + hi) >> 1;
-        if (empty(mid)) lo = mid;
-        else hi = mid;
-    }
-    return lo;
-}
-
-// One wave per cycle position: cand[p] = 0 (none), 1 (plain ear), 2 (fan through N) or 3 (fan
-// through P), fan[p] = the fan's far end; candidates claim their spans in claims[round & 1].
-__global__ __launch_bounds__(64 * EAR_WAVES) void k_ear_cand(MeshDev m, int B, int *bnd, const int *hull_off,
-                                                            const int *hull_cnt, unsigned long long *claims,
-                                                            int round)
-{
-    if (round > 0 && *ear_count(m, round - 1) == 0) return;
-    __shared__ int s_run[EAR_WAVES][FAN_CAP];
-    EarCycle e = ear_cycle(bnd, B);
-    const int lane = threadIdx.x & 63;
-    int *run = s_run[threadIdx.x >> 6];
-    unsigned long long *claim = claims + (size_t)(round & 1) * B;
-    const int wave = (xcd_block() * blockDim.x + threadIdx.x) >> 6, nw = (gridDim.x * blockDim.x) >> 6;
-    for (int p = wave; p < B; p += nw) {
-        int c = 0, lo = 0, hi = 0, end = -1, off = 0, h = 0;
-        if (e.alive[p]) {
-            int kp = e.prv[p], kn = e.nxt[p];
-            if (kp != kn) {
-                double2 P = e.bpos[kp], C = e.bpos[p], N = e.bpos[kn];
-                if (orient_dev(m, P, C, N) < 0) {
-                    const int s = e.pset[p];
-                    off = hull_off[s];
-                    h = hull_cnt[s];
-                    const double *pr = e.param + 5 * (size_t)s;
-                    if (ear_empty_wave(m, e, off, h, pr, P, N, C, kp, kn)) {
-                        c = 1; lo = kp; hi = kn;
-                        int k2 = e.nxt[kn];
-                        if (k2 != kp && orient_dev(m, C, N, e.bpos[k2]) == 0) {
-                            int R = ear_run_wave(m, e, off, h, kn, 1, C, N, run);
-                            if (R > 0) R = ear_fan_delaunay(m, e, run, R, 1, kp, e.prv[kp], kn);
-                            int f = R > 0 ? ear_fan_end(m, e, off, h, pr, run, R, 1, P, C, N, kp, kn) : -1;
-                            if (f >= 0) { c = 2; end = run[f]; hi = end; }
-                        }
-                        int k0 = e.prv[kp];
-                        if (c == 1 && k0 != kn && orient_dev(m, C, P, e.bpos[k0]) == 0) {
-                            int R = ear_run_wave(m, e, off, h, kp, -1, C, P, run);
-                            if (R > 0) R = ear_fan_delaunay(m, e, run, R, -1, kn, e.nxt[kn], kp);
-                            int f = R > 0 ? ear_fan_end(m, e, off, h, pr, run, R, -1, P, C, N, kp, kn) : -1;
-                            if (f >= 0) { c = 3; end = run[f]; lo = end; }
-                        }
-                    }
+    const double2 P = m.pos[p], Q = m.pos[q];
+    const int gp = h.bidx[p] >> 6, gq = h.bidx[q] >> 6;
+    HullBest c{-1, P};
+    hull_chunk(m, h, P, Q, p, q, gp, b0, b1, lane, c);
+    if (gq != gp) hull_chunk(m, h, P, Q, p, q, gq, b0, b1, lane, c);
+    const double ux = Q.x - P.x, uy = Q.y - P.y;
+    const int g1 = (b1 - 1) >> 6;
+    for (int gb = b0 >> 6; gb <= g1; gb += 64) {
+        const int g = gb + lane;
+        const bool in = g <= g1 && g != gp && g != gq;
+        const HullBox bx = h.bbox[min(g, g1)];
+        // largest cross product (Q - P) x (X - P) over the box
+        const double ex = (uy > 0 ? bx.lx : bx.hx) - P.x, ey = (ux > 0 ? bx.hy : bx.ly) - P.y;
+        const double l = ux * ey, r = uy * ex;
+        const bool left = in && l - r >= -1e-14 * (fabs(l) + fabs(r));
+        for (unsigned long long todo = __ballot(left); todo;) {
+            if (c.v >= 0) {
+                // circle of (P, Q, C): centre P + (ox, oy)
+                const double vx = c.X.x - P.x, vy = c.X.y - P.y;
+                const double a = ux * vy, b = uy * vx, cr = a - b;
+                if (cr > 1e-6 * (fabs(a) + fabs(b))) {
+                    const double uu = ux * ux + uy * uy, vv = vx * vx + vy * vy, f = 0.5 / cr;
+                    const double ox = f * (vy * uu - uy * vv), oy = f * (ux * vv - vx * uu);
+                    const double dx = fmax(fmax(bx.lx - P.x - ox, P.x + ox - bx.hx), 0.0);
+                    const double dy = fmax(fmax(bx.ly - P.y - oy, P.y + oy - bx.hy), 0.0);
+                    const double rad = sqrt(ox * ox + oy * oy);
+                    // the centre's cancellation error, the relative error of f and of the differences
+                    const double reach = rad * (1.0 + 1e-8) + 1e-14 * (fabs(P.x) + fabs(P.y) + rad) +
+                                         1e-14 * f * ((fabs(vx) + fabs(vy)) * uu + (fabs(ux) + fabs(uy)) * vv);
+                    const bool out = dx * dx + dy * dy > reach * reach;
+                    todo &= ~__ballot(out);
+                    if (!todo) break;
                 }
             }
-        }
-        if (c) {
-            const unsigned long long key = ear_key(p, round, c > 1);
-            const int len = ear_span(lo, hi, h);
-            for (int k = lane; k < len; k += 64) atomicMax(&claim[ear_wrap(lo + k, off, h)], key);
-        }
-        if (lane == 0) {
-            e.cand[p] = c;
-            e.win[p] = end;
-            if (c) atomicAdd(ear_count(m, round), 1);
+            const int k = __ffsll((long long)todo) - 1;
+            todo &= todo - 1;
+            hull_chunk(m, h, P, Q, p, q, gb + k, b0, b1, lane, c);
         }
     }
+    return c.v;
 }
 
-// The fan of winner p in direction d (+1: run through N, apex P; -1: run through P, apex N) up to
-// position `end`, by the whole wave: the run's live positions q_1 .. q_R after p, triangle i
-// between q_i and q_{i+1} (q_0 = p), consecutive triangles linked across their shared apex edges.
-GA_INLINE void ear_fan_cut(const MeshDev &m, const EarCycle &e, int p, int d, int end, int off, int h, int kp, int kn,
-                           int *list_out, int cnt_out_slot, int op)
+// Creates the triangle (p, q, c) unless another demand did, in *slot when the wave has one (then
+// -1), else in one from the pool or a new one; pushes the far sides that nothing is known of on the
+// wave's stack (next[] links the demands, *head the first).  One wave; lanes 0, 1 and 2 take a side each.
+__device__ void hull_create(const MeshDev &m, const HullDev &h, int H, int it0, int p, int q, int c, int lane,
+                            int *slot, int *head)
 {
-    const int lane = threadIdx.x & 63;
-    const int len = ear_span(d > 0 ? p : end, d > 0 ? end : p, h) - 1;   // positions p + d .. end
-    int R = 0;
-    for (int b = 0; b < len; b += 64) {
-        int k = b + lane + 1;
-        bool live = k <= len && e.alive[ear_wrap(p + d * k, off, h)];
-        R += __popcll(__ballot(live));
+    u64 *own = h.table + H;
+    // the sides from the smallest vertex a; the wave that sets the left of a -> b creates the triangle
+    const int r = p < q ? (p < c ? 0 : 2) : (q < c ? 1 : 2);
+    const int a = r == 0 ? p : (r == 1 ? q : c), b = r == 0 ? q : (r == 1 ? c : p), d = r == 0 ? c : (r == 1 ? p : q);
+    const int su = lane == 0 ? a : (lane == 1 ? b : d), sv = lane == 0 ? b : (lane == 1 ? d : a);
+    const int k = lane == 0 ? 2 : (lane == 1 ? 0 : 1);   // the side lies opposite vertex k of (a, b, d)
+    int it = 0, T = *slot;
+    if (lane < 3) it = 2 * hull_entry(m, h, H, su, sv) + (su < sv ? 0 : 1);
+    if (T < 0 && lane == 0) {
+        // the pool's shares are taken one by one, so that no counter serves all waves
+        const int s = (int)((blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) % HULL_SHARES);
+        const int x = s + HULL_SHARES * atomicAdd(&h.share[s * HULL_SHARE_INTS], 1);
+        T = x < m.counters[C_HULL_POOL] ? h.pool[x] : atomicAdd(m.ntri, 1);
     }
-    int T0 = 0;
-    if (lane == 0) T0 = atomicAdd(m.ntri, R);
-    T0 = __shfl(T0, 0, 64);
-    if (T0 + R > m.cap) {
+    T = __shfl(T, 0, 64);
+    if (T >= m.cap) {
         if (lane == 0) atomicOr(m.status, GA_ERR_CAPACITY);
         return;
     }
-    const int apex = d > 0 ? kp : kn, va = e.verts[apex];
-    int carry = p, i0 = 0;
-    for (int b = 0; b < len; b += 64) {
-        int k = b + lane + 1;
-        int q = k <= len ? ear_wrap(p + d * k, off, h) : -1;
-        bool live = q >= 0 && e.alive[q];
-        unsigned long long lm = __ballot(live), below = lm & ((1ull << lane) - 1);
-        int src = below ? 63 - __clzll((long long)below) : lane;
-        int qprev = __shfl(q, src, 64);
-        if (live) {
-            const int i = i0 + __popcll(below), T = T0 + i;
-            const int qi = below ? qprev : carry;
-            const int vi = e.verts[qi], vn = e.verts[q];
-            int4 tn;
-            if (d > 0) {
-                // (P, q_{i+1}, q_i): edge 0 faces the boundary edge q_i -> q_{i+1}, edge 1 the apex edge
-                const int X0 = e.owner[qi], X1 = i == 0 ? e.owner[kp] : enc(T - 1, 2);
-                m.tv[T] = make_int4(va, vn, vi, 0);
-                tn = make_int4(X0, X1, i == R - 1 ? -1 : enc(T + 1, 1), 0);
-                if (X0 >= 0) set_link(m, enc_t(X0), enc_j(X0), enc(T, 0));
-                if (i == 0 && X1 >= 0) set_link(m, enc_t(X1), enc_j(X1), enc(T, 1));
-            } else {
-                // (q_{i+1}, N, q_i): edge 1 faces the boundary edge q_{i+1} -> q_i, edge 0 the apex edge
-                const int Y0 = i == 0 ? e.owner[p] : enc(T - 1, 2), Y1 = e.owner[q];
-                m.tv[T] = make_int4(vn, va, vi, 0);
-                tn = make_int4(Y0, Y1, i == R - 1 ? -1 : enc(T + 1, 0), 0);
-                if (Y1 >= 0) set_link(m, enc_t(Y1), enc_j(Y1), enc(T, 1));
-                if (i == 0 && Y0 >= 0) set_link(m, enc_t(Y0), enc_j(Y0), enc(T, 0));
-            }
-            m.tn[T] = tn;
-            m.stamp[T] = op;
-            if (atomicExch(&m.lmark[T], m.list_op) != m.list_op)
-                list_out[atomicAdd(&m.counters[cnt_out_slot], 1)] = T;
-            e.alive[qi] = 0;
-            m.vt[vi] = T;
-            m.vt[vn] = T;
-            if (i == 0) m.vt[va] = T;
-        }
-        if (lm) carry = __shfl(q, 63 - __clzll((long long)lm), 64);
-        i0 += __popcll(lm);
-    }
+    *slot = T;
+    const unsigned val = hull_value(T, k) << 1;
+    bool won = false;
     if (lane == 0) {
-        const int Tl = T0 + R - 1;
-        if (d > 0) {
-            e.owner[kp] = enc(Tl, 2);
-            e.nxt[kp] = end;
-            e.prv[end] = kp;
+        unsigned *half = (unsigned *)&own[it >> 1];   // a < b: the low half
+        unsigned w = it == it0 ? HULL_LISTED : 0u;
+        while (w <= HULL_LISTED) {
+            const unsigned seen = atomicCAS(half, w, val | w);
+            if (seen == w) { won = true; break; }
+            w = seen;
+        }
+    }
+    if (!__shfl((int)won, 0, 64)) return;
+    *slot = -1;
+    bool more = false;
+    if (lane < 3) {
+        const int dir = it & 1;
+        const u64 w = (lane == 0 ? 0ull : (u64)val << (32 * dir)) | ((u64)HULL_LISTED << (32 * (1 - dir)));
+        const unsigned o = hull_half(atomicOr(&own[it >> 1], w), 1 - dir);
+        const unsigned ov = o >> 1;
+        if (ov == HULL_EDGE) set_link(m, T, k, -1);
+        else if (ov) bond(m, T, k, enc((int)((ov - 1) / 3u), (int)((ov - 1) % 3u)));
+        else more = o == 0;   // this wave has listed it
+    }
+    if (lane == 0) m.tv[T] = make_int4(a, b, d, 0);
+    const unsigned long long mb = __ballot(more);
+    for (int s = 0; s < 3; s++) {
+        if (!((mb >> s) & 1)) continue;
+        const int x = __shfl(it, s, 64) ^ 1;
+        if (lane == 0) h.next[x] = *head;
+        *head = x;
+    }
+}
+
+// Drops the frame vertices and the frame triangles left, and fills what they covered: one wave per
+// first demand (with its frame triangle's slot) and per boundary vertex without a real edge.  For such
+// a vertex the edge to its nearest boundary vertex is a Delaunay edge (the circle on it as diameter is
+// empty) with nothing known on either side.
+__global__ __launch_bounds__(256) void k_hull_fill(MeshDev m, HullDev h)
+{
+    const int H = hull_table(m, h), nd = m.counters[C_HULL], B = hull_b(m, h);
+    u64 *own = h.table + H;
+    GRID_STRIDE(k, m.V - m.n) {
+        const int f = m.n + k;
+        if (m.vstate[f] == VS_IN_MESH) m.vstate[f] = VS_REMOVED;
+        m.vt[f] = -1;
+    }
+    const int lane = threadIdx.x & 63, nw = (gridDim.x * blockDim.x) >> 6;
+    for (int i = (blockIdx.x * blockDim.x + threadIdx.x) >> 6; i < nd + B; i += nw) {
+        int head = -1, slot = -1, b0, b1;
+        if (i < nd) {
+            const int2 f = h.list[i];
+            head = f.x;
+            slot = f.y;
+            if (lane == 0) h.next[head] = -1;
+            const int v = (int)((h.table[head >> 1] - 1) >> 32);
+            const SetDesc &sd = m.sets[m.vset[v]];
+            b0 = h.bidx[sd.poff];
+            b1 = h.bidx[sd.poff + sd.n];
         } else {
-            e.owner[end] = enc(Tl, 2);
-            e.nxt[end] = kn;
-            e.prv[kn] = end;
+            const int v = h.blist[i - nd];
+            if (h.mark[v] == 3) continue;
+            const SetDesc &sd = m.sets[m.vset[v]];
+            b0 = h.bidx[sd.poff];
+            b1 = h.bidx[sd.poff + sd.n];
+            const int w = hull_nearest(m, h, i - nd, b0, b1, lane);
+            if (w < 0) continue;
+            int e = 0;
+            u64 old = 0;
+            if (lane == 0) {
+                e = hull_entry(m, h, H, v, w);
+                old = atomicOr(&own[e], (u64)HULL_LISTED << 32 | HULL_LISTED);
+            }
+            e = __shfl(e, 0, 64);
+            old = __shfl(old, 0, 64);
+            for (int d = 0; d < 2; d++)
+                if (hull_half(old, d) == 0) {
+                    if (lane == 0) h.next[2 * e + d] = head;
+                    head = 2 * e + d;
+                }
         }
+        while (head >= 0) {
+            const int it = head;
+            int nx = 0, known = 0;
+            u64 key = 0;
+            if (lane == 0) {
+                nx = h.next[it];
+                const u64 w = __hip_atomic_load(&own[it >> 1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                known = hull_half(w, it & 1) > HULL_LISTED;   // found from another side
+                key = __hip_atomic_load(&h.table[it >> 1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) - 1;
+            }
+            head = __shfl(nx, 0, 64);
+            if (__shfl(known, 0, 64)) continue;
+            key = __shfl(key, 0, 64);
+            const int lo = (int)(key >> 32), hi = (int)(key & 0xffffffffull);
+            const int p = it & 1 ? hi : lo, q = it & 1 ? lo : hi;
+            const int c = hull_apex(m, h, p, q, b0, b1, lane);
+            if (c >= 0) {
+                hull_create(m, h, H, it, p, q, c, lane, &slot, &head);
+            } else if (lane == 0) {
+                const int d = it & 1;
+                const unsigned ov = hull_half(atomicOr(&own[it >> 1], (u64)(HULL_EDGE << 1) << (32 * d)), 1 - d) >> 1;
+                if (ov && ov != HULL_EDGE) set_link(m, (int)((ov - 1) / 3u), (int)((ov - 1) % 3u), -1);
+            }
+        }
+        if (slot >= 0 && lane == 0) m.tv[slot] = make_int4(GA_DEAD, GA_DEAD, GA_DEAD, 0);
     }
 }
 
-// One wave per candidate: a winner (its key at every position of its span) cuts its ear or fan.
-// Clears the claims of the next round (written two rounds ago, read by the previous apply).
-__global__ __launch_bounds__(64 * EAR_WAVES) void k_ear_apply(MeshDev m, int B, int *bnd, const int *hull_off,
-                                                             const int *hull_cnt, unsigned long long *claims,
-                                                             int round, int *list_out, int cnt_out_slot, int op)
+void launch_hull(MeshDev &m, const HullDev &h, int op, void *scan_tmp, hipStream_t st)
 {
-    bool any = *ear_count(m, round) != 0;
-    if (blockIdx.x == 0 && threadIdx.x == 0) *ear_count(m, round + 1) = 0;
-    if (!any) return;
-    EarCycle e = ear_cycle(bnd, B);
-    const unsigned long long *claim = claims + (size_t)(round & 1) * B;
-    unsigned long long *other = claims + (size_t)((round + 1) & 1) * B;
-    GRID_STRIDE(k, B) other[k] = 0;
-    const int lane = threadIdx.x & 63;
-    const int wave = (xcd_block() * blockDim.x + threadIdx.x) >> 6, nw = (gridDim.x * blockDim.x) >> 6;
-    for (int p = wave; p < B; p += nw) {
-        const int c = e.cand[p];
-        if (!c) continue;
-        const unsigned long long key = ear_key(p, round, c > 1);
-        // a winner holds p, so no other winner changes p's links or its span
-        if (claim[p] != key) continue;
-        const int s = e.pset[p], off = hull_off[s], h = hull_cnt[s];
-        const int kp = e.prv[p], kn = e.nxt[p], end = e.win[p];
-        const int lo = c == 3 ? end : kp, hi = c == 2 ? end : kn, len = ear_span(lo, hi, h);
-        bool lost = false;
-        for (int k = lane; k < len; k += 64)
-            if (claim[ear_wrap(lo + k, off, h)] != key) lost = true;
-        if (__any(lost)) continue;
-        if (c == 1) {
-            if (lane == 0) ear_cut(m, e, p, list_out, cnt_out_slot, op);
-        } else {
-            ear_fan_cut(m, e, p, c == 2 ? 1 : -1, end, off, h, kp, kn, list_out, cnt_out_slot, op);
-        }
-    }
-}
-
-// All rounds of every set in one launch, one workgroup per set (batches of many small sets);
-// counters[C_EAR] = the most rounds a set ran.
-__global__ __launch_bounds__(EAR_THREADS) void k_ear_sets(MeshDev m, int B, int *bnd, const int *hull_cnt,
-                                                          const int *hull_off, int *list_out, int cnt_out_slot,
-                                                          int op)
-{
-    const int s = blockIdx.x, h = hull_cnt[s], off = hull_off[s];
-    if (h < 3) return;
-    EarCycle e = ear_cycle(bnd, B);
-    ear_build_grid(e, s, h, off);
-    const int tid = threadIdx.x;
-    __shared__ int s_cut, s_stop;
-    for (int round = 0;; round++) {
-        if (round > h + 8) {   // every round with a candidate cuts at least one ear
-            if (tid == 0) atomicOr(m.status, GA_ERR_WALK);
-            break;
-        }
-        for (int k = tid; k < h; k += EAR_THREADS) e.cand[off + k] = ear_candidate(m, e, off + k, off);
-        __syncthreads();
-        if (tid == 0) { s_cut = 0; s_stop = 0; }
-        for (int k = tid; k < h; k += EAR_THREADS) e.win[off + k] = ear_winner(e, off + k, round);
-        __syncthreads();
-        for (int k = tid; k < h; k += EAR_THREADS) {
-            if (!e.win[off + k]) continue;
-            if (ear_cut(m, e, off + k, list_out, cnt_out_slot, op)) s_cut = 1;
-            else s_stop = 1;
-        }
-        __syncthreads();
-        bool done = !s_cut || s_stop;
-        if (done) {
-            if (tid == 0) atomicMax(&m.counters[C_EAR], round + 1);
-            break;
-        }
-        __syncthreads();
-    }
-}
-
-void launch_bnd_detect(MeshDev &m, int *outdeg, int *cover, int *hull_cnt, int *hull_start, int *badset,
-                       int *blist, int *bidx, hipStream_t st)
-{
-    GA_LAUNCH(k_bnd_edges, dim3(FIXED_GRID), dim3(256), 0, st, m, outdeg, cover, hull_cnt, hull_start, badset);
-    GA_LAUNCH(k_bnd_cover, dim3(FIXED_GRID), dim3(256), 0, st, m, (const int *)cover, badset, blist, bidx,
-              m.counters + C_BND);
-}
-
-void launch_bnd_rank(MeshDev &m, int B, int rounds, const int *blist, const int *bidx, const int *hull_start,
-                     const int *hull_cnt, const int *hull_off, int *badset, int *bnd, hipStream_t st)
-{
-    int *succ[2] = {bnd, bnd + B}, *d[2] = {bnd + 2 * B, bnd + 3 * B};
-    int *verts = bnd + 4 * B, *owner = bnd + 5 * B, *nxt = bnd + 6 * B, *prv = bnd + 7 * B, *alive = bnd + 8 * B,
-        *pset = bnd + 9 * B;
-    int g = std::min(4096, (B + 255) / 256);
-    GA_LAUNCH(k_bnd_rank_init, dim3(g), dim3(256), 0, st, m, B, blist, bidx, hull_start, succ[0], d[0], badset);
-    int cur = 0;
-    if (B <= RANK_BLOCK * RANK_PER) {
-        GA_LAUNCH(k_bnd_rank_block, dim3(1), dim3(RANK_BLOCK), 0, st, B, rounds, succ[0], d[0]);
-    } else {
-        for (int r = 0; r < rounds; r++) {
-            GA_LAUNCH(k_bnd_rank_step, dim3(g), dim3(256), 0, st, B, (const int *)succ[cur], (const int *)d[cur],
-                      succ[1 - cur], d[1 - cur]);
-            cur = 1 - cur;
-        }
-    }
-    launch_fill_i32(verts, -1, (size_t)B, st);
-    GA_LAUNCH(k_bnd_place, dim3(g), dim3(256), 0, st, m, B, blist, (const int *)succ[cur], (const int *)d[cur],
-              hull_cnt, hull_off, badset, verts, owner, nxt, prv, alive, pset, (double2 *)(bnd + bnd_pos_off(B)));
-}
-
-void launch_kill_frame(MeshDev &m, hipStream_t st)
-{
-    GA_LAUNCH(k_kill_frame, dim3(FIXED_GRID), dim3(256), 0, st, m);
-}
-
-// claim keys of the grid-wide rounds: two arrays of B, after the grid parameters of the sets
-static unsigned long long *ear_claims(int *bnd, int B, int nsets)
-{
-    return (unsigned long long *)(bnd + ((bnd_pos_off(B) + 4 * B + 10 * nsets + 1) & ~1));
-}
-
-// the grid of every set, and cleared claims for the grid-wide rounds
-void launch_ear_grid(MeshDev &m, int B, int *bnd, const int *hull_cnt, const int *hull_off, int nsets, hipStream_t st)
-{
-    GA_LAUNCH(k_ear_grid, dim3(nsets), dim3(EAR_THREADS), 0, st, m, B, bnd, hull_cnt, hull_off);
-    // claims zero, and the first round's candidate count
-    IntFills f;
-    f.add(ear_claims(bnd, B, nsets), 4 * (size_t)B, 0);
-    f.add(m.counters + C_EAR, 1, 0);
-    launch_fill_multi(f, st);
-}
-
-// rounds r0 .. r0 + k - 1 as grid-wide kernels, one wave per cycle position
-void launch_ear_rounds(MeshDev &m, int B, int *bnd, const int *hull_cnt, const int *hull_off, int nsets, int r0,
-                       int k, int *list_out, int cnt_out_slot, int op, hipStream_t st)
-{
-    unsigned long long *claims = ear_claims(bnd, B, nsets);
-    int gw = std::min(4096, (B + EAR_WAVES - 1) / EAR_WAVES);
-    gw = (gw + 7) & ~7;
-    for (int r = r0; r < r0 + k; r++) {
-        GA_LAUNCH(k_ear_cand, dim3(gw), dim3(64 * EAR_WAVES), 0, st, m, B, bnd, hull_off, hull_cnt, claims, r);
-        GA_LAUNCH(k_ear_apply, dim3(gw), dim3(64 * EAR_WAVES), 0, st, m, B, bnd, hull_off, hull_cnt, claims, r,
-                  list_out, cnt_out_slot, op);
-    }
-}
-
-// every set's ear rounds in one workgroup; counters[C_EAR] = the most rounds any set ran
-void launch_ear_sets(MeshDev &m, int B, int *bnd, const int *hull_cnt, const int *hull_off, int nsets,
-                     int *list_out, int cnt_out_slot, int op, hipStream_t st)
-{
-    GA_LAUNCH(k_ear_sets, dim3(nsets), dim3(EAR_THREADS), 0, st, m, B, bnd, hull_cnt, hull_off, list_out,
-              cnt_out_slot, op);
+    GA_LAUNCH(k_hull_scan, dim3(FIXED_GRID), dim3(256), 0, st, m, h, op);
+    launch_exclusive_scan(h.mark, h.bidx, (size_t)m.n + 1, scan_tmp, st);
+    GA_LAUNCH(k_hull_place, dim3(FIXED_GRID), dim3(256), 0, st, m, h);
+    GA_LAUNCH(k_hull_edges, dim3(FIXED_GRID), dim3(256), 0, st, m, h, op);
+    GA_LAUNCH(k_hull_fill, dim3(FIXED_GRID), dim3(256), 0, st, m, h);
 }
 
 // ---- canonical output ----------------------------------------------------------------------------

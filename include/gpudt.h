@@ -176,10 +176,10 @@ typedef struct {
     long long incircleTests, incircleExact, orientExact;
     long long alphaExactCompares, alphaExactAttach, alphaClusters, alphaMaxCluster;
     double ms_pba, ms_recon, ms_shift, ms_missing, ms_boundary, ms_flip, ms_canon, ms_alpha, ms_total;
-    /* work counts of the last run: frame vertices examined by the frame-removal kernel, sum of the
-       fan lengths of removed frame vertices, triangles listed for the flip tests */
+    /* frameSeen, frameChain: 0 (kept for the layout); flipListed: triangles listed for the flip
+       tests of the last run */
     long long frameSeen, frameChain, flipListed;
-    /* 1 when the frame was removed in bulk (one boundary cycle per set), 0 round by round */
+    /* 1 once the frame was removed; launches that filled what it covered */
     int frameBulk, earRounds;
     /* constrained runs: cavity insertion rounds, and the time of the constraint stage (insertion
        and the constrained flips) */
@@ -189,7 +189,7 @@ typedef struct {
        and the master list */
     double ms_alpha_rho, ms_alpha_order, ms_alpha_lists;
     /* per mesh stage (0: shifting, missing-site insertion and the flips after them; 1: frame
-       removal and the final flips; 2: constraints and canonical output): triangles listed for
+       removal; 2: constraints and canonical output): triangles listed for
        flip tests, incircle tests, exact incircle and exact orientation evaluations */
     long long stageListed[3], stageIncircleTests[3], stageIncircleExact[3], stageOrientExact[3];
     /* flip passes run back to back by the single-workgroup tail on short lists, and the triangles
