@@ -44,7 +44,7 @@ ALGO_BYTES = {
         "gather_bytes": lambda st, T, n: 156.0 * (st["flipListed"] - st["flipTailListed"])},
     "k_pba_color": {
         "model": "8 B per pixel (envelope read 4 + label written 4)",
-        "bytes": lambda st, T, n: 8.0 * T * T * st["pbaIterations"]},
+        "bytes": lambda st, T, n: 8.0 * T * T},
 }
 
 

@@ -589,7 +589,7 @@ static BatchPlan plan_batch(const int *n, const int *T, const double *bb5, int n
         acc[BM_STACK] += (Ts / 64) * m;
         acc[BM_MERGE] += (Ts / 64) * std::max(1LL, m / 2);
         acc[BM_COLOR] += (Ts / 64) * m;
-        acc[BM_PIX] += Ts * Ts / 256;
+        acc[BM_PIX] += Ts * Ts / 1024;
         acc[BM_RECON] += (Ts / 16) * (Ts / 16);   // one tile per 16 x 16-pixel cell
     }
     for (int k = 0; k < BM_COUNT; k++) b.blocks[k] = (int)acc[k];
@@ -662,16 +662,17 @@ static void run_pba(galpha_ctx *c, const double *d_xy, const BatchDev &bd, int *
     PbaBuffers b{c->smap.as<int>(), c->g.as<short>(), c->S.as<int>(), c->cnt.as<int>(), c->plo.as<int>(),
                  c->E.as<int>(), c->ecnt.as<int>(), c->vor.as<int>()};
     int it = 0, isl = 0;
+    int *cnt = c->counters.as<int>();
+    c->mlist.ensure(4 * (size_t)bd.ntot);   // (free until the shifting: the removed sites)
+    launch_pba(b, bd, st);
+    launch_islands(c->vor.as<int>(), c->pix.as<int>(), bd, c->bad.as<int>(), cnt + C_FLAG, st);
     for (; it < 16; it++) {
-        launch_pba(b, bd, st);
-        if (it > 0) ctx_counter_set(c, C_FLAG, 0);
-        launch_islands(c->vor.as<int>(), c->pix.as<int>(), bd, c->bad.as<int>(), c->counters.as<int>() + C_FLAG, st);
         int cv[C_ISLAND_SITES + 1];   // the flag and the island count in one read
         ctx_counters_read(c, cv, 0, C_ISLAND_SITES + 1);
         isl = cv[C_ISLAND_SITES];
         if (cv[C_FLAG] == 0) break;
-        launch_remove_bad(c->bad.as<int>(), c->pix.as<int>(), bd, c->smap.as<int>(),
-                          c->counters.as<int>() + C_ISLAND_SITES, st);
+        launch_island_repair(b, bd, c->bad.as<int>(), c->pix.as<int>(), cnt + C_ISLAND_SITES, isl, c->mlist.as<int>(),
+                             cnt + C_CHANGED, cnt + C_FLAG, st);
     }
     if (it == 16) throw GalphaError("discrete Voronoi diagram did not settle (island certificate)");
     *iters = it + 1;

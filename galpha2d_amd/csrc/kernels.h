@@ -156,7 +156,7 @@ struct HullDev {
 #define C_TESTS_INCIRCLE 14
 #define C_TESTS_ORIENT 15
 #define C_RECON_TRIS 16
-#define C_SHIFT_BAD 17
+#define C_CHANGED 17          // pixels relabelled by an island repair
 #define C_DELETED 18
 #define C_ISLAND_SITES 19
 #define C_HSTART 20
@@ -203,7 +203,9 @@ void launch_renumber(const double2 *xy, const BatchDev &b, int *cell, int *ccoun
                      void *scan_tmp, int *perm, double2 *xys, hipStream_t st);
 void launch_pba(const PbaBuffers &p, const BatchDev &b, hipStream_t st);
 void launch_islands(const int *vor, const int *pix, const BatchDev &b, int *bad, int *flag, hipStream_t st);
-void launch_remove_bad(int *bad, const int *pix, const BatchDev &b, int *smap, int *removed, hipStream_t st);
+// repairs the diagram around the sites that the certificate flagged (see pba.hip)
+void launch_island_repair(const PbaBuffers &p, const BatchDev &b, int *bad, const int *pix, int *removed, int first,
+                          int *rlist, int *nchanged, int *flag, hipStream_t st);
 
 // util.hip: up to four segments of device ints copied into one contiguous device array
 struct IntSegments {

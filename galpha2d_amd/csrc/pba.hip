@@ -19,7 +19,8 @@
 // The island certificate replaces the reference's iterate-and-recolour loop
 // (kernelIslandDetection, CPU colorIsland): a pixel must have a same-labelled neighbour
 // one step toward its site (dx, dy or the diagonal).  Sites failing it are taken out of
-// the site map and the diagram is recomputed, so every label stays an exact nearest site.
+// the site map and the diagram is repaired: their columns get new nearest sites, their pixels
+// the nearest site that is left, so every label stays an exact nearest site.
 #include "dev_common.h"
 #include "kernels.h"
 
@@ -146,8 +147,65 @@ __global__ void k_splat_frame(const int *__restrict__ fpix, BatchDev b, int *__r
 }
 
 // ---- phase 1: nearest site per column --------------------------------------------------
-// block = 256 (4 waves, one column each); g[x*T + y] = row of the nearest site in column x
-// (ties to the lower row), -1 for an empty column.
+// One column, one wave (every wave of the block calls it): g[y] = row of the nearest site of the
+// column (ties to the lower row), -1 for an empty column.  masks, prv, nxt: 256 LDS entries of the
+// wave.
+GA_INLINE void pba_column(const int *__restrict__ col, short *__restrict__ gc, int nch, int lane,
+                          unsigned long long *masks, short *prv, short *nxt)
+{
+    for (int c = 0; c < nch; c++) {
+        int v = col[(c << 6) + lane];
+        unsigned long long m = __ballot(v != PBA_EMPTY);
+        if (lane == 0) masks[c] = m;
+    }
+    __syncthreads();
+    // previous / next nonempty chunk, 64 chunks per ballot group
+    int carry_prev = -1;
+    for (int gbase = 0; gbase < nch; gbase += 64) {
+        int c = gbase + lane;
+        bool nz = c < nch && masks[c] != 0ull;
+        unsigned long long b = __ballot(nz);
+        unsigned long long below = lane ? (b & ((1ull << lane) - 1ull)) : 0ull;
+        int pv = below ? gbase + 63 - __clzll(below) : carry_prev;
+        if (c < nch) prv[c] = (short)pv;
+        if (b) carry_prev = gbase + 63 - __clzll(b);
+    }
+    int carry_next = nch;
+    for (int gbase = ((nch - 1) >> 6) << 6; gbase >= 0; gbase -= 64) {
+        int c = gbase + lane;
+        bool nz = c < nch && masks[c] != 0ull;
+        unsigned long long b = __ballot(nz);
+        unsigned long long above = (lane == 63) ? 0ull : (b & (~0ull << (lane + 1)));
+        int nx = above ? gbase + __ffsll((long long)above) - 1 : carry_next;
+        if (c < nch) nxt[c] = (short)nx;
+        if (b) carry_next = gbase + __ffsll((long long)b) - 1;
+    }
+    __syncthreads();
+    for (int c = 0; c < nch; c++) {
+        unsigned long long m = masks[c];
+        int y = (c << 6) + lane;
+        unsigned long long mb = (lane == 63) ? m : (m & ((2ull << lane) - 1ull));
+        int yb = -1, ya = -1;
+        if (mb) yb = (c << 6) + 63 - __clzll(mb);
+        else {
+            int p = prv[c];
+            if (p >= 0) yb = (p << 6) + 63 - __clzll(masks[p]);
+        }
+        unsigned long long ma = m & (~0ull << lane);
+        if (ma) ya = (c << 6) + __ffsll((long long)ma) - 1;
+        else {
+            int q = nxt[c];
+            if (q < nch) ya = (q << 6) + __ffsll((long long)masks[q]) - 1;
+        }
+        int r;
+        if (yb < 0) r = ya;
+        else if (ya < 0) r = yb;
+        else r = (y - yb <= ya - y) ? yb : ya;
+        gc[y] = (short)r;
+    }
+}
+
+// block = 256 (4 waves, one column each)
 __global__ __launch_bounds__(256) void k_pba_cols(const int *__restrict__ smap_all,
                                                   short *__restrict__ g_all, BatchDev bd)
 {
@@ -156,64 +214,9 @@ __global__ __launch_bounds__(256) void k_pba_cols(const int *__restrict__ smap_a
     const int *bm = bd.bmap(BM_COLS);
     int set = set_of(bm, bd.nsets, blockIdx.x);
     const SetDesc &sd = bd.sets[set];
-    int logT = sd.logT;
-    const int *smap = smap_all + sd.toff;
-    short *g = g_all + sd.toff;
-    int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    int T = 1 << logT, nch = T >> 6;
-    int x = (blockIdx.x - bm[set]) * 4 + wave;
-    const int *col = smap + ((size_t)x << logT);
-    for (int c = 0; c < nch; c++) {
-        int v = col[(c << 6) + lane];
-        unsigned long long m = __ballot(v != PBA_EMPTY);
-        if (lane == 0) masks[wave][c] = m;
-    }
-    __syncthreads();
-    // previous / next nonempty chunk, 64 chunks per ballot group
-    int carry_prev = -1;
-    for (int gbase = 0; gbase < nch; gbase += 64) {
-        int c = gbase + lane;
-        bool nz = c < nch && masks[wave][c] != 0ull;
-        unsigned long long b = __ballot(nz);
-        unsigned long long below = lane ? (b & ((1ull << lane) - 1ull)) : 0ull;
-        int pv = below ? gbase + 63 - __clzll(below) : carry_prev;
-        if (c < nch) prv[wave][c] = (short)pv;
-        if (b) carry_prev = gbase + 63 - __clzll(b);
-    }
-    int carry_next = nch;
-    for (int gbase = ((nch - 1) >> 6) << 6; gbase >= 0; gbase -= 64) {
-        int c = gbase + lane;
-        bool nz = c < nch && masks[wave][c] != 0ull;
-        unsigned long long b = __ballot(nz);
-        unsigned long long above = (lane == 63) ? 0ull : (b & (~0ull << (lane + 1)));
-        int nx = above ? gbase + __ffsll((long long)above) - 1 : carry_next;
-        if (c < nch) nxt[wave][c] = (short)nx;
-        if (b) carry_next = gbase + __ffsll((long long)b) - 1;
-    }
-    __syncthreads();
-    short *gc = g + ((size_t)x << logT);
-    for (int c = 0; c < nch; c++) {
-        unsigned long long m = masks[wave][c];
-        int y = (c << 6) + lane;
-        unsigned long long mb = (lane == 63) ? m : (m & ((2ull << lane) - 1ull));
-        int yb = -1, ya = -1;
-        if (mb) yb = (c << 6) + 63 - __clzll(mb);
-        else {
-            int p = prv[wave][c];
-            if (p >= 0) yb = (p << 6) + 63 - __clzll(masks[wave][p]);
-        }
-        unsigned long long ma = m & (~0ull << lane);
-        if (ma) ya = (c << 6) + __ffsll((long long)ma) - 1;
-        else {
-            int q = nxt[wave][c];
-            if (q < nch) ya = (q << 6) + __ffsll((long long)masks[wave][q]) - 1;
-        }
-        int r;
-        if (yb < 0) r = ya;
-        else if (ya < 0) r = yb;
-        else r = (y - yb <= ya - y) ? yb : ya;
-        gc[y] = (short)r;
-    }
+    const int wave = threadIdx.x >> 6;
+    const size_t off = sd.toff + ((size_t)((blockIdx.x - bm[set]) * 4 + wave) << sd.logT);
+    pba_column(smap_all + off, g_all + off, (1 << sd.logT) >> 6, threadIdx.x & 63, masks[wave], prv[wave], nxt[wave]);
 }
 
 // ---- phase 2: proximate-site stacks per (row, band) ------------------------------------
@@ -433,46 +436,179 @@ __global__ __launch_bounds__(64) void k_pba_color(const int *__restrict__ E_all,
 }
 
 // ---- island certificate ------------------------------------------------------------------
-// blocks of 256 pixels (a texture has T*T >= 4096 pixels, a multiple of 256)
+// bad[s]: 0, BAD_SITE (a pixel of s fails the certificate), BAD_REMOVED (taken out of the site map)
+#define BAD_SITE 1
+#define BAD_REMOVED 2
+GA_INLINE void island_fail(int s, int *bad, int *flag)
+{
+    bad[s] = BAD_SITE;
+    *flag = 1;
+}
+
+// Blocks of 1,024 pixels (a texture has T * T >= 4096 pixels, T >= 64), four consecutive rows per
+// thread, so a wave reads whole lines of its own and its neighbour columns; XCD k takes one
+// contiguous eighth of the blocks, whose neighbour columns are then in its own L2.  Bound by the
+// reads of the diagram: 136 us at T = 8192 (2.0 TB/s); one pixel per thread, in launch order, took 226 us,
+// and 1,640 us against 754 us on a batch of 1,024 textures (357M pixels).
 __global__ __launch_bounds__(256) void k_islands(const int *__restrict__ vor_all, const int *__restrict__ pix,
                                                  BatchDev bd, int *__restrict__ bad, int *__restrict__ flag)
 {
+    const unsigned nb = gridDim.x, q8 = nb >> 3;   // the last nb % 8 blocks keep their numbers
+    const unsigned blk = blockIdx.x < 8 * q8 ? (blockIdx.x & 7u) * q8 + (blockIdx.x >> 3) : blockIdx.x;
     const int *bm = bd.bmap(BM_PIX);
-    int set = set_of(bm, bd.nsets, blockIdx.x);
+    int set = set_of(bm, bd.nsets, (int)blk);
     const SetDesc &sd = bd.sets[set];
     int logT = sd.logT;
     int T = 1 << logT;
     const int *vor = vor_all + sd.toff;
-    size_t idx = (size_t)(blockIdx.x - bm[set]) * 256 + threadIdx.x;
-    int x = (int)(idx >> logT), y = (int)(idx & (T - 1));
-    int s = vor[idx];
-    if (s < 0) return;
-    int sp = pix[s];
-    int sx = sp >> 16, sy = sp & 0xffff;
-    int dx = (sx > x) - (sx < x), dy = (sy > y) - (sy < y);
-    if (dx == 0 && dy == 0) return;
-    bool ok = false;
-    if (dx != 0 && vor[idx + ((long long)dx << logT)] == s) ok = true;
-    if (!ok && dy != 0 && vor[idx + dy] == s) ok = true;
-    if (!ok && dx != 0 && dy != 0 && vor[idx + ((long long)dx << logT) + dy] == s) ok = true;
-    if (!ok) {
-        bad[s] = 1;
-        *flag = 1;
+    size_t idx = (size_t)((int)blk - bm[set]) * 1024 + 4 * threadIdx.x;
+    const int x = (int)(idx >> logT), y0 = (int)(idx & (T - 1));
+    const int4 own = *(const int4 *)(vor + idx);
+    const int lab[4] = {own.x, own.y, own.z, own.w};
+    int sp[4], need = 0;   // need: 1 the left column, 2 the right one
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        sp[j] = lab[j] < 0 ? (x << 16) | (y0 + j) : (j && lab[j] == lab[j - 1] ? sp[j - 1] : pix[lab[j]]);
+        const int sx = sp[j] >> 16;
+        need |= sx < x ? 1 : (sx > x ? 2 : 0);
+    }
+    // (a site lies inside the texture, so the column one step toward it does too)
+    int4 left = make_int4(-1, -1, -1, -1), right = left;
+    if (need & 1) left = *(const int4 *)(vor + idx - T);
+    if (need & 2) right = *(const int4 *)(vor + idx + T);
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const int s = lab[j], sx = sp[j] >> 16, sy = sp[j] & 0xffff, y = y0 + j;
+        const int dx = (sx > x) - (sx < x), dy = (sy > y) - (sy < y);
+        if (dx == 0 && dy == 0) continue;
+        const int lj = j == 0 ? left.x : (j == 1 ? left.y : (j == 2 ? left.z : left.w));
+        const int rj = j == 0 ? right.x : (j == 1 ? right.y : (j == 2 ? right.z : right.w));
+        bool ok = dx != 0 && (dx < 0 ? lj : rj) == s;
+        if (!ok && dy != 0) {
+            const int k = j + dy;
+            const int v = k < 0 || k > 3 ? vor[idx + k] : (k == 0 ? own.x : (k == 1 ? own.y : (k == 2 ? own.z : own.w)));
+            ok = v == s;
+        }
+        if (!ok && dx != 0 && dy != 0) ok = vor[idx + j + dy + ((long long)dx << logT)] == s;
+        if (!ok) island_fail(s, bad, flag);
     }
 }
 
-// Take sites flagged by the certificate out of the site map (counted in *removed).
+// Takes the sites flagged by the certificate out of the site map, and lists them (count in *removed).
 __global__ void k_remove_bad(int *__restrict__ bad, const int *__restrict__ pix, BatchDev bd,
-                             int *__restrict__ smap, int *__restrict__ removed)
+                             int *__restrict__ smap, int *__restrict__ removed, int *__restrict__ rlist,
+                             int *__restrict__ setbad)
 {
     int s = blockIdx.x * blockDim.x + threadIdx.x;
-    bool r = s < bd.ntot && bad[s];
-    wave_count_full(removed, r ? 1 : 0);
+    bool r = s < bd.ntot && bad[s] == BAD_SITE;
+    const int k = wave_reserve(removed, r);
     if (!r) return;
-    bad[s] = 0;
-    const SetDesc &sd = bd.sets[bd.vset[s]];
+    bad[s] = BAD_REMOVED;
+    rlist[k] = s;
+    const int set = bd.vset[s];
+    setbad[set] = 1;
+    const SetDesc &sd = bd.sets[set];
     int sp = pix[s];
     smap[sd.toff + ((size_t)(sp >> 16) << sd.logT) + (sp & 0xffff)] = PBA_EMPTY;
+}
+
+// phase 1 again for the columns of the removed sites [first, *removed) (one wave per block)
+__global__ __launch_bounds__(64) void k_repair_cols(const int *__restrict__ rlist, int first,
+                                                    const int *__restrict__ removed, const int *__restrict__ pix,
+                                                    BatchDev bd, const int *__restrict__ smap_all,
+                                                    short *__restrict__ g_all)
+{
+    __shared__ unsigned long long masks[256];
+    __shared__ short prv[256], nxt[256];
+    const int n = *removed;
+    for (int k = first + blockIdx.x; k < n; k += gridDim.x) {
+        const int s = rlist[k];
+        const SetDesc &sd = bd.sets[bd.vset[s]];
+        const size_t off = sd.toff + ((size_t)(pix[s] >> 16) << sd.logT);
+        pba_column(smap_all + off, g_all + off, (1 << sd.logT) >> 6, threadIdx.x, masks, prv, nxt);
+        __syncthreads();
+    }
+}
+
+// The pixels of removed sites get the nearest site that is left, from the column field: columns at
+// growing distance k on both sides while k * k can still win, with phase 3's ties (lower column).
+// A wave holds 64 rows of one column, so its column reads are whole lines; four distances are in
+// flight.  A repair takes 0.15 ms at T = 2048 and 0.3 ms at T = 8192, where a whole second diagram took
+// 0.4 and 2.2 ms, and a batch of 1,024 sets (10-20% of them repaired, three times) 1.5 instead of 17 ms.
+// Only these pixels need the certificate again (any other keeps its label, and the
+// neighbour that certified it had the same one): they are listed.  Blocks of 1,024 pixels; sets
+// without a removed site return at once.
+__global__ __launch_bounds__(256) void k_relabel(int *__restrict__ vor_all, const short *__restrict__ g_all,
+                                                 const int *__restrict__ smap_all, const int *__restrict__ bad,
+                                                 const int *__restrict__ setbad, BatchDev bd,
+                                                 unsigned *__restrict__ changed, int *__restrict__ chset,
+                                                 int *__restrict__ nchanged)
+{
+    const int *bm = bd.bmap(BM_PIX);
+    int set = set_of(bm, bd.nsets, blockIdx.x);
+    if (!setbad[set]) return;
+    const SetDesc &sd = bd.sets[set];
+    const int logT = sd.logT, T = 1 << logT;
+    int *vor = vor_all + sd.toff;
+    const short *g = g_all + sd.toff;
+    const int *smap = smap_all + sd.toff;
+    for (int q = 0; q < 4; q++) {
+        const size_t idx = (size_t)(blockIdx.x - bm[set]) * 1024 + q * 256 + threadIdx.x;
+        const int s = vor[idx];
+        const bool act = s >= 0 && bad[s] == BAD_REMOVED;
+        if (!__any(act)) continue;
+        const int x = (int)(idx >> logT), y = (int)(idx & (T - 1));
+        long long best = act ? 0x7fffffffffffffffll : -1;
+        int bx = -1, by = 0;
+        for (int k = 0; k < T && __any((long long)k * k <= best); k += 4) {
+            short gl[4], gr[4];
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                gl[u] = x - k - u >= 0 ? g[((size_t)(x - k - u) << logT) + y] : (short)-1;
+                gr[u] = x + k + u < T ? g[((size_t)(x + k + u) << logT) + y] : (short)-1;
+            }
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                const long long kk = (long long)(k + u) * (k + u);
+                if (gl[u] >= 0) {
+                    const long long d = kk + (long long)(gl[u] - y) * (gl[u] - y);
+                    if (d <= best) { best = d; bx = x - k - u; by = gl[u]; }
+                }
+                if (gr[u] >= 0) {
+                    const long long d = kk + (long long)(gr[u] - y) * (gr[u] - y);
+                    if (d < best) { best = d; bx = x + k + u; by = gr[u]; }
+                }
+            }
+        }
+        const int c = wave_reserve(nchanged, act);
+        if (!act) continue;
+        vor[idx] = bx < 0 ? -1 : smap[((size_t)bx << logT) + by];
+        changed[c] = (unsigned)idx;
+        chset[c] = set;
+    }
+}
+
+// the certificate of the relabelled pixels (set and pixel of each)
+__global__ void k_recheck(const int *__restrict__ vor_all, const int *__restrict__ pix, BatchDev bd,
+                          const unsigned *__restrict__ changed, const int *__restrict__ chset,
+                          const int *__restrict__ nchanged, int *__restrict__ bad, int *__restrict__ flag)
+{
+    const int n = *nchanged;
+    for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < n; c += gridDim.x * blockDim.x) {
+        const SetDesc &sd = bd.sets[chset[c]];
+        const size_t idx = changed[c];
+        const int logT = sd.logT, T = 1 << logT;
+        const int *vor = vor_all + sd.toff;
+        const int s = vor[idx];
+        if (s < 0) continue;
+        const int x = (int)(idx >> logT), y = (int)(idx & (T - 1)), sp = pix[s], sx = sp >> 16, sy = sp & 0xffff;
+        const int dx = (sx > x) - (sx < x), dy = (sy > y) - (sy < y);
+        if (dx == 0 && dy == 0) continue;
+        bool ok = dx != 0 && vor[idx + ((long long)dx << logT)] == s;
+        if (!ok && dy != 0) ok = vor[idx + dy] == s;
+        if (!ok && dx != 0 && dy != 0) ok = vor[idx + ((long long)dx << logT) + dy] == s;
+        if (!ok) island_fail(s, bad, flag);
+    }
 }
 
 // ---- host-side launchers ---------------------------------------------------------------
@@ -531,8 +667,26 @@ void launch_islands(const int *vor, const int *pix, const BatchDev &b, int *bad,
     GA_LAUNCH(k_islands, dim3(b.blocks[BM_PIX]), dim3(256), 0, st, vor, pix, b, bad, flag);
 }
 
-void launch_remove_bad(int *bad, const int *pix, const BatchDev &b, int *smap, int *removed, hipStream_t st)
+// removes the flagged sites (listed in rlist from position `first`, the number removed before) and
+// repairs the diagram around them, then checks the pixels that changed; zeroes *flag and *nchanged
+void launch_island_repair(const PbaBuffers &p, const BatchDev &b, int *bad, const int *pix, int *removed, int first,
+                          int *rlist, int *nchanged, int *flag, hipStream_t st)
 {
-    if (b.ntot > 0)
-        GA_LAUNCH(k_remove_bad, dim3((b.ntot + 255) / 256), dim3(256), 0, st, bad, pix, b, smap, removed);
+    // free after phase 3: the band ends, stacks and envelopes (every texture has 64 T band ends and T * T
+    // entries of the others)
+    int *setbad = p.cnt, *chset = p.E;
+    unsigned *changed = (unsigned *)p.S;
+    if (b.ntot <= 0) return;
+    IntFills f;
+    f.add(setbad, (size_t)b.nsets, 0);
+    f.add(nchanged, 1, 0);
+    f.add(flag, 1, 0);
+    launch_fill_multi(f, st);
+    GA_LAUNCH(k_remove_bad, dim3((b.ntot + 255) / 256), dim3(256), 0, st, bad, pix, b, p.smap, removed, rlist, setbad);
+    GA_LAUNCH(k_repair_cols, dim3(1024), dim3(64), 0, st, (const int *)rlist, first, (const int *)removed, pix, b,
+              (const int *)p.smap, p.g);
+    GA_LAUNCH(k_relabel, dim3(b.blocks[BM_PIX]), dim3(256), 0, st, p.vor, (const short *)p.g, (const int *)p.smap,
+              (const int *)bad, (const int *)setbad, b, changed, chset, nchanged);
+    GA_LAUNCH(k_recheck, dim3(1024), dim3(256), 0, st, (const int *)p.vor, pix, b, (const unsigned *)changed,
+              (const int *)chset, (const int *)nchanged, bad, flag);
 }
