@@ -42,9 +42,9 @@ ALGO_BYTES = {
         "gather_model": "156 B per listed triangle (list entry 4, vertices + links 32, three neighbour "
                         "stamps and far vertices 24, six positions 96)",
         "gather_bytes": lambda st, T, n: 156.0 * (st["flipListed"] - st["flipTailListed"])},
-    "k_pba_color": {
-        "model": "8 B per pixel (envelope read 4 + label written 4)",
-        "bytes": lambda st, T, n: 8.0 * T * T},
+    "k_pba_label": {
+        "model": "6 B per pixel (column field read 2 + label written 4)",
+        "bytes": lambda st, T, n: 6.0 * T * T},
 }
 
 

@@ -101,9 +101,9 @@ struct galpha_ctx {
     hipStream_t stream = nullptr;
     std::string err;
     // PBA
-    DevBuf smap, g, S, cnt, E, ecnt, vor, bad, fpix;
+    DevBuf smap, g, hmin, far, setfar, vor, bad, fpix;
+    DevBuf chg, chgset;   // island repair: relabelled pixels and their sets
     // mesh
-    DevBuf plo;   // phase-2 band range starts
     DevBuf perm, xys, pcell, ccount, ccursor;   // spatial numbering of the real points
     DevBuf cls;                                  // alpha-complex classes (host queries)
     DevBuf tv, tn, remap, stamp, claim, modA, modB, cand, pos, vt, vstate, pix, deg, off, fill, fan,
@@ -527,10 +527,9 @@ struct BatchPlan {
     std::vector<SetDesc> sets;
     std::vector<int> bm;              // BM_COUNT x (nsets + 1)
     int blocks[BM_COUNT] = {0};
-    int max_m2 = 1;                   // largest phase-2 band count
     int ncells = 0;                   // 16 x 16-pixel cells of all textures
     std::vector<int> fpix;            // frame pixels of all sets, in set order
-    int ntot = 0, V = 0, sumT = 0;
+    int ntot = 0, V = 0, maxT = 0, far_rows = 2, far_lds = 0;
     size_t P = 0;
     int nsets() const { return (int)sets.size(); }
 };
@@ -540,7 +539,7 @@ static BatchPlan plan_batch(const int *n, const int *T, const double *bb5, int n
 {
     BatchPlan b;
     b.sets.resize(nsets);
-    long long poff = 0, nftot = 0, roff = 0;
+    long long poff = 0, nftot = 0;
     size_t toff = 0;
     std::vector<int> nfs(nsets);
     for (int s = 0; s < nsets; s++) {
@@ -554,26 +553,27 @@ static BatchPlan plan_batch(const int *n, const int *T, const double *bb5, int n
         d.n = n[s];
         d.poff = (int)poff;
         d.nf = (int)fp.size();
-        d.roff = (int)roff;
-        // bands per row: 64 columns each, at most 64 (T / 64 is a power of two)
-        d.m2 = d.m3 = std::max(1, std::min(64, T[s] / 64));
         d.coff = b.ncells;
         b.ncells += (T[s] / 16) * (T[s] / 16);
-        b.max_m2 = std::max(b.max_m2, d.m2);
         d.margin = margin_for(T[s]);
         d.shx = sg.shx; d.shy = sg.shy; d.scale = sg.scale; d.inv = sg.inv;
         nfs[s] = d.nf;
         b.fpix.insert(b.fpix.end(), fp.begin(), fp.end());
         poff += n[s];
         nftot += d.nf;
-        roff += T[s];
         toff += (size_t)T[s] * T[s];
     }
     check_slot_capacity(poff + nftot);
     b.ntot = (int)poff;
     b.V = (int)(poff + nftot);
-    b.sumT = (int)roff;
     b.P = toff;
+    // two blocks of k_pba_far_rows per CU: fewer rows per block when the textures are few and small
+    long long sumT = 0;
+    for (int s = 0; s < nsets; s++) {
+        b.maxT = std::max(b.maxT, T[s]);
+        sumT += T[s];
+    }
+    while (b.far_rows < 16 && sumT / (2 * b.far_rows) >= 512) b.far_rows *= 2;
     long long fb = poff;
     for (int s = 0; s < nsets; s++) { b.sets[s].fbase = (int)fb; fb += nfs[s]; }
     b.bm.assign((size_t)BM_COUNT * (nsets + 1), 0);
@@ -584,11 +584,12 @@ static BatchPlan plan_batch(const int *n, const int *T, const double *bb5, int n
             b.bm[(size_t)k * (nsets + 1) + s] = (int)acc[k];
         }
         if (s == nsets) break;
-        long long Ts = T[s], m = std::max(1, std::min(64, T[s] / 64));
+        long long Ts = T[s];
         acc[BM_COLS] += Ts / 4;
-        acc[BM_STACK] += (Ts / 64) * m;
-        acc[BM_MERGE] += (Ts / 64) * std::max(1LL, m / 2);
-        acc[BM_COLOR] += (Ts / 64) * m;
+        acc[BM_LABEL] += (Ts / 64) * (Ts / 64);
+        const int rb = pba_far_rows(log2i(T[s]), b.far_rows);
+        if (rb) acc[BM_ROWS] += Ts / rb;
+        b.far_lds = std::max(b.far_lds, pba_far_lds(T[s], rb));
         acc[BM_PIX] += Ts * Ts / 1024;
         acc[BM_RECON] += (Ts / 16) * (Ts / 16);   // one tile per 16 x 16-pixel cell
     }
@@ -601,11 +602,9 @@ static void ensure_pba(galpha_ctx *c, const BatchPlan &b)
     size_t P = b.P;
     c->smap.ensure(4 * P);
     c->g.ensure(2 * P);
-    c->S.ensure(4 * P);
-    c->cnt.ensure(4 * (size_t)64 * b.sumT);
-    c->plo.ensure(4 * (size_t)64 * b.sumT);
-    c->E.ensure(4 * P);
-    c->ecnt.ensure(4 * (size_t)b.sumT);
+    c->hmin.ensure(P / 8);
+    c->far.ensure(P / 256);
+    c->setfar.ensure(4 * (size_t)b.nsets() + 16);
     c->vor.ensure(4 * P);
     c->bad.ensure(4 * (size_t)(b.V + 1));
     c->fpix.ensure(4 * (size_t)(b.V - b.ntot + 1));
@@ -639,7 +638,9 @@ static BatchDev upload_plan(galpha_ctx *c, const BatchPlan &b)
     d.vset = c->vset.as<int>();
     d.ntot = b.ntot;
     d.V = b.V;
-    d.max_m2 = b.max_m2;
+    d.maxT = b.maxT;
+    d.far_rows = b.far_rows;
+    d.far_lds = b.far_lds;
     d.P = b.P;
     return d;
 }
@@ -657,22 +658,26 @@ static void run_pba(galpha_ctx *c, const double *d_xy, const BatchDev &bd, int *
         f.add(c->bad.p, (size_t)bd.V + 1, 0);
         f.add(c->counters.as<int>() + C_ISLAND_SITES, 1, 0);
         f.add(c->counters.as<int>() + C_FLAG, 1, 0);
+        f.add(c->setfar.p, (size_t)bd.nsets, 0);
+        f.add(c->far.p, 4 * (size_t)bd.blocks[BM_LABEL], 0);
         launch_fill_multi(f, st);
     }
-    PbaBuffers b{c->smap.as<int>(), c->g.as<short>(), c->S.as<int>(), c->cnt.as<int>(), c->plo.as<int>(),
-                 c->E.as<int>(), c->ecnt.as<int>(), c->vor.as<int>()};
+    PbaBuffers b{c->smap.as<int>(), c->g.as<short>(), c->hmin.as<short>(), c->far.as<int>(), c->setfar.as<int>(),
+                 c->vor.as<int>()};
     int it = 0, isl = 0;
     int *cnt = c->counters.as<int>();
-    c->mlist.ensure(4 * (size_t)bd.ntot);   // (free until the shifting: the removed sites)
-    launch_pba(b, bd, st);
+    launch_pba(b, c->pix.as<int>(), bd, st);
     launch_islands(c->vor.as<int>(), c->pix.as<int>(), bd, c->bad.as<int>(), cnt + C_FLAG, st);
     for (; it < 16; it++) {
         int cv[C_ISLAND_SITES + 1];   // the flag and the island count in one read
         ctx_counters_read(c, cv, 0, C_ISLAND_SITES + 1);
         isl = cv[C_ISLAND_SITES];
         if (cv[C_FLAG] == 0) break;
+        c->mlist.ensure(4 * (size_t)bd.ntot);   // (free until the shifting: the removed sites)
+        c->chg.ensure(4 * bd.P);
+        c->chgset.ensure(4 * bd.P);
         launch_island_repair(b, bd, c->bad.as<int>(), c->pix.as<int>(), cnt + C_ISLAND_SITES, isl, c->mlist.as<int>(),
-                             cnt + C_CHANGED, cnt + C_FLAG, st);
+                             c->chg.as<unsigned>(), c->chgset.as<int>(), cnt + C_CHANGED, cnt + C_FLAG, st);
     }
     if (it == 16) throw GalphaError("discrete Voronoi diagram did not settle (island certificate)");
     *iters = it + 1;
@@ -1368,14 +1373,14 @@ galpha_ctx *galphaCreate(int device)
 
 static void release_all(galpha_ctx *c)
 {
-    DevBuf *bufs[] = {&c->smap, &c->g, &c->S, &c->cnt, &c->E, &c->ecnt, &c->vor, &c->bad, &c->fpix, &c->tv,
+    DevBuf *bufs[] = {&c->smap, &c->g, &c->hmin, &c->far, &c->setfar, &c->chg, &c->chgset, &c->vor, &c->bad, &c->fpix, &c->tv,
                       &c->tn, &c->remap, &c->stamp, &c->claim, &c->modA, &c->modB, &c->cand, &c->pos, &c->vt,
                       &c->vstate, &c->pix, &c->deg, &c->off, &c->fill, &c->fan, &c->moved, &c->decide, &c->mx,
                       &c->mlist, &c->loc, &c->lt, &c->scratch, &c->keys, &c->keys2,
                       &c->vals, &c->vals2, &c->rot, &c->newid, &c->out9, &c->counters, &c->status, &c->xy,
                       &c->scanTmp, &c->sortTmp, &c->tileCnt, &c->tileOff, &c->dellist, &c->dbg,
                       &c->setsD, &c->bmD, &c->vset, &c->setFirst,
-                      &c->offsD, &c->bboxTmp, &c->lmark, &c->plo,
+                      &c->offsD, &c->bboxTmp, &c->lmark,
                       &c->perm, &c->xys, &c->pcell, &c->ccount, &c->ccursor, &c->cls,
                       &c->kin, &c->kv, &c->kinv, &c->kdone, &c->kcnt, &c->krs, &c->kroff, &c->kwork, &c->khash, &c->rdbuf};
     for (DevBuf *b : bufs) b->release();
@@ -1387,14 +1392,14 @@ static void release_all(galpha_ctx *c)
 // device bytes held by a context (all grown buffers)
 size_t galpha_ctx_device_bytes(galpha_ctx *c)
 {
-    DevBuf *bufs[] = {&c->smap, &c->g, &c->S, &c->cnt, &c->E, &c->ecnt, &c->vor, &c->bad, &c->fpix, &c->tv,
+    DevBuf *bufs[] = {&c->smap, &c->g, &c->hmin, &c->far, &c->setfar, &c->chg, &c->chgset, &c->vor, &c->bad, &c->fpix, &c->tv,
                       &c->tn, &c->remap, &c->stamp, &c->claim, &c->modA, &c->modB, &c->cand, &c->pos, &c->vt,
                       &c->vstate, &c->pix, &c->deg, &c->off, &c->fill, &c->fan, &c->moved, &c->decide, &c->mx,
                       &c->mlist, &c->loc, &c->lt, &c->scratch, &c->keys, &c->keys2,
                       &c->vals, &c->vals2, &c->rot, &c->newid, &c->out9, &c->counters, &c->status, &c->xy,
                       &c->scanTmp, &c->sortTmp, &c->tileCnt, &c->tileOff, &c->dellist, &c->dbg,
                       &c->setsD, &c->bmD, &c->vset, &c->setFirst,
-                      &c->offsD, &c->bboxTmp, &c->lmark, &c->plo,
+                      &c->offsD, &c->bboxTmp, &c->lmark,
                       &c->perm, &c->xys, &c->pcell, &c->ccount, &c->ccursor, &c->cls,
                       &c->kin, &c->kv, &c->kinv, &c->kdone, &c->kcnt, &c->krs, &c->kroff, &c->kwork, &c->khash, &c->rdbuf};
     size_t t = 0;

@@ -25,8 +25,6 @@ struct SetDesc {
     int logT;            // texture side T = 1 << logT
     int n, poff;         // real points and the global id of the first one
     int nf, fbase;       // frame vertices and the global id of the first one
-    int roff;            // sum of the texture sides of the previous sets (row / column arrays)
-    int m2, m3;          // PBA bands for phases 2 and 3
     int coff;            // first 16 x 16-pixel cell of the set (spatial numbering of the points)
     int margin;
     double shx, shy, scale, inv;   // snap grid: snapped = sh + (pixel - margin) * scale
@@ -45,7 +43,17 @@ GA_INLINE_HOST_DEVICE int set_of(const int *start, int nsets, int b)
 }
 
 // per-launch block maps (device arrays of nsets + 1 entries each)
-enum { BM_COLS, BM_STACK, BM_MERGE, BM_COLOR, BM_PIX, BM_RECON, BM_COUNT };
+enum { BM_COLS, BM_LABEL, BM_ROWS, BM_PIX, BM_RECON, BM_COUNT };
+// rows of a block of k_pba_far_rows for a texture of side 1 << logT (0 above 4096, see pba.hip); want: rows
+// for blocks enough to fill the chip
+GA_INLINE_HOST_DEVICE int pba_far_rows(int logT, int want)
+{
+    if (logT > 12) return 0;
+    const int lo = logT < 10 ? 1 << (10 - logT) : 1, hi = logT > 10 ? 1 << (14 - logT) : 16;
+    return want < lo ? lo : (want > hi ? hi : want);
+}
+// LDS bytes of its block
+inline int pba_far_lds(int T, int rows) { return 2 * T * rows * 133 / 64; }
 struct BatchDev {
     const SetDesc *sets;   // [nsets]
     int nsets;
@@ -53,7 +61,9 @@ struct BatchDev {
     int blocks[BM_COUNT];  // total blocks per map (host copy of bm[k][nsets])
     const int *vset;       // [V] set of every vertex
     int ntot, V;           // real points, all vertices
-    int max_m2;            // largest phase-2 band count of the sets
+    int maxT;              // largest texture side
+    int far_rows;          // rows wanted per block of k_pba_far_rows
+    int far_lds;           // its largest LDS size
     size_t P;              // pixels of all textures
     GA_INLINE_HOST_DEVICE const int *bmap(int k) const { return bm + (size_t)k * (nsets + 1); }
 };
@@ -61,11 +71,9 @@ struct BatchDev {
 struct PbaBuffers {
     int *smap;     // T*T site id per pixel (0x7fffffff = empty)
     short *g;      // T*T nearest-site row per column
-    int *S;        // T*T band stacks
-    int *cnt;      // 64*T per set: end (hi) of each band's envelope range
-    int *lo;       // 64*T per set: start (lo) of each band's envelope range
-    int *E;        // T*T compacted envelopes
-    int *ecnt;     // T envelope sizes
+    short *hmin;   // T*T/16 smallest row distance of 16 columns
+    int *far;      // T*T/1024 tile parts with far pixels
+    int *setfar;   // [nsets] sets with far pixels (zero on entry)
     int *vor;      // T*T nearest site id
 };
 
@@ -201,11 +209,11 @@ void launch_splat(const double2 *xy, const BatchDev &b, const int *perm, int *sm
 // ccount (ncells + 1 ints) zero on entry
 void launch_renumber(const double2 *xy, const BatchDev &b, int *cell, int *ccount, int *cursor, int ncells,
                      void *scan_tmp, int *perm, double2 *xys, hipStream_t st);
-void launch_pba(const PbaBuffers &p, const BatchDev &b, hipStream_t st);
+void launch_pba(const PbaBuffers &p, const int *pix, const BatchDev &b, hipStream_t st);
 void launch_islands(const int *vor, const int *pix, const BatchDev &b, int *bad, int *flag, hipStream_t st);
 // repairs the diagram around the sites that the certificate flagged (see pba.hip)
 void launch_island_repair(const PbaBuffers &p, const BatchDev &b, int *bad, const int *pix, int *removed, int first,
-                          int *rlist, int *nchanged, int *flag, hipStream_t st);
+                          int *rlist, unsigned *changed, int *chset, int *nchanged, int *flag, hipStream_t st);
 
 // util.hip: up to four segments of device ints copied into one contiguous device array
 struct IntSegments {

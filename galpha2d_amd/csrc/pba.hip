@@ -8,11 +8,8 @@
 //   * phase 1 (nearest site in each column) is one wave per column: a 64-bit ballot per
 //     64-row chunk marks the sites, and the nearest site above/below each pixel comes from
 //     bit scans over those masks held in LDS -- the site map is read once;
-//   * phase 2 builds per-(row, band) stacks of proximate sites with lanes = rows, stored as
-//     arrays (no pointer chasing), integer-exact dominance tests;
-//   * phase 2b merges band stacks per row and compacts the envelope contiguously;
-//   * phase 3 colours pixels with lanes = rows, binary-searching the start element of its
-//     pixel band in the compacted envelope.
+//   * phases 2 and 3 are one search of the column field outward from every pixel, in LDS
+//     tiles; only pixels far from every site take a second kernel (see there).
 // All distances are exact integers; every pixel receives a site at minimal Euclidean
 // distance (ties go to the lower column, then the lower row).
 //
@@ -219,220 +216,381 @@ __global__ __launch_bounds__(256) void k_pba_cols(const int *__restrict__ smap_a
     pba_column(smap_all + off, g_all + off, (1 << sd.logT) >> 6, threadIdx.x & 63, masks[wave], prv[wave], nxt[wave]);
 }
 
-// ---- phase 2: proximate-site stacks per (row, band) ------------------------------------
-#define PBA_MAXB 64   // bands per texture row at most (m2, m3 <= 64)
-GA_INLINE int pk(int x, int h) { return (x << 16) | (h & 0xffff); }
-GA_INLINE int pk_x(int e) { return (int)((unsigned)e >> 16); }
-GA_INLINE int pk_h(int e) { return (int)(short)(e & 0xffff); }
+// ---- phases 2 and 3: nearest site per pixel ---------------------------------------------
+// The nearest site of pixel (x, y) lies in column x +- k with k * k no larger than the best squared
+// distance so far, so the columns are searched outward from x.  With 16 pixels and more per point
+// that ends after a few columns: k_pba_label holds the squared row distances of a 64 x 64-pixel tile
+// and 16 columns on either side in LDS and finds nearly every label of an evenly filled texture
+// there, in one pass.  Pixels that are further from every site (the empty space between
+// clusters) are left to the far kernels, which skip 16 and 64 columns at a time by their smallest
+// row distance.  k_pba_label is bound by its LDS reads, the far kernels by their instructions; a
+// stack of each row's envelope (a band of 64 columns per thread, then pairwise merges, compaction
+// and a colouring pass) is one serial chain per row and took, at T = 4096 (1M uniform points), 284 us
+// against 47; at T = 8192 (4M) 1,344 against 332; at T = 2048 with 8 clusters (mostly far pixels)
+// 259 against 99.
+#define LAB_R 16                     // columns searched on either side in the tile
+#define LAB_W (64 + 2 * LAB_R)
+#define LAB_EMPTY 0x3fffffff         // above every squared distance
+#define LAB_FAR (-2)                 // label of a pixel left to the far kernels
+#define FAR_ROWS_T 4096              // largest texture side of k_pba_far_rows
+#define FAR_EMPTY 12000              // its row offset of an empty column: the square is above FAR_NONE, and 16 times
+                                     // a squared distance with it is below 2^32
+#define FAR_NONE 100000000           // above the squared distances of textures up to FAR_ROWS_T
 
-// b is dominated by a (left) and c (right): the a|b bisector is not left of the b|c one
-GA_INLINE bool dominated(int a, int b, int c)
+GA_INLINE int site_at(const int *smap, const short *g, int logT, int x, int y)
 {
-    long long xa = pk_x(a), ha = pk_h(a), xb = pk_x(b), hb = pk_h(b), xc = pk_x(c), hc = pk_h(c);
-    long long fa = xa * xa + ha * ha, fb = xb * xb + hb * hb, fc = xc * xc + hc * hc;
-    return (fb - fa) * (xc - xb) >= (fc - fb) * (xb - xa);
+    const size_t c = (size_t)x << logT;
+    return smap[c + g[c + y]];
 }
 
-// grid (T/64, m2), block 64: lanes are rows.  Stack entries of band b live in
-// S[(b*Wb + k) * T + y], k < hi[b*T + y]; lo[b*T + y] = 0 (the merge steps move both ends).
-// The column reads of a band do not depend on the stack, so they are issued 8 at a time ahead
-// of the dominance tests.
-__global__ __launch_bounds__(64) void k_pba_stack(const short *__restrict__ g_all, int *__restrict__ S_all,
-                                                  int *__restrict__ hi_all, int *__restrict__ lo_all, BatchDev bd)
+// One 64 x 64-pixel tile per block.  A lane takes two neighbouring rows of a column: both keys of a
+// candidate are one LDS word, 64 * (squared distance) + 16 + (its column - x), so that the smaller key is the
+// nearer site and, in ties, the lower column, and two rows take a packed add and a packed minimum
+// (with a separate distance and column per row the compares and selects bound it: 1,510 us in a
+// batch of 1,024 sets, 268M pixels, against 954).  far[4 * tile + k] tells whether pixels of columns 16 k ..
+// 16 k + 15 are left, setfar[set] whether any of the set's are (both zero on entry).  16 waves
+// when there are fewer than 1,024 tiles (T = 512: 64 tiles, 23 us with 4 waves, 10 with 16), else 4, whose
+// longer runs of columns share more of the site reads.
+typedef unsigned short us2 __attribute__((ext_vector_type(2)));
+
+template <int W>
+__global__ __launch_bounds__(64 * W) void k_pba_label(const short *__restrict__ g_all, const int *__restrict__ smap_all,
+                                                      int *__restrict__ vor_all, int *__restrict__ far,
+                                                      int *__restrict__ setfar, BatchDev bd)
 {
-    const int *bm = bd.bmap(BM_STACK);
-    int set = set_of(bm, bd.nsets, blockIdx.x);
+    __shared__ int4 s_q[LAB_W * 8];
+    us2 *s_d = (us2 *)s_q;   // [LAB_W][32] row pairs: 64 * dy^2, 0x7fff above LAB_R and in empty columns
+    const int *bm = bd.bmap(BM_LABEL);
+    const int set = set_of(bm, bd.nsets, blockIdx.x);
     const SetDesc &sd = bd.sets[set];
-    int logT = sd.logT;
-    int T = 1 << logT, nbx = T >> 6, Wb = T / sd.m2;
-    int lb = blockIdx.x - bm[set];
+    const int logT = sd.logT, T = 1 << logT, nb = T >> 6;
+    const int lb = blockIdx.x - bm[set], x0 = (lb / nb) * 64, y0 = (lb % nb) * 64;
     const short *g = g_all + sd.toff;
-    int *S = S_all + sd.toff;
-    size_t roff = (size_t)PBA_MAXB * sd.roff;
-    int y = (lb % nbx) * 64 + threadIdx.x;
-    int b = lb / nbx;
-    int x0 = b * Wb;
-    int top = 0, e0 = 0, e1 = 0;
-    for (int xb = x0; xb < x0 + Wb; xb += 8) {
-        short gv[8];
-#pragma unroll
-        for (int u = 0; u < 8; u++) gv[u] = xb + u < x0 + Wb ? g[((size_t)(xb + u) << logT) + y] : (short)-1;
-#pragma unroll
-        for (int u = 0; u < 8; u++) {
-            int gy = gv[u];
-            if (gy < 0) continue;
-            int c = pk(xb + u, gy - y);
-            while (top >= 2 && dominated(e0, e1, c)) {
-                top--;
-                e1 = e0;
-                if (top >= 2) e0 = S[((size_t)(x0 + top - 2) << logT) + y];
-            }
-            S[((size_t)(x0 + top) << logT) + y] = c;
-            top++;
-            e0 = e1;
-            e1 = c;
-        }
-    }
-    hi_all[roff + (size_t)b * T + y] = top;
-    lo_all[roff + (size_t)b * T + y] = 0;
-}
-
-// ---- phase 2b: merge band envelopes pairwise, then compact ------------------------------
-// Step s merges, for every row, the envelope of bands [j*2^s, j*2^s + 2^(s-1)) with that of
-// the next 2^(s-1) bands: the left chain's last element and the right chain's first are
-// popped while the triple at the junction shows one of them dominated (the same exact test
-// as the stacks).  A chain runs through the nonempty [lo, hi) ranges of its bands in order.
-// The lower envelope of a row is unique, so the merge order does not change it.
-// grid (T/64) * (m2/2) blocks of 64 (lanes are rows); blocks whose group does not exist at
-// this step return.
-__global__ __launch_bounds__(64) void k_pba_merge_step(const int *__restrict__ S_all, int *__restrict__ hi_all,
-                                                       int *__restrict__ lo_all, BatchDev bd, int s)
-{
-    const int *bm = bd.bmap(BM_MERGE);
-    int set = set_of(bm, bd.nsets, blockIdx.x);
-    const SetDesc &sd = bd.sets[set];
-    int logT = sd.logT;
-    int T = 1 << logT, nbx = T >> 6, m2 = sd.m2, Wb = T / m2;
-    int gsz = 1 << s, half = gsz >> 1;
-    int lb = blockIdx.x - bm[set];
-    int j = lb / nbx;
-    if ((j + 1) * gsz > m2) return;
-    const int *S = S_all + sd.toff;
-    size_t roff = (size_t)PBA_MAXB * sd.roff;
-    int y = (lb % nbx) * 64 + threadIdx.x;
-    int *HI = hi_all + roff + y, *LO = lo_all + roff + y;   // band b at [b * T]
-#define ELEM(B, I) S[((size_t)((B) * Wb + (I)) << logT) + y]
-    int b0 = j * gsz, bmid = b0 + half, b1 = b0 + gsz;
-    // L: last nonempty band of the left half; R: first nonempty band of the right half
-    int L = bmid - 1;
-    while (L >= b0 && HI[(size_t)L * T] <= LO[(size_t)L * T]) L--;
-    int R = bmid;
-    while (R < b1 && HI[(size_t)R * T] <= LO[(size_t)R * T]) R++;
-    if (L < b0 || R >= b1) return;
-    int Llo = LO[(size_t)L * T], Lhi = HI[(size_t)L * T];
-    int Rlo = LO[(size_t)R * T], Rhi = HI[(size_t)R * T];
-    for (;;) {
-        int l1 = ELEM(L, Lhi - 1), r1 = ELEM(R, Rlo);
-        // element before l1 on the left chain
-        bool has0 = false;
-        int l0 = 0;
-        if (Lhi - 1 > Llo) { l0 = ELEM(L, Lhi - 2); has0 = true; }
-        else {
-            int P = L - 1;
-            while (P >= b0 && HI[(size_t)P * T] <= LO[(size_t)P * T]) P--;
-            if (P >= b0) { l0 = ELEM(P, HI[(size_t)P * T] - 1); has0 = true; }
-        }
-        if (has0 && dominated(l0, l1, r1)) {
-            Lhi--;
-            HI[(size_t)L * T] = Lhi;
-            if (Lhi == Llo) {
-                L--;
-                while (L >= b0 && HI[(size_t)L * T] <= LO[(size_t)L * T]) L--;
-                if (L < b0) break;
-                Llo = LO[(size_t)L * T]; Lhi = HI[(size_t)L * T];
-            }
-            continue;
-        }
-        // element after r1 on the right chain
-        bool has2 = false;
-        int r2 = 0;
-        if (Rlo + 1 < Rhi) { r2 = ELEM(R, Rlo + 1); has2 = true; }
-        else {
-            int Q = R + 1;
-            while (Q < b1 && HI[(size_t)Q * T] <= LO[(size_t)Q * T]) Q++;
-            if (Q < b1) { r2 = ELEM(Q, LO[(size_t)Q * T]); has2 = true; }
-        }
-        if (has2 && dominated(l1, r1, r2)) {
-            Rlo++;
-            LO[(size_t)R * T] = Rlo;
-            if (Rlo == Rhi) {
-                R++;
-                while (R < b1 && HI[(size_t)R * T] <= LO[(size_t)R * T]) R++;
-                if (R >= b1) break;
-                Rlo = LO[(size_t)R * T]; Rhi = HI[(size_t)R * T];
-            }
-            continue;
-        }
-        break;
-    }
-#undef ELEM
-}
-
-// grid (T/64) * m2 blocks of 64 (lanes are rows): band b's [lo, hi) goes to the row's compacted
-// envelope after the ranges of bands 0 .. b-1; the last band writes the envelope size
-__global__ __launch_bounds__(64) void k_pba_compact(const int *__restrict__ S_all, const int *__restrict__ hi_all,
-                                                    const int *__restrict__ lo_all, int *__restrict__ E_all,
-                                                    int *__restrict__ ecnt_all, BatchDev bd)
-{
-    const int *bm = bd.bmap(BM_STACK);
-    int set = set_of(bm, bd.nsets, blockIdx.x);
-    const SetDesc &sd = bd.sets[set];
-    int logT = sd.logT;
-    int T = 1 << logT, nbx = T >> 6, m2 = sd.m2, Wb = T / m2;
-    int lb = blockIdx.x - bm[set];
-    int b = lb / nbx;
-    int y = (lb % nbx) * 64 + threadIdx.x;
-    size_t roff = (size_t)PBA_MAXB * sd.roff;
-    const int *HI = hi_all + roff + y, *LO = lo_all + roff + y;
-    int off = 0;
-    for (int q = 0; q < b; q++) off += HI[(size_t)q * T] - LO[(size_t)q * T];
-    int lo = LO[(size_t)b * T], hi = HI[(size_t)b * T];
-    const int *S = S_all + sd.toff;
-    int *E = E_all + sd.toff;
-    for (int i = lo; i < hi; i++) E[((size_t)(off + i - lo) << logT) + y] = S[((size_t)(b * Wb + i) << logT) + y];
-    if (b == m2 - 1) ecnt_all[sd.roff + y] = off + (hi > lo ? hi - lo : 0);
-}
-
-// ---- phase 3: colour ------------------------------------------------------------------
-GA_INLINE long long fdist(int e, int i)
-{
-    long long dx = i - pk_x(e), h = pk_h(e);
-    return dx * dx + h * h;
-}
-
-// grid (T/64, m3), block 64; vor[x*T + y] = site id
-__global__ __launch_bounds__(64) void k_pba_color(const int *__restrict__ E_all, const int *__restrict__ ecnt_all,
-                                                  const int *__restrict__ smap_all, int *__restrict__ vor_all,
-                                                  BatchDev bd)
-{
-    const int *bm = bd.bmap(BM_COLOR);
-    int set = set_of(bm, bd.nsets, blockIdx.x);
-    const SetDesc &sd = bd.sets[set];
-    int logT = sd.logT;
-    int T = 1 << logT, nbx = T >> 6, Wp = T / sd.m3;
-    int lb = blockIdx.x - bm[set];
-    const int *E = E_all + sd.toff;
-    const int *ecnt = ecnt_all + sd.roff;
     const int *smap = smap_all + sd.toff;
     int *vor = vor_all + sd.toff;
-    int y = (lb % nbx) * 64 + threadIdx.x;
-    int ps = (lb / nbx) * Wp, pe = ps + Wp;
-    int n = ecnt[y];
-    if (n <= 0) {
-        for (int i = ps; i < pe; i++) vor[((size_t)i << logT) + y] = -1;
-        return;
-    }
-#define EL(K) E[((size_t)(K) << logT) + y]
-    int lo = 0, hi = n - 1;
-    while (lo < hi) {
-        int mid = (lo + hi) >> 1;
-        if (fdist(EL(mid + 1), ps) < fdist(EL(mid), ps)) lo = mid + 1;
-        else hi = mid;
-    }
-    int k = lo;
-    int e = EL(k);
-    int en = (k + 1 < n) ? EL(k + 1) : 0;
-    int id = smap[((size_t)pk_x(e) << logT) + (y + pk_h(e))];
-    for (int i = ps; i < pe; i++) {
-        while (k + 1 < n && fdist(en, i) < fdist(e, i)) {
-            k++;
-            e = en;
-            en = (k + 1 < n) ? EL(k + 1) : 0;
-            id = smap[((size_t)pk_x(e) << logT) + (y + pk_h(e))];
+    // 8 rows per thread and step: 16 bytes of one column
+    for (int q = threadIdx.x; q < LAB_W * 8; q += 64 * W) {
+        const int c = q >> 3, r = (q & 7) * 8, x = x0 - LAB_R + c;
+        short v[8];
+        unsigned short o[8];
+        int4 t = {-1, -1, -1, -1};
+        if (x >= 0 && x < T) t = *(const int4 *)(g + ((size_t)x << logT) + y0 + r);
+        __builtin_memcpy(v, &t, 16);
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const int dy = abs(v[i] - (y0 + r + i));
+            o[i] = v[i] >= 0 && dy <= LAB_R ? (unsigned short)(64 * dy * dy) : (unsigned short)0x7fff;
         }
-        vor[((size_t)i << logT) + y] = id;
+        __builtin_memcpy(&t, o, 16);
+        s_q[q] = t;
     }
-#undef EL
+    __syncthreads();
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, y = y0 + 2 * (lane & 31);
+    int pb0 = -1, pb1 = -1, id0 = 0, id1 = 0;    // the columns and sites of the pixels before
+    bool left = false;
+    for (int i = 0; i < 32 / W; i++) {
+        const int xi = (64 / W) * w + (32 / W) * (lane >> 5) + i;
+        const us2 *p = s_d + (LAB_R + xi) * 32 + (lane & 31);
+        us2 best = p[0] + (unsigned short)16;
+#pragma unroll
+        for (int k0 = 1; k0 <= LAB_R; k0 += 4) {
+            if (!__any(max(best.x, best.y) >= 64 * k0 * k0)) break;
+#pragma unroll
+            for (int k = k0; k < k0 + 4; k++) {
+                best = __builtin_elementwise_min(best, p[-32 * k] + (unsigned short)(64 * k * k + 16 - k));
+                best = __builtin_elementwise_min(best, p[32 * k] + (unsigned short)(64 * k * k + 16 + k));
+            }
+        }
+        const bool d0 = best.x < 64 * (LAB_R + 1) * (LAB_R + 1), d1 = best.y < 64 * (LAB_R + 1) * (LAB_R + 1);
+        const int b0 = x0 + xi - 16 + (best.x & 63), b1 = x0 + xi - 16 + (best.y & 63);
+        if (d0 && b0 != pb0) id0 = site_at(smap, g, logT, pb0 = b0, y);
+        if (d1 && b1 != pb1) id1 = site_at(smap, g, logT, pb1 = b1, y + 1);
+        *(int2 *)(vor + ((size_t)(x0 + xi) << logT) + y) = make_int2(d0 ? id0 : LAB_FAR, d1 ? id1 : LAB_FAR);
+        left |= !(d0 && d1);
+    }
+    if (__any(left) && lane == 0) {
+        far[4 * (size_t)blockIdx.x + (64 / W) * w / 16] = 1;
+        setfar[set] = 1;
+    }
+}
+
+// smallest row distance of 16 consecutive columns in every row (0x7fff: no site in them); only for
+// sets with far pixels
+__global__ __launch_bounds__(256) void k_pba_blockmin(const short *__restrict__ g_all, short *__restrict__ hmin_all,
+                                                      const int *__restrict__ setfar, BatchDev bd)
+{
+    const int *bm = bd.bmap(BM_LABEL);
+    const int set = set_of(bm, bd.nsets, blockIdx.x);
+    const SetDesc &sd = bd.sets[set];
+    const int logT = sd.logT, T = 1 << logT, nb = T >> 6;
+    if (!setfar[set] || T <= FAR_ROWS_T) return;
+    const int lb = blockIdx.x - bm[set], xb = (lb / nb) * 4 + (threadIdx.x >> 6), y = (lb % nb) * 64 + (threadIdx.x & 63);
+    const short *g = g_all + sd.toff;
+    int mn = 0x7fff;
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+        const int v = g[((size_t)(16 * xb + i) << logT) + y];
+        if (v >= 0) mn = min(mn, abs(v - y));
+    }
+    hmin_all[(sd.toff >> 4) + ((size_t)xb << logT) + y] = (short)mn;
+}
+
+// The far pixels of textures up to FAR_ROWS_T: one block holds the whole column field of up to 16 rows in
+// LDS (8 at T = 2048, 4 at 4096; fewer where that leaves less than two blocks per CU: a search is a
+// few thousand cycles of one wave, and 16 rows at T = 512 are 32 blocks: 68 us against 23 with 2).
+// Lanes are rows times 4 to 32 neighbouring columns (a group of columns); a wave takes up to 16
+// groups.  The nearest column of a row does not decrease from pixel to pixel (for columns i < j the
+// difference of the squared distances grows with x), so between two known pixels only the columns
+// between theirs can win: each wave's first group comes first, then the middles of ever shorter
+// intervals, and in the wide cells of empty space both ends mostly have the same site and nothing
+// is left to search.  A search goes outward from x and is ruled out by the smallest row distance of
+// 64 columns at a time, then of 16.
+// Without the LDS copy every step of a search is a dependent read of L2: k_pba_far takes 186 us at
+// T = 512 (12,007 points in 8 clusters) and 278 us at T = 2048 (250,001), this 15 and 81 us.
+__global__ __launch_bounds__(1024) void k_pba_far_rows(const short *__restrict__ g_all, const int *__restrict__ smap_all,
+                                                       const int *__restrict__ pix, int *__restrict__ vor_all,
+                                                       const int *__restrict__ far_all,
+                                                       const int *__restrict__ setfar, BatchDev bd)
+{
+    // [T / 4][RB][4] row offset of the column's site (FAR_EMPTY: none); [T][RB] nearest column of the waves'
+    // pixels (-1: not known yet); the smallest magnitude of an offset in 16 columns [T / 16][RB], in 64
+    extern __shared__ int4 s_far4[];
+    short *s_dy = (short *)s_far4;
+    const int *bm = bd.bmap(BM_ROWS);
+    const int set = set_of(bm, bd.nsets, blockIdx.x);
+    if (!setfar[set]) return;
+    const SetDesc &sd = bd.sets[set];
+    const int logT = sd.logT, T = 1 << logT, nb = T >> 6, RB = pba_far_rows(logT, bd.far_rows), lr = __ffs(RB) - 1;
+    const int y0 = (blockIdx.x - bm[set]) << lr, tid = threadIdx.x;
+    // parts of 16 columns with far pixels in the tiles of these rows
+    const int *far = far_all + 4 * (size_t)bd.bmap(BM_LABEL)[set];
+    int any = 0;
+    for (int p = tid; p < (T >> 4); p += 1024) any |= far[4 * ((p >> 2) * nb + (y0 >> 6)) + (p & 3)];
+    if (!__syncthreads_or(any)) return;
+    const short *g = g_all + sd.toff;
+    short *s_mn = s_dy + ((size_t)T << (lr + 1)), *s_m4 = s_mn + ((size_t)(T >> 4) << lr);
+    auto at = [&](int c, int row) { return ((((c >> 2) << lr) + row) << 2) + (c & 3); };
+    // (four reads in flight per thread in this and the next loop)
+    for (int q0 = tid; q0 < (T << lr); q0 += 4096) {
+        short v[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const int q = min(q0 + 1024 * u, (T << lr) - 1);
+            v[u] = g[((size_t)(q >> lr) << logT) + y0 + (q & (RB - 1))];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const int q = q0 + 1024 * u, row = q & (RB - 1);
+            if (q < (T << lr)) s_dy[at(q >> lr, row)] = v[u] < 0 ? (short)FAR_EMPTY : (short)(v[u] - (y0 + row));
+        }
+    }
+    const int *smap = smap_all + sd.toff;
+    int *vor = vor_all + sd.toff;
+    const int lane = tid & 63, w = tid >> 6, r = lane & (RB - 1), y = y0 + r;
+    const int step = 64 >> lr, nG = (T >> 4) / step;   // columns of a group, groups of a wave
+    const int xw = w * (T >> 4) + (lane >> lr);        // the lane's column in group 0
+    short *s_wave = s_dy + ((size_t)T << lr) + (size_t)w * nG * 64, *s_col = s_wave + lane;   // group k at [64 k]
+    unsigned open = 0;   // groups whose pixel is far
+    for (int k0 = 0; k0 < nG; k0 += 4) {
+        int v[4], sp[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) v[u] = vor[((size_t)(xw + min(k0 + u, nG - 1) * step) << logT) + y];
+#pragma unroll
+        for (int u = 0; u < 4; u++) sp[u] = v[u] < 0 ? -1 : pix[v[u]];
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+            if (k0 + u < nG) {
+                s_col[64 * (k0 + u)] = (short)(sp[u] >> 16);
+                open |= (unsigned)(v[u] == LAB_FAR) << (k0 + u);
+            }
+    }
+    __syncthreads();
+    for (int q = tid; q < ((T >> 4) << lr); q += 1024) {
+        int mn = FAR_EMPTY;
+        for (int u = 0; u < 16; u++) mn = min(mn, abs((int)s_dy[at(16 * (q >> lr) + u, q & (RB - 1))]));
+        s_mn[q] = (short)mn;
+    }
+    __syncthreads();
+    for (int q = tid; q < ((T >> 6) << lr); q += 1024) {
+        const int c = ((q >> lr) << (lr + 2)) + (q & (RB - 1));
+        s_m4[q] = min(min(s_mn[c], s_mn[c + RB]), min(s_mn[c + 2 * RB], s_mn[c + 3 * RB]));
+    }
+    __syncthreads();
+    // the nearest column of the pixels of group k among [lo, hi] (lanes with act; lo, hi: nearest
+    // columns of known pixels of the row on either side, or the outermost columns)
+    auto search = [&](int k, int lo, int hi, bool act) {
+        const int x = xw + k * step, X = (w * (T >> 4) + k * step) >> 6;   // (a group lies in 64 columns)
+        int best = -1, bx = -1;
+        if (act) {
+            best = FAR_NONE;
+            const int vl = s_dy[at(lo, r)], vh = s_dy[at(hi, r)];
+            const int el = __mul24(x - lo, x - lo) + __mul24(vl, vl), eh = __mul24(x - hi, x - hi) + __mul24(vh, vh);
+            if (el < best) { best = el; bx = lo; }
+            if (eh < best) { best = eh; bx = hi; }
+        }
+        // 64 columns that can hold a nearer site for some lane; 16 * (squared distance) + column as one
+        // key: the smallest is the nearest of 16 columns, in ties the lower
+        auto visit = [&](int B) {
+            for (int b = 4 * B; b < 4 * B + 4; b++) {
+                const int h = s_mn[(b << lr) + r], d = max(max(16 * b - x, x - (16 * b + 15)), 0);
+                if (!__any(16 * b + 15 >= lo && 16 * b <= hi && __mul24(d, d) + __mul24(h, h) <= best)) continue;
+                const int2 *p = (const int2 *)s_dy + ((4 * b) << lr) + r;
+                const int a = x - 16 * b;
+                int dx2 = __mul24(a, a);
+                unsigned key = ~0u;
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    const int2 t = p[q << lr];
+                    const short v[4] = {(short)t.x, (short)(t.x >> 16), (short)t.y, (short)(t.y >> 16)};
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        const int u = 4 * q + e;
+                        key = min(key, ((unsigned)(v[e] * v[e] + dx2) << 4) + u);
+                        dx2 += 2 * u + 1 - 2 * a;
+                    }
+                }
+                const int dd = (int)(key >> 4), cx = 16 * b + (int)(key & 15);
+                if (dd < best || (dd == best && cx < bx)) { best = dd; bx = cx; }
+            }
+        };
+        if (__any(act && 64 * X + 63 >= lo && 64 * X <= hi)) visit(X);
+        for (int j = 1; j < nb; j++) {
+            const int bl = X - j, br = X + j, dl = x - (64 * bl + 63), dr = 64 * br - x;
+            const bool inl = bl >= 0 && __mul24(dl, dl) <= best && 64 * bl + 63 >= lo;
+            const bool inr = br < nb && __mul24(dr, dr) <= best && 64 * br <= hi;
+            if (!__any(inl || inr)) break;
+            const int hl = inl && 64 * bl <= hi ? s_m4[(bl << lr) + r] : FAR_EMPTY;
+            const int hr = inr && 64 * br + 63 >= lo ? s_m4[(br << lr) + r] : FAR_EMPTY;
+            if (__any(__mul24(dl, dl) + __mul24(hl, hl) <= best)) visit(bl);
+            if (__any(__mul24(dr, dr) + __mul24(hr, hr) <= best)) visit(br);
+        }
+        if (act) s_col[64 * k] = (short)bx;
+    };
+    {
+        const bool act = s_col[0] < 0;
+        if (__any(act)) search(0, 0, T - 1, act);
+    }
+    __syncthreads();
+    if (!__any(open)) return;
+    const int end = w < 15 ? s_wave[nG * 64 + r] : T - 1;   // nearest column of the next wave's first pixel
+    for (int s = nG >> 1; s; s >>= 1)
+        for (int k = s; k < nG; k += 2 * s) {
+            const int lo = s_col[64 * (k - s)], hi = k + s < nG ? s_col[64 * (k + s)] : end;
+            const bool mine = s_col[64 * k] < 0;
+            if (mine && lo == hi) s_col[64 * k] = (short)lo;
+            const bool act = mine && lo != hi;
+            if (__any(act)) search(k, lo, hi, act);
+        }
+#pragma unroll 4
+    for (int k = 0; k < nG; k++) {
+        const int c = s_col[64 * k];
+        if ((open >> k) & 1)
+            vor[((size_t)(xw + k * step) << logT) + y] = smap[((size_t)c << logT) + y + s_dy[at(c, r)]];
+    }
+}
+
+// The far pixels of larger textures, by tiles (64 x 64 pixels per block, lanes are rows).  The nearest
+// column of a row does not decrease from pixel to pixel (for columns i < j the difference of the squared distances
+// grows with x), so between two known pixels only the columns between theirs can win.  The two
+// outer columns of the tile are searched in full, then the middles of ever shorter intervals; in
+// the wide empty regions both ends mostly have the same site and nothing is left to search.  A
+// search goes outward from x by blocks of 16 columns, into those whose smallest row distance (hmin)
+// can beat the best so far.  One wave per pixel column in sequence, from the pixel before, took
+// 443 us at T = 2048 with 8 clusters, this 278 us.
+__global__ __launch_bounds__(256) void k_pba_far(const short *__restrict__ g_all, const short *__restrict__ hmin_all,
+                                                 const int *__restrict__ smap_all, const int *__restrict__ pix,
+                                                 int *__restrict__ vor_all, const int *__restrict__ far, BatchDev bd)
+{
+    __shared__ short s_col[64][64];   // nearest column of pixel (x, y), -1: not known yet
+    __shared__ unsigned char s_far[64][64];
+    const int4 parts = *(const int4 *)(far + 4 * (size_t)blockIdx.x);
+    if (!(parts.x | parts.y | parts.z | parts.w)) return;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int *bm = bd.bmap(BM_LABEL);
+    const int set = set_of(bm, bd.nsets, blockIdx.x);
+    const SetDesc &sd = bd.sets[set];
+    const int logT = sd.logT, T = 1 << logT, nb = T >> 6, nblk = T >> 4;
+    if (T <= FAR_ROWS_T) return;
+    const int lb = blockIdx.x - bm[set], x0 = (lb / nb) * 64, y = (lb % nb) * 64 + lane;
+    const short *g = g_all + sd.toff + y, *hmin = hmin_all + (sd.toff >> 4) + y;
+    const int *smap = smap_all + sd.toff;
+    int *vor = vor_all + sd.toff + y;
+    for (int i = w; i < 64; i += 4) {
+        const int v = vor[(size_t)(x0 + i) << logT];
+        s_far[i][lane] = v == LAB_FAR;
+        s_col[i][lane] = v == LAB_FAR ? (short)-1 : (short)(pix[v] >> 16);
+    }
+    __syncthreads();
+    // the nearest column of pixel x0 + i among [lo, hi] (lanes with act)
+    auto search = [&](int i, int lo, int hi, bool act) {
+        const int x = x0 + i;
+        int best = -1, bx = -1;
+        if (act) {
+            best = LAB_EMPTY;
+            const int vl = g[(size_t)lo << logT], vh = g[(size_t)hi << logT];   // the ends' own sites bound it
+            if (vl >= 0) { best = (x - lo) * (x - lo) + (vl - y) * (vl - y); bx = lo; }
+            if (vh >= 0) {
+                const int d = (x - hi) * (x - hi) + (vh - y) * (vh - y);
+                if (d < best) { best = d; bx = hi; }
+            }
+        }
+        const int b0 = lo >> 4, b1 = hi >> 4, xb = x >> 4;
+        auto look = [&](int b) {
+#pragma unroll
+            for (int u = 0; u < 16; u++) {
+                const int cx = 16 * b + u, v = g[(size_t)cx << logT];
+                const int d = (x - cx) * (x - cx) + (v - y) * (v - y);
+                if (v >= 0 && (d < best || (d == best && cx < bx))) { best = d; bx = cx; }
+            }
+        };
+        if (__any(act && xb >= b0 && xb <= b1)) look(xb);
+        for (int j = 1; j < nblk; j += 4) {
+            int hl[4], hr[4];
+            bool more = false;
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                const int bl = xb - j - u, br = xb + j + u, dl = x - (16 * bl + 15), dr = 16 * br - x;
+                const bool inl = dl * dl <= best && bl >= 0, inr = dr * dr <= best && br < nblk;
+                more |= (inl && bl >= b0) || (inr && br <= b1);
+                hl[u] = inl && bl >= b0 && bl <= b1 ? hmin[(size_t)bl << logT] : 0x7fff;
+                hr[u] = inr && br <= b1 && br >= b0 ? hmin[(size_t)br << logT] : 0x7fff;
+            }
+            if (!__any(more)) break;
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                const int bl = xb - j - u, br = xb + j + u, dl = x - (16 * bl + 15), dr = 16 * br - x;
+                if (__any(hl[u] != 0x7fff && dl * dl + hl[u] * hl[u] <= best)) look(bl);
+                if (__any(hr[u] != 0x7fff && dr * dr + hr[u] * hr[u] <= best)) look(br);
+            }
+        }
+        if (act) s_col[i][lane] = (short)bx;
+    };
+    if (w < 2) {
+        const int i = w ? 63 : 0;
+        const bool act = s_col[i][lane] < 0;
+        if (__any(act)) search(i, 0, T - 1, act);
+    }
+    for (int s = 32; s; s >>= 1) {
+        __syncthreads();
+        for (int i = s * (2 * w + 1); i < 63; i += 8 * s) {
+            const int lo = s_col[i - s][lane], hi = s_col[min(i + s, 63)][lane];
+            const bool open = s_col[i][lane] < 0;
+            if (open && lo == hi) s_col[i][lane] = (short)lo;
+            const bool act = open && lo != hi;
+            if (__any(act)) search(i, lo, hi, act);
+        }
+    }
+    __syncthreads();
+    int pc = -1, pid = 0;
+    for (int i = 16 * w; i < 16 * w + 16; i++) {
+        if (!s_far[i][lane]) continue;
+        const int c = s_col[i][lane];
+        if (c != pc) {
+            pid = smap[((size_t)c << logT) + g[(size_t)c << logT]];
+            pc = c;
+        }
+        vor[(size_t)(x0 + i) << logT] = pid;
+    }
 }
 
 // ---- island certificate ------------------------------------------------------------------
@@ -651,15 +809,28 @@ void launch_splat(const double2 *xy, const BatchDev &b, const int *perm, int *sm
         GA_LAUNCH(k_splat_frame, dim3((nf + 255) / 256), dim3(256), 0, st, fpix, b, smap, pix);
 }
 
-void launch_pba(const PbaBuffers &p, const BatchDev &b, hipStream_t st)
+void launch_pba(const PbaBuffers &p, const int *pix, const BatchDev &b, hipStream_t st)
 {
     GA_LAUNCH(k_pba_cols, dim3(b.blocks[BM_COLS]), dim3(256), 0, st, p.smap, p.g, b);
-    GA_LAUNCH(k_pba_stack, dim3(b.blocks[BM_STACK]), dim3(64), 0, st, p.g, p.S, p.cnt, p.lo, b);
-    for (int s = 1; (1 << s) <= b.max_m2; s++)
-        GA_LAUNCH(k_pba_merge_step, dim3(b.blocks[BM_MERGE]), dim3(64), 0, st, (const int *)p.S, p.cnt, p.lo, b, s);
-    GA_LAUNCH(k_pba_compact, dim3(b.blocks[BM_STACK]), dim3(64), 0, st, (const int *)p.S, (const int *)p.cnt,
-              (const int *)p.lo, p.E, p.ecnt, b);
-    GA_LAUNCH(k_pba_color, dim3(b.blocks[BM_COLOR]), dim3(64), 0, st, p.E, p.ecnt, p.smap, p.vor, b);
+    const int tiles = b.blocks[BM_LABEL];
+    if (tiles < 1024)
+        GA_LAUNCH(k_pba_label<16>, dim3(tiles), dim3(1024), 0, st, (const short *)p.g, (const int *)p.smap, p.vor, p.far,
+                  p.setfar, b);
+    else
+        GA_LAUNCH(k_pba_label<4>, dim3(tiles), dim3(256), 0, st, (const short *)p.g, (const int *)p.smap, p.vor, p.far,
+                  p.setfar, b);
+    if (b.maxT > FAR_ROWS_T) {
+        GA_LAUNCH(k_pba_blockmin, dim3(b.blocks[BM_LABEL]), dim3(256), 0, st, (const short *)p.g, p.hmin,
+                  (const int *)p.setfar, b);
+        GA_LAUNCH(k_pba_far, dim3(b.blocks[BM_LABEL]), dim3(256), 0, st, (const short *)p.g, (const short *)p.hmin,
+                  (const int *)p.smap, pix, p.vor, (const int *)p.far, b);
+    }
+    if (b.blocks[BM_ROWS] > 0) {
+        if (b.far_lds > 65536)
+            (void)hipFuncSetAttribute((const void *)k_pba_far_rows, hipFuncAttributeMaxDynamicSharedMemorySize, b.far_lds);
+        GA_LAUNCH(k_pba_far_rows, dim3(b.blocks[BM_ROWS]), dim3(1024), b.far_lds, st, (const short *)p.g, (const int *)p.smap, pix,
+                  p.vor, (const int *)p.far, (const int *)p.setfar, b);
+    }
 }
 
 void launch_islands(const int *vor, const int *pix, const BatchDev &b, int *bad, int *flag, hipStream_t st)
@@ -670,12 +841,10 @@ void launch_islands(const int *vor, const int *pix, const BatchDev &b, int *bad,
 // removes the flagged sites (listed in rlist from position `first`, the number removed before) and
 // repairs the diagram around them, then checks the pixels that changed; zeroes *flag and *nchanged
 void launch_island_repair(const PbaBuffers &p, const BatchDev &b, int *bad, const int *pix, int *removed, int first,
-                          int *rlist, int *nchanged, int *flag, hipStream_t st)
+                          int *rlist, unsigned *changed, int *chset, int *nchanged, int *flag, hipStream_t st)
 {
-    // free after phase 3: the band ends, stacks and envelopes (every texture has 64 T band ends and T * T
-    // entries of the others)
-    int *setbad = p.cnt, *chset = p.E;
-    unsigned *changed = (unsigned *)p.S;
+    // (free after phase 3)
+    int *setbad = p.setfar;
     if (b.ntot <= 0) return;
     IntFills f;
     f.add(setbad, (size_t)b.nsets, 0);
