@@ -237,10 +237,50 @@ GA_INLINE int min_ulp_exp(const double *v, int n)
     return s == 100000 ? 0 : s;
 }
 
+// Sign of ax by - ax cy - cx by - ay bx + ay cx + cy bx (the terms cx cy cancel) by floating-point
+// expansions (Shewchuk 1997): each product is a rounded value and its exact error, and the
+// twelve terms are added one by one to an expansion of non-overlapping components, whose largest nonzero
+// one has the sign.  Exact while no product or error leaves the range of normal numbers.
+// A lone test of this kind holds up its whole launch: the big integers below live in scratch
+// memory, the expansion in registers (the slowest deletion round at 12,007 points in clusters: 54 us
+// with the former, 39 with the latter).
+GA_INLINE int orient_expansion(double2 a, double2 b, double2 c)
+{
+    const double f[6] = {a.x, -a.x, -c.x, -a.y, a.y, c.y}, g[6] = {b.y, c.y, b.y, b.x, c.x, b.x};
+    double e[12] = {};
+#pragma unroll
+    for (int k = 0; k < 12; k++) {
+        const double p = f[k / 2] * g[k / 2];
+        double q = k & 1 ? p : fma(f[k / 2], g[k / 2], -p);
+#pragma unroll
+        for (int i = 0; i <= k; i++) {   // q + e[0 .. k - 1]: the error of each sum stays, the sum goes on
+            if (i == k) {
+                e[i] = q;
+                break;
+            }
+            const double s = q + e[i], bv = s - q;
+            e[i] = (q - (s - bv)) + (e[i] - bv);
+            q = s;
+        }
+    }
+    double top = 0.0;
+#pragma unroll
+    for (int i = 0; i < 12; i++)
+        if (e[i] != 0.0) top = e[i];
+    return top > 0.0 ? 1 : (top < 0.0 ? -1 : 0);
+}
+
 // exact orientation sign (ovf set when the capacity would be exceeded)
 GA_INLINE int orient_exact(double2 a, double2 b, double2 c, int *ovf)
 {
-    double v[6] = {a.x, a.y, b.x, b.y, c.x, c.y};
+    double v[6] = {a.x, a.y, b.x, b.y, c.x, c.y}, lo = INFINITY, hi = 0.0;
+    for (int i = 0; i < 6; i++) {
+        if (v[i] != 0.0) lo = fmin(lo, fabs(v[i]));
+        hi = fmax(hi, fabs(v[i]));
+    }
+    // All products and their errors are normal numbers.  (Wider spreads go to the big integers, which
+    // refuse what exceeds their capacity; 60 bits never do.)
+    if (lo > 1e-130 && hi < 1e130 && hi <= lo * 0x1p60) return orient_expansion(a, b, c);
     int s = min_ulp_exp(v, 6);
     BigInt<12> ax, ay, bx, by, cx, cy, t1, t2, t3, t4, r;
     bi_from_double(ax, a.x, s, ovf); bi_from_double(ay, a.y, s, ovf);
