@@ -26,15 +26,26 @@
 #include <algorithm>
 
 // Workgroups go to the 8 XCDs round-robin by blockIdx.x, and each XCD has its own L2.  Grid-
-// stride loops renumber their blocks so that XCD k runs the blocks [k G / 8, (k + 1) G / 8) of
-// every sweep: neighbouring indices (triangle slots and vertices are numbered in spatial order)
-// then share one L2 instead of being spread over all eight.
-GA_INLINE int xcd_block()
+// stride loops give XCD k the k-th eighth of the range, and its blocks stride through that:
+// neighbouring indices (triangle slots and vertices are numbered in spatial order) then share
+// one L2 instead of being spread over all eight, and every XCD has the same share whatever the
+// range and the grid are.  (With the k-th eighth of the blocks of every sweep instead, a list
+// shorter than the grid ran on the first XCDs alone: at 65K points k_fanfill took 36 us against
+// 19, a pass of k_flip_commit up to 18 against 10.)
+struct XcdRange {
+    int begin, end, step;
+};
+// of a block that takes `unit` indices per step, from its index `at` on
+GA_INLINE XcdRange xcd_range(int n, int unit, int at)
 {
-    unsigned g = gridDim.x, b = blockIdx.x;
-    return (g & 7u) ? (int)b : (int)((b & 7u) * (g >> 3) + (b >> 3));
+    const int g = (int)gridDim.x, b = (int)blockIdx.x;
+    if (g & 7) return {b * unit + at, n, g * unit};
+    const int share = (n + 8 * unit - 1) / (8 * unit) * unit, first = (b & 7) * share;
+    return {first + (b >> 3) * unit + at, first + share < n ? first + share : n, (g >> 3) * unit};
 }
-#define GRID_STRIDE(i, n) for (int i = xcd_block() * blockDim.x + threadIdx.x; i < (n); i += gridDim.x * blockDim.x)
+#define XCD_STRIDE(i, n, unit) for (auto [i, i##_end, i##_step] = xcd_range(n, unit, 0); i < i##_end; i += i##_step)
+#define GRID_STRIDE(i, n) \
+    for (auto [i, i##_end, i##_step] = xcd_range(n, (int)blockDim.x, (int)threadIdx.x); i < i##_end; i += i##_step)
 #define FIXED_GRID 2048
 
 GA_INLINE int ic(const int4 &a, int i) { return i == 0 ? a.x : (i == 1 ? a.y : a.z); }
@@ -287,7 +298,7 @@ __global__ __launch_bounds__(256) void k_deg(const int4 *__restrict__ tv, const 
     __shared__ int cnt[ADJ_WIN];
     __shared__ int s_red[4];
     const int n = *ntri;
-    for (int c0 = xcd_block() * ADJ_CHUNK; c0 < n; c0 += gridDim.x * ADJ_CHUNK) {
+    XCD_STRIDE(c0, n, ADJ_CHUNK) {
         const int base = adj_chunk_min(tv, c0, n, s_red);
         for (int i = threadIdx.x; i < ADJ_WIN; i += 256) cnt[i] = 0;
         __syncthreads();
@@ -322,7 +333,7 @@ __global__ __launch_bounds__(256) void k_fanfill(const int4 *__restrict__ tv, co
     __shared__ int cnt[ADJ_WIN];
     __shared__ int s_red[4];
     const int n = *ntri;
-    for (int c0 = xcd_block() * ADJ_CHUNK; c0 < n; c0 += gridDim.x * ADJ_CHUNK) {
+    XCD_STRIDE(c0, n, ADJ_CHUNK) {
         const int base = adj_chunk_min(tv, c0, n, s_red);
         for (int i = threadIdx.x; i < ADJ_WIN; i += 256) cnt[i] = 0;
         __syncthreads();
@@ -548,7 +559,7 @@ void launch_shift_commit(MeshDev &m, const unsigned char *moved, hipStream_t st)
 // skipped by its state test.
 __global__ __launch_bounds__(256) void k_pending_list(MeshDev m)
 {
-    for (int b0 = blockIdx.x * 1024; b0 < m.n; b0 += gridDim.x * 1024) {
+    XCD_STRIDE(b0, m.n, 1024) {
         unsigned bits = 0;
         for (int j = 0; j < 4; j++) {
             int v = b0 + j * 256 + (int)threadIdx.x;
@@ -823,7 +834,7 @@ GA_INLINE void missing_anchor(const MeshDev &m, const int *__restrict__ vor, int
 __global__ __launch_bounds__(256) void k_missing_init(MeshDev m, const int *__restrict__ vor, int *mlist, int *loc)
 {
     // block-uniform loop: 1024 vertices per block and step, one list reservation per step
-    for (int b0 = blockIdx.x * 1024; b0 < m.n; b0 += gridDim.x * 1024) {
+    XCD_STRIDE(b0, m.n, 1024) {
         unsigned bits = 0;
         for (int j = 0; j < 4; j++) {
             int v = b0 + j * 256 + (int)threadIdx.x;
@@ -1076,7 +1087,7 @@ GA_INLINE void flip_test_body(const MeshDev &m, const int *list, int n, int prev
     int tests = 0;
     const int bd = (int)blockDim.x;
     int per = n > 4 * (int)(gridDim.x * bd) ? 4 : 1;
-    for (int b0 = xcd_block() * bd * per; b0 < n; b0 += gridDim.x * bd * per) {
+    XCD_STRIDE(b0, n, bd * per) {
         unsigned bits = 0;   // bit 3j + i: edge i of the j-th triangle of this thread wants a flip
         int tj[4];
 #pragma unroll
@@ -1155,7 +1166,7 @@ GA_INLINE void flip_commit_body(const MeshDev &m, int n, int op, int *list_out, 
     int flips = 0;
     const int bd = (int)blockDim.x;
     const int per = n > 4 * (int)(gridDim.x * bd) ? 4 : 1;
-    for (int b0 = xcd_block() * bd * per; b0 < n; b0 += gridDim.x * bd * per) {
+    XCD_STRIDE(b0, n, bd * per) {
         int tq[4], uq[4];
         unsigned outs = 0;   // bit 2j: slot t of the j-th candidate joins the next list, 2j + 1: slot u
 #pragma unroll
@@ -1396,7 +1407,7 @@ GA_INLINE int hull_entry(const MeshDev &m, const HullDev &h, int H, int a, int b
 __global__ __launch_bounds__(256) void k_hull_scan(MeshDev m, HullDev h, int op)
 {
     const int n = ntri_used(m);
-    for (int b0 = xcd_block() * 1024; b0 < n; b0 += gridDim.x * 1024) {
+    XCD_STRIDE(b0, n, 1024) {
         unsigned bits = 0;
 #pragma unroll
         for (int j = 0; j < 4; j++) {
@@ -1750,6 +1761,17 @@ void launch_hull(MeshDev &m, const HullDev &h, int op, void *scan_tmp, hipStream
     GA_LAUNCH(k_hull_fill, dim3(FIXED_GRID), dim3(256), 0, st, m, h);
 }
 
+// Ranges in canonical order: input order inside a set (not spatial), one set after another.  A
+// batch's sets are shared out to the XCDs, a single set is not (k_canon_emit: 1M points 129 us against
+// 165 with shares, 1,024 sets 1,534 against 1,362).
+GA_INLINE XcdRange canon_range(const MeshDev &m, int n)
+{
+    const int bd = (int)blockDim.x, tid = (int)threadIdx.x;
+    if (m.nsets > 1) return xcd_range(n, bd, tid);
+    return {(int)blockIdx.x * bd + tid, n, (int)gridDim.x * bd};
+}
+#define CANON_STRIDE(i, n) for (auto [i, i##_end, i##_step] = canon_range(m, n); i < i##_end; i += i##_step)
+
 // ---- canonical output ----------------------------------------------------------------------------
 // Output order: (v0, v1, v2) of input indices with v0 the smallest vertex; input indices of the sets
 // of a batch are consecutive ranges in set order, so this is also set order.  Every directed edge
@@ -1851,7 +1873,7 @@ __global__ void k_canon_newid(int *order, const unsigned *skey, const unsigned *
 __global__ void k_canon_emit(MeshDev m, const int *order, const int *newid, const int *dF, int *out9, int *rset)
 {
     const int F = *dF;
-    GRID_STRIDE(r, F) {
+    CANON_STRIDE(r, F) {
         const int s = order[r];
         const int4 v = m.tv[s];
         const int ro = newid[s] & 3;
@@ -1884,7 +1906,7 @@ __global__ void k_canon_set_first(MeshDev m, const int *rset, const int *dF, int
         if (blockIdx.x == 0 && threadIdx.x == 0 && F > 0) set_first[0] = 0;
         return;
     }
-    GRID_STRIDE(r, F) {
+    CANON_STRIDE(r, F) {
         int set = rset[r];
         if (r == 0 || rset[r - 1] != set) set_first[set] = r;
     }
