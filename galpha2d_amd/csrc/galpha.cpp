@@ -107,8 +107,8 @@ struct galpha_ctx {
     DevBuf perm, xys, pcell, ccount, ccursor;   // spatial numbering of the real points
     DevBuf cls;                                  // alpha-complex classes (host queries)
     DevBuf tv, tn, remap, stamp, claim, modA, modB, cand, pos, vt, vstate, pix, deg, off, fill, fan,
-        moved, decide, mx, mlist, loc, lt, scratch, keys, keys2, vals, vals2, rot, newid,
-        out9, counters, status, xy, scanTmp, sortTmp, tileCnt, tileOff, dellist, dbg;
+        moved, mark, mx, mlist, loc, lt, scratch, keys, keys2, vals, vals2, rot, newid,
+        out9, counters, status, xy, scanTmp, sortTmp, tileCnt, tileOff, dbg;
     // batch plan on the device
     DevBuf setsD, bmD, vset, setFirst, offsD, bboxTmp, lmark;
     // constrained DT: input pairs, vertex-id pairs, inverse numbering, flags, walk counts, region
@@ -367,18 +367,11 @@ static void ctx_counters_read(galpha_ctx *c, int *dst, int slot, int n, bool fol
     HIPCHK(hipStreamSynchronize(c->stream));
     memcpy(dst, c->hsnap, sizeof(int) * n);
 }
-static int ctx_counter(galpha_ctx *c, int slot)
-{
-    int v = 0;
-    ctx_counters_read(c, &v, slot, 1);
-    return v;
-}
 // stream-ordered read of device memory (the caller's stream may be non-blocking)
 static void ctx_read(galpha_ctx *c, void *dst, const void *src, size_t bytes)
 {
     stage_d2h(c->stage, dst, src, bytes, c->stream);
 }
-static int ctx_status(galpha_ctx *c) { return ctx_counter(c, C_STATUS); }
 
 // Device int segments (up to four) in one host read: gathered into one device array, then one copy
 // through pinned memory and one wait (each copy into pageable memory waits a round trip of its own).
@@ -412,17 +405,7 @@ static void ctx_read_segments(galpha_ctx *c, std::initializer_list<std::pair<con
         stage_d2h(c->stage, dst, c->rdbuf.p, 4 * tot, c->stream);
     }
 }
-static void ctx_counter_set(galpha_ctx *c, int slot, int v)
-{
-    HIPCHK(hipMemsetD32Async((hipDeviceptr_t)(c->counters.as<int>() + slot), v, 1, c->stream));
-}
-// striped statistics (see kernels.h): fold the stripes on the device, then read
-static int ctx_stat(galpha_ctx *c, int k)
-{
-    int v = 0;
-    ctx_counters_read(c, &v, C_FOLD + k, 1, true);
-    return v;
-}
+// striped statistics (see kernels.h) are folded on the device, then read
 // all single-word counters, the status word and the folded statistics in one read:
 // snap[k] = counter k, snap[C_FOLD + k] = statistic k
 struct Snap {
@@ -720,7 +703,7 @@ static Snap remove_frame(galpha_ctx *c, MeshDev &m, hipStream_t st)
     // table takes 6 B entries of 16 bytes or the whole fan buffer, 4.5 V and more)
     HullDev h{};
     h.ftri = m.modA;
-    h.mark = m.decide;
+    h.mark = m.mark;
     h.bidx = c->off.as<int>();
     h.blist = c->mlist.as<int>();
     h.bpos = c->scratch.as<double2>();
@@ -729,7 +712,7 @@ static Snap remove_frame(galpha_ctx *c, MeshDev &m, hipStream_t st)
     h.list = (int2 *)m.cand;
     h.next = (int *)m.remap;
     h.pool = m.modB;
-    h.share = m.dellist;
+    h.share = (int *)(h.bbox + m.n / 64 + 2);
     h.room = (int)std::min<size_t>({c->fan.bytes / 16, c->remap.bytes / 8, (size_t)1 << 30});
     {
         IntFills f;
@@ -812,14 +795,13 @@ static int run_batch(galpha_ctx *c, const double *d_xy, const BatchPlan &plan)
     c->fill.ensure(4 * (size_t)(V + 1));
     c->fan.ensure(8 * 3 * (size_t)cap);
     c->moved.ensure((size_t)V);
-    c->decide.ensure(4 * (size_t)V);
+    c->mark.ensure(4 * (size_t)V);
     c->mx.ensure(8 * (size_t)V);
     c->mlist.ensure(4 * (size_t)n);
     c->loc.ensure(4 * (size_t)n);
     c->lt.ensure(4 * (size_t)n);
     size_t scap = std::max((size_t)4 * 8192 + 64, (size_t)(8 * V) + 4096);
     c->scratch.ensure(4 * scap);
-    c->dellist.ensure(4 * (size_t)cap);
     c->lmark.ensure(4 * (size_t)cap);
     // Slot tags (stamp, claim keys, list marks) carry the context's op number, and the removal
     // rounds (deletion, frame) tag their per-vertex priority maxima with a round number; both
@@ -867,8 +849,9 @@ static int run_batch(galpha_ctx *c, const double *d_xy, const BatchPlan &plan)
     c->dbg.ensure(64 * sizeof(double));
     m.dbg = c->dbg.as<double>();
     m.deg = c->deg.as<int>();
-    m.decide = c->decide.as<int>();
-    m.dellist = c->dellist.as<int>();
+    m.mark = c->mark.as<int>();
+    m.off = c->off.as<int>();
+    m.fan = c->fan.as<int2>();
     m.lt = c->lt.as<int>();
     m.lmark = c->lmark.as<int>();
 
@@ -877,96 +860,7 @@ static int run_batch(galpha_ctx *c, const double *d_xy, const BatchPlan &plan)
                  c->scanTmp.p, st);
     launch_adjacency(m, c->deg.as<int>(), c->off.as<int>(), c->fill.as<int>(), c->fan.as<int2>(), c->scanTmp.p, st);
     launch_init_positions(m, st);
-    {
-        int cv[C_NCOUNTERS];   // slot count (40) and status word
-        ctx_counters_read(c, cv, 0, C_NCOUNTERS);
-        S.reconTris = cv[40];
-        if (cv[40] > cap) throw GalphaError("triangle capacity exceeded in reconstruction");
-        if (cv[C_STATUS])
-            throw GalphaError("reconstruction produced an invalid triangle (status " + std::to_string(cv[C_STATUS]) + ")");
-    }
     ev_mark(c, 2, st);
-    // ---- shifting
-    // revert moved vertices of non-ccw triangles until every triangle is ccw (monotone)
-    // Round loops launch several rounds per host read of their counters: a round after
-    // convergence finds nothing to do, so over-running is harmless.
-    {
-        // worklists in the flip lists (free until the flips), marks in decide[] (free until the
-        // greedy rounds)
-        // Lists alternate between two buffers; their counts rotate through three slots, so each
-        // pass zeroes the next pass's output count (the slot the pass before it read) itself.
-        unsigned char *moved = c->moved.as<unsigned char>();
-        int *wl[2] = {m.modA, m.modB};
-        const int slot[3] = {C_MODN, C_MODN2, C_MODN3};
-        launch_shift_bulk(m, moved, m.decide, wl[0], slot[0], slot[1], st);   // (zeroes decide[])
-        for (int it = 0;; it += 4) {
-            if (it > 100000) throw GalphaError("bulk shifting did not converge");
-            for (int k = it; k < it + 4; k++)
-                launch_shift_star(m, moved, m.decide, wl[k & 1], slot[k % 3], wl[(k + 1) & 1], slot[(k + 1) % 3],
-                                  slot[(k + 2) % 3], st);
-            if (ctx_counter(c, slot[(it + 4) % 3]) == 0) break;
-        }
-    }
-    launch_shift_commit(m, c->moved.as<unsigned char>(), st);
-    // the missing-site list is free until the missing stage: it holds the pending vertices
-    m.plist = c->mlist.as<int>();
-    launch_pending_list(m, st);
-    int pend = ctx_stat(c, C_PEND);
-    S.shiftBad = pend;
-    int moved_before = 0;
-    // Eight greedy rounds (two batches of four per host read), then deletion takes the rest.
-    // Later rounds move few vertices each and cost more than deleting and reinserting them:
-    // on 1M uniform points the shifting stage took 1.68 ms with up to 48 rounds, 1.40 ms with 8.
-    const int pgrid = round_grid(pend);   // the pending list keeps its length (done entries are skipped)
-    // (all eight before one read: a round after convergence moves nothing)
-    // Sets of 256K points and more always leave vertices to delete after the greedy rounds, so
-    // their moved count comes with the deletion loop's first snapshot instead of a read of its own.
-    const bool large = m.n >= (1 << 18);
-    if (pend > 0) {
-        for (int k = 0; k < 8; k++) launch_shift_greedy(m, k, pgrid, st);
-        if (!large) {
-            int moved_total = ctx_stat(c, C_MOVED);
-            pend -= moved_total - moved_before;
-            moved_before = moved_total;
-        }
-    }
-    int deleted_before = 0;
-    // three rounds per read; sets of 256K points and more start with six (1M uniform points take
-    // six), saving a read
-    for (int r = 0, per = large ? 6 : 3; pend > 0; r += per, per = 3) {
-        if (r > 10000) throw GalphaError("vertex deletion did not finish");
-        for (int k = 0; k < per; k++) {
-            // (k_del_prio zeroes C_SCR and C_MODN; rounds with nothing pending return at once)
-            launch_delete_round(m, c->mx.as<unsigned int>(), next_prio_round(), c->op++, pgrid, st);
-        }
-        Snap sn = ctx_snapshot(c);
-        int after = sn.stat(C_DELETED);
-        const int moved_total = sn.stat(C_MOVED);
-        pend -= (after - deleted_before) + (moved_total - moved_before);
-        moved_before = moved_total;
-        deleted_before = after;
-        int stt = sn.status();
-        if (stt) {
-            int dbg[16];
-            ctx_counters_read(c, dbg, C_DBG, 16);
-            std::string d = " [v=" + std::to_string(dbg[1]) + " poly(" + std::to_string(dbg[2]) + "):";
-            for (int k = 0; k < 12 && k < dbg[2]; k++) d += " " + std::to_string(dbg[3 + k]);
-            double dp[48];
-            ctx_read(c, dp, c->dbg.p, sizeof(dp));
-            char buf[64];
-            d += " pos:";
-            for (int k = 0; k < 2 + 2 * std::min(dbg[2], 15); k++) {
-                snprintf(buf, sizeof(buf), " %.17g", dp[k]);
-                d += buf;
-            }
-            d += " states:";
-            for (int k = 0; k < std::min(dbg[2], 15); k++) d += " " + std::to_string((int)dp[32 + k]);
-            throw GalphaError("vertex deletion failed (status " + std::to_string(stt) + ")" + d + "]");
-        }
-    }
-    S.deleted = deleted_before;
-    ev_mark(c, 3, st);
-
     // Flip helpers: Lawson passes over the list of triangles to test; a pass with no flip has no candidate
     // left (the highest candidate always wins), so three passes run per host read.
     // `last` keeps the snapshot of the final check (counters, statistics and status after the
@@ -1042,44 +936,108 @@ static int run_batch(galpha_ctx *c, const double *d_xy, const BatchPlan &plan)
     };
     auto flip_all = [&]() {
         int opn = c->op++;
-        ctx_counter_set(c, C_MODN, 0);
         launch_flip_all(m, opn, m.modA, st);
         flip_until_done(m.modA, C_MODN, m.modB, C_MODN2, opn, -1);
     };
-    // ---- missing sites
-    // Inserted into the mesh as it is after shifting (every triangle counter-clockwise, not yet
-    // Delaunay): the walks and splits only need a valid triangulation, and one flip phase over
-    // all triangles afterwards makes the mesh Delaunay, instead of flip passes after every
-    // insertion round.
-    // (C_MISS is zero since the run's start: only the missing stage counts it)
-    launch_missing_init(m, c->vor.as<int>(), c->mlist.as<int>(), c->loc.as<int>(), st);
-    last = ctx_snapshot(c);
-    int nmiss = last.v[C_MISS];
-    S.missing = nmiss;
-    for (int r = 0; r < 100000; r++) {
-        // `last`: the snapshot after the previous round (or after the list was built)
-        int left = nmiss - last.stat(C_INSERTED) - last.stat(C_DUPS);
-        if (left <= 0) break;
-        if (last.status())
-            throw GalphaError("missing-site insertion failed (status " + std::to_string(last.status()) + ")");
-        if (r > 5000) throw GalphaError("missing-site insertion did not finish");
-        // two rounds per read (a round after the last insertion finds every entry done); sets of
-        // 256K points and more start with four (1M uniform points take four), saving a read
-        const int per = r == 0 && m.n >= (1 << 18) ? 4 : 2;
-        for (int k = 0; k < per; k++) {
-            int opn = c->op++;
-            launch_insert_round(m, c->mlist.as<int>(), c->loc.as<int>(), opn, round_grid(nmiss), st);   // (zeroes C_MODN)
-            launch_relink(m, m.modA, C_MODN, opn, round_grid(4LL * left), st);
-            S.insertRounds++;
+    // ---- shifting, deletion, insertion and the flips to a Delaunay mesh, in one chain of launches
+    // All the rounds that most inputs need are launched one behind the other, and their counters
+    // are read once, after the flips: a round that finds nothing to do returns at once (a few us),
+    // a host read between two stages costs 20 to 30 us.  A stage that the rounds before it left
+    // unfinished lists nothing (C_SHIFTING, C_PLEFT, C_MLEFT); the loop then launches more of the
+    // rounds that were short.
+    //   bulk shifting: moved vertices of non-ccw triangles revert until every triangle is ccw;
+    //   eight greedy rounds, then deletion takes the rest: later rounds move few vertices each and
+    //   cost more than deleting and reinserting them (1M uniform points: 1.68 ms of shifting
+    //   with up to 48 rounds, 1.40 ms with 8);
+    //   deletion rounds (1M uniform points take six) and insertion rounds (four).  Missing sites go into the mesh as
+    //   it is after shifting (every triangle counter-clockwise, not yet Delaunay): the walks and
+    //   splits only need a valid triangulation, and one flip phase over all triangles
+    //   afterwards makes the mesh Delaunay, instead of flip passes after every insertion round.
+    {
+        // worklists in the buffers of the missing sites' walks (nothing touches them until bulk
+        // shifting has ended).  Lists alternate between two buffers; their counts rotate through three
+        // slots, so each pass zeroes the next pass's output count (the slot the pass before it read)
+        // itself.
+        unsigned char *moved = c->moved.as<unsigned char>();
+        int *wl[2] = {c->loc.as<int>(), m.lt};
+        const int slot[3] = {C_STAR, C_STAR + 1, C_STAR + 2};
+        // the missing-site list is free until the missing stage: it holds the pending vertices
+        m.plist = c->mlist.as<int>();
+        launch_shift_bulk(m, moved, m.mark, wl[0], slot[0], slot[1], st);   // (zeroes mark[])
+        int stars = 0;
+        bool shifting = true, deleting = true;
+        // grids before the lists' lengths are known: one vertex in 8 pending, one in 4 missing
+        int pgrid = round_grid(m.n), dgrid = round_grid(m.n / 2), mgrid = round_grid(m.n / 4);
+        for (int r = 0;; r++) {
+            if (shifting) {
+                for (int k = stars; k < stars + 4; k++)
+                    launch_shift_star(m, moved, m.mark, wl[k & 1], slot[k % 3], wl[(k + 1) & 1], slot[(k + 1) % 3],
+                                      slot[(k + 2) % 3], st);
+                stars += 4;
+                if (stars > 100000) throw GalphaError("bulk shifting did not converge");
+                launch_shift_commit(m, moved, slot[stars % 3], st);
+                for (int k = 0; k < 8; k++) launch_shift_greedy(m, k, m.mark, pgrid, st);
+            }
+            if (deleting) {
+                // (k_del_prio zeroes C_SCR and C_PLEFT)
+                for (int k = 0; k < 6; k++)
+                    launch_delete_round(m, c->mx.as<unsigned int>(), next_prio_round(), dgrid, st);
+                ev_mark(c, 3, st);
+                // (C_MISS is zero since the run's start: only the missing stage counts it)
+                launch_missing_init(m, c->vor.as<int>(), c->mlist.as<int>(), c->loc.as<int>(), st);
+            }
+            for (int k = 0; k < 4; k++) {
+                int opn = c->op++;
+                launch_insert_round(m, c->mlist.as<int>(), c->loc.as<int>(), opn, mgrid, st);   // (zeroes C_MODN, C_MLEFT)
+                launch_relink(m, m.modA, C_MODN, opn, mgrid, st);
+                S.insertRounds++;
+            }
+            ev_mark(c, 4, st);
+            flip_all();
+            S.reconTris = last.v[C_RECON_SLOTS];
+            if (last.v[C_RECON_SLOTS] > cap) throw GalphaError("triangle capacity exceeded in reconstruction");
+            if (last.v[C_RECON_STATUS])
+                throw GalphaError("reconstruction produced an invalid triangle (status " +
+                                  std::to_string(last.v[C_RECON_STATUS]) + ")");
+            shifting = last.v[C_SHIFTING] != 0;
+            deleting = shifting || last.v[C_PLEFT] != 0;
+            if (int stt = last.status()) {
+                if (!last.v[C_DBG])
+                    throw GalphaError((deleting ? "vertex deletion failed (status " : "missing-site insertion failed (status ") +
+                                      std::to_string(stt) + ")");
+                int dbg[16];
+                ctx_counters_read(c, dbg, C_DBG, 16);
+                std::string d = " [v=" + std::to_string(dbg[1]) + " poly(" + std::to_string(dbg[2]) + "):";
+                for (int k = 0; k < 12 && k < dbg[2]; k++) d += " " + std::to_string(dbg[3 + k]);
+                double dp[48];
+                ctx_read(c, dp, c->dbg.p, sizeof(dp));
+                char buf[64];
+                d += " pos:";
+                for (int k = 0; k < 2 + 2 * std::min(dbg[2], 15); k++) {
+                    snprintf(buf, sizeof(buf), " %.17g", dp[k]);
+                    d += buf;
+                }
+                d += " states:";
+                for (int k = 0; k < std::min(dbg[2], 15); k++) d += " " + std::to_string((int)dp[32 + k]);
+                throw GalphaError("vertex deletion failed (status " + std::to_string(stt) + ")" + d + "]");
+            }
+            if (!deleting && !last.v[C_MLEFT]) break;
+            if (r > 10000) throw GalphaError(deleting ? "vertex deletion did not finish" : "missing-site insertion did not finish");
+            pgrid = round_grid(8LL * last.v[C_PLIST]);
+            dgrid = round_grid(4LL * last.v[C_PLIST]);
+            mgrid = round_grid(last.v[C_MISS]);
+            if (shifting) pgrid = round_grid(m.n);
+            if (deleting) {
+                if (shifting) dgrid = round_grid(m.n / 2);
+                mgrid = round_grid(m.n / 4);
+            }
         }
-        last = ctx_snapshot(c);
     }
+    S.shiftBad = last.v[C_PLIST];
+    S.deleted = last.stat(C_DELETED);
+    S.missing = last.v[C_MISS];
     S.inserted = last.stat(C_INSERTED);
     S.duplicates = last.stat(C_DUPS);
-    ev_mark(c, 4, st);
-
-    // ---- flips to a Delaunay mesh of the current vertices
-    flip_all();
     ev_mark(c, 5, st);
     const Snap after_main = last;   // per-stage statistics: shifting, insertion and these flips
 
@@ -1375,10 +1333,10 @@ static void release_all(galpha_ctx *c)
 {
     DevBuf *bufs[] = {&c->smap, &c->g, &c->hmin, &c->far, &c->setfar, &c->chg, &c->chgset, &c->vor, &c->bad, &c->fpix, &c->tv,
                       &c->tn, &c->remap, &c->stamp, &c->claim, &c->modA, &c->modB, &c->cand, &c->pos, &c->vt,
-                      &c->vstate, &c->pix, &c->deg, &c->off, &c->fill, &c->fan, &c->moved, &c->decide, &c->mx,
+                      &c->vstate, &c->pix, &c->deg, &c->off, &c->fill, &c->fan, &c->moved, &c->mark, &c->mx,
                       &c->mlist, &c->loc, &c->lt, &c->scratch, &c->keys, &c->keys2,
                       &c->vals, &c->vals2, &c->rot, &c->newid, &c->out9, &c->counters, &c->status, &c->xy,
-                      &c->scanTmp, &c->sortTmp, &c->tileCnt, &c->tileOff, &c->dellist, &c->dbg,
+                      &c->scanTmp, &c->sortTmp, &c->tileCnt, &c->tileOff, &c->dbg,
                       &c->setsD, &c->bmD, &c->vset, &c->setFirst,
                       &c->offsD, &c->bboxTmp, &c->lmark,
                       &c->perm, &c->xys, &c->pcell, &c->ccount, &c->ccursor, &c->cls,
@@ -1394,10 +1352,10 @@ size_t galpha_ctx_device_bytes(galpha_ctx *c)
 {
     DevBuf *bufs[] = {&c->smap, &c->g, &c->hmin, &c->far, &c->setfar, &c->chg, &c->chgset, &c->vor, &c->bad, &c->fpix, &c->tv,
                       &c->tn, &c->remap, &c->stamp, &c->claim, &c->modA, &c->modB, &c->cand, &c->pos, &c->vt,
-                      &c->vstate, &c->pix, &c->deg, &c->off, &c->fill, &c->fan, &c->moved, &c->decide, &c->mx,
+                      &c->vstate, &c->pix, &c->deg, &c->off, &c->fill, &c->fan, &c->moved, &c->mark, &c->mx,
                       &c->mlist, &c->loc, &c->lt, &c->scratch, &c->keys, &c->keys2,
                       &c->vals, &c->vals2, &c->rot, &c->newid, &c->out9, &c->counters, &c->status, &c->xy,
-                      &c->scanTmp, &c->sortTmp, &c->tileCnt, &c->tileOff, &c->dellist, &c->dbg,
+                      &c->scanTmp, &c->sortTmp, &c->tileCnt, &c->tileOff, &c->dbg,
                       &c->setsD, &c->bmD, &c->vset, &c->setFirst,
                       &c->offsD, &c->bboxTmp, &c->lmark,
                       &c->perm, &c->xys, &c->pcell, &c->ccount, &c->ccursor, &c->cls,

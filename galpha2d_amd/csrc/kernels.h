@@ -107,8 +107,9 @@ struct MeshDev {
     double *dbg;         // failure dump: positions (K + up to 15 polygon vertices) and states
     // per-context work buffers (never process globals: contexts run concurrently)
     int *deg;            // [V + 1] vertex degrees of the reconstruction
-    int *decide;         // [V] greedy shifting decisions
-    int *dellist;        // [cap] triangles created by a deletion round
+    int *mark;           // [V] state of the shifting rounds (see mesh.hip)
+    const int *off;      // [V + 1] corners of every vertex in the reconstruction: fan[off[v]] .. fan[off[v + 1]]
+    const int2 *fan;     // (enc(triangle, corner), next vertex)
     int *lt;             // [n] located type of every missing site
     int *lmark;          // [cap] operation that last put the slot in a flip list (one entry per pass)
     // constraint edges (set of (min << 32 | max) + 1 keys, open addressing, 0 = empty); NULL when
@@ -154,7 +155,7 @@ struct HullDev {
 #define C_WIN 4
 #define C_SCR 5
 #define C_MISS 6
-#define C_PEND 7
+#define C_SHIFTING 7          // bulk shifting has not come to an end yet
 #define C_EXACT_ORIENT 8
 #define C_EXACT_INCIRCLE 9
 #define C_FLIPS 10
@@ -173,15 +174,18 @@ struct HullDev {
 #define C_FTRI 25             // frame triangles listed by k_hull_scan
 #define C_HULL 26             // first demands of frame removal
 #define C_HULL_POOL 27        // other frame triangles (free slots)
-#define C_MOVED 28            // vertices moved by greedy shifting rounds (statistic)
+#define C_PLEFT 28            // vertices are left to delete
+#define C_MLEFT 29            // vertices are left to insert
 #define C_PLIST 30            // entries of the pending-vertex list (MeshDev::plist)
+#define C_RECON_STATUS 31     // status word and slot count after the reconstruction
+#define C_RECON_SLOTS 39
 #define C_STATUS 32           // device status word (GA_ERR_* bits); MeshDev::status points here
 #define C_CONS_PEND 33        // constraints still to insert (the current insertion round's walk)
 #define C_CONS_MOD 34         // slots rewritten by the current insertion round
 #define C_TAIL_PASSES 35      // passes run by the last single-workgroup flip tail
 #define C_TAIL_DONE 36        // 1 when that tail ended with a pass without flips
 #define C_TAIL_LISTED 37      // triangles listed by flip tails (also counted in C_FLIP_LISTED)
-#define C_MODN3 38            // third list count of the bulk shifting passes (with C_MODN, C_MODN2)
+#define C_STAR 41             // 41..43: list counts of the bulk shifting passes
 #define TAIL_LIST 2048        // longest flip list the single-workgroup tail takes
 // status bits of constraint insertion (the other GA_ERR_* bits are in dev_common.h)
 #define GA_ERR_CONS_POINT 128     // a point lies inside a constraint segment
@@ -194,8 +198,8 @@ struct HullDev {
 #define GA_STRIPE_INTS 1024
 #endif
 #define C_FOLD 64             // counters[C_FOLD + k] = stripe sum of statistic k after a fold
-// Counters C_PEND, C_EXACT_*, C_INSERTED, C_DUPS, C_TESTS_INCIRCLE, C_RECON_TRIS, C_DELETED,
-// C_FLIPS_TOTAL and C_MOVED are striped statistics (MeshDev::stats); the others are single words.
+// Counters C_EXACT_*, C_INSERTED, C_DUPS, C_TESTS_INCIRCLE, C_RECON_TRIS, C_DELETED
+// and C_FLIPS_TOTAL are striped statistics (MeshDev::stats); the others are single words.
 #define C_DBG 48          // 48..63: first failure dump
 #define C_NCOUNTERS 64
 
@@ -253,11 +257,11 @@ void launch_shift_bulk(MeshDev &m, unsigned char *moved, int *mark, int *wl_out,
                        int cnt_next_slot, hipStream_t st);
 void launch_shift_star(MeshDev &m, unsigned char *moved, int *mark, const int *wl_in, int cnt_in_slot, int *wl_out,
                        int cnt_out_slot, int cnt_next_slot, hipStream_t st);
-// lists the vertices still pending into m.plist (count in counters[C_PLIST])
-void launch_pending_list(MeshDev &m, hipStream_t st);
-void launch_shift_commit(MeshDev &m, const unsigned char *moved, hipStream_t st);
-void launch_shift_greedy(MeshDev &m, int round, int grid, hipStream_t st);
-void launch_delete_round(MeshDev &m, unsigned int *mx, int round, int op, int grid, hipStream_t st);
+// once counters[cnt_slot] is zero: commits, and lists the vertices still pending into m.plist (count in
+// counters[C_PLIST])
+void launch_shift_commit(MeshDev &m, const unsigned char *moved, int cnt_slot, hipStream_t st);
+void launch_shift_greedy(MeshDev &m, int round, int *mark, int grid, hipStream_t st);
+void launch_delete_round(MeshDev &m, unsigned int *mx, int round, int grid, hipStream_t st);
 void launch_missing_init(MeshDev &m, const int *vor, int *mlist, int *loc, hipStream_t st);
 void launch_insert_round(MeshDev &m, int *mlist, int *loc, int op, int grid, hipStream_t st);
 void launch_relink(MeshDev &m, const int *modlist, int cnt_slot, int op, int grid, hipStream_t st);

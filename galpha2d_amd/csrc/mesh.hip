@@ -454,12 +454,14 @@ GA_INLINE double2 cand_pos(const MeshDev &m, const unsigned char *moved, int v)
 // and later passes only at the stars of the vertices reverted by the pass before (a worklist;
 // mark[] lists each vertex once).
 // also zeroes the revert marks, the count of k_shift_bulk's output list and that of the first
-// star pass's
+// star pass's, and keeps what the reconstruction left in the slot count and the status word
 __global__ void k_shift_init(MeshDev m, unsigned char *moved, int *mark, int cnt_out_slot, int cnt_next_slot)
 {
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         m.counters[cnt_out_slot] = 0;
         m.counters[cnt_next_slot] = 0;
+        m.counters[C_RECON_SLOTS] = *m.ntri;
+        m.counters[C_RECON_STATUS] = *m.status;
     }
     GRID_STRIDE(v, m.n) moved[v] = (m.vstate[v] == VS_PENDING) ? 1 : 0;
     GRID_STRIDE(v, m.V) mark[v] = 0;
@@ -501,6 +503,11 @@ __global__ void k_shift_bulk(MeshDev m, unsigned char *moved, int *mark, int *wl
     }
 }
 
+// Until a vertex is deleted the links are those of the reconstruction and its fans (off, fan: the
+// corners of every vertex) list the stars.  Eight lanes share a star: its triangles are
+// read at once, where a walk over the links is a chain of two dependent reads per triangle.
+#define FAN_LANES 8
+
 // cnt_next_slot: the output count of the next pass (neither this pass's input nor its output),
 // zeroed here so that no launch is needed between passes
 __global__ void k_shift_star(MeshDev m, unsigned char *moved, int *mark, const int *wl_in, int cnt_in_slot,
@@ -508,17 +515,10 @@ __global__ void k_shift_star(MeshDev m, unsigned char *moved, int *mark, const i
 {
     if (blockIdx.x == 0 && threadIdx.x == 0) m.counters[cnt_next_slot] = 0;
     int nw = m.counters[cnt_in_slot];
-    GRID_STRIDE(k, nw) {
+    for (auto [k, end, step] = xcd_range(nw, 256 / FAN_LANES, threadIdx.x / FAN_LANES); k < end; k += step) {
         int v = wl_in[k];
-        int t0 = m.vt[v], t = t0, i = slot_of(m.tv[t0], v), guard = 0;
-        do {
-            shift_check(m, moved, mark, m.tv[t], wl_out, cnt_out_slot);
-            int e = ic(m.tn[t], p1(i));
-            if (e < 0) { atomicOr(m.status, GA_ERR_WALK); break; }
-            t = enc_t(e);
-            i = p1(enc_j(e));
-            if (++guard > 100000) { atomicOr(m.status, GA_ERR_WALK); break; }
-        } while (t != t0);
+        for (int f = m.off[v] + threadIdx.x % FAN_LANES, f1 = m.off[v + 1]; f < f1; f += FAN_LANES)
+            shift_check(m, moved, mark, m.tv[enc_t(m.fan[f].x)], wl_out, cnt_out_slot);
     }
 }
 
@@ -536,34 +536,25 @@ void launch_shift_star(MeshDev &m, unsigned char *moved, int *mark, const int *w
               cnt_out_slot, cnt_next_slot);
 }
 
-__global__ void k_shift_commit(MeshDev m, const unsigned char *moved)
+// Commits the moves once the star passes have come to an end (cnt_slot: the output count of the last
+// one) and lists the few percent of the vertices that are still pending: the greedy and
+// deletion rounds only look at these; a listed vertex that has left the pending state since is skipped by
+// its state.  Before the end it only says so in C_SHIFTING: the list stays empty, so the
+// rounds launched behind it find nothing to do.
+__global__ __launch_bounds__(256) void k_shift_commit(MeshDev m, const unsigned char *moved, int cnt_slot)
 {
-    GRID_STRIDE(v, m.n) {
-        bool pend = m.vstate[v] == VS_PENDING;
-        if (pend && moved[v]) {
-            m.pos[v] = m.xy[v];
-            m.vstate[v] = VS_IN_MESH;
-            pend = false;
-        }
-        stat_inc(m.stats, C_PEND, pend);
-    }
-}
-
-void launch_shift_commit(MeshDev &m, const unsigned char *moved, hipStream_t st)
-{
-    GA_LAUNCH(k_shift_commit, dim3(FIXED_GRID), dim3(256), 0, st, m, moved);
-}
-
-// The greedy and deletion rounds only look at vertices that are still pending after bulk
-// shifting (a few percent), listed once; a listed vertex that has left the pending state since is
-// skipped by its state test.
-__global__ __launch_bounds__(256) void k_pending_list(MeshDev m)
-{
+    const bool open = m.counters[cnt_slot] != 0;
+    if (blockIdx.x == 0 && threadIdx.x == 0) m.counters[C_SHIFTING] = open;
+    if (open || *m.status) return;
     XCD_STRIDE(b0, m.n, 1024) {
         unsigned bits = 0;
         for (int j = 0; j < 4; j++) {
             int v = b0 + j * 256 + (int)threadIdx.x;
-            if (v < m.n && m.vstate[v] == VS_PENDING) bits |= 1u << j;
+            if (v >= m.n || m.vstate[v] != VS_PENDING) continue;
+            if (moved[v]) {
+                m.pos[v] = m.xy[v];
+                m.vstate[v] = VS_IN_MESH;
+            } else bits |= 1u << j;
         }
         int k = block_reserve(&m.counters[C_PLIST], __popc(bits));
         for (int j = 0; j < 4; j++)
@@ -571,65 +562,53 @@ __global__ __launch_bounds__(256) void k_pending_list(MeshDev m)
     }
 }
 
-void launch_pending_list(MeshDev &m, hipStream_t st)
+void launch_shift_commit(MeshDev &m, const unsigned char *moved, int cnt_slot, hipStream_t st)
 {
-    GA_LAUNCH(k_pending_list, dim3(FIXED_GRID), dim3(256), 0, st, m);
+    GA_LAUNCH(k_shift_commit, dim3(round_grid((m.n + 3) / 4)), dim3(256), 0, st, m, moved, cnt_slot);
 }
 
 GA_INLINE uint32_t vprio(int v, int round) { return hash32((uint32_t)v * 0x9E3779B1u ^ hash32((uint32_t)round + 0x1234567u)); }
 
 // Greedy round: a pending vertex whose pending neighbours all have lower priority moves to
-// its true position when all its star triangles stay counter-clockwise.  Decisions only;
-// the commit kernel applies them (so every decision sees the same snapshot).
-__global__ void k_shift_greedy(MeshDev m, int round, int *decide)
+// its true position when all its star triangles stay counter-clockwise.  mark[v] is 1 for a
+// pending vertex (the bulk passes reverted it), round + 2 once it has moved.  Whoever was
+// pending when the round began (1 or round + 2) counts as pending all round, so of two
+// neighbours only the one with the higher priority can move, whether or not the other sees it
+// move: one launch decides and moves.  (With one lane per vertex walking the links, and a launch
+// of its own for the moves, a round took 20 us at 1M points and
+// 18 at 12,007 in clusters, now 5.5 and 3.2.)
+__global__ __launch_bounds__(256) void k_shift_greedy(MeshDev m, int round, int *mark)
 {
     int np = m.counters[C_PLIST];
-    GRID_STRIDE(k, np) {
-        decide[k] = 0;
+    const int sub = threadIdx.x % FAN_LANES, shift = __lane_id() - sub;
+    for (auto [k, end, step] = xcd_range(np, 256 / FAN_LANES, threadIdx.x / FAN_LANES); k < end; k += step) {
         int v = m.plist[k];
-        if (m.vstate[v] != VS_PENDING) continue;
+        if (mark[v] != 1) continue;
         uint32_t p = vprio(v, round);
-        int t0 = m.vt[v];
-        int t = t0, i = slot_of(m.tv[t0], v);
-        bool ok = true, winner = true;
         double2 q = m.xy[v];
-        int guard = 0;
-        do {
-            int4 tt = m.tv[t];
-            int a = ic(tt, p1(i)), b = ic(tt, m1(i));
-            if (a < m.n && m.vstate[a] == VS_PENDING) {
+        bool no = false;
+        for (int f = m.off[v] + sub, f1 = m.off[v + 1]; f < f1 && !no; f += FAN_LANES) {
+            int2 e = m.fan[f];
+            int a = e.y, b = ic(m.tv[enc_t(e.x)], m1(enc_j(e.x)));
+            int sa = a < m.n ? mark[a] : 0;
+            if (sa == 1 || sa == round + 2) {
                 uint32_t pa = vprio(a, round);
-                if (pa > p || (pa == p && a > v)) { winner = false; break; }
+                no = pa > p || (pa == p && a > v);
             }
-            if (ok && orient_dev(m, q, m.pos[a], m.pos[b]) <= 0) ok = false;
-            int e = ic(m.tn[t], p1(i));
-            if (e < 0) { atomicOr(m.status, GA_ERR_WALK); winner = false; break; }
-            t = enc_t(e);
-            i = p1(enc_j(e));
-            if (++guard > 100000) { atomicOr(m.status, GA_ERR_WALK); winner = false; break; }
-        } while (t != t0);
-        if (winner && ok) decide[k] = 1;
-    }
-}
-
-__global__ void k_shift_greedy_commit(MeshDev m, const int *decide)
-{
-    int np = m.counters[C_PLIST];
-    GRID_STRIDE(k, np) {
-        bool d = decide[k] != 0;
-        if (d) {
-            int v = m.plist[k];
-            m.pos[v] = m.xy[v];
-            m.vstate[v] = VS_IN_MESH;
+            if (!no) no = orient_dev(m, q, m.pos[a], m.pos[b]) <= 0;
         }
-        stat_inc(m.stats, C_MOVED, d);
+        bool any = (__ballot(no) >> shift) & ((1u << FAN_LANES) - 1u);
+        if (!any && sub == 0) {
+            m.pos[v] = q;
+            m.vstate[v] = VS_IN_MESH;
+            mark[v] = round + 2;
+        }
     }
 }
 
-void launch_shift_greedy(MeshDev &m, int round, int grid, hipStream_t st)
+void launch_shift_greedy(MeshDev &m, int round, int *mark, int grid, hipStream_t st)
 {
-    GA_LAUNCH(k_shift_greedy, dim3(grid), dim3(256), 0, st, m, round, m.decide);
-    GA_LAUNCH(k_shift_greedy_commit, dim3(grid), dim3(256), 0, st, m, (const int *)m.decide);
+    GA_LAUNCH(k_shift_greedy, dim3(grid), dim3(256), 0, st, m, round, mark);
 }
 
 // ---- deletion of vertices that cannot move (star-shaped hole, ear clipping) --------------------
@@ -642,12 +621,12 @@ GA_INLINE unsigned long long prio64(int v, int round)
 }
 
 // distance-2 independence: every vertex records the largest priority in its closed neighbourhood
-// also zeroes the scratch and modified-list counts that k_del_apply of this round fills
+// also zeroes the scratch count and the flag of pending vertices that k_del_apply of this round sets
 __global__ void k_del_prio(MeshDev m, unsigned long long *mx, int round)
 {
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         m.counters[C_SCR] = 0;
-        m.counters[C_MODN] = 0;
+        m.counters[C_PLEFT] = 0;
     }
     int np = m.counters[C_PLIST];
     GRID_STRIDE(k, np) {
@@ -677,120 +656,248 @@ GA_INLINE void bond(const MeshDev &m, int T, int k, int X)
     if (X >= 0) set_link(m, enc_t(X), enc_j(X), enc(T, k));
 }
 
-__global__ void k_del_apply(MeshDev m, const unsigned long long *mx, int round, int op, int *list_out)
+// The hole is star-shaped from K (v's position): K lies left of every polygon edge.
+// An ear (A, B, C) is cut when it is counter-clockwise and K is left of or on the new
+// edge A -> C; that keeps K left of or on every edge of the remaining polygon, so the
+// ear holds no other polygon vertex (they are in angular order around K) and an ear
+// always exists.  (K strictly inside the ear is excluded by the same test.)
+template <class F>
+GA_INLINE void del_failed(const MeshDev &m, int v, int msz, F poly)
 {
-    int np = m.counters[C_PLIST];
-    GRID_STRIDE(kk, np) {
-        int v = m.plist[kk];
-        if (m.vstate[v] != VS_PENDING) continue;
-        unsigned long long p = prio64(v, round);
-        if (mx[v] != p) continue;
-        int t0 = m.vt[v], t = t0, i = slot_of(m.tv[t0], v), d = 0, guard = 0;
-        bool win = true;
-        do {
-            int a = ic(m.tv[t], p1(i));
-            if (mx[a] != p) { win = false; break; }
-            int e = ic(m.tn[t], p1(i));
-            if (e < 0) { atomicOr(m.status, GA_ERR_WALK); win = false; break; }
-            t = enc_t(e);
-            i = p1(enc_j(e));
-            d++;
-            if (++guard > 100000) { win = false; break; }
-        } while (t != t0);
-        if (!win) continue;
-        // scratch: poly[d], plink[d], slots[d]; list slots for the d - 2 new triangles
-        int base = wave_reserve_n<28>(&m.counters[C_SCR], 3 * d);
-        int lbase = wave_reserve_n<28>(&m.counters[C_MODN], d >= 2 ? d - 2 : 0);
-        if ((size_t)(base + 3 * d) > m.scratch_cap) {
-            atomicOr(m.status, GA_ERR_SCRATCH);
-            for (int k = 0; k < d - 2; k++) list_out[lbase + k] = -1;
-            continue;
-        }
-        int *poly = m.scratch + base, *plink = poly + d, *slots = plink + d;
-        t = t0; i = slot_of(m.tv[t0], v);
-        for (int k = 0; k < d; k++) {
-            int4 tt = m.tv[t];
-            poly[k] = ic(tt, p1(i));                 // triangle (v, l_k, l_k+1)
-            plink[k] = ic(m.tn[t], i);               // outer side of edge (l_k, l_k+1)
-            slots[k] = t;
-            int e = ic(m.tn[t], p1(i));
-            t = enc_t(e);
-            i = p1(enc_j(e));
-        }
-        // The hole is star-shaped from K (v's position): K lies left of every polygon edge.
-        // An ear (A, B, C) is cut when it is counter-clockwise and K is left of or on the new
-        // edge A -> C; that keeps K left of or on every edge of the remaining polygon, so the
-        // ear holds no other polygon vertex (they are in angular order around K) and an ear
-        // always exists.  (K strictly inside the ear is excluded by the same test.)
-        double2 K = m.pos[v];
-        int msz = d, used = 0;
-        while (msz > 3) {
-            int pick = -1;
-            for (int k = 0; k < msz && pick < 0; k++) {
-                int kp = k == 0 ? msz - 1 : k - 1, kn = k == msz - 1 ? 0 : k + 1;
-                double2 A = m.pos[poly[kp]], B = m.pos[poly[k]], C = m.pos[poly[kn]];
-                if (orient_dev(m, A, B, C) <= 0) continue;
-                if (orient_dev(m, A, C, K) < 0) continue;
-                pick = k;
-            }
-            if (pick < 0) {
-                atomicOr(m.status, GA_ERR_PATCH);
-                if (atomicCAS(&m.counters[C_DBG], 0, 1) == 0) {
-                    m.counters[C_DBG + 1] = v;
-                    m.counters[C_DBG + 2] = msz;
-                    for (int k = 0; k < msz && k < 12; k++) m.counters[C_DBG + 3 + k] = poly[k];
-                    m.dbg[0] = K.x; m.dbg[1] = K.y;
-                    for (int k = 0; k < msz && k < 15; k++) {
-                        m.dbg[2 + 2 * k] = m.pos[poly[k]].x;
-                        m.dbg[3 + 2 * k] = m.pos[poly[k]].y;
-                        m.dbg[32 + k] = (double)m.vstate[poly[k]];
-                    }
-                }
-                break;
-            }
-            int kp = pick == 0 ? msz - 1 : pick - 1, kn = pick == msz - 1 ? 0 : pick + 1;
-            int T = slots[used++];
-            int A = poly[kp], B = poly[pick], C = poly[kn];
-            m.tv[T] = make_int4(A, B, C, 0);
-            m.tn[T] = make_int4(-1, -1, -1, 0);
-            // slot 2 (opp C) = edge (A,B) -> plink[kp]; slot 0 (opp A) = edge (B,C) -> plink[pick]
-            bond(m, T, 2, plink[kp]);
-            bond(m, T, 0, plink[pick]);
-            m.vt[A] = T; m.vt[B] = T; m.vt[C] = T;
-            m.stamp[T] = op;
-            list_out[lbase + used - 1] = T;
-            // new polygon edge (A, C): its other side is slot 1 (opp B) of T
-            plink[kp] = enc(T, 1);
-            for (int k = pick; k < msz - 1; k++) { poly[k] = poly[k + 1]; plink[k] = plink[k + 1]; }
-            msz--;
-        }
-        if (msz == 3) {
-            if (orient_dev(m, m.pos[poly[0]], m.pos[poly[1]], m.pos[poly[2]]) <= 0) atomicOr(m.status, GA_ERR_PATCH);
-            int T = slots[used++];
-            m.tv[T] = make_int4(poly[0], poly[1], poly[2], 0);
-            m.tn[T] = make_int4(-1, -1, -1, 0);
-            bond(m, T, 2, plink[0]);   // (p0,p1)
-            bond(m, T, 0, plink[1]);   // (p1,p2)
-            bond(m, T, 1, plink[2]);   // (p2,p0)
-            m.vt[poly[0]] = T; m.vt[poly[1]] = T; m.vt[poly[2]] = T;
-            m.stamp[T] = op;
-            list_out[lbase + used - 1] = T;
-        }
-        for (int k = used; k < d - 2; k++) list_out[lbase + k] = -1;   // only after a failure
-        for (int k = used; k < d; k++) m.tv[slots[k]] = make_int4(GA_DEAD, GA_DEAD, GA_DEAD, 0);
-        m.vstate[v] = VS_MISSING;
-        m.vt[v] = slots[0];      // anchor for the re-insertion walk
-        m.pos[v] = m.xy[v];
-        stat_inc(m.stats, C_DELETED, true);
+    atomicOr(m.status, GA_ERR_PATCH);
+    if (atomicCAS(&m.counters[C_DBG], 0, 1) != 0) return;
+    m.counters[C_DBG + 1] = v;
+    m.counters[C_DBG + 2] = msz;
+    for (int k = 0; k < msz && k < 12; k++) m.counters[C_DBG + 3 + k] = poly(k);
+    m.dbg[0] = m.pos[v].x; m.dbg[1] = m.pos[v].y;
+    for (int k = 0; k < msz && k < 15; k++) {
+        m.dbg[2 + 2 * k] = m.pos[poly(k)].x;
+        m.dbg[3 + 2 * k] = m.pos[poly(k)].y;
+        m.dbg[32 + k] = (double)m.vstate[poly(k)];
     }
 }
 
-void launch_delete_round(MeshDev &m, unsigned int *mxraw, int round, int op, int grid, hipStream_t st)
+// one lane, any number d of corners (the polygon in the scratch arena); returns the first slot, -1 when
+// the arena is full
+__device__ __noinline__ int del_serial(const MeshDev &m, int v, int d)
+{
+    // scratch: poly[d], plink[d], slots[d]
+    int base = atomicAdd(&m.counters[C_SCR], 3 * d);
+    if ((size_t)(base + 3 * d) > m.scratch_cap) {
+        atomicOr(m.status, GA_ERR_SCRATCH);
+        return -1;
+    }
+    int *poly = m.scratch + base, *plink = poly + d, *slots = plink + d;
+    int t = m.vt[v], i = slot_of(m.tv[t], v);
+    for (int k = 0; k < d; k++) {
+        int4 tt = m.tv[t];
+        poly[k] = ic(tt, p1(i));                 // triangle (v, l_k, l_k+1)
+        plink[k] = ic(m.tn[t], i);               // outer side of edge (l_k, l_k+1)
+        slots[k] = t;
+        int e = ic(m.tn[t], p1(i));
+        t = enc_t(e);
+        i = p1(enc_j(e));
+    }
+    double2 K = m.pos[v];
+    int msz = d, used = 0;
+    while (msz > 3) {
+        int pick = -1;
+        for (int k = 0; k < msz && pick < 0; k++) {
+            int kp = k == 0 ? msz - 1 : k - 1, kn = k == msz - 1 ? 0 : k + 1;
+            double2 A = m.pos[poly[kp]], B = m.pos[poly[k]], C = m.pos[poly[kn]];
+            if (orient_dev(m, A, B, C) <= 0) continue;
+            if (orient_dev(m, A, C, K) < 0) continue;
+            pick = k;
+        }
+        if (pick < 0) {
+            del_failed(m, v, msz, [&](int k) { return poly[k]; });
+            break;
+        }
+        int kp = pick == 0 ? msz - 1 : pick - 1, kn = pick == msz - 1 ? 0 : pick + 1;
+        int T = slots[used++];
+        int A = poly[kp], B = poly[pick], C = poly[kn];
+        m.tv[T] = make_int4(A, B, C, 0);
+        m.tn[T] = make_int4(-1, -1, -1, 0);
+        // slot 2 (opp C) = edge (A,B) -> plink[kp]; slot 0 (opp A) = edge (B,C) -> plink[pick]
+        bond(m, T, 2, plink[kp]);
+        bond(m, T, 0, plink[pick]);
+        m.vt[A] = T; m.vt[B] = T; m.vt[C] = T;
+        // new polygon edge (A, C): its other side is slot 1 (opp B) of T
+        plink[kp] = enc(T, 1);
+        for (int k = pick; k < msz - 1; k++) { poly[k] = poly[k + 1]; plink[k] = plink[k + 1]; }
+        msz--;
+    }
+    if (msz == 3) {
+        if (orient_dev(m, m.pos[poly[0]], m.pos[poly[1]], m.pos[poly[2]]) <= 0) atomicOr(m.status, GA_ERR_PATCH);
+        int T = slots[used++];
+        m.tv[T] = make_int4(poly[0], poly[1], poly[2], 0);
+        m.tn[T] = make_int4(-1, -1, -1, 0);
+        bond(m, T, 2, plink[0]);   // (p0,p1)
+        bond(m, T, 0, plink[1]);   // (p1,p2)
+        bond(m, T, 1, plink[2]);   // (p2,p0)
+        m.vt[poly[0]] = T; m.vt[poly[1]] = T; m.vt[poly[2]] = T;
+    }
+    for (int k = used; k < d; k++) m.tv[slots[k]] = make_int4(GA_DEAD, GA_DEAD, GA_DEAD, 0);
+    return slots[0];
+}
+
+// LDS written by one lane and read by another of the same wave
+GA_INLINE void wave_lds_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+#define DEL_LANES 16         // lanes of a vertex
+#define DEL_MAX 64           // most corners of its polygon in LDS
+#define DEL_GROUPS (256 / DEL_LANES)
+
+// Bound by dependent reads: a block takes 64 listed vertices, keeps those that hold the maximum at
+// themselves, and gives each of them to 16 lanes.  One lane walks the star and puts the polygon into
+// LDS; the lanes check its corners' maxima and then test all ears at once (the one with the lowest index
+// is cut, and only its two neighbours are tested again).  One lane per vertex, walking the
+// star twice and testing ears one after another from memory, took 37 us per round at 1M points and
+// 40, up to 106, at 12,007 in clusters (long polygons), this 27 and 14, up to 40.
+__global__ __launch_bounds__(256) void k_del_apply(MeshDev m, const unsigned long long *mx, int round)
+{
+    __shared__ int s_poly[DEL_GROUPS][DEL_MAX], s_link[DEL_GROUPS][DEL_MAX], s_slot[DEL_GROUPS][DEL_MAX];
+    __shared__ double2 s_pos[DEL_GROUPS][DEL_MAX];
+    __shared__ unsigned char s_prv[DEL_GROUPS][DEL_MAX], s_nxt[DEL_GROUPS][DEL_MAX];
+    __shared__ int s_cand[64], s_nc;
+    const int np = m.counters[C_PLIST], tid = threadIdx.x, grp = tid / DEL_LANES, l = tid % DEL_LANES;
+    const int shift = (tid & 63) - l;
+    int *poly = s_poly[grp], *link = s_link[grp], *slot = s_slot[grp];
+    double2 *pos = s_pos[grp];
+    unsigned char *prv = s_prv[grp], *nxt = s_nxt[grp];
+    auto group = [&](bool b) { return (unsigned)(__ballot(b) >> shift) & ((1u << DEL_LANES) - 1u); };
+    bool left = false;   // a vertex stays pending
+    XCD_STRIDE(b0, np, 64) {
+        if (tid < 64) {
+            int v = b0 + tid < np ? m.plist[b0 + tid] : -1;
+            bool pend = v >= 0 && m.vstate[v] == VS_PENDING, cand = pend && mx[v] == prio64(v, round);
+            unsigned long long b = __ballot(cand);
+            if (cand) s_cand[__popcll(b & ((1ull << tid) - 1ull))] = v;
+            if (tid == 0) s_nc = __popcll(b);
+            left |= pend && !cand;
+        }
+        __syncthreads();
+        for (int q = grp, nc = s_nc; q < nc; q += DEL_GROUPS) {
+            const int v = s_cand[q];
+            const unsigned long long p = prio64(v, round);
+            int d = 0;
+            if (l == 0) {
+                int t0 = m.vt[v], t = t0, i = slot_of(m.tv[t0], v);
+                do {
+                    int4 tt = m.tv[t], tn = m.tn[t];
+                    if (d < DEL_MAX) {
+                        poly[d] = ic(tt, p1(i));   // triangle (v, l_k, l_k+1)
+                        link[d] = ic(tn, i);       // outer side of edge (l_k, l_k+1)
+                        slot[d] = t;
+                    } else if (mx[ic(tt, p1(i))] != p) { d = 0; break; }
+                    int e = ic(tn, p1(i));
+                    if (e < 0) { atomicOr(m.status, GA_ERR_WALK); d = 0; break; }
+                    t = enc_t(e);
+                    i = p1(enc_j(e));
+                    if (++d > 100000) { d = 0; break; }
+                } while (t != t0);
+            }
+            d = __shfl(d, shift, 64);
+            wave_lds_sync();
+            bool ok = d > 0;
+            for (int k = l; k < min(d, DEL_MAX); k += DEL_LANES) {
+                ok = ok && mx[poly[k]] == p;
+                pos[k] = m.pos[poly[k]];
+                prv[k] = (unsigned char)(k == 0 ? d - 1 : k - 1);
+                nxt[k] = (unsigned char)(k == d - 1 ? 0 : k + 1);
+            }
+            if (group(!ok)) { left = true; continue; }
+            int anchor = -1;
+            if (d > DEL_MAX) {
+                if (l == 0) anchor = del_serial(m, v, d);
+            } else {
+                wave_lds_sync();
+                const double2 K = m.pos[v];
+                auto ear = [&](int k) {
+                    double2 A = pos[prv[k]], B = pos[k], C = pos[nxt[k]];
+                    return orient_dev(m, A, B, C) > 0 && orient_dev(m, A, C, K) >= 0;
+                };
+                unsigned ears = 0;   // bit j: corner l + 16 j is an ear
+                if (d > 3)
+                    for (int k = l, j = 0; k < d; k += DEL_LANES, j++) ears |= (unsigned)ear(k) << j;
+                int msz = d, used = 0, A = 0;
+                for (; msz > 3; msz--, used++) {
+                    int pick = -1;
+                    for (int j = 0; j < DEL_MAX / DEL_LANES && pick < 0; j++) {
+                        unsigned b = group((ears >> j) & 1u);
+                        if (b) pick = DEL_LANES * j + __ffs((int)b) - 1;
+                    }
+                    if (pick < 0) break;
+                    A = prv[pick];
+                    const int C = nxt[pick];
+                    wave_lds_sync();
+                    if (l == 0) {
+                        const int T = slot[used], LA = link[A], LB = link[pick];
+                        const int a = poly[A], b = poly[pick], c = poly[C];
+                        m.tv[T] = make_int4(a, b, c, 0);
+                        // slot 2 (opposite c) = edge (a, b), slot 0 = edge (b, c), slot 1 = the new polygon edge (a, c)
+                        m.tn[T] = make_int4(-1, -1, -1, 0);
+                        bond(m, T, 2, LA);
+                        bond(m, T, 0, LB);
+                        m.vt[a] = T; m.vt[b] = T; m.vt[c] = T;
+                        link[A] = enc(T, 1);
+                        nxt[A] = (unsigned char)C;
+                        prv[C] = (unsigned char)A;
+                    }
+                    wave_lds_sync();
+                    if (pick % DEL_LANES == l) ears &= ~(1u << (pick / DEL_LANES));
+                    if (msz > 4)
+                        for (int e = 0; e < 2; e++) {
+                            const int k = e ? C : A, j = k / DEL_LANES;
+                            if (k % DEL_LANES == l) ears = (ears & ~(1u << j)) | ((unsigned)ear(k) << j);
+                        }
+                }
+                if (l == 0) {
+                    if (msz > 3) {
+                        // the corners that are left, from A on
+                        del_failed(m, v, msz, [&](int k) {
+                            int x = A;
+                            while (k--) x = nxt[x];
+                            return poly[x];
+                        });
+                    } else {
+                        int x = A, y = nxt[x], z = nxt[y];
+                        if (orient_dev(m, pos[x], pos[y], pos[z]) <= 0) atomicOr(m.status, GA_ERR_PATCH);
+                        const int T = slot[used++];
+                        m.tv[T] = make_int4(poly[x], poly[y], poly[z], 0);
+                        m.tn[T] = make_int4(-1, -1, -1, 0);
+                        bond(m, T, 2, link[x]);   // (x, y)
+                        bond(m, T, 0, link[y]);   // (y, z)
+                        bond(m, T, 1, link[z]);   // (z, x)
+                        m.vt[poly[x]] = T; m.vt[poly[y]] = T; m.vt[poly[z]] = T;
+                    }
+                    for (int k = used; k < d; k++) m.tv[slot[k]] = make_int4(GA_DEAD, GA_DEAD, GA_DEAD, 0);
+                    anchor = slot[0];
+                }
+                wave_lds_sync();
+            }
+            if (l == 0 && anchor >= 0) {
+                m.vstate[v] = VS_MISSING;
+                m.vt[v] = anchor;      // for the re-insertion walk
+                m.pos[v] = m.xy[v];
+                stat_inc(m.stats, C_DELETED, true);
+            }
+        }
+        __syncthreads();
+    }
+    if (__syncthreads_or(left) && tid == 0) m.counters[C_PLEFT] = 1;
+}
+
+void launch_delete_round(MeshDev &m, unsigned int *mxraw, int round, int grid, hipStream_t st)
 {
     unsigned long long *mx = (unsigned long long *)mxraw;
     GA_LAUNCH(k_del_prio, dim3(grid), dim3(256), 0, st, m, mx, round);
-    GA_LAUNCH(k_del_apply, dim3(grid), dim3(256), 0, st, m, (const unsigned long long *)mx, round, op,
-                       m.dellist);
+    GA_LAUNCH(k_del_apply, dim3(std::max(8, grid / 4 & ~7)), dim3(256), 0, st, m, (const unsigned long long *)mx, round);
 }
 
 // ---- missing-site insertion ------------------------------------------------------------------
@@ -833,6 +940,8 @@ GA_INLINE void missing_anchor(const MeshDev &m, const int *__restrict__ vor, int
 
 __global__ __launch_bounds__(256) void k_missing_init(MeshDev m, const int *__restrict__ vor, int *mlist, int *loc)
 {
+    // launched behind rounds that may not have been enough: nothing is listed then
+    if (m.counters[C_SHIFTING] || m.counters[C_PLEFT] || *m.status) return;
     // block-uniform loop: 1024 vertices per block and step, one list reservation per step
     XCD_STRIDE(b0, m.n, 1024) {
         unsigned bits = 0;
@@ -855,11 +964,14 @@ void launch_missing_init(MeshDev &m, const int *vor, int *mlist, int *loc, hipSt
 }
 
 // located: lt = (type << 2) | edge ; type 1 inside, 2 on edge, 3 duplicate ; -1 not located
-// also zeroes the modified-slot count that k_insert of this round fills (the previous round's
-// relink, which read it, has finished)
+// also zeroes the modified-slot count and the flag of missing vertices that k_insert of this round
+// sets (the previous round's relink, which read the count, has finished)
 __global__ void k_locate(MeshDev m, const int *mlist, int *loc, int *lt, int op)
 {
-    if (blockIdx.x == 0 && threadIdx.x == 0) m.counters[C_MODN] = 0;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        m.counters[C_MODN] = 0;
+        m.counters[C_MLEFT] = 0;
+    }
     int nm = m.counters[C_MISS];
     GRID_STRIDE(k, nm) {
         int v = mlist[k];
@@ -919,10 +1031,14 @@ __global__ void k_locate(MeshDev m, const int *mlist, int *loc, int *lt, int op)
 __global__ void k_insert(MeshDev m, const int *mlist, const int *loc, const int *lt, int op, int *list_out)
 {
     int nm = m.counters[C_MISS];
+    bool left = false;   // a vertex stays missing
     GRID_STRIDE(k, nm) {
         int L = lt[k];
-        if (L < 0) continue;
         int v = mlist[k];
+        if (L < 0) {
+            left |= m.vstate[v] == VS_MISSING;
+            continue;
+        }
         int t = loc[k];
         unsigned long long key = ((unsigned long long)op << 32) | (0xffffffffu - (unsigned)oid(m, v));
         int type = L >> 2, i = L & 3;
@@ -933,7 +1049,10 @@ __global__ void k_insert(MeshDev m, const int *mlist, const int *loc, const int 
         int q0 = wave_reserve_mult(&m.counters[C_MODN], win, 4);
         int q1 = q0 + 1, q2 = q0 + 2, q3 = q0 + 3;
         int s = wave_reserve_mult(m.ntri, win, 2);
-        if (!win) continue;
+        if (!win) {
+            left = true;
+            continue;
+        }
         if (type == 1) {
             if (s + 2 > m.cap) {
                 atomicOr(m.status, GA_ERR_CAPACITY);
@@ -986,6 +1105,8 @@ __global__ void k_insert(MeshDev m, const int *mlist, const int *loc, const int 
         m.pos[v] = m.xy[v];
         stat_inc(m.stats, C_INSERTED, true);
     }
+    // (one store per block: a million to the one word took 0.4 ms)
+    if (__syncthreads_or(left) && threadIdx.x == 0) m.counters[C_MLEFT] = 1;
 }
 
 void launch_insert_round(MeshDev &m, int *mlist, int *loc, int op, int grid, hipStream_t st)
@@ -1060,10 +1181,12 @@ GA_INLINE bool cons_has(const MeshDev &m, int a, int b)
 }
 
 // ---- flipping ---------------------------------------------------------------------------------
-// every slot in use (dead ones are skipped by the test); no atomics: the list is the identity
+// every slot in use (dead ones are skipped by the test); no atomics: the list is the identity.
+// Launched behind rounds that may not have been enough: the list is empty then.
 __global__ void k_flip_all(MeshDev m, int op, int *list, int cnt_slot)
 {
-    int n = ntri_used(m);
+    const bool early = m.counters[C_SHIFTING] || m.counters[C_PLEFT] || m.counters[C_MLEFT] || *m.status;
+    int n = early ? 0 : ntri_used(m);
     GRID_STRIDE(t, n) {
         m.stamp[t] = op;
         list[t] = t;
