@@ -57,7 +57,7 @@ class _Alpha(C.Structure):
 # every symbol include/gpudt.h declares
 EXPORTS = ["gpudtComputeDT", "gpudtReleaseDTOutput", "gpudtGetLastError", "gpudtComputeAlpha",
            "gpudtReleaseAlpha", "galphaCreate", "galphaDestroy", "galphaLastError",
-           "galphaComputeHost", "galphaComputeDevice", "galphaDeviceTriangles",
+           "galphaComputeHost", "galphaComputeDevice", "galphaComputeHostAlpha", "galphaDeviceTriangles",
            "galphaCopyTriangles", "galphaGetStats", "galphaVoronoi", "galphaCopyAlpha",
            "galphaTextureFor", "galphaAutotune", "galphaBatch", "galphaBatchDevice", "galphaBatchTriangles", "galphaBatchCopyAlpha", "galphaFree", "galphaAutoTexture", "galphaKernelProbe",
            "galphaKernelProbeResult", "galphaServerCreate", "galphaServerDestroy", "galphaServerSubmit",
@@ -101,6 +101,8 @@ def lib():
     L.galphaComputeHost.restype = C.c_int
     L.galphaComputeDevice.argtypes = [vp, vp, C.c_int, C.c_int, C.c_int, vp]
     L.galphaComputeDevice.restype = C.c_int
+    L.galphaComputeHostAlpha.argtypes = [vp, C.POINTER(C.c_double), C.c_int, C.c_int]
+    L.galphaComputeHostAlpha.restype = C.c_int
     L.galphaComputeDeviceNoAlloc.argtypes = [C.c_int, vp, C.c_int, C.c_int, vp, C.c_int, vp]
     L.galphaComputeDeviceNoAlloc.restype = C.c_int
     L.galphaDeviceTriangles.argtypes = [vp, C.POINTER(vp), ip]
@@ -288,26 +290,44 @@ def auto_texture(n):
     return lib().galphaAutoTexture(int(n))
 
 
+class _HostArray:
+    """A host array that the library allocated, handed over to numpy (the base of the array made
+    from it): freed with the last view of it."""
+    __slots__ = ("__array_interface__", "_free", "_ptr")
+
+    def __init__(self, ptr, shape, dtype):
+        self._ptr = C.cast(ptr, C.c_void_p)
+        self._free = lib().galphaFree
+        self.__array_interface__ = dict(data=(self._ptr.value, False), shape=shape, typestr=np.dtype(dtype).str, version=3)
+
+    def __del__(self):
+        self._free(self._ptr)
+
+
 def _alpha_to_numpy(A):
+    """Takes the arrays out of a result (what is left of it is still to be released)."""
     a = A.contents
 
-    def arr(p, n, dt):
-        if n <= 0:
+    def arr(name, n, dt):
+        p = getattr(a, name)
+        if n <= 0 or not p:
             return np.zeros(0, dtype=dt)
-        return np.ctypeslib.as_array(p, shape=(n,)).astype(dt, copy=True)
+        owner = _HostArray(p, (n,), dt)
+        setattr(a, name, type(p)())
+        return np.asarray(owner)
     return dict(
-        spectrum=arr(a.spectrum, a.specSize, np.float64),
-        tri_ro_rank=arr(a.tri_ro_rank, a.nTris, np.int32),
-        edge_t=arr(a.edge_t, a.nEdges, np.int32), edge_vopp=arr(a.edge_vopp, a.nEdges, np.int32),
-        edge_ro_rank=arr(a.edge_ro_rank, a.nEdges, np.int32),
-        edge_nu_min=arr(a.edge_nu_min_rank, a.nEdges, np.int32),
-        edge_nu_max=arr(a.edge_nu_max_rank, a.nEdges, np.int32),
-        vert_nu_min=arr(a.vert_nu_min_rank, a.nPoints, np.int32),
-        vert_nu_max=arr(a.vert_nu_max_rank, a.nPoints, np.int32),
-        master_simplex=arr(a.master_simplex, a.masterSize, np.int32),
-        master_st=arr(a.master_st, a.masterSize, np.int32),
-        master_at=arr(a.master_at, a.masterSize, np.int32),
-        spec_pointers=arr(a.spec_pointers, a.nSpecPointers, np.int32))
+        spectrum=arr("spectrum", a.specSize, np.float64),
+        tri_ro_rank=arr("tri_ro_rank", a.nTris, np.int32),
+        edge_t=arr("edge_t", a.nEdges, np.int32), edge_vopp=arr("edge_vopp", a.nEdges, np.int32),
+        edge_ro_rank=arr("edge_ro_rank", a.nEdges, np.int32),
+        edge_nu_min=arr("edge_nu_min_rank", a.nEdges, np.int32),
+        edge_nu_max=arr("edge_nu_max_rank", a.nEdges, np.int32),
+        vert_nu_min=arr("vert_nu_min_rank", a.nPoints, np.int32),
+        vert_nu_max=arr("vert_nu_max_rank", a.nPoints, np.int32),
+        master_simplex=arr("master_simplex", a.masterSize, np.int32),
+        master_st=arr("master_st", a.masterSize, np.int32),
+        master_at=arr("master_at", a.masterSize, np.int32),
+        spec_pointers=arr("spec_pointers", a.nSpecPointers, np.int32))
 
 
 _ALPHA_ARRAYS = (("spectrum", "spectrum", C.c_double), ("tri_ro_rank", "tri_ro_rank", C.c_int),
@@ -712,9 +732,6 @@ def compute_alpha_shapes(points, fbo_size):
     (AlphaShape/Alpha_Shapes_2D.cu:206-233): DT + alpha spectrum, intervals and master list."""
     ctx = default_context()
     xy = np.ascontiguousarray(points, dtype=np.float64)
-    d = DeviceBuffer(xy)
-    ctx.compute_device(d.ptr, xy.shape[0], fbo_size, with_alpha=True)
-    tris = ctx.triangles()
-    res = ctx.alpha()
-    d.free()
-    return tris, res
+    if ctx._L.galphaComputeHostAlpha(ctx._h, _dp(xy), xy.shape[0], int(fbo_size)) < 0:
+        ctx._err("galphaComputeDevice")
+    return ctx.triangles(), ctx.alpha()

@@ -1972,16 +1972,41 @@ void alpha_run_batch(AlphaDev &d, const double *d_xy, int n, const int *d_tris9,
     }
 }
 
+// the arrays of a result being copied to the host
+struct AlphaCopy {
+    void **dst[16];
+    CopyPart part[16];
+    int n = 0;
+    void add(void **to, const void *src, size_t bytes)
+    {
+        dst[n] = to;
+        part[n++] = CopyPart{src, bytes};
+    }
+    void run(HostStage &stage, hipStream_t st)
+    {
+        for (int k = 0; k < n; k++) {
+            *dst[k] = galpha_host_alloc(part[k].bytes);
+            if (!*dst[k]) throw GalphaError("host allocation failed");
+        }
+        const char *p = stage_gather(stage, part, n, st);
+        for (int k = 0; k < n; k++) {
+            if (p) {
+                memcpy(*dst[k], p, part[k].bytes);
+                p += (part[k].bytes + 15) & ~(size_t)15;
+            } else if (part[k].bytes) {
+                stage_d2h(stage, *dst[k], part[k].src, part[k].bytes, st);
+            }
+        }
+    }
+};
+
 PGPUDTALPHA alpha_copy_to_host(AlphaDev &d, HostStage &stage, hipStream_t st)
 {
     PGPUDTALPHA A = (PGPUDTALPHA)calloc(1, sizeof(GPUDTALPHA));
     A->nPoints = d.n; A->nEdges = d.E; A->nTris = d.F; A->specSize = d.specSize;
     A->masterSize = d.M; A->nSpecPointers = d.nsp;
-    auto cp = [&](void **dst, int idx, size_t bytes) {
-        *dst = galpha_host_alloc(bytes);
-        if (!*dst) throw GalphaError("host allocation failed");
-        if (bytes) stage_d2h(stage, *dst, d.b[idx].p, bytes, st);
-    };
+    AlphaCopy c;
+    auto cp = [&](void **dst, int idx, size_t bytes) { c.add(dst, d.b[idx].p, bytes); };
     cp((void **)&A->spectrum, AB_SPEC, 8 * (size_t)d.specSize);
     cp((void **)&A->tri_ro_rank, AB_TRANK, 4 * (size_t)d.F);
     cp((void **)&A->edge_t, AB_ET, 4 * (size_t)d.E);
@@ -1995,6 +2020,7 @@ PGPUDTALPHA alpha_copy_to_host(AlphaDev &d, HostStage &stage, hipStream_t st)
     cp((void **)&A->master_st, AB_OVAL, 4 * (size_t)d.M);
     cp((void **)&A->master_at, AB_MKEY, 4 * (size_t)d.M);
     cp((void **)&A->spec_pointers, AB_SP, 4 * (size_t)d.nsp);
+    c.run(stage, st);
     return A;
 }
 
@@ -2011,10 +2037,9 @@ PGPUDTALPHA alpha_copy_set_to_host(AlphaDev &d, int set, HostStage &stage, hipSt
     if (!A) throw GalphaError("host allocation failed");
     A->nPoints = np; A->nEdges = ne; A->nTris = nt; A->specSize = ns;
     A->masterSize = nm; A->nSpecPointers = ns;
+    AlphaCopy c;
     auto cp = [&](void **dst, int idx, size_t elem, size_t first, size_t count) {
-        *dst = galpha_host_alloc(count * elem);
-        if (!*dst) throw GalphaError("host allocation failed");
-        if (count) stage_d2h(stage, *dst, (char *)d.b[idx].p + first * elem, count * elem, st);
+        c.add(dst, (char *)d.b[idx].p + first * elem, count * elem);
     };
     cp((void **)&A->spectrum, AB_SPEC, 8, s0, ns);
     cp((void **)&A->tri_ro_rank, AB_TRANK, 4, t0, nt);
@@ -2031,6 +2056,7 @@ PGPUDTALPHA alpha_copy_set_to_host(AlphaDev &d, int set, HostStage &stage, hipSt
     // spec pointers of rank r >= 1 of this set: distinct key number specstart - set + r - 1
     int R = ns - 1;
     cp((void **)&A->spec_pointers, AB_SP, 4, R > 0 ? (size_t)(1 + s0 - set) - 1 : 0, R > 0 ? (size_t)R + 1 : 1);
+    c.run(stage, st);
     A->spec_pointers[0] = -1;
     for (int r = 1; r <= R; r++) A->spec_pointers[r] -= m0;
     for (int k = 0; k < ne; k++) A->edge_t[k] -= t0;

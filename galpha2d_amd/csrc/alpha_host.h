@@ -43,7 +43,14 @@ struct HostStage {
     size_t half = 0;
     hipEvent_t ev[2] = {nullptr, nullptr};
     CopyPool *pool = nullptr;    // started on the first large copy, joined by stage_free
+    bool busy = false;           // an upload from the first half may be in flight (event 0)
 };
+struct CopyPart {
+    const void *src;             // device, 4-byte aligned
+    size_t bytes;                // a multiple of 4
+};
+// n <= 16 device arrays into the pinned staging; the first one's host address (see galpha.cpp)
+const char *stage_gather(HostStage &s, const CopyPart *parts, int n, hipStream_t st);
 // dst (host) <- src (device); returns when dst holds the data
 void stage_d2h(HostStage &s, void *dst, const void *src, size_t bytes, hipStream_t st);
 // dst (device) <- src (host); returns when src may be reused (the copies are ordered on st)

@@ -285,6 +285,10 @@ static unsigned long long host_hash(HostStage &s, const void *p, size_t n)
 
 static void stage_ensure(HostStage &s)
 {
+    if (s.busy) {   // an upload that was not waited for may still read the first half
+        s.busy = false;
+        HIPCHK(hipEventSynchronize(s.ev[0]));
+    }
     if (s.p) return;
     if (t_arena) throw GalphaError("pinned staging is not available in a no-allocation call");
     HIPCHK(hipHostMalloc((void **)&s.p, 2 * STAGE_HALF, hipHostMallocDefault));
@@ -344,9 +348,37 @@ void stage_h2d_hash(HostStage &s, void *dst, const void *src, size_t bytes, hipS
         HIPCHK(hipMemcpyAsync((char *)dst + off, s.p + (i & 1) * s.half, len, hipMemcpyHostToDevice, st));
         HIPCHK(hipEventRecord(s.ev[i & 1], st));
     }
-    // the staging halves are free again once their last DMAs ended
+    // the staging halves are free again once their last DMAs ended (the next use of the staging waits
+    // for a single one)
+    if (nch == 1) {
+        s.busy = true;
+        return;
+    }
     HIPCHK(hipEventSynchronize(s.ev[(nch - 1) & 1]));
     if (nch >= 2) HIPCHK(hipEventSynchronize(s.ev[nch & 1]));
+}
+
+// Arrays of up to STAGE_GATHER bytes together: one launch writes them into the pinned staging (16-byte
+// aligned, one after another) and one wait follows, where a copy and a wait each took 15 to 30 us.
+// Returns the address of the first, NULL when they are too large.
+static const size_t STAGE_GATHER = (size_t)16 << 20;
+
+const char *stage_gather(HostStage &s, const CopyPart *parts, int n, hipStream_t st)
+{
+    CopyParts g{};
+    size_t at = 0;
+    for (int k = 0; k < n; k++) {
+        g.src[k] = (const int *)parts[k].src;
+        g.at[k] = at / 4;
+        g.words[k] = parts[k].bytes / 4;
+        at += (parts[k].bytes + 15) & ~(size_t)15;
+    }
+    if (at > STAGE_GATHER) return nullptr;
+    stage_ensure(s);
+    g.n = n;
+    launch_gather_parts(g, (int *)s.p, at / 4, st);
+    HIPCHK(hipStreamSynchronize(st));
+    return s.p;
 }
 
 static const int SNAP_INTS = 256;
@@ -634,7 +666,7 @@ static void run_pba(galpha_ctx *c, const double *d_xy, const BatchDev &bd, int *
 {
     hipStream_t st = c->stream;
     launch_fill_i32(c->smap.as<int>(), 0x7fffffff, bd.P, st);
-    launch_vset(bd, c->vset.as<int>(), st);
+    if (!perm) launch_vset(bd, c->vset.as<int>(), st);   // (else the renumbering has done it)
     launch_splat((const double2 *)d_xy, bd, perm, c->smap.as<int>(), c->pix.as<int>(), c->fpix.as<int>(), st);
     {
         IntFills f;   // island marks, and the island counters of the first pass
@@ -1524,6 +1556,34 @@ int galphaComputeDevice(galpha_ctx *c, const double *d_xy, int n, int fboSize, i
             throw;
         }
         c->stream = own;
+        return F;
+    } catch (const std::exception &e) {
+        return fail(c, e);
+    }
+}
+
+// DT and alpha shapes of n host points; the results stay on the device (galphaCopyTriangles,
+// galphaCopyAlpha), as after galphaComputeDevice.  The points go through the context's own buffer: an
+// allocation and its release around every call cost some 60 us.
+int galphaComputeHostAlpha(galpha_ctx *c, const double *xy, int n, int fboSize)
+{
+    if (!c) return -1;
+    try {
+        HIPCHK(hipSetDevice(c->device));
+        double bb[5] = {0, 0, 1, 1, 0};
+        check_texture(fboSize);
+        if (n >= 3) check_slot_capacity((long long)n + frame_count(fboSize));
+        if (n > 0) bbox_host(xy, n, bb);
+        c->xy.ensure(16 * (size_t)std::max(n, 1));
+        if (n > 0) stage_h2d(c->stage, c->xy.p, xy, 16 * (size_t)n, c->stream);
+        int F = run_dt(c, c->xy.as<double>(), n, fboSize, bb);
+        c->last_alpha = false;
+        auto t0 = std::chrono::steady_clock::now();
+        alpha_run(c->alpha, c->xy.as<double>(), n, c->out9.as<int>(), F, c->stream, &c->stats);
+        c->last_alpha = true;
+        HIPCHK(hipStreamSynchronize(c->stream));
+        auto t1 = std::chrono::steady_clock::now();
+        c->stats.ms_alpha = std::chrono::duration<double, std::milli>(t1 - t0).count();
         return F;
     } catch (const std::exception &e) {
         return fail(c, e);

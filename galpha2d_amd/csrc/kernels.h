@@ -226,6 +226,13 @@ struct IntSegments {
     int n;
 };
 void launch_gather_segments(const IntSegments &g, int *dst, hipStream_t st);
+// up to 16 int arrays of any size to dst + at[k] (multiples of 4; dst: pinned host memory)
+struct CopyParts {
+    const int *src[16];
+    size_t at[16], words[16];
+    int n;
+};
+void launch_gather_parts(const CopyParts &g, int *dst, size_t words, hipStream_t st);
 // up to eight device int arrays, each set to one value, in one launch
 struct IntFills {
     int *p[8];

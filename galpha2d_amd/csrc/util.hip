@@ -113,6 +113,30 @@ void launch_gather_segments(const IntSegments &g, int *dst, hipStream_t st)
     GA_LAUNCH(k_gather_segments, dim3(blocks), dim3(256), 0, st, g, dst);
 }
 
+// several device arrays into pinned host memory, at 16-byte aligned places (the host waits on the stream)
+__global__ __launch_bounds__(256) void k_gather_parts(CopyParts g, int *dst)
+{
+    const size_t tid = blockIdx.x * (size_t)blockDim.x + threadIdx.x, nth = (size_t)gridDim.x * blockDim.x;
+    for (int k = 0; k < g.n; k++) {
+        const int *src = g.src[k];
+        int *to = dst + g.at[k];
+        const size_t n = g.words[k];
+        size_t head = 0;
+        if (((uintptr_t)src & 15) == 0) {
+            for (size_t i = tid; i < n / 4; i += nth) ((int4 *)to)[i] = ((const int4 *)src)[i];
+            head = n & ~(size_t)3;
+        }
+        for (size_t i = head + tid; i < n; i += nth) to[i] = src[i];
+    }
+    __threadfence_system();
+}
+
+void launch_gather_parts(const CopyParts &g, int *dst, size_t words, hipStream_t st)
+{
+    const int blocks = (int)std::max((size_t)1, std::min((size_t)1024, (words / 4 + 255) / 256));
+    GA_LAUNCH(k_gather_parts, dim3(blocks), dim3(256), 0, st, g, dst);
+}
+
 // several device int arrays, each set to one value, in one launch (16-byte stores where a
 // segment's start is 16-byte aligned)
 __global__ void k_fill_multi(IntFills f)

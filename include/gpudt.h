@@ -212,6 +212,8 @@ int galphaComputeHost(galpha_ctx *ctx, const double *xy, int n, int fboSize,
  * stream is a hipStream_t (NULL = the context's own stream). */
 int galphaComputeDevice(galpha_ctx *ctx, const double *d_xy, int n, int fboSize, int with_alpha,
                         void *stream);
+/* The same with the alpha result for n points in host memory (results on the device as well). */
+int galphaComputeHostAlpha(galpha_ctx *ctx, const double *xy, int n, int fboSize);
 /* Constraint edges (n pairs of point indices, the layout of GPUDTPARAMS::constraints) for the
  * following single-set runs of this context (galphaComputeHost / galphaComputeDevice), until set
  * again; n = 0 clears them.  Batches and serving reject a context that holds constraints. */
