@@ -770,12 +770,13 @@ static const double *renumber_points(galpha_ctx *c, const double *d_xy, const Ba
     c->perm.ensure(4 * (size_t)n + 64);
     c->xys.ensure(16 * (size_t)n + 64);
     c->pcell.ensure(4 * (size_t)n + 64);
+    c->lt.ensure(4 * (size_t)n);   // (the missing sites' later)
     c->ccount.ensure(4 * nc + 64);
     c->ccursor.ensure(4 * nc + 64);
     c->scanTmp.ensure(scan_temp_bytes(nc) + 4096);
     launch_vset(bd, c->vset.as<int>(), st);
     HIPCHK(hipMemsetAsync(c->ccount.p, 0, 4 * nc, st));
-    launch_renumber((const double2 *)d_xy, bd, c->pcell.as<int>(), c->ccount.as<int>(), c->ccursor.as<int>(),
+    launch_renumber((const double2 *)d_xy, bd, c->pcell.as<int>(), c->lt.as<int>(), c->ccount.as<int>(), c->ccursor.as<int>(),
                     plan.ncells, c->scanTmp.p, c->perm.as<int>(), c->xys.as<double2>(), st);
     return c->xys.as<double>();
 }

@@ -211,7 +211,7 @@ void launch_splat(const double2 *xy, const BatchDev &b, const int *perm, int *sm
                   hipStream_t st);
 // spatial numbering of the real points: perm[new] = input index, xys[new] = xy[perm[new]];
 // ccount (ncells + 1 ints) zero on entry
-void launch_renumber(const double2 *xy, const BatchDev &b, int *cell, int *ccount, int *cursor, int ncells,
+void launch_renumber(const double2 *xy, const BatchDev &b, int *cell, int *slot, int *ccount, int *first, int ncells,
                      void *scan_tmp, int *perm, double2 *xys, hipStream_t st);
 void launch_pba(const PbaBuffers &p, const int *pix, const BatchDev &b, hipStream_t st);
 void launch_islands(const int *vor, const int *pix, const BatchDev &b, int *bad, int *flag, hipStream_t st);

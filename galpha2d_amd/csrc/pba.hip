@@ -77,24 +77,57 @@ GA_INLINE unsigned spread14(unsigned v)
     return v;
 }
 
-__global__ void k_cell_count(const double2 *__restrict__ xy, BatchDev b, int *__restrict__ cell,
-                             int *__restrict__ ccount)
+// Bound by the atomics on the cells' counts: those of one block of 1,024 * PER points go through a table
+// in LDS first, so that a cell takes one per block.  (One per point, and a second one in the scatter: 48
+// + 78 us for 1M uniform points, 52 + 15 now; 137 + 97 for 250K in 8 clusters, whose cells are few and
+// full, so that their atomics queue up on a few lines, 29 + under 10 now.)  PER is 4 from 128K points on, where that
+// leaves blocks enough (250K in clusters: 69 us with 1, 29 with 4).  slot[i]: the point's place in its cell.
+template <int PER>
+__global__ __launch_bounds__(1024) void k_cell_count(const double2 *__restrict__ xy, BatchDev b, int *__restrict__ cell,
+                                                     int *__restrict__ slot, int *__restrict__ ccount)
 {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= b.ntot) return;
-    const SetDesc &sd = b.sets[b.vset[i]];
-    int px, py;
-    point_pixel(sd, xy[i], &px, &py);
-    int c = sd.coff + (int)((spread14((unsigned)px >> 4) << 1) | spread14((unsigned)py >> 4));
-    cell[i] = c;
-    atomicAdd(&ccount[c], 1);
+    constexpr int TAB = 2048 * PER;
+    __shared__ int s_key[TAB], s_cnt[TAB];
+    for (int k = threadIdx.x; k < TAB; k += 1024) {
+        s_key[k] = -1;
+        s_cnt[k] = 0;
+    }
+    __syncthreads();
+    const int i0 = blockIdx.x * 1024 * PER + threadIdx.x;
+    int h[PER], at[PER];
+#pragma unroll
+    for (int u = 0; u < PER; u++) {
+        const int i = i0 + 1024 * u;
+        h[u] = at[u] = 0;
+        if (i >= b.ntot) continue;
+        const SetDesc &sd = b.sets[b.vset[i]];
+        int px, py;
+        point_pixel(sd, xy[i], &px, &py);
+        const int c = sd.coff + (int)((spread14((unsigned)px >> 4) << 1) | spread14((unsigned)py >> 4));
+        cell[i] = c;
+        for (h[u] = (int)(((unsigned)c * 0x9E3779B1u) % TAB);; h[u] = (h[u] + 1) % TAB) {
+            const int k = atomicCAS(&s_key[h[u]], -1, c);
+            if (k == -1 || k == c) break;
+        }
+        at[u] = atomicAdd(&s_cnt[h[u]], 1);
+    }
+    __syncthreads();
+    for (int k = threadIdx.x; k < TAB; k += 1024)
+        if (s_cnt[k]) s_cnt[k] = atomicAdd(&ccount[s_key[k]], s_cnt[k]);
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < PER; u++) {
+        const int i = i0 + 1024 * u;
+        if (i < b.ntot) slot[i] = s_cnt[h[u]] + at[u];
+    }
 }
 
-// cursor = exclusive prefix of the cell counts; perm[new index] = input index
-__global__ void k_cell_scatter(const int *__restrict__ cell, int n, int *__restrict__ cursor, int *__restrict__ perm)
+// first = exclusive prefix of the cell counts; perm[new index] = input index
+__global__ void k_cell_scatter(const int *__restrict__ cell, const int *__restrict__ slot, int n,
+                               const int *__restrict__ first, int *__restrict__ perm)
 {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) perm[atomicAdd(&cursor[cell[i]], 1)] = i;
+    if (i < n) perm[first[cell[i]] + slot[i]] = i;
 }
 
 __global__ void k_gather_xy(const double2 *__restrict__ xy, const int *__restrict__ perm, int n,
@@ -785,14 +818,18 @@ void launch_vset(const BatchDev &b, int *vset, hipStream_t st)
 }
 
 // ccount (ncells + 1 entries) must be zero on entry
-void launch_renumber(const double2 *xy, const BatchDev &b, int *cell, int *ccount, int *cursor, int ncells,
+void launch_renumber(const double2 *xy, const BatchDev &b, int *cell, int *slot, int *ccount, int *first, int ncells,
                      void *scan_tmp, int *perm, double2 *xys, hipStream_t st)
 {
     int n = b.ntot;
     if (n <= 0) return;
-    GA_LAUNCH(k_cell_count, dim3((n + 255) / 256), dim3(256), 0, st, xy, b, cell, ccount);
-    launch_exclusive_scan(ccount, cursor, (size_t)ncells + 1, scan_tmp, st);
-    GA_LAUNCH(k_cell_scatter, dim3((n + 255) / 256), dim3(256), 0, st, (const int *)cell, n, cursor, perm);
+    if (n >= (1 << 17))
+        GA_LAUNCH(k_cell_count<4>, dim3((n + 4095) / 4096), dim3(1024), 0, st, xy, b, cell, slot, ccount);
+    else
+        GA_LAUNCH(k_cell_count<1>, dim3((n + 1023) / 1024), dim3(1024), 0, st, xy, b, cell, slot, ccount);
+    launch_exclusive_scan(ccount, first, (size_t)ncells + 1, scan_tmp, st);
+    GA_LAUNCH(k_cell_scatter, dim3((n + 255) / 256), dim3(256), 0, st, (const int *)cell, (const int *)slot, n,
+              (const int *)first, perm);
     GA_LAUNCH(k_gather_xy, dim3((n + 255) / 256), dim3(256), 0, st, xy, (const int *)perm, n, xys);
 }
 
