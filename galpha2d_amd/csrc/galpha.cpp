@@ -606,7 +606,7 @@ static BatchPlan plan_batch(const int *n, const int *T, const double *bb5, int n
         if (rb) acc[BM_ROWS] += Ts / rb;
         b.far_lds = std::max(b.far_lds, pba_far_lds(T[s], rb));
         acc[BM_PIX] += Ts * Ts / 1024;
-        acc[BM_RECON] += (Ts / 16) * (Ts / 16);   // one tile per 16 x 16-pixel cell
+        acc[BM_RECON] += (Ts / 16) * (Ts / 16) / RECON_TILES;   // one tile per 16 x 16-pixel cell
     }
     for (int k = 0; k < BM_COUNT; k++) b.blocks[k] = (int)acc[k];
     return b;
@@ -627,7 +627,7 @@ static void ensure_pba(galpha_ctx *c, const BatchPlan &b)
     c->vset.ensure(4 * (size_t)(b.V + 1));
     c->counters.ensure(COUNTER_BYTES);
     c->status.ensure(sizeof(int) * 4);
-    size_t ntiles = (size_t)std::max(b.blocks[BM_RECON], 1);
+    size_t ntiles = (size_t)RECON_TILES * std::max(b.blocks[BM_RECON], 1);
     c->tileCnt.ensure(4 * ntiles);
     c->tileOff.ensure(4 * ntiles);
     c->scanTmp.ensure(scan_temp_bytes(std::max(ntiles, (size_t)(b.V + 2))) + 4096);

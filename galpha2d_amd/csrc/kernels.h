@@ -43,6 +43,7 @@ GA_INLINE_HOST_DEVICE int set_of(const int *start, int nsets, int b)
 }
 
 // per-launch block maps (device arrays of nsets + 1 entries each)
+#define RECON_TILES 16   // 16 x 16-pixel tiles of a workgroup of the reconstruction (a 64 x 64 texture has 16)
 enum { BM_COLS, BM_LABEL, BM_ROWS, BM_PIX, BM_RECON, BM_COUNT };
 // rows of a block of k_pba_far_rows for a texture of side 1 << logT (0 above 4096, see pba.hip); want: rows
 // for blocks enough to fill the chip

@@ -152,75 +152,61 @@ GA_INLINE unsigned compact_bits(unsigned v)
 
 // Tiles of 16 x 16 2x2-block origins, one per 16 x 16-pixel cell, in the Morton order of the
 // cells (the order the real points are numbered in), so triangles are emitted in the spatial
-// order of their vertices.  Set s owns tiles [bm[s], bm[s + 1]) of the BM_RECON map; thread k of
-// a tile takes the block at (16 cx + k / 16, 16 cy + k % 16).
-GA_INLINE void recon_block(int lt, int *x, int *y)
+// order of their vertices.  A workgroup of the BM_RECON map takes RECON_TILES tiles of one set, a wave one
+// tile at a time; lane k takes the four blocks at (16 cx + k / 4, 16 cy + 4 (k % 4) ..): two 16-byte
+// reads and two single ones, where a thread per block read 16 labels for the same four.  Bound by
+// the labels read twice and, in the emission, by the gathers of the corners' pixels (T = 4096, 1M
+// points: 23 and 55 us, 43 and 85 with a thread per block and a workgroup per tile; 1,024 sets,
+// 268M pixels: 437 and 676 us, 1,673 and 2,065 with a search of the sets per tile).
+struct ReconLane {
+    int a[5], b[5];   // labels of column x and x + 1, rows y .. y + 4
+    int c[4], sum;    // triangles of the four blocks
+};
+GA_INLINE ReconLane recon_lane(const int *vor, int logT, int lt, int lane)
 {
-    *x = (int)(compact_bits((unsigned)lt >> 1) << 4) + (int)(threadIdx.x >> 4);
-    *y = (int)(compact_bits((unsigned)lt) << 4) + (int)(threadIdx.x & 15);
+    ReconLane r;
+    const int T = 1 << logT;
+    const int x = (int)(compact_bits((unsigned)lt >> 1) << 4) + (lane >> 2);
+    const int y = (int)(compact_bits((unsigned)lt) << 4) + 4 * (lane & 3);
+    r.sum = 0;
+    if (x < T - 1) {
+        const int *p = vor + ((size_t)x << logT) + y, *q = p + T;
+        const int4 u = *(const int4 *)p, w = *(const int4 *)q;
+        const int more = y + 4 < T ? 4 : 3;   // the texture's last row starts no block
+        r.a[0] = u.x; r.a[1] = u.y; r.a[2] = u.z; r.a[3] = u.w; r.a[4] = p[more];
+        r.b[0] = w.x; r.b[1] = w.y; r.b[2] = w.z; r.b[3] = w.w; r.b[4] = q[more];
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            r.c[k] = y + k < T - 1 ? recon_count(r.a[k], r.b[k], r.b[k + 1], r.a[k + 1]) : 0;
+            r.sum += r.c[k];
+        }
+    } else {
+#pragma unroll
+        for (int k = 0; k < 4; k++) r.c[k] = 0;
+    }
+    return r;
 }
 
 __global__ __launch_bounds__(256) void k_recon_count(const int *__restrict__ vor_all, BatchDev bd,
                                                      int *__restrict__ tile_cnt)
 {
     const int *bm = bd.bmap(BM_RECON);
-    int set = set_of(bm, bd.nsets, blockIdx.x);
+    const int set = set_of(bm, bd.nsets, blockIdx.x);
     const SetDesc &sd = bd.sets[set];
-    int logT = sd.logT;
-    int T = 1 << logT;
-    const int *vor = vor_all + sd.toff;
-    int tile = blockIdx.x;
-    int x, y;
-    recon_block(tile - bm[set], &x, &y);
-    int c = 0;
-    if (x < T - 1 && y < T - 1) {
-        size_t i0 = ((size_t)x << logT) + y, i1 = i0 + T;
-        c = recon_count(vor[i0], vor[i1], vor[i1 + 1], vor[i0 + 1]);
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int t0 = RECON_TILES * (int)blockIdx.x, l0 = RECON_TILES * ((int)blockIdx.x - bm[set]);
+#pragma unroll
+    for (int k = w; k < RECON_TILES; k += 4) {
+        int s = recon_lane(vor_all + sd.toff, sd.logT, l0 + k, lane).sum;
+        for (int d = 32; d > 0; d >>= 1) s += __shfl_down(s, d, 64);
+        if (lane == 0) tile_cnt[t0 + k] = s;
     }
-    __shared__ int ws[4];
-    int s = c;
-    for (int d = 32; d > 0; d >>= 1) s += __shfl_down(s, d, 64);
-    if ((threadIdx.x & 63) == 0) ws[threadIdx.x >> 6] = s;
-    __syncthreads();
-    if (threadIdx.x == 0) tile_cnt[tile] = ws[0] + ws[1] + ws[2] + ws[3];
 }
 
-__global__ __launch_bounds__(256) void k_recon_emit(const int *__restrict__ vor_all, const int *__restrict__ pix,
-                                                    BatchDev bd, const int *__restrict__ tile_off,
-                                                    int4 *__restrict__ tv, int4 *__restrict__ tn,
-                                                    int *__restrict__ status, int cap)
+// the triangles of one block from slot off on; tn is left to k_match, which writes all of it
+GA_INLINE void recon_emit_block(int a, int b, int cc, int d, int c, int off, const int *__restrict__ pix,
+                                int4 *__restrict__ tv, int *__restrict__ status)
 {
-    const int *bm = bd.bmap(BM_RECON);
-    int set = set_of(bm, bd.nsets, blockIdx.x);
-    const SetDesc &sd = bd.sets[set];
-    int logT = sd.logT;
-    int T = 1 << logT;
-    const int *vor = vor_all + sd.toff;
-    int tile = blockIdx.x;
-    int x, y;
-    recon_block(tile - bm[set], &x, &y);
-    int c = 0, a = 0, b = 0, cc = 0, d = 0;
-    if (x < T - 1 && y < T - 1) {
-        size_t i0 = ((size_t)x << logT) + y, i1 = i0 + T;
-        a = vor[i0]; b = vor[i1]; cc = vor[i1 + 1]; d = vor[i0 + 1];
-        c = recon_count(a, b, cc, d);
-    }
-    // block exclusive scan of c
-    __shared__ int ws[4];
-    int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    int inc = c;
-    for (int k = 1; k < 64; k <<= 1) {
-        int t = __shfl_up(inc, k, 64);
-        if (lane >= k) inc += t;
-    }
-    if (lane == 63) ws[w] = inc;
-    __syncthreads();
-    int off = tile_off[tile];
-    for (int i = 0; i < w; i++) off += ws[i];
-    off += inc - c;
-    if (c == 0) return;
-    if (off + c > cap) { atomicOr(status, GA_ERR_CAPACITY); return; }
-    int4 none = make_int4(-1, -1, -1, 0);
     if (c == 1) {
         int t0, t1, t2;
         if (a == b) { t0 = a; t1 = cc; t2 = d; }
@@ -228,40 +214,65 @@ __global__ __launch_bounds__(256) void k_recon_emit(const int *__restrict__ vor_
         else { t0 = a; t1 = b; t2 = cc; }   // c == d or d == a
         if (iorient(pix[t0], pix[t1], pix[t2]) <= 0) atomicOr(status, GA_ERR_RECON);
         tv[off] = make_int4(t0, t1, t2, 0);
-        tn[off] = none;
+        return;
+    }
+    int pa = pix[a], pb = pix[b], pc = pix[cc], pd = pix[d];
+    if (iorient(pa, pb, pc) > 0 && iorient(pa, pc, pd) > 0) {
+        tv[off] = make_int4(a, b, cc, 0);
+        tv[off + 1] = make_int4(a, cc, d, 0);
+    } else if (iorient(pb, pc, pd) > 0 && iorient(pb, pd, pa) > 0) {
+        tv[off] = make_int4(b, cc, d, 0);
+        tv[off + 1] = make_int4(b, d, a, 0);
     } else {
-        int pa = pix[a], pb = pix[b], pc = pix[cc], pd = pix[d];
-        if (iorient(pa, pb, pc) > 0 && iorient(pa, pc, pd) > 0) {
-            tv[off] = make_int4(a, b, cc, 0);
-            tv[off + 1] = make_int4(a, cc, d, 0);
-        } else if (iorient(pb, pc, pd) > 0 && iorient(pb, pd, pa) > 0) {
-            tv[off] = make_int4(b, cc, d, 0);
-            tv[off + 1] = make_int4(b, d, a, 0);
-        } else {
-            atomicOr(status, GA_ERR_RECON);
-            tv[off] = make_int4(a, b, cc, 0);
-            tv[off + 1] = make_int4(a, cc, d, 0);
-        }
-        tn[off] = none;
-        tn[off + 1] = none;
+        atomicOr(status, GA_ERR_RECON);
+        tv[off] = make_int4(a, b, cc, 0);
+        tv[off + 1] = make_int4(a, cc, d, 0);
     }
 }
 
-__global__ void k_set_ntri(const int *tile_cnt, const int *tile_off, int ntiles, int *ntri, int cap)
+__global__ __launch_bounds__(256) void k_recon_emit(const int *__restrict__ vor_all, const int *__restrict__ pix,
+                                                    BatchDev bd, const int *__restrict__ tile_cnt,
+                                                    const int *__restrict__ tile_off, int4 *__restrict__ tv,
+                                                    int *__restrict__ status, int *__restrict__ ntri, int cap)
 {
-    int F = tile_off[ntiles - 1] + tile_cnt[ntiles - 1];
-    *ntri = F > cap ? cap : F;
+    const int *bm = bd.bmap(BM_RECON);
+    const int set = set_of(bm, bd.nsets, blockIdx.x);
+    const SetDesc &sd = bd.sets[set];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int t0 = RECON_TILES * (int)blockIdx.x, l0 = RECON_TILES * ((int)blockIdx.x - bm[set]);
+    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) {
+        const int last = t0 + RECON_TILES - 1;
+        *ntri = min(tile_off[last] + tile_cnt[last], cap);
+    }
+    for (int k = w; k < RECON_TILES; k += 4) {
+        if (tile_cnt[t0 + k] == 0) continue;
+        const ReconLane r = recon_lane(vor_all + sd.toff, sd.logT, l0 + k, lane);
+        int inc = r.sum;
+        for (int d = 1; d < 64; d <<= 1) {
+            const int t = __shfl_up(inc, d, 64);
+            if (lane >= d) inc += t;
+        }
+        int off = tile_off[t0 + k] + inc - r.sum;
+        if (r.sum && off + r.sum > cap) {
+            atomicOr(status, GA_ERR_CAPACITY);
+            continue;
+        }
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            if (r.c[j]) recon_emit_block(r.a[j], r.b[j], r.b[j + 1], r.a[j + 1], r.c[j], off, pix, tv, status);
+            off += r.c[j];
+        }
+    }
 }
 
 void launch_recon(const int *vor, const int *pix, const BatchDev &b, MeshDev &m, int *tile_cnt, int *tile_off,
                   void *scan_tmp, hipStream_t st)
 {
-    int ntiles = b.blocks[BM_RECON];
-    GA_LAUNCH(k_recon_count, dim3(ntiles), dim3(256), 0, st, vor, b, tile_cnt);
-    launch_exclusive_scan(tile_cnt, tile_off, ntiles, scan_tmp, st);
-    GA_LAUNCH(k_recon_emit, dim3(ntiles), dim3(256), 0, st, vor, pix, b, tile_off, m.tv, m.tn,
-                       m.status, m.cap);
-    GA_LAUNCH(k_set_ntri, dim3(1), dim3(1), 0, st, tile_cnt, tile_off, ntiles, m.ntri, m.cap);
+    const int blocks = b.blocks[BM_RECON];
+    GA_LAUNCH(k_recon_count, dim3(blocks), dim3(256), 0, st, vor, b, tile_cnt);
+    launch_exclusive_scan(tile_cnt, tile_off, RECON_TILES * blocks, scan_tmp, st);
+    GA_LAUNCH(k_recon_emit, dim3(blocks), dim3(256), 0, st, vor, pix, b, (const int *)tile_cnt, (const int *)tile_off,
+              m.tv, m.status, m.ntri, m.cap);
 }
 
 // ---- adjacency from scratch ----------------------------------------------------------------
