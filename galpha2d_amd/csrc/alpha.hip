@@ -199,6 +199,7 @@ struct AlphaK {
 #define A_BADMESH 6      // caller triangles that fail k_mesh_check
 #define A_EXCLU 7        // small clusters left to the exact kernel (list in xclu)
 #define A_ATT_LIST 8     // edges whose attachment the filter leaves open (list in xatt)
+#define A_RANKS 10       // single set: number of ranks, set by k_spec_values
 #define A_MK 9           // master-list entries with a rank (the sorted list's length), set by k_master_decode
 // Counters that every wave of a large grid updates live in stripes 128 bytes apart (atomics on
 // one address or line from many waves serialise at about 11 ns each), chosen by the wave's
@@ -1159,13 +1160,6 @@ __global__ void k_big_ends(const int *flag, int S0, const int *cstart, int nbig,
     }
 }
 
-// inclusive = exclusive + flag (in place over the flag array)
-// incl[i] = excl[i] + flag[i] (incl may be flag)
-__global__ void k_incl_from_excl(const int *excl, const int *flag, int *incl, int n)
-{
-    GS(i, n) incl[i] = excl[i] + flag[i];
-}
-
 GA_INLINE int entry_tri(const AlphaK &a, int id) { return id < a.F ? id : a.edge_t[id - a.F]; }
 GA_INLINE int tri_set(const AlphaK &a, int t) { return a.vset ? a.vset[tv(a, t, 0)] : 0; }
 
@@ -1177,7 +1171,7 @@ GA_INLINE double entry_value(const AlphaK &a, int id)
     return rho_edge(cpt(a, t, pl1(i)), cpt(a, t, mi1(i)));
 }
 
-// single set: rank = incl[k] (1-based); the spectrum value of a rank is the smallest FP64 value
+// single set: rank = group starts up to and at k (excl[k] + gflag[k], 1-based); the spectrum value of a rank is the smallest FP64 value
 // of its members
 // An entry alone in its certified cluster is never moved by the exact sorts, so key2[k] (single
 // set) still holds its FP64 value bits, and it is alone in its rank (plain store).  Entries of larger clusters
@@ -1204,7 +1198,7 @@ GA_INLINE void spec_value(const AlphaK &a, int S0, int k, int id, int slot, bool
     if (need && (lane == 63 || next != sl)) atomicMin(&a.specbits[slot], v);
 }
 
-__global__ void k_ranks(AlphaK a, int S0, const int *incl)
+__global__ void k_ranks(AlphaK a, int S0, const int *excl)
 {
     if (big_pending(a)) return;
     for (int base = blockIdx.x * blockDim.x; base < S0; base += gridDim.x * blockDim.x) {
@@ -1212,7 +1206,7 @@ __global__ void k_ranks(AlphaK a, int S0, const int *incl)
         const bool act = k < S0;
         int r = 0, id = 0;
         if (act) {
-            r = incl[k];
+            r = excl[k] + a.gflag[k];
             id = a.id2[k];
             if (id < a.F) a.tri_rank[id] = r;
             else a.edge_rank[id - a.F] = r;
@@ -1222,42 +1216,26 @@ __global__ void k_ranks(AlphaK a, int S0, const int *incl)
 }
 
 // batches: entries are in (set, exact value) order, so the global group ranks count up through
-// the sets; local ranks count the groups inside the set.
-__global__ void k_iota(int n, int *a)
-{
-    GS(k, n) a[k] = k;
-}
-
-__global__ void k_batch_flags(int S0, const unsigned int *sset2, const int *order2, const int *incl, int *flags2)
+// the sets, and every set starts a group (a certified cluster never spans sets): the rank inside the set is
+// the count since its first entry
+// global rank of the first and last entry of every set (sets without entries keep -1)
+__global__ void k_set_bounds(int S0, const int *sset, const int *excl, const int *gflag, int *first, int *last)
 {
     GS(j, S0) {
-        int f = 1;
-        if (j > 0) f = sset2[j] != sset2[j - 1] || incl[order2[j]] != incl[order2[j - 1]];
-        flags2[j] = f;
+        const int s = sset[j];
+        if (j == 0 || sset[j - 1] != s) first[s] = excl[j] + gflag[j];
+        if (j == S0 - 1 || sset[j + 1] != s) last[s] = excl[j] + gflag[j];
     }
 }
 
-// first / last inclusive local count of every set (sets without entries keep -1)
-__global__ void k_set_bounds(int S0, const unsigned int *sset2, const int *incl2, int *first, int *last)
-{
-    GS(j, S0) {
-        int s = (int)sset2[j];
-        if (j == 0 || sset2[j - 1] != sset2[j]) first[s] = incl2[j];
-        if (j == S0 - 1 || sset2[j + 1] != sset2[j]) last[s] = incl2[j];
-    }
-}
-
-__global__ void k_ranks_batch(AlphaK a, int S0, const unsigned int *sset2, const int *order2, const int *incl2,
-                              const int *first)
+__global__ void k_ranks_batch(AlphaK a, int S0, const int *sset, const int *excl, const int *first)
 {
     for (int base = blockIdx.x * blockDim.x; base < S0; base += gridDim.x * blockDim.x) {
-        const int j = base + threadIdx.x;
-        const bool act = j < S0;
-        int k = 0, id = 0, slot = 0;
+        const int k = base + threadIdx.x;
+        const bool act = k < S0;
+        int id = 0, slot = 0;
         if (act) {
-            int s = (int)sset2[j];
-            int r = incl2[j] - first[s] + 1;
-            k = order2[j];
+            const int s = sset[k], r = excl[k] + a.gflag[k] - first[s] + 1;
             id = a.id2[k];
             if (id < a.F) a.tri_rank[id] = r;
             else a.edge_rank[id - a.F] = r;
@@ -1382,37 +1360,52 @@ __global__ void k_master_decode(int n, int E, int M, unsigned int none, const un
 // least the entry of its own value, so the keys of set s are exactly specstart[s] + 1 ..
 // specstart[s + 1] - 1 (single set: 1 .. R), and key K of set s is distinct key number
 // K - s - 1: no scan over the entries is needed.  specstart[0] = 0.
-__global__ void k_spec_pointers(AlphaK a, int M, unsigned int none, const unsigned int *skey, const int *specstart,
-                                int nsets, int *sp, int cap)
+// A block takes SP_TILE keys at a time and searches the sets of the first and the last, between which the
+// others' lie (mostly one set: 144M entries of 1,024 sets 373 us, 1,315 with a search through all
+// sets per distinct key).
+#define SP_TILE 4096
+__global__ __launch_bounds__(256) void k_spec_pointers(AlphaK a, int M, unsigned int none, const unsigned int *skey,
+                                                       const int *specstart, int nsets, int *sp, int cap)
 {
+    __shared__ int s_set[2];
     if (big_pending(a)) return;
-    GS(k, M) {
-        const unsigned K = skey[k];
-        if (K >= none || (k > 0 && skey[k - 1] == K)) continue;
-        int s = 0;
-        if (nsets > 1) {
-            // largest s with specstart[s] < K
-            int lo = 0, hi = nsets - 1;
-            while (lo < hi) {
-                const int mid = (lo + hi + 1) >> 1;
-                if ((unsigned)specstart[mid] < K) lo = mid;
-                else hi = mid - 1;
-            }
-            s = lo;
+    // largest s in [lo, hi] with specstart[s] < K
+    auto set_at = [&](unsigned K, int lo, int hi) {
+        while (lo < hi) {
+            const int mid = (lo + hi + 1) >> 1;
+            if ((unsigned)specstart[mid] < K) lo = mid;
+            else hi = mid - 1;
         }
-        if ((int)K - s < cap) sp[(int)K - s] = k;
+        return lo;
+    };
+    for (long long base = (long long)blockIdx.x * SP_TILE; base < M; base += (long long)gridDim.x * SP_TILE) {
+        const int end = (int)min(base + SP_TILE, (long long)M);
+        if (nsets > 1) {
+            __syncthreads();
+            if (threadIdx.x < 2) s_set[threadIdx.x] = set_at(skey[threadIdx.x ? end - 1 : (int)base], 0, nsets - 1);
+            __syncthreads();
+        }
+        for (int k = (int)base + threadIdx.x; k < end; k += 256) {
+            const unsigned K = skey[k];
+            if (K >= none || (k > 0 && skey[k - 1] == K)) continue;
+            const int s = nsets > 1 ? set_at(K, s_set[0], s_set[1]) : 0;
+            if ((int)K - s < cap) sp[(int)K - s] = k;
+        }
     }
     if (blockIdx.x == 0 && threadIdx.x == 0) sp[0] = -1;
 }
 
 // slots without a member (rank 0 of every set) read as 0; ~0 is a NaN pattern, never a value.
-// nslots < 0: a single set whose rank count R is incl[0] (the inclusive rank of the last entry),
-// nslots = R + 1
+// nslots < 0: a single set whose rank count R is the rank of the last entry (S0 - 1), kept in
+// counters[A_RANKS]; nslots = R + 1
 // also sets every vertex's working interval pair to (INT_MAX, -1) for k_edge_intervals
-__global__ void k_spec_values(const unsigned long long *bits, int nslots, const int *incl_last, double *spec,
+__global__ void k_spec_values(AlphaK a, int S0, const unsigned long long *bits, int nslots, const int *excl, double *spec,
                               int2 *vnum, int n)
 {
-    if (nslots < 0) nslots = *incl_last + 1;
+    if (nslots < 0) {
+        nslots = excl[S0 - 1] + a.gflag[S0 - 1] + 1;
+        if (blockIdx.x == 0 && threadIdx.x == 0) a.counters[A_RANKS] = nslots - 1;
+    }
     GS(r, nslots) spec[r] = bits[r] == ~0ull ? 0.0 : __longlong_as_double((long long)bits[r]);
     GS(v, n) vnum[v] = make_int2(0x7fffffff, -1);
 }
@@ -1451,7 +1444,7 @@ enum {
     AB_ID2, AB_LO, AB_HI, AB_SLO, AB_SHI, AB_FLAG, AB_RANK, AB_SPECBITS, AB_VMIN, AB_VMAX, AB_STATUS, AB_CNTRS,
     AB_TMP, AB_SCAN, AB_NEG, AB_PMAX, AB_NSMIN, AB_MKEY, AB_MVAL, AB_MFLAG, AB_MPOS, AB_OKEY, AB_OVAL,
     AB_SKEY, AB_SVAL, AB_SPEC, AB_SP, AB_MISC, AB_BIG0, AB_BIG1, AB_BIG2, AB_BIG3, AB_BIGL,
-    AB_BS0, AB_BS1, AB_BS2, AB_BS3, AB_BS4, AB_BSET, AB_MSET, AB_VHULL, AB_RANKQ, AB_RD, AB_XATT, AB_XCLU, AB_XPAIR, AB_VNUM, AB_CXY, AB_COUNT
+    AB_BS0, AB_BS1, AB_BSET, AB_MSET, AB_VHULL, AB_RANKQ, AB_RD, AB_XATT, AB_XCLU, AB_XPAIR, AB_VNUM, AB_CXY, AB_COUNT
 };
 static_assert(AB_COUNT <= 64, "AlphaDev holds 64 buffers");
 
@@ -1815,32 +1808,16 @@ void alpha_run_batch(AlphaDev &d, const double *d_xy, int n, const int *d_tris9,
         R = h4[0] + h4[1];
         nslots = R + 1;
     }
-    // incl = excl + flag: single set into the free NEG buffer (gflag stays for a second pass),
-    // batches into the group-flag buffer
-    int *incl = nsets == 1 ? AP<int>(d, AB_NEG) : a.gflag;
-    GA_LAUNCH(k_incl_from_excl, dim3(AGRID), dim3(256), 0, st, (const int *)a.rank, (const int *)a.gflag, incl, S0);
+    const int *excl = a.rank;
     if (nsets == 1) {
-        GA_LAUNCH(k_ranks, dim3(AGRID), dim3(256), 0, st, a, S0, (const int *)incl);
+        GA_LAUNCH(k_ranks, dim3(AGRID), dim3(256), 0, st, a, S0, excl);
     } else {
-        // entries are already in (set, exact value) order; sset[j] is the set of position j
-        ab(d, AB_BS3, 4 * (size_t)S0 + 64);
-        ab(d, AB_BS4, 4 * (size_t)S0 + 64);
+        // entries are already in (set, exact value) order; sset[k] is the set of position k
         ab(d, AB_BSET, 4 * 3 * (size_t)(nsets + 1));
-        const unsigned *sset2 = (const unsigned *)sset;
-        int *pos = sset_rev;   // free: the reversed sets were only needed by the scan
-        int *order2 = AP<int>(d, AB_BS3), *flags2 = AP<int>(d, AB_BS4);
         int *first = AP<int>(d, AB_BSET), *last = first + (nsets + 1), *sstart = last + (nsets + 1);
-        GA_LAUNCH(k_iota, dim3(AGRID), dim3(256), 0, st, S0, order2);
-        GA_LAUNCH(k_batch_flags, dim3(AGRID), dim3(256), 0, st, S0, (const unsigned *)sset2, (const int *)order2,
-                  (const int *)incl, flags2);
-        int *incl2 = pos;   // pos is free after the sort
-        launch_exclusive_scan(flags2, incl2, S0, d.b[AB_SCAN].p, st);
-        GA_LAUNCH(k_incl_from_excl, dim3(AGRID), dim3(256), 0, st, (const int *)incl2, (const int *)flags2, flags2,
-                  S0);
-        incl2 = flags2;
         launch_fill_i32(first, -1, 2 * (size_t)(nsets + 1), st);
-        GA_LAUNCH(k_set_bounds, dim3(AGRID), dim3(256), 0, st, S0, (const unsigned *)sset2, (const int *)incl2,
-                  first, last);
+        GA_LAUNCH(k_set_bounds, dim3(AGRID), dim3(256), 0, st, S0, (const int *)sset, excl, (const int *)a.gflag, first,
+                  last);
         std::vector<int> hf(nsets), hl(nsets);
         chk(hipMemcpyAsync(hf.data(), first, 4 * (size_t)nsets, hipMemcpyDeviceToHost, st), "copy");
         chk(hipMemcpyAsync(hl.data(), last, 4 * (size_t)nsets, hipMemcpyDeviceToHost, st), "copy");
@@ -1860,13 +1837,12 @@ void alpha_run_batch(AlphaDev &d, const double *d_xy, int n, const int *d_tris9,
         IntFills f;
         f.add(a.specbits, 2 * (size_t)nslots, -1);
         launch_fill_multi(f, st);
-        GA_LAUNCH(k_ranks_batch, dim3(AGRID), dim3(256), 0, st, a, S0, (const unsigned *)sset2, (const int *)order2,
-                  (const int *)incl2, (const int *)first);
+        GA_LAUNCH(k_ranks_batch, dim3(AGRID), dim3(256), 0, st, a, S0, (const int *)sset, excl, (const int *)first);
     }
     const int slot_bound = nsets == 1 ? S0 + 1 : nslots;   // spectrum slots, or a bound of them
     ab(d, AB_SPEC, 8 * (size_t)(slot_bound + 1));
-    GA_LAUNCH(k_spec_values, dim3(AGRID), dim3(256), 0, st, (const unsigned long long *)a.specbits, nslots,
-              (const int *)(incl + S0 - 1), AP<double>(d, AB_SPEC), a.vnum, n);
+    GA_LAUNCH(k_spec_values, dim3(AGRID), dim3(256), 0, st, a, S0, (const unsigned long long *)a.specbits, nslots, excl,
+              AP<double>(d, AB_SPEC), a.vnum, n);
     chk(hipEventRecord(d.ev[2], st), "event");
     // intervals (k_master_keys splits the vertex pairs into the output arrays)
     GA_LAUNCH(k_edge_intervals, dim3(AGRID), dim3(256), 0, st, a, E);
@@ -1931,10 +1907,9 @@ void alpha_run_batch(AlphaDev &d, const double *d_xy, int n, const int *d_tris9,
     chk(hipEventRecord(d.ev[3], st), "event");
     // counters, status, the single set's rank count and the ranked master entries in one read
     int fin[11];
-    const int *zero = a.counters + A_BADMESH;   // 0 here: only caller meshes with errors set it
     read_ints(d, st,
               {a.counters + 0, a.counters + 1, a.counters + 2, a.counters + 3, a.counters + 4, a.counters + 5,
-               a.counters + 6, a.counters + 7, a.status, nsets == 1 ? incl + S0 - 1 : zero, pMk},
+               a.counters + 6, a.counters + 7, a.status, a.counters + A_RANKS, pMk},
               fin, &a);   // the statistics folded on the way
     if (!big_done && fin[A_BIGCLUSTER] > 0) {
         big_clusters(d, a, S0, fin[A_BIGCLUSTER], st);
