@@ -1142,7 +1142,7 @@ static int run_batch(galpha_ctx *c, const double *d_xy, const BatchPlan &plan)
     c->rot.ensure(4 * (size_t)nslots + 64);
     c->newid.ensure(4 * (size_t)nslots + 64);
     // one key (v0, v1) of 2B bits, input indices below 2^B (a batch's sets are consecutive ranges);
-    // up to B = 20 a 32-bit key (v0, top bits of v1) whose rare ties k_canon_newid orders
+    // up to B = 24 a 32-bit key (v0, top bits of v1 - v0) whose ties k_canon_newid orders
     int kb = 2;
     while ((1LL << kb) < (long long)n) kb++;
     if (2 * kb > 64) throw GalphaError("too many points for the canonical key");
@@ -1173,7 +1173,7 @@ static int run_batch(galpha_ctx *c, const double *d_xy, const BatchPlan &plan)
     // the live-triangle count stays on the device (folded statistic) until the final read
     c->out9.ensure(36 * (size_t)nslots + 64);
     launch_fold_stats(c->counters.as<int>(), st);
-    launch_canon_emit(m, order, skey32, v1s, c->rot.as<int>(), c->newid.as<int>(),
+    launch_canon_emit(m, order, skey32, v1s, vals, c->rot.as<int>(), c->newid.as<int>(),
                       c->counters.as<int>() + C_FOLD + C_RECON_TRIS, c->out9.as<int>(), c->setFirst.as<int>(),
                       c->keys2.as<int>(), st);   // keys2 (v1s) is free after k_canon_newid: output sets
     ev_mark(c, 8, st);

@@ -204,6 +204,9 @@ struct HullDev {
 #define C_DBG 48          // 48..63: first failure dump
 #define C_NCOUNTERS 64
 
+// Sorts of up to this many pairs go by merging, longer ones by radix passes (250K points, sorts of
+// 0.66M and 1.05M pairs: 283 us by merging, 231 by eight passes; 65K, 139K pairs: 57 and 85).
+#define SORT_MERGE_LIMIT (512 * 1024)
 // pba.hip
 void launch_fill_i32(int *a, int v, size_t n, hipStream_t st);
 void launch_vset(const BatchDev &b, int *vset, hipStream_t st);
@@ -305,10 +308,11 @@ void launch_cons_insert(MeshDev &m, const int2 *cv, int nc, int *done, const int
 void launch_hull(MeshDev &m, const HullDev &h, int op, void *scan_tmp, hipStream_t st);
 // canonical order: key (v0 << B) | v1 of input indices below 2^B, sorted on its low 2B bits
 void launch_canon_keys(MeshDev &m, unsigned long long *keys, int *vals, int *rot, int B, hipStream_t st);
-// canonical keys of 32 bits up to input indices below 2^CANON_KEY32_BITS (ties within 256 triangles)
-#define CANON_KEY32_BITS 20
+// canonical keys of 32 bits up to input indices below 2^CANON_KEY32_BITS
+#define CANON_KEY32_BITS 24
 void launch_canon_keys32(MeshDev &m, unsigned *keys, unsigned *v1s, int *vals, int *rot, int B, hipStream_t st);
-void launch_canon_emit(MeshDev &m, int *order, const unsigned *skey, const unsigned *v1s, const int *rot, int *newid,
+// out: [nslots] the order when skey is given (32-bit keys)
+void launch_canon_emit(MeshDev &m, const int *order, const unsigned *skey, const unsigned *v1s, int *out, const int *rot, int *newid,
                        const int *dF, int *out9,
                        int *set_first, int *rset, hipStream_t st);
 int sort_pairs_u64(unsigned long long *keys_in, int *vals_in, unsigned long long *keys_out, int *vals_out,

@@ -17,7 +17,8 @@ int sort_pairs_u64(unsigned long long *keys_in, int *vals_in, unsigned long long
 using SortCfgU32 = rocprim::radix_sort_config<
     rocprim::default_config, rocprim::default_config,
     rocprim::radix_sort_onesweep_config<rocprim::kernel_config<1024, 8>, rocprim::kernel_config<1024, 8>, 8,
-                                        rocprim::block_radix_rank_algorithm::match>>;
+                                        rocprim::block_radix_rank_algorithm::match>,
+    SORT_MERGE_LIMIT>;
 
 int sort_pairs_u32(unsigned int *keys_in, int *vals_in, unsigned int *keys_out, int *vals_out,
                    int n, int begin_bit, int end_bit, void *temp, size_t *temp_bytes, hipStream_t st)
