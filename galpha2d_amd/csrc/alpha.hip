@@ -40,7 +40,8 @@
 using SortCfg32 = rocprim::radix_sort_config<
     rocprim::default_config, rocprim::default_config,
     rocprim::radix_sort_onesweep_config<rocprim::kernel_config<1024, 8>, rocprim::kernel_config<1024, 8>, 8,
-                                        rocprim::block_radix_rank_algorithm::match>>;
+                                        rocprim::block_radix_rank_algorithm::match>,
+    SORT_MERGE_LIMIT>;
 #define U53 1.1102230246251565e-16
 
 GA_INLINE double2 P(const double2 *xy, int v) { return xy[v]; }
@@ -164,7 +165,7 @@ struct AlphaK {
     int *cnt, *eoff;     // [F]
     int *edge_t, *edge_v, *edge_att, *edge_rank, *edge_numin, *edge_numax;  // [E]
     int *tri_rank;       // [F]
-    unsigned long long *key;   // [S0] single set: FP64 value bits of the triangles; batches: sort keys
+    unsigned long long *key;   // [S0] FP64 value bits of the triangles; batches: then the sort keys
     int *id, *id2;       // [S0] entry ids (t or F + e)
     unsigned long long *key2;
     EntryIv *iv;         // [F + E] per entry id: certified interval (lo, hi) and FP64 value
@@ -230,6 +231,7 @@ GA_INLINE void stat_add(int *counters, int k, int v)
 
 GA_INLINE int tv(const AlphaK &a, int t, int i) { return a.tris[(size_t)t * 9 + 3 + i]; }
 GA_INLINE int tn(const AlphaK &a, int t, int i) { return a.tris[(size_t)t * 9 + i]; }
+GA_INLINE int tri_set(const AlphaK &a, int t) { return a.vset ? a.vset[tv(a, t, 0)] : 0; }
 GA_INLINE int pl1(int i) { return i == 2 ? 0 : i + 1; }
 // first pass of a single set that found large clusters: the rest is redone after their order
 GA_INLINE bool big_pending(const AlphaK &a) { return a.skip_if_big && a.counters[A_BIGCLUSTER] > 0; }
@@ -340,12 +342,12 @@ __device__ Key32Map key32_map(const AlphaK &a)
 }
 GA_INLINE unsigned key32(const Key32Map &m, unsigned long long u) { return (unsigned)((u >> m.sh) - m.base); }
 GA_INLINE unsigned long long value_bits(double v) { return (unsigned long long)__double_as_longlong(v); }
-// Batches order entries by (set, value): the set above the value's top 40 bits, so certified
+// Batches order entries by (set, value): the set above the top vbits of the 32-bit key, so certified
 // clusters never span sets (equal values in different sets, e.g. repeated requests, are never
-// compared).  The low value bits are not kept; they are recomputed where needed.
-GA_INLINE unsigned long long batch_key(int set, double v)
+// compared).
+GA_INLINE unsigned long long batch_key(int set, unsigned k, int vbits)
 {
-    return ((unsigned long long)set << 40) | ((unsigned long long)__double_as_longlong(v) >> 24);
+    return ((unsigned long long)set << vbits) | (k >> (32 - vbits));
 }
 
 // relative error bound of the certified rho estimate used for ordering
@@ -360,7 +362,7 @@ __global__ void k_tri_rho(AlphaK a)
             a.cxy[(size_t)t * 3 + 2] = Cc;
             double v = rho_tri(A, B, Cc);
             const unsigned long long u = value_bits(v);
-            a.key[t] = a.vset ? batch_key(a.vset[tv(a, t, 0)], v) : u;
+            a.key[t] = u;
             a.id[t] = t;
             // ar with Shewchuk's orient2d bound: |ar - det| <= eb
             double detleft = (A.x - Cc.x) * (B.y - Cc.y), detright = (A.y - Cc.y) * (B.x - Cc.x);
@@ -385,7 +387,7 @@ __global__ void k_tri_rho(AlphaK a)
             mc = max(mc, ~u);
         }
     }
-    if (!a.vset) range_note(a, mx, mc);
+    range_note(a, mx, mc);
 }
 
 // attachment of edge (p, q) to the apex k by the FP64 filter: 1 attached, 0 not, -1 open
@@ -432,7 +434,7 @@ __global__ void k_attached(AlphaK a, int Emax)
             mc = max(mc, ~u);
         }
     }
-    if (!a.vset) range_note(a, mx, mc);
+    range_note(a, mx, mc);
 }
 
 // the edges left open by k_attached: both sides with the exact predicate where the filter fails
@@ -467,14 +469,15 @@ __global__ void k_attached_exact(AlphaK a)
     stat_add(a.counters, ST_EXACT_ATT, natt);
 }
 
-// unattached edges appended after the triangles (flag scanned into rank[] positions).  Single
-// set: the 32-bit sort keys of every entry go to k32 (the triangles' from their value bits in
-// key[]); batches: 64-bit (set, value) keys in key[].
-__global__ void k_edge_entries(AlphaK a, int E, unsigned *k32)
+// unattached edges appended after the triangles (flag scanned into rank[] positions).  The sort
+// keys of every entry (the triangles' from their value bits in key[]): single set, 32 bits in k32;
+// batches, 64 bits of set and value in key[].
+__global__ void k_edge_entries(AlphaK a, int E, unsigned *k32, int vbits)
 {
-    Key32Map m{0, 0};
-    if (!a.vset) {
-        m = key32_map(a);
+    const Key32Map m = key32_map(a);
+    if (a.vset) {
+        GS(t, a.F) a.key[t] = batch_key(tri_set(a, t), key32(m, a.key[t]), vbits);
+    } else {
         GS(t, a.F) k32[t] = key32(m, a.key[t]);
     }
     GS(e, E) {
@@ -482,24 +485,23 @@ __global__ void k_edge_entries(AlphaK a, int E, unsigned *k32)
         int k = a.F + a.rank[e];
         int t = a.edge_t[e], i = a.edge_v[e];
         double v = rho_edge(cpt(a, t, pl1(i)), cpt(a, t, mi1(i)));
-        if (a.vset) a.key[k] = batch_key(a.vset[tv(a, t, 0)], v);
-        else k32[k] = key32(m, value_bits(v));
+        const unsigned kv = key32(m, value_bits(v));
+        if (a.vset) a.key[k] = batch_key(tri_set(a, t), kv, vbits);
+        else k32[k] = kv;
         a.id[k] = a.F + e;
     }
 }
 
 // batches: sorted intervals, the set of every position (and reversed) and the negated lo values
-// reversed, for the segmented scans of the cluster flags
-__global__ void k_gather_iv(AlphaK a, int S0, double *neg_lo_rev, int *sset, int *sset_rev)
+// reversed, for the segmented scans of the cluster flags; key2 gets the value for spec_value
+__global__ void k_gather_iv(AlphaK a, int S0, int vbits, double *neg_lo_rev, int *sset, int *sset_rev)
 {
     GS(k, S0) {
-        if (sset) {
-            int s = (int)(a.key2[k] >> 40);
-            sset[k] = s;
-            sset_rev[S0 - 1 - k] = s;
-        }
-        int id = a.id2[k];
+        const int s = (int)(a.key2[k] >> vbits), id = a.id2[k];
+        sset[k] = s;
+        sset_rev[S0 - 1 - k] = s;
         const EntryIv w = a.iv[id];
+        a.key2[k] = value_bits(w.v);
         a.shi[k] = w.hi;
         a.slo[k] = w.lo;
         neg_lo_rev[S0 - 1 - k] = -w.lo;
@@ -1161,20 +1163,12 @@ __global__ void k_big_ends(const int *flag, int S0, const int *cstart, int nbig,
 }
 
 GA_INLINE int entry_tri(const AlphaK &a, int id) { return id < a.F ? id : a.edge_t[id - a.F]; }
-GA_INLINE int tri_set(const AlphaK &a, int t) { return a.vset ? a.vset[tv(a, t, 0)] : 0; }
-
-GA_INLINE double entry_value(const AlphaK &a, int id)
-{
-    if (id < a.F) return rho_tri(cpt(a, id, 0), cpt(a, id, 1), cpt(a, id, 2));
-    int e = id - a.F;
-    int t = a.edge_t[e], i = a.edge_v[e];
-    return rho_edge(cpt(a, t, pl1(i)), cpt(a, t, mi1(i)));
-}
 
 // single set: rank = group starts up to and at k (excl[k] + gflag[k], 1-based); the spectrum value of a rank is the smallest FP64 value
 // of its members
-// An entry alone in its certified cluster is never moved by the exact sorts, so key2[k] (single
-// set) still holds its FP64 value bits, and it is alone in its rank (plain store).  Entries of larger clusters
+// An entry alone in its certified cluster is never moved by the exact sorts, so key2[k] still holds
+// its FP64 value bits, and it is alone in its rank (plain store; 1,024 sets: 971 us, 2,180 with the
+// value recomputed from the points).  Entries of larger clusters
 // recompute their value and take the minimum: first over the lanes of the wave that hold the same
 // slot (slots do not decrease from lane to lane), then one atomicMin per slot and wave (a
 // lattice's triangles can put a million entries in one rank).  Called by every lane of the wave;
@@ -1182,12 +1176,11 @@ GA_INLINE double entry_value(const AlphaK &a, int id)
 GA_INLINE void spec_value(const AlphaK &a, int S0, int k, int id, int slot, bool act)
 {
     const bool alone = act && a.flag[k] && (k + 1 == S0 || a.flag[k + 1]);
-    if (alone && !a.vset) a.specbits[slot] = a.key2[k];
-    else if (alone) a.specbits[slot] = (unsigned long long)__double_as_longlong(entry_value(a, id));
+    if (alone) a.specbits[slot] = a.key2[k];
     const bool need = act && !alone;
     if (!__any(need)) return;
     const int lane = threadIdx.x & 63;
-    unsigned long long v = need ? (unsigned long long)__double_as_longlong(entry_value(a, id)) : ~0ull;
+    unsigned long long v = need ? value_bits(a.iv[id].v) : ~0ull;
     const int sl = need ? slot : -1;
     for (int d = 1; d < 64; d <<= 1) {
         unsigned long long ov = __shfl_up(v, d, 64);
@@ -1713,10 +1706,15 @@ void alpha_run_batch(AlphaDev &d, const double *d_xy, int n, const int *d_tris9,
     d.S = S0;
     // single set: 32-bit keys in and out side by side in key2 (free until the gather below)
     unsigned *k32 = (unsigned *)a.key2;
-    GA_LAUNCH(k_edge_entries, dim3(AGRID), dim3(256), 0, st, a, E, k32);
+    // batches: 28 value bits or more, as many as whole radix digits leave room for beside the set (1,024
+    // sets: 30 of 40, 5 passes; the top 40 bits of the value took 7)
+    int sbits = 0;
+    while ((1LL << sbits) < (long long)nsets) sbits++;
+    const int vbits = std::min(32, (28 + sbits + 7) / 8 * 8 - sbits);
+    GA_LAUNCH(k_edge_entries, dim3(AGRID), dim3(256), 0, st, a, E, k32, vbits);
     chk(hipEventRecord(d.ev[1], st), "event");
     // radix sort by value: single set, 32-bit monotone keys (4 passes; see key32); batches, the
-    // set above the top 40 bits of the FP64 value.  The cluster boundaries below only need
+    // set above the top vbits of those.  The cluster boundaries below only need
     // "everything before is certainly smaller than everything after", which holds for any order,
     // so entries that tie on their key end in one cluster and are put in exact order there.
     size_t tb = 0;
@@ -1729,9 +1727,7 @@ void alpha_run_batch(AlphaDev &d, const double *d_xy, int n, const int *d_tris9,
                                                  32u, st),
             "sort");
     } else {
-        unsigned sbits = 0;   // set bits above the 40 value bits
-        while ((1LL << sbits) < (long long)nsets) sbits++;
-        const unsigned kbits = 40u + sbits;
+        const unsigned kbits = (unsigned)(vbits + sbits);
         chk(rocprim::radix_sort_pairs(nullptr, tb, a.key, a.key2, a.id, a.id2, (unsigned)S0, 0u, kbits, st), "sort");
         ab(d, AB_TMP, tb + 256);
         tb = d.b[AB_TMP].bytes;
@@ -1755,7 +1751,7 @@ void alpha_run_batch(AlphaDev &d, const double *d_xy, int n, const int *d_tris9,
         GA_LAUNCH(k_cluster_flags_tiles, dim3(ntiles), dim3(256), 0, st, a, S0, (const double *)tmax,
                   (const double *)tmin);
     } else {
-        GA_LAUNCH(k_gather_iv, dim3(AGRID), dim3(256), 0, st, a, S0, neg, sset, sset_rev);
+        GA_LAUNCH(k_gather_iv, dim3(AGRID), dim3(256), 0, st, a, S0, vbits, neg, sset, sset_rev);
         tb = 0;
         chk(rocprim::inclusive_scan_by_key(nullptr, tb, sset, a.shi, pmax, (size_t)S0, rocprim::maximum<double>(),
                                            rocprim::equal_to<int>(), st), "scan");
