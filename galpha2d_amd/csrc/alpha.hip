@@ -407,24 +407,25 @@ GA_INLINE int attached_filter(double2 p, double2 q, double2 k)
 
 // Edges decided by the filter; an edge it leaves open goes to xatt for k_attached_exact (which
 // carries the expansion arithmetic and its scratch, so this kernel runs at full occupancy).
-__global__ void k_attached(AlphaK a, int Emax)
+// One reservation of list entries per block and step (a lattice leaves a third of its edges open:
+// 2M points 221 us, 609 with one per wave).
+__global__ __launch_bounds__(256) void k_attached(AlphaK a, int Emax)
 {
     int E = a.eoff[a.F - 1] + a.cnt[a.F - 1];
     unsigned long long mx = 0, mc = 0;   // value-bit range of every edge (a superset of the entries)
-    GS(e, Emax) {
-        if (e >= E) a.flag[e] = 0;   // the scan of unattached edges runs to Emax
-        else {
+    for (int base = blockIdx.x * 256; base < Emax; base += gridDim.x * 256) {
+        const int e = base + threadIdx.x;
+        bool open = false;
+        if (e >= E) {
+            if (e < Emax) a.flag[e] = 0;   // the scan of unattached edges runs to Emax
+        } else {
             int t = a.edge_t[e], i = a.edge_v[e];
             double2 p = cpt(a, t, pl1(i)), q = cpt(a, t, mi1(i));
             int nb = tn(a, t, i);
             int att = attached_filter(p, q, cpt(a, t, i));
             if (att == 0 && nb >= 0) att = attached_filter(p, q, cpt(a, nb >> 2, nb & 3));
-            const bool open = att < 0;
-            int slot = wave_reserve(&a.counters[A_ATT_LIST], open);
-            if (open) {
-                a.xatt[slot] = e;
-                att = 0;   // set by k_attached_exact before the flags are scanned again
-            }
+            open = att < 0;
+            if (open) att = 0;   // set by k_attached_exact before the flags are scanned again
             a.edge_att[e] = att;
             a.flag[e] = !att;
             double v = rho_edge(p, q);
@@ -432,6 +433,10 @@ __global__ void k_attached(AlphaK a, int Emax)
             a.iv[a.F + e] = EntryIv{v * (1.0 - 8.0 * U53), v * (1.0 + 8.0 * U53), v, 0.0};
             mx = max(mx, u);
             mc = max(mc, ~u);
+        }
+        if (__syncthreads_or(open)) {
+            const int slot = block_reserve(&a.counters[A_ATT_LIST], open);
+            if (open) a.xatt[slot] = e;
         }
     }
     range_note(a, mx, mc);
