@@ -903,6 +903,7 @@ static int run_batch(galpha_ctx *c, const double *d_xy, const BatchPlan &plan)
     // passes size their grids by the list length of the last read (lists shrink from pass to pass).
     // Lists of at most TAIL_LIST triangles go to the single-workgroup tail, which runs passes
     // back to back without launches or host reads until one flips nothing.
+    int after_exact = 0;   // exact incircle tests up to the last read
     auto flip_until_done = [&](int *listA, int cntA, int *listB, int cntB, int prev, long long hint) {
         int *lin = listA, *lout = listB, sin = cntA, sout = cntB;
         int pass_count = 0;
@@ -910,6 +911,8 @@ static int run_batch(galpha_ctx *c, const double *d_xy, const BatchPlan &plan)
         long long next = hint;   // length of the next pass's list, when known
         launch_reset_counters(c->counters.as<int>(), C_CAND, -1, -1, -1, st);
         const int maxp = 512;
+        bool many_exact = false;   // the passes before the last read took thousands of exact tests
+        int exact_before = after_exact;
         // the tail's passes after a read: returns true when the flips are done
         auto tail_result = [&](int op0) {
             const int p = last.v[C_TAIL_PASSES];
@@ -939,7 +942,7 @@ static int run_batch(galpha_ctx *c, const double *d_xy, const BatchPlan &plan)
             }
             for (int k = 0; k < 3; k++) {
                 int opn = c->op++;
-                launch_flip_pass(m, lin, sin, lout, sout, prev, opn, grid, st);
+                launch_flip_pass(m, lin, sin, lout, sout, prev, opn, grid, many_exact || (next >= 0 ? next : 2LL * m.n) >= FLIP_SPLIT, st);
                 prev = opn;
                 std::swap(lin, lout);
                 std::swap(sin, sout);
@@ -952,6 +955,8 @@ static int run_batch(galpha_ctx *c, const double *d_xy, const BatchPlan &plan)
             c->op += maxp;
             launch_flip_tail(m, lin, sin, lout, sout, prev, op0, maxp, st);
             last = ctx_snapshot(c);
+            many_exact = last.stat(C_EXACT_INCIRCLE) - exact_before > 4096;
+            exact_before = after_exact = last.stat(C_EXACT_INCIRCLE);
             const int p = last.v[C_TAIL_PASSES];
             if (p == 0) {
                 c->op = op0;

@@ -171,6 +171,7 @@ struct HullDev {
 #define C_ISLAND_SITES 19
 #define C_HSTART 20
 #define C_FLIPS_TOTAL 21
+#define C_XFLIP 22            // edges left to k_flip_exact
 #define C_FLIP_LISTED 24      // triangles listed for k_flip_test (all launches)
 #define C_FTRI 25             // frame triangles listed by k_hull_scan
 #define C_HULL 26             // first demands of frame removal
@@ -187,6 +188,8 @@ struct HullDev {
 #define C_TAIL_DONE 36        // 1 when that tail ended with a pass without flips
 #define C_TAIL_LISTED 37      // triangles listed by flip tails (also counted in C_FLIP_LISTED)
 #define C_STAR 41             // 41..43: list counts of the bulk shifting passes
+#define FLIP_SPLIT (1 << 20)  // flip lists from this length on, and those behind passes with many exact tests, leave the
+                              // exact tests to a launch of their own
 #define TAIL_LIST 2048        // longest flip list the single-workgroup tail takes
 // status bits of constraint insertion (the other GA_ERR_* bits are in dev_common.h)
 #define GA_ERR_CONS_POINT 128     // a point lies inside a constraint segment
@@ -286,7 +289,7 @@ void launch_flip_all(MeshDev &m, int op, int *list, hipStream_t st);
 void launch_flip_tail(MeshDev &m, int *lA, int sA, int *lB, int sB, int prev_op, int op0, int max_passes,
                       hipStream_t st);
 void launch_flip_pass(MeshDev &m, const int *list_in, int cnt_in_slot, int *list_out, int cnt_out_slot,
-                      int prev_op, int op, int grid, hipStream_t st);
+                      int prev_op, int op, int grid, bool split, hipStream_t st);
 // Blocks of 256 threads for a round over about `items` list entries: enough for one entry per
 // thread, a multiple of 8 (one share per XCD), at most 2048 (grid-stride loops cover any rest).
 // Lists that shrink from round to round then do not launch thousands of idle blocks.

@@ -1216,6 +1216,14 @@ void launch_flip_all(MeshDev &m, int op, int *list, hipStream_t st)
 // per step: per = 4 for lists longer than four times the grid (fewer reservations), else 1 (more
 // waves in flight for the latency-bound gathers).
 // block-uniform: every thread of the block runs the same iterations (block_reserve inside)
+// SPLIT: edges that the filter leaves open are listed in m.scratch (an edge is tested from at most
+// two sides: 6 V entries; counters[C_XFLIP]) for k_flip_exact.  The exact test takes registers and
+// scratch memory that leave three waves per SIMD to the whole kernel, and on a lattice a few lanes
+// of every wave take it (first pass at 1M uniform points: 117 us, 80 split; the passes over a
+// lattice and clusters of 2M points together 2,600 us, 1,470 split).  Lists of less than FLIP_SPLIT
+// triangles keep it inside unless the passes before took many exact tests: the launch more costs
+// what it gives there (250K points in clusters: 3.35 ms, all passes split 3.44).
+template <bool SPLIT>
 GA_INLINE void flip_test_body(const MeshDev &m, const int *list, int n, int prev_op, int op)
 {
     int tests = 0;
@@ -1223,6 +1231,7 @@ GA_INLINE void flip_test_body(const MeshDev &m, const int *list, int n, int prev
     int per = n > 4 * (int)(gridDim.x * bd) ? 4 : 1;
     XCD_STRIDE(b0, n, bd * per) {
         unsigned bits = 0;   // bit 3j + i: edge i of the j-th triangle of this thread wants a flip
+        unsigned open = 0;   // the same: the filter leaves it open
         int tj[4];
 #pragma unroll
         for (int j = 0; j < 4; j++) {
@@ -1262,7 +1271,14 @@ GA_INLINE void flip_test_body(const MeshDev &m, const int *list, int n, int prev
             for (int i = 0; i < 3; i++) {
                 if (uu[i] < 0) continue;
                 tests++;
-                if (incircle_at(m, pa, pb, pc, pd[i], tt.x, tt.y, tt.z, dd[i]) > 0) {
+                int in;
+                if (SPLIT) {
+                    in = incircle_filter(pa, pb, pc, pd[i]);
+                    open |= (unsigned)(in == 0) << (3 * j + i);
+                } else {
+                    in = incircle_at(m, pa, pb, pc, pd[i], tt.x, tt.y, tt.z, dd[i]);
+                }
+                if (in > 0) {
                     unsigned long long key = ((unsigned long long)op << 32) | (0xffffffffu - (unsigned)(t * 3 + i));
                     atomicMax(&m.claim[t], key);
                     atomicMax(&m.claim[uu[i]], key);
@@ -1275,10 +1291,18 @@ GA_INLINE void flip_test_body(const MeshDev &m, const int *list, int n, int prev
         for (int j = 0; j < 4; j++)
             for (int i = 0; i < 3; i++)
                 if ((bits >> (3 * j + i)) & 1) m.cand[slot++] = tj[j] * 3 + i;
+        if (SPLIT && __syncthreads_or(open)) {
+            slot = block_reserve(&m.counters[C_XFLIP], __popc(open));
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                for (int i = 0; i < 3; i++)
+                    if ((open >> (3 * j + i)) & 1) m.scratch[slot++] = tj[j] * 3 + i;
+        }
     }
     stat_add_full(m.stats, C_TESTS_INCIRCLE, tests);
 }
 
+template <bool SPLIT>
 __global__ __launch_bounds__(256) void k_flip_test(MeshDev m, const int *list, int cnt_slot, int prev_op, int op,
                                                    int cnt_out_slot)
 {
@@ -1289,7 +1313,27 @@ __global__ __launch_bounds__(256) void k_flip_test(MeshDev m, const int *list, i
         m.counters[cnt_out_slot] = 0;
         m.counters[C_FLIPS] = 0;
     }
-    flip_test_body(m, list, n, prev_op, op);
+    flip_test_body<SPLIT>(m, list, n, prev_op, op);
+}
+
+// the edges that k_flip_test<true> left open
+__global__ __launch_bounds__(256) void k_flip_exact(MeshDev m, int op)
+{
+    const int n = m.counters[C_XFLIP];
+    GRID_STRIDE(k, n) {
+        const int c = m.scratch[k], t = c / 3, i = c % 3;
+        const int4 tt = m.tv[t];
+        const int e = ic(m.tn[t], i), u = enc_t(e), d = ic(m.tv[u], enc_j(e));
+        stat_inc(m.stats, C_EXACT_INCIRCLE, true);
+        const bool in = incircle_slow(m.pos[tt.x], oid(m, tt.x), m.pos[tt.y], oid(m, tt.y), m.pos[tt.z], oid(m, tt.z),
+                                      m.pos[d], oid(m, d), m.status) > 0;
+        const int slot = wave_reserve(&m.counters[C_CAND], in);
+        if (!in) continue;
+        const unsigned long long key = ((unsigned long long)op << 32) | (0xffffffffu - (unsigned)c);
+        atomicMax(&m.claim[t], key);
+        atomicMax(&m.claim[u], key);
+        m.cand[slot] = c;
+    }
 }
 
 // Block-uniform loop (block_reserve inside): up to four candidates per thread and step, and one
@@ -1359,6 +1403,7 @@ GA_INLINE void flip_commit_body(const MeshDev &m, int n, int op, int *list_out, 
 
 __global__ void k_flip_commit(MeshDev m, int op, int *list_out, int cnt_out_slot)
 {
+    if (blockIdx.x == 0 && threadIdx.x == 0) m.counters[C_XFLIP] = 0;
     flip_commit_body(m, m.counters[C_CAND], op, list_out, cnt_out_slot);
 }
 
@@ -1385,7 +1430,7 @@ __global__ __launch_bounds__(TAIL_THREADS) void k_flip_tail(MeshDev m, int *lA, 
             m.counters[C_FLIPS] = 0;
         }
         __syncthreads();
-        flip_test_body(m, lin, n, prev, op);
+        flip_test_body<false>(m, lin, n, prev, op);
         __syncthreads();
         flip_commit_body(m, m.counters[C_CAND], op, lout, sout);
         __syncthreads();
@@ -1415,13 +1460,18 @@ void launch_flip_tail(MeshDev &m, int *lA, int sA, int *lB, int sB, int prev_op,
     GA_LAUNCH(k_flip_tail, dim3(1), dim3(TAIL_THREADS), 0, st, m, lA, sA, lB, sB, prev_op, op0, max_passes);
 }
 
-// Three launches per pass and no counter resets of their own: the test clears the output list's
+// Three launches per pass (four with the exact tests split off) and no counter resets of their own: the test clears the output list's
 // count and the flip flag, and the relink clears the candidate count for the next pass (it must
 // be zero before the first pass).
 void launch_flip_pass(MeshDev &m, const int *list_in, int cnt_in_slot, int *list_out, int cnt_out_slot,
-                      int prev_op, int op, int grid, hipStream_t st)
+                      int prev_op, int op, int grid, bool split, hipStream_t st)
 {
-    GA_LAUNCH(k_flip_test, dim3(grid), dim3(256), 0, st, m, list_in, cnt_in_slot, prev_op, op, cnt_out_slot);
+    if (split) {
+        GA_LAUNCH(k_flip_test<true>, dim3(grid), dim3(256), 0, st, m, list_in, cnt_in_slot, prev_op, op, cnt_out_slot);
+        GA_LAUNCH(k_flip_exact, dim3(std::min(grid, 512)), dim3(256), 0, st, m, op);
+    } else {
+        GA_LAUNCH(k_flip_test<false>, dim3(grid), dim3(256), 0, st, m, list_in, cnt_in_slot, prev_op, op, cnt_out_slot);
+    }
     GA_LAUNCH(k_flip_commit, dim3(grid), dim3(256), 0, st, m, op, list_out, cnt_out_slot);
     GA_LAUNCH(k_relink, dim3(grid), dim3(256), 0, st, m, (const int *)list_out, cnt_out_slot, op, C_CAND);
 }
