@@ -909,8 +909,7 @@ static int run_batch(galpha_ctx *c, const double *d_xy, const BatchPlan &plan)
         int pass_count = 0;
         int grid = hint >= 0 ? round_grid(2 * hint) : 2048;
         long long next = hint;   // length of the next pass's list, when known
-        launch_reset_counters(c->counters.as<int>(), C_CAND, -1, -1, -1, st);
-        const int maxp = 512;
+        const int maxp = 512, limit = m.n <= INSERT_TAIL_POINTS ? TAIL_LIST_SMALL : TAIL_LIST;
         bool many_exact = false;   // the passes before the last read took thousands of exact tests
         int exact_before = after_exact;
         // the tail's passes after a read: returns true when the flips are done
@@ -928,17 +927,17 @@ static int run_batch(galpha_ctx *c, const double *d_xy, const BatchPlan &plan)
             return last.v[C_TAIL_DONE] != 0;
         };
         for (pass_count = 0; pass_count < 100000;) {
-            if (next >= 0 && next <= TAIL_LIST) {
+            if (next >= 0 && next <= limit) {
                 const int op0 = c->op;
                 c->op += maxp;
-                launch_flip_tail(m, lin, sin, lout, sout, prev, op0, maxp, st);
+                launch_flip_tail(m, lin, sin, lout, sout, prev, op0, maxp, limit, st);
                 last = ctx_snapshot(c);
                 const int p = last.v[C_TAIL_PASSES];
                 if (tail_result(op0)) return;
                 next = last.v[sin];
                 grid = round_grid(2LL * next);
-                if (p == maxp && next <= TAIL_LIST) continue;
-                next = TAIL_LIST + 1;   // the list outgrew the tail: grid passes first
+                if (p == maxp && next <= limit) continue;
+                next = limit + 1;   // the list outgrew the tail: grid passes first
             }
             for (int k = 0; k < 3; k++) {
                 int opn = c->op++;
@@ -950,10 +949,10 @@ static int run_batch(galpha_ctx *c, const double *d_xy, const BatchPlan &plan)
             S.flipPasses += 3;
             pass_count += 3;
             // the tail right behind the grid passes, before the read: it returns at once while the
-            // list is longer than TAIL_LIST (no passes), else it usually finishes the flips
+            // list is longer than limit (no passes), else it usually finishes the flips
             const int op0 = c->op;
             c->op += maxp;
-            launch_flip_tail(m, lin, sin, lout, sout, prev, op0, maxp, st);
+            launch_flip_tail(m, lin, sin, lout, sout, prev, op0, maxp, limit, st);
             last = ctx_snapshot(c);
             many_exact = last.stat(C_EXACT_INCIRCLE) - exact_before > 4096;
             exact_before = after_exact = last.stat(C_EXACT_INCIRCLE);
@@ -965,8 +964,8 @@ static int run_batch(galpha_ctx *c, const double *d_xy, const BatchPlan &plan)
             } else {
                 if (tail_result(op0)) return;
                 next = last.v[sin];
-                if (p == maxp && next <= TAIL_LIST) continue;
-                next = TAIL_LIST + 1;
+                if (p == maxp && next <= limit) continue;
+                next = limit + 1;
             }
             grid = round_grid(2LL * next);
         }
@@ -974,8 +973,9 @@ static int run_batch(galpha_ctx *c, const double *d_xy, const BatchPlan &plan)
     };
     auto flip_all = [&]() {
         int opn = c->op++;
-        launch_flip_all(m, opn, m.modA, st);
-        flip_until_done(m.modA, C_MODN, m.modB, C_MODN2, opn, -1);
+        launch_flip_all(m, opn, m.modA, st);   // (zeroes C_CAND)
+        // small sets start with the tail (a list above its limit comes back for grid passes)
+        flip_until_done(m.modA, C_MODN, m.modB, C_MODN2, opn, m.n <= INSERT_TAIL_POINTS ? TAIL_LIST_SMALL : -1);
     };
     // ---- shifting, deletion, insertion and the flips to a Delaunay mesh, in one chain of launches
     // All the rounds that most inputs need are launched one behind the other, and their counters
@@ -1006,8 +1006,16 @@ static int run_batch(galpha_ctx *c, const double *d_xy, const BatchPlan &plan)
         bool shifting = true, deleting = true;
         // grids before the lists' lengths are known: one vertex in 8 pending, one in 4 missing
         int pgrid = round_grid(m.n), dgrid = round_grid(m.n / 2), mgrid = round_grid(m.n / 4);
+        const bool tail = m.n <= SHIFT_TAIL_POINTS;
         for (int r = 0;; r++) {
-            if (shifting) {
+            if (tail && deleting) {
+                const int max_rounds = 64, round0 = c->prio_round + 1;
+                c->prio_round += max_rounds - 1;
+                next_prio_round();
+                launch_shift_tail(m, moved, m.mark, wl[0], wl[1], C_STAR, c->mx.as<unsigned int>(), round0, max_rounds,
+                                  r > 0, st);
+            }
+            if (shifting && !tail) {
                 for (int k = stars; k < stars + 4; k++)
                     launch_shift_star(m, moved, m.mark, wl[k & 1], slot[k % 3], wl[(k + 1) & 1], slot[(k + 1) % 3],
                                       slot[(k + 2) % 3], st);
@@ -1018,13 +1026,17 @@ static int run_batch(galpha_ctx *c, const double *d_xy, const BatchPlan &plan)
             }
             if (deleting) {
                 // (k_del_prio zeroes C_SCR and C_PLEFT)
-                for (int k = 0; k < 6; k++)
+                for (int k = 0; k < 6 && !tail; k++)
                     launch_delete_round(m, c->mx.as<unsigned int>(), next_prio_round(), dgrid, st);
                 ev_mark(c, 3, st);
                 // (C_MISS is zero since the run's start: only the missing stage counts it)
                 launch_missing_init(m, c->vor.as<int>(), c->mlist.as<int>(), c->loc.as<int>(), st);
             }
-            for (int k = 0; k < 4; k++) {
+            if (m.n <= INSERT_TAIL_POINTS) {
+                launch_insert_tail(m, c->mlist.as<int>(), c->loc.as<int>(), c->op, 64, st);
+                c->op += 64;
+            }
+            for (int k = 0; k < 4 && m.n > INSERT_TAIL_POINTS; k++) {
                 int opn = c->op++;
                 launch_insert_round(m, c->mlist.as<int>(), c->loc.as<int>(), opn, mgrid, st);   // (zeroes C_MODN, C_MLEFT)
                 launch_relink(m, m.modA, C_MODN, opn, mgrid, st);
@@ -1032,6 +1044,7 @@ static int run_batch(galpha_ctx *c, const double *d_xy, const BatchPlan &plan)
             }
             ev_mark(c, 4, st);
             flip_all();
+            if (m.n <= INSERT_TAIL_POINTS) S.insertRounds += last.v[C_INSERT_ROUNDS];
             S.reconTris = last.v[C_RECON_SLOTS];
             if (last.v[C_RECON_SLOTS] > cap) throw GalphaError("triangle capacity exceeded in reconstruction");
             if (last.v[C_RECON_STATUS])

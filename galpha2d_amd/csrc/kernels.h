@@ -172,6 +172,7 @@ struct HullDev {
 #define C_HSTART 20
 #define C_FLIPS_TOTAL 21
 #define C_XFLIP 22            // edges left to k_flip_exact
+#define C_INSERT_ROUNDS 23    // rounds run by the last k_insert_tail
 #define C_FLIP_LISTED 24      // triangles listed for k_flip_test (all launches)
 #define C_FTRI 25             // frame triangles listed by k_hull_scan
 #define C_HULL 26             // first demands of frame removal
@@ -190,7 +191,8 @@ struct HullDev {
 #define C_STAR 41             // 41..43: list counts of the bulk shifting passes
 #define FLIP_SPLIT (1 << 20)  // flip lists from this length on, and those behind passes with many exact tests, leave the
                               // exact tests to a launch of their own
-#define TAIL_LIST 2048        // longest flip list the single-workgroup tail takes
+#define TAIL_LIST 2048        // longest flip list the single-workgroup tail takes, and of sets of up to
+#define TAIL_LIST_SMALL 16384 // INSERT_TAIL_POINTS points, whose passes cost less there than their launches
 // status bits of constraint insertion (the other GA_ERR_* bits are in dev_common.h)
 #define GA_ERR_CONS_POINT 128     // a point lies inside a constraint segment
 #define GA_ERR_CONS_CROSS 256     // two constraints cross
@@ -276,6 +278,13 @@ void launch_shift_star(MeshDev &m, unsigned char *moved, int *mark, const int *w
 void launch_shift_commit(MeshDev &m, const unsigned char *moved, int cnt_slot, hipStream_t st);
 void launch_shift_greedy(MeshDev &m, int round, int *mark, int grid, hipStream_t st);
 void launch_delete_round(MeshDev &m, unsigned int *mx, int round, int grid, hipStream_t st);
+// small sets (see mesh.hip): everything from the bulk passes' first worklist to the deletions, and the
+// insertion rounds, one workgroup each
+#define SHIFT_TAIL_POINTS 8192
+#define INSERT_TAIL_POINTS 2048
+void launch_shift_tail(MeshDev &m, unsigned char *moved, int *mark, int *wlA, int *wlB, int slot, unsigned int *mx,
+                       int round0, int max_rounds, bool more, hipStream_t st);
+void launch_insert_tail(MeshDev &m, int *mlist, int *loc, int op0, int max_rounds, hipStream_t st);
 void launch_missing_init(MeshDev &m, const int *vor, int *mlist, int *loc, hipStream_t st);
 void launch_insert_round(MeshDev &m, int *mlist, int *loc, int op, int grid, hipStream_t st);
 void launch_relink(MeshDev &m, const int *modlist, int cnt_slot, int op, int grid, hipStream_t st);
@@ -287,7 +296,7 @@ void launch_counters_to_host(int *counters, int slot, int n, int fold, int *host
 void launch_flip_all(MeshDev &m, int op, int *list, hipStream_t st);
 // flip passes on short lists in one workgroup (see k_flip_tail)
 void launch_flip_tail(MeshDev &m, int *lA, int sA, int *lB, int sB, int prev_op, int op0, int max_passes,
-                      hipStream_t st);
+                      int limit, hipStream_t st);
 void launch_flip_pass(MeshDev &m, const int *list_in, int cnt_in_slot, int *list_out, int cnt_out_slot,
                       int prev_op, int op, int grid, bool split, hipStream_t st);
 // Blocks of 256 threads for a round over about `items` list entries: enough for one entry per

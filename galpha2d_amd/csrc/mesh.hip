@@ -47,6 +47,7 @@ GA_INLINE XcdRange xcd_range(int n, int unit, int at)
 #define GRID_STRIDE(i, n) \
     for (auto [i, i##_end, i##_step] = xcd_range(n, (int)blockDim.x, (int)threadIdx.x); i < i##_end; i += i##_step)
 #define FIXED_GRID 2048
+#define TAIL_THREADS 1024    // of the single-workgroup insertion rounds and flip passes
 
 GA_INLINE int ic(const int4 &a, int i) { return i == 0 ? a.x : (i == 1 ? a.y : a.z); }
 GA_INLINE void sc(int4 &a, int i, int v)
@@ -519,18 +520,23 @@ __global__ void k_shift_bulk(MeshDev m, unsigned char *moved, int *mark, int *wl
 // read at once, where a walk over the links is a chain of two dependent reads per triangle.
 #define FAN_LANES 8
 
+GA_INLINE void shift_star_body(const MeshDev &m, unsigned char *moved, int *mark, const int *wl_in, int nw, int *wl_out,
+                               int cnt_out_slot)
+{
+    for (auto [k, end, step] = xcd_range(nw, (int)blockDim.x / FAN_LANES, (int)threadIdx.x / FAN_LANES); k < end; k += step) {
+        int v = wl_in[k];
+        for (int f = m.off[v] + threadIdx.x % FAN_LANES, f1 = m.off[v + 1]; f < f1; f += FAN_LANES)
+            shift_check(m, moved, mark, m.tv[enc_t(m.fan[f].x)], wl_out, cnt_out_slot);
+    }
+}
+
 // cnt_next_slot: the output count of the next pass (neither this pass's input nor its output),
 // zeroed here so that no launch is needed between passes
 __global__ void k_shift_star(MeshDev m, unsigned char *moved, int *mark, const int *wl_in, int cnt_in_slot,
                              int *wl_out, int cnt_out_slot, int cnt_next_slot)
 {
     if (blockIdx.x == 0 && threadIdx.x == 0) m.counters[cnt_next_slot] = 0;
-    int nw = m.counters[cnt_in_slot];
-    for (auto [k, end, step] = xcd_range(nw, 256 / FAN_LANES, threadIdx.x / FAN_LANES); k < end; k += step) {
-        int v = wl_in[k];
-        for (int f = m.off[v] + threadIdx.x % FAN_LANES, f1 = m.off[v + 1]; f < f1; f += FAN_LANES)
-            shift_check(m, moved, mark, m.tv[enc_t(m.fan[f].x)], wl_out, cnt_out_slot);
-    }
+    shift_star_body(m, moved, mark, wl_in, m.counters[cnt_in_slot], wl_out, cnt_out_slot);
 }
 
 void launch_shift_bulk(MeshDev &m, unsigned char *moved, int *mark, int *wl_out, int cnt_out_slot,
@@ -552,15 +558,13 @@ void launch_shift_star(MeshDev &m, unsigned char *moved, int *mark, const int *w
 // deletion rounds only look at these; a listed vertex that has left the pending state since is skipped by
 // its state.  Before the end it only says so in C_SHIFTING: the list stays empty, so the
 // rounds launched behind it find nothing to do.
-__global__ __launch_bounds__(256) void k_shift_commit(MeshDev m, const unsigned char *moved, int cnt_slot)
+GA_INLINE void shift_commit_body(const MeshDev &m, const unsigned char *moved)
 {
-    const bool open = m.counters[cnt_slot] != 0;
-    if (blockIdx.x == 0 && threadIdx.x == 0) m.counters[C_SHIFTING] = open;
-    if (open || *m.status) return;
-    XCD_STRIDE(b0, m.n, 1024) {
+    const int bd = (int)blockDim.x;
+    XCD_STRIDE(b0, m.n, 4 * bd) {
         unsigned bits = 0;
         for (int j = 0; j < 4; j++) {
-            int v = b0 + j * 256 + (int)threadIdx.x;
+            int v = b0 + j * bd + (int)threadIdx.x;
             if (v >= m.n || m.vstate[v] != VS_PENDING) continue;
             if (moved[v]) {
                 m.pos[v] = m.xy[v];
@@ -569,8 +573,16 @@ __global__ __launch_bounds__(256) void k_shift_commit(MeshDev m, const unsigned 
         }
         int k = block_reserve(&m.counters[C_PLIST], __popc(bits));
         for (int j = 0; j < 4; j++)
-            if ((bits >> j) & 1) m.plist[k++] = b0 + j * 256 + (int)threadIdx.x;
+            if ((bits >> j) & 1) m.plist[k++] = b0 + j * bd + (int)threadIdx.x;
     }
+}
+
+__global__ __launch_bounds__(256) void k_shift_commit(MeshDev m, const unsigned char *moved, int cnt_slot)
+{
+    const bool open = m.counters[cnt_slot] != 0;
+    if (blockIdx.x == 0 && threadIdx.x == 0) m.counters[C_SHIFTING] = open;
+    if (open || *m.status) return;
+    shift_commit_body(m, moved);
 }
 
 void launch_shift_commit(MeshDev &m, const unsigned char *moved, int cnt_slot, hipStream_t st)
@@ -588,11 +600,11 @@ GA_INLINE uint32_t vprio(int v, int round) { return hash32((uint32_t)v * 0x9E377
 // move: one launch decides and moves.  (With one lane per vertex walking the links, and a launch
 // of its own for the moves, a round took 20 us at 1M points and
 // 18 at 12,007 in clusters, now 5.5 and 3.2.)
-__global__ __launch_bounds__(256) void k_shift_greedy(MeshDev m, int round, int *mark)
+GA_INLINE bool shift_greedy_body(const MeshDev &m, int round, int *mark, int np)
 {
-    int np = m.counters[C_PLIST];
+    bool moves = false;   // this lane moved a vertex
     const int sub = threadIdx.x % FAN_LANES, shift = __lane_id() - sub;
-    for (auto [k, end, step] = xcd_range(np, 256 / FAN_LANES, threadIdx.x / FAN_LANES); k < end; k += step) {
+    for (auto [k, end, step] = xcd_range(np, (int)blockDim.x / FAN_LANES, (int)threadIdx.x / FAN_LANES); k < end; k += step) {
         int v = m.plist[k];
         if (mark[v] != 1) continue;
         uint32_t p = vprio(v, round);
@@ -613,8 +625,15 @@ __global__ __launch_bounds__(256) void k_shift_greedy(MeshDev m, int round, int 
             m.pos[v] = q;
             m.vstate[v] = VS_IN_MESH;
             mark[v] = round + 2;
+            moves = true;
         }
     }
+    return moves;
+}
+
+__global__ __launch_bounds__(256) void k_shift_greedy(MeshDev m, int round, int *mark)
+{
+    shift_greedy_body(m, round, mark, m.counters[C_PLIST]);
 }
 
 void launch_shift_greedy(MeshDev &m, int round, int *mark, int grid, hipStream_t st)
@@ -632,14 +651,8 @@ GA_INLINE unsigned long long prio64(int v, int round)
 }
 
 // distance-2 independence: every vertex records the largest priority in its closed neighbourhood
-// also zeroes the scratch count and the flag of pending vertices that k_del_apply of this round sets
-__global__ void k_del_prio(MeshDev m, unsigned long long *mx, int round)
+GA_INLINE void del_prio_body(const MeshDev &m, unsigned long long *mx, int round, int np)
 {
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        m.counters[C_SCR] = 0;
-        m.counters[C_PLEFT] = 0;
-    }
-    int np = m.counters[C_PLIST];
     GRID_STRIDE(k, np) {
         int v = m.plist[k];
         if (m.vstate[v] != VS_PENDING) continue;
@@ -656,6 +669,16 @@ __global__ void k_del_prio(MeshDev m, unsigned long long *mx, int round)
             if (++guard > 100000) break;
         } while (t != t0);
     }
+}
+
+// also zeroes the scratch count and the flag of pending vertices that k_del_apply of this round sets
+__global__ void k_del_prio(MeshDev m, unsigned long long *mx, int round)
+{
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        m.counters[C_SCR] = 0;
+        m.counters[C_PLEFT] = 0;
+    }
+    del_prio_body(m, mx, round, m.counters[C_PLIST]);
 }
 
 // link two (triangle, slot) sides of one edge; X < 0 means hull
@@ -762,34 +785,45 @@ GA_INLINE void wave_lds_sync()
 
 #define DEL_LANES 16         // lanes of a vertex
 #define DEL_MAX 64           // most corners of its polygon in LDS
-#define DEL_GROUPS (256 / DEL_LANES)
 
-// Bound by dependent reads: a block takes 64 listed vertices, keeps those that hold the maximum at
+// Bound by dependent reads: a block takes 64 listed vertices (ENT), keeps those that hold the maximum at
 // themselves, and gives each of them to 16 lanes.  One lane walks the star and puts the polygon into
 // LDS; the lanes check its corners' maxima and then test all ears at once (the one with the lowest index
 // is cut, and only its two neighbours are tested again).  One lane per vertex, walking the
 // star twice and testing ears one after another from memory, took 37 us per round at 1M points and
 // 40, up to 106, at 12,007 in clusters (long polygons), this 27 and 14, up to 40.
-__global__ __launch_bounds__(256) void k_del_apply(MeshDev m, const unsigned long long *mx, int round)
+template <int BD, int ENT>
+GA_INLINE bool del_apply_body(const MeshDev &m, const unsigned long long *mx, int round, int np)
 {
+    constexpr int DEL_GROUPS = BD / DEL_LANES;
     __shared__ int s_poly[DEL_GROUPS][DEL_MAX], s_link[DEL_GROUPS][DEL_MAX], s_slot[DEL_GROUPS][DEL_MAX];
     __shared__ double2 s_pos[DEL_GROUPS][DEL_MAX];
     __shared__ unsigned char s_prv[DEL_GROUPS][DEL_MAX], s_nxt[DEL_GROUPS][DEL_MAX];
-    __shared__ int s_cand[64], s_nc;
-    const int np = m.counters[C_PLIST], tid = threadIdx.x, grp = tid / DEL_LANES, l = tid % DEL_LANES;
+    __shared__ int s_cand[ENT], s_nc;
+    const int tid = threadIdx.x, grp = tid / DEL_LANES, l = tid % DEL_LANES;
     const int shift = (tid & 63) - l;
     int *poly = s_poly[grp], *link = s_link[grp], *slot = s_slot[grp];
     double2 *pos = s_pos[grp];
     unsigned char *prv = s_prv[grp], *nxt = s_nxt[grp];
     auto group = [&](bool b) { return (unsigned)(__ballot(b) >> shift) & ((1u << DEL_LANES) - 1u); };
     bool left = false;   // a vertex stays pending
-    XCD_STRIDE(b0, np, 64) {
-        if (tid < 64) {
+    XCD_STRIDE(b0, np, ENT) {
+        if (ENT > 64) {
+            if (tid == 0) s_nc = 0;
+            __syncthreads();
+        }
+        if (tid < ENT) {
             int v = b0 + tid < np ? m.plist[b0 + tid] : -1;
             bool pend = v >= 0 && m.vstate[v] == VS_PENDING, cand = pend && mx[v] == prio64(v, round);
             unsigned long long b = __ballot(cand);
-            if (cand) s_cand[__popcll(b & ((1ull << tid) - 1ull))] = v;
-            if (tid == 0) s_nc = __popcll(b);
+            int at = 0;
+            if (ENT > 64) {
+                if ((tid & 63) == 0) at = atomicAdd(&s_nc, (int)__popcll(b));
+                at = __shfl(at, 0, 64);
+            } else if (tid == 0) {
+                s_nc = __popcll(b);
+            }
+            if (cand) s_cand[at + __popcll(b & ((1ull << (tid & 63)) - 1ull))] = v;
             left |= pend && !cand;
         }
         __syncthreads();
@@ -901,7 +935,58 @@ __global__ __launch_bounds__(256) void k_del_apply(MeshDev m, const unsigned lon
         }
         __syncthreads();
     }
-    if (__syncthreads_or(left) && tid == 0) m.counters[C_PLEFT] = 1;
+    return __syncthreads_or(left);
+}
+
+__global__ __launch_bounds__(256) void k_del_apply(MeshDev m, const unsigned long long *mx, int round)
+{
+    if (del_apply_body<256, 64>(m, mx, round, m.counters[C_PLIST]) && threadIdx.x == 0) m.counters[C_PLEFT] = 1;
+}
+
+// Small sets: bulk shifting from its first worklist on, the commit, the greedy rounds and the
+// deletions in one workgroup, phases separated by barriers.  A launch of a few thousand lanes costs the host
+// about 5 us and the device 2.5, and there are 25 of them (1,000 points: 840 us for the call with them, 770;
+// 5,003 points 762 and 699); from some ten thousand points on the rounds keep more than one CU busy.
+// more: only further deletion rounds (the ones before were not enough).
+#define SHIFT_TAIL_THREADS 512
+__global__ __launch_bounds__(SHIFT_TAIL_THREADS) void k_shift_tail(MeshDev m, unsigned char *moved, int *mark, int *wlA,
+                                                                   int *wlB, int slot, unsigned long long *mx, int round0,
+                                                                   int max_rounds, int more)
+{
+    int *lin = wlA, *lout = wlB;
+    for (int s = 0; !more; s++) {   // counters[slot + s % 2]: the pass's worklist (every vertex is listed once)
+        const int nw = m.counters[slot + (s & 1)];
+        if (nw == 0) break;
+        __syncthreads();
+        if (threadIdx.x == 0) m.counters[slot + 1 - (s & 1)] = 0;
+        __syncthreads();
+        shift_star_body(m, moved, mark, lin, nw, lout, slot + 1 - (s & 1));
+        __syncthreads();
+        int *t = lin; lin = lout; lout = t;
+    }
+    if (threadIdx.x == 0) m.counters[C_SHIFTING] = 0;
+    if (__syncthreads_or(*m.status != 0)) return;
+    if (!more) shift_commit_body(m, moved);
+    __syncthreads();
+    const int np = m.counters[C_PLIST];
+    bool left = np > 0;
+    for (int r = 0; r < 8 && left && !more; r++)
+        if (!__syncthreads_or(shift_greedy_body(m, r, mark, np))) break;
+    for (int r = 0; r < max_rounds && left; r++) {
+        if (threadIdx.x == 0) m.counters[C_SCR] = 0;
+        del_prio_body(m, mx, round0 + r, np);
+        __syncthreads();
+        left = del_apply_body<SHIFT_TAIL_THREADS, SHIFT_TAIL_THREADS>(m, mx, round0 + r, np);
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) m.counters[C_PLEFT] = left;
+}
+
+void launch_shift_tail(MeshDev &m, unsigned char *moved, int *mark, int *wlA, int *wlB, int slot, unsigned int *mx,
+                       int round0, int max_rounds, bool more, hipStream_t st)
+{
+    GA_LAUNCH(k_shift_tail, dim3(1), dim3(SHIFT_TAIL_THREADS), 0, st, m, moved, mark, wlA, wlB, slot,
+              (unsigned long long *)mx, round0, max_rounds, more ? 1 : 0);
 }
 
 void launch_delete_round(MeshDev &m, unsigned int *mxraw, int round, int grid, hipStream_t st)
@@ -977,13 +1062,8 @@ void launch_missing_init(MeshDev &m, const int *vor, int *mlist, int *loc, hipSt
 // located: lt = (type << 2) | edge ; type 1 inside, 2 on edge, 3 duplicate ; -1 not located
 // also zeroes the modified-slot count and the flag of missing vertices that k_insert of this round
 // sets (the previous round's relink, which read the count, has finished)
-__global__ void k_locate(MeshDev m, const int *mlist, int *loc, int *lt, int op)
+GA_INLINE void locate_body(const MeshDev &m, const int *mlist, int *loc, int *lt, int op, int nm)
 {
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        m.counters[C_MODN] = 0;
-        m.counters[C_MLEFT] = 0;
-    }
-    int nm = m.counters[C_MISS];
     GRID_STRIDE(k, nm) {
         int v = mlist[k];
         lt[k] = -1;
@@ -1039,9 +1119,17 @@ __global__ void k_locate(MeshDev m, const int *mlist, int *loc, int *lt, int op)
     }
 }
 
-__global__ void k_insert(MeshDev m, const int *mlist, const int *loc, const int *lt, int op, int *list_out)
+__global__ void k_locate(MeshDev m, const int *mlist, int *loc, int *lt, int op)
 {
-    int nm = m.counters[C_MISS];
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        m.counters[C_MODN] = 0;
+        m.counters[C_MLEFT] = 0;
+    }
+    locate_body(m, mlist, loc, lt, op, m.counters[C_MISS]);
+}
+
+GA_INLINE bool insert_body(const MeshDev &m, const int *mlist, const int *loc, const int *lt, int op, int *list_out, int nm)
+{
     bool left = false;   // a vertex stays missing
     GRID_STRIDE(k, nm) {
         int L = lt[k];
@@ -1116,8 +1204,13 @@ __global__ void k_insert(MeshDev m, const int *mlist, const int *loc, const int 
         m.pos[v] = m.xy[v];
         stat_inc(m.stats, C_INSERTED, true);
     }
+    return __syncthreads_or(left);
+}
+
+__global__ void k_insert(MeshDev m, const int *mlist, const int *loc, const int *lt, int op, int *list_out)
+{
     // (one store per block: a million to the one word took 0.4 ms)
-    if (__syncthreads_or(left) && threadIdx.x == 0) m.counters[C_MLEFT] = 1;
+    if (insert_body(m, mlist, loc, lt, op, list_out, m.counters[C_MISS]) && threadIdx.x == 0) m.counters[C_MLEFT] = 1;
 }
 
 void launch_insert_round(MeshDev &m, int *mlist, int *loc, int op, int grid, hipStream_t st)
@@ -1164,6 +1257,31 @@ void launch_relink(MeshDev &m, const int *modlist, int cnt_slot, int op, int gri
     GA_LAUNCH(k_relink, dim3(grid), dim3(256), 0, st, m, modlist, cnt_slot, op, -1);
 }
 
+// Small sets: the insertion rounds in one workgroup until nothing is missing or max_rounds run out
+__global__ __launch_bounds__(TAIL_THREADS) void k_insert_tail(MeshDev m, int *mlist, int *loc, int op0, int max_rounds)
+{
+    const int nm = m.counters[C_MISS];
+    bool left = nm > 0;
+    int r = 0;
+    for (; r < max_rounds && left; r++) {
+        if (threadIdx.x == 0) m.counters[C_MODN] = 0;
+        locate_body(m, mlist, loc, m.lt, op0 + r, nm);
+        __syncthreads();
+        left = insert_body(m, mlist, loc, m.lt, op0 + r, m.modA, nm);
+        relink_body(m, m.modA, m.counters[C_MODN], op0 + r);
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) {
+        m.counters[C_MLEFT] = left;
+        m.counters[C_INSERT_ROUNDS] = r;
+    }
+}
+
+void launch_insert_tail(MeshDev &m, int *mlist, int *loc, int op0, int max_rounds, hipStream_t st)
+{
+    GA_LAUNCH(k_insert_tail, dim3(1), dim3(TAIL_THREADS), 0, st, m, mlist, loc, op0, max_rounds);
+}
+
 // ---- constraint edge set ----------------------------------------------------------------------
 // key of the undirected edge {a, b}; never 0 (the empty mark)
 GA_INLINE unsigned long long cons_key(int a, int b)
@@ -1202,7 +1320,10 @@ __global__ void k_flip_all(MeshDev m, int op, int *list, int cnt_slot)
         m.stamp[t] = op;
         list[t] = t;
     }
-    if (blockIdx.x == 0 && threadIdx.x == 0) m.counters[cnt_slot] = n;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        m.counters[cnt_slot] = n;
+        m.counters[C_CAND] = 0;
+    }
 }
 
 void launch_flip_all(MeshDev &m, int op, int *list, hipStream_t st)
@@ -1409,17 +1530,16 @@ __global__ void k_flip_commit(MeshDev m, int op, int *list_out, int cnt_out_slot
 
 // Short lists: the remaining passes in one workgroup, phases separated by block barriers instead
 // of launches, until a pass flips nothing (counters[C_TAIL_DONE] = 1) or the list outgrows
-// TAIL_LIST or max_passes run out (the host goes on with grid passes).  Pass k uses op op0 + k;
+// limit or max_passes run out (the host goes on with grid passes).  Pass k uses op op0 + k;
 // counters[C_TAIL_PASSES] = passes run (odd: the lists have swapped).
-#define TAIL_THREADS 1024
 __global__ __launch_bounds__(TAIL_THREADS) void k_flip_tail(MeshDev m, int *lA, int sA, int *lB, int sB,
-                                                            int prev_op, int op0, int max_passes)
+                                                            int prev_op, int op0, int max_passes, int limit)
 {
     int *lin = lA, *lout = lB, sin = sA, sout = sB;
     int prev = prev_op, pass = 0, done = 0;
     for (; pass < max_passes; pass++) {
         const int n = m.counters[sin];
-        if (n > TAIL_LIST) break;
+        if (n > limit) break;
         const int op = op0 + pass;
         __syncthreads();   // every thread has read n before the counters are reset
         if (threadIdx.x == 0) {
@@ -1455,9 +1575,9 @@ __global__ __launch_bounds__(TAIL_THREADS) void k_flip_tail(MeshDev m, int *lA, 
 }
 
 void launch_flip_tail(MeshDev &m, int *lA, int sA, int *lB, int sB, int prev_op, int op0, int max_passes,
-                      hipStream_t st)
+                      int limit, hipStream_t st)
 {
-    GA_LAUNCH(k_flip_tail, dim3(1), dim3(TAIL_THREADS), 0, st, m, lA, sA, lB, sB, prev_op, op0, max_passes);
+    GA_LAUNCH(k_flip_tail, dim3(1), dim3(TAIL_THREADS), 0, st, m, lA, sA, lB, sB, prev_op, op0, max_passes, limit);
 }
 
 // Three launches per pass (four with the exact tests split off) and no counter resets of their own: the test clears the output list's
