@@ -1191,16 +1191,20 @@ static int run_batch(galpha_ctx *c, const double *d_xy, const BatchPlan &plan)
     // the live-triangle count stays on the device (folded statistic) until the final read
     c->out9.ensure(36 * (size_t)nslots + 64);
     launch_fold_stats(c->counters.as<int>(), st);
-    launch_canon_emit(m, order, skey32, v1s, vals, c->rot.as<int>(), c->newid.as<int>(),
+    // (records in the fan buffer, 24 bytes per slot)
+    launch_canon_emit(m, order, skey32, v1s, vals, c->rot.as<int>(), c->newid.as<int>(), c->fan.as<int2>(),
                       c->counters.as<int>() + C_FOLD + C_RECON_TRIS, c->out9.as<int>(), c->setFirst.as<int>(),
                       c->keys2.as<int>(), st);   // keys2 (v1s) is free after k_canon_newid: output sets
     ev_mark(c, 8, st);
     Snap fin;
     std::vector<int> sfv((size_t)nsets + sizeof(fin.v) / 4);   // first triangle of every set, then the counters
-    ctx_read_segments(c, {{c->setFirst.as<int>(), nsets}, {c->counters.as<int>(), (int)(sizeof(fin.v) / 4)}},
-                      sfv.data());
+    if (nsets > 1)
+        ctx_read_segments(c, {{c->setFirst.as<int>(), nsets}, {c->counters.as<int>(), (int)(sizeof(fin.v) / 4)}},
+                          sfv.data());
+    else
+        ctx_read_segments(c, {{c->counters.as<int>(), (int)(sizeof(fin.v) / 4)}}, sfv.data() + 1);
     memcpy(fin.v, sfv.data() + nsets, sizeof(fin.v));
-    const int *sf = sfv.data();
+    const int *sf = sfv.data();   // (a single set's: 0)
     if (fin.status()) throw GalphaError("canonical output failed (status " + std::to_string(fin.status()) + ")");
     int F = fin.stat(C_RECON_TRIS);
     // sets without triangles start where the next set starts

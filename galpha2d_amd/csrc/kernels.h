@@ -323,10 +323,9 @@ void launch_canon_keys(MeshDev &m, unsigned long long *keys, int *vals, int *rot
 // canonical keys of 32 bits up to input indices below 2^CANON_KEY32_BITS
 #define CANON_KEY32_BITS 24
 void launch_canon_keys32(MeshDev &m, unsigned *keys, unsigned *v1s, int *vals, int *rot, int B, hipStream_t st);
-// out: [nslots] the order when skey is given (32-bit keys)
-void launch_canon_emit(MeshDev &m, const int *order, const unsigned *skey, const unsigned *v1s, int *out, const int *rot, int *newid,
-                       const int *dF, int *out9,
-                       int *set_first, int *rset, hipStream_t st);
+// out: [nslots] the order when skey is given (32-bit keys); rec: 24 bytes per slot; set_first: batches only
+void launch_canon_emit(MeshDev &m, const int *order, const unsigned *skey, const unsigned *v1s, int *out, const int *rot,
+                       int *newid, int2 *rec, const int *dF, int *out9, int *set_first, int *rset, hipStream_t st);
 int sort_pairs_u64(unsigned long long *keys_in, int *vals_in, unsigned long long *keys_out, int *vals_out,
                    int n, int begin_bit, int end_bit, void *temp, size_t *temp_bytes, hipStream_t st);
 int sort_pairs_u32(unsigned int *keys_in, int *vals_in, unsigned int *keys_out, int *vals_out,

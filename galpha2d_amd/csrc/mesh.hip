@@ -2065,17 +2065,6 @@ void launch_hull(MeshDev &m, const HullDev &h, int op, void *scan_tmp, hipStream
     GA_LAUNCH(k_hull_fill, dim3(FIXED_GRID), dim3(256), 0, st, m, h);
 }
 
-// Ranges in canonical order: input order inside a set (not spatial), one set after another.  A
-// batch's sets are shared out to the XCDs, a single set is not (k_canon_emit: 1M points 129 us against
-// 165 with shares, 1,024 sets 1,534 against 1,362).
-GA_INLINE XcdRange canon_range(const MeshDev &m, int n)
-{
-    const int bd = (int)blockDim.x, tid = (int)threadIdx.x;
-    if (m.nsets > 1) return xcd_range(n, bd, tid);
-    return {(int)blockIdx.x * bd + tid, n, (int)gridDim.x * bd};
-}
-#define CANON_STRIDE(i, n) for (auto [i, i##_end, i##_step] = canon_range(m, n); i < i##_end; i += i##_step)
-
 // ---- canonical output ----------------------------------------------------------------------------
 // Output order: (v0, v1, v2) of input indices with v0 the smallest vertex; input indices of the sets
 // of a batch are consecutive ranges in set order, so this is also set order.  Every directed edge
@@ -2170,15 +2159,57 @@ __global__ void k_canon_newid(const int *order, const unsigned *skey, const unsi
     }
 }
 
-// out9 holds global vertex ids and global triangle positions.  One thread per output record r,
-// from the slot order[r] that k_canon_newid left there (the inverse of newid): neighbouring lanes
-// write whole records (75 MB written at 1M points, 319 MB when each slot scattered its record),
-// and the slot reads become gathers, since the canonical order follows input ids.
-// Batches: rset[r] = set of output triangle r, for k_canon_set_first.
-__global__ void k_canon_emit(MeshDev m, const int *order, const int *newid, const int *dF, int *out9, int *rset)
+// out9 holds global vertex ids and global triangle positions.  The slots are in spatial order and the
+// output is in the order of the input indices, so one of the two sides is scattered whatever the
+// order of the work: k_canon_records makes the six words of a slot's record in slot order (its
+// neighbours' positions and its vertices' ids lie close together there), and k_canon_emit, one thread
+// per output record, gathers them, so that neighbouring lanes write whole records (gathering vertices,
+// links, positions and ids per output record instead took 565 us at 4M points, this 356; 129 and 84 at
+// 1M).  A batch's sets are small enough that the gathers of a set stay in its L2: there
+// k_canon_emit_sets makes the records on the way (1,024 sets: 1,354 us, in two steps 1,608).
+__global__ __launch_bounds__(256) void k_canon_records(MeshDev m, const int *newid, int2 *rec)
+{
+    const int n = ntri_used(m);
+    GRID_STRIDE(t, n) {
+        const int4 v = m.tv[t];
+        if (v.x == GA_DEAD) continue;
+        const int4 nb = m.tn[t];
+        const int ro = newid[t] & 3;
+        int w[6];
+#pragma unroll
+        for (int i = 0; i < 3; i++) {
+            const int si = (i + ro) % 3;
+            w[3 + i] = oid(m, ic(v, si));
+            const int e = ic(nb, si);
+            w[i] = -1;
+            if (e >= 0) {
+                const int nu = newid[enc_t(e)];
+                w[i] = enc(nu >> 2, (enc_j(e) - (nu & 3) + 3) % 3);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 3; i++) rec[3 * (size_t)t + i] = make_int2(w[2 * i], w[2 * i + 1]);
+    }
+}
+
+__global__ __launch_bounds__(256) void k_canon_emit(const int *order, const int2 *rec, const int *dF, int *out9)
 {
     const int F = *dF;
-    CANON_STRIDE(r, F) {
+    for (int r = blockIdx.x * 256 + threadIdx.x; r < F; r += gridDim.x * 256) {
+        const int2 *w = rec + 3 * (size_t)order[r];
+        const int2 a = w[0], b = w[1], c = w[2];
+        int *o = out9 + (size_t)r * 9;
+        o[0] = a.x; o[1] = a.y; o[2] = b.x;
+        o[3] = b.y; o[4] = c.x; o[5] = c.y;
+        o[6] = 0; o[7] = 0; o[8] = 0;
+    }
+}
+
+// rset[r] = set of output triangle r, for k_canon_set_first
+__global__ void k_canon_emit_sets(MeshDev m, const int *order, const int *newid, const int *dF, int *out9, int *rset)
+{
+    const int F = *dF;
+    GRID_STRIDE(r, F) {
         const int s = order[r];
         const int4 v = m.tv[s];
         const int ro = newid[s] & 3;
@@ -2199,7 +2230,7 @@ __global__ void k_canon_emit(MeshDev m, const int *order, const int *newid, cons
         int *o = out9 + (size_t)r * 9;
 #pragma unroll
         for (int i = 0; i < 9; i++) o[i] = rec[i];
-        if (m.nsets > 1) rset[r] = m.vset[v.x];
+        rset[r] = m.vset[v.x];
     }
 }
 
@@ -2207,23 +2238,24 @@ __global__ void k_canon_emit(MeshDev m, const int *order, const int *newid, cons
 __global__ void k_canon_set_first(MeshDev m, const int *rset, const int *dF, int *set_first)
 {
     int F = *dF;
-    if (m.nsets == 1) {
-        if (blockIdx.x == 0 && threadIdx.x == 0 && F > 0) set_first[0] = 0;
-        return;
-    }
-    CANON_STRIDE(r, F) {
+    GRID_STRIDE(r, F) {
         int set = rset[r];
         if (r == 0 || rset[r - 1] != set) set_first[set] = r;
     }
 }
 
-void launch_canon_emit(MeshDev &m, const int *order, const unsigned *skey, const unsigned *v1s, int *out, const int *rot, int *newid,
-                       const int *dF, int *out9, int *set_first, int *rset, hipStream_t st)
+void launch_canon_emit(MeshDev &m, const int *order, const unsigned *skey, const unsigned *v1s, int *out, const int *rot,
+                       int *newid, int2 *rec, const int *dF, int *out9, int *set_first, int *rset, hipStream_t st)
 {
-    launch_fill_i32(set_first, -1, (size_t)m.nsets, st);
     GA_LAUNCH(k_canon_newid, dim3(FIXED_GRID), dim3(256), 0, st, order, skey, v1s, rot, dF, newid, out);
-    GA_LAUNCH(k_canon_emit, dim3(FIXED_GRID), dim3(256), 0, st, m, skey ? (const int *)out : order, (const int *)newid, dF, out9,
-              rset);
+    const int *sorted = skey ? out : order;
+    if (m.nsets == 1) {   // (its first triangle is triangle 0)
+        GA_LAUNCH(k_canon_records, dim3(FIXED_GRID), dim3(256), 0, st, m, (const int *)newid, rec);
+        GA_LAUNCH(k_canon_emit, dim3(FIXED_GRID), dim3(256), 0, st, sorted, (const int2 *)rec, dF, out9);
+        return;
+    }
+    GA_LAUNCH(k_canon_emit_sets, dim3(FIXED_GRID), dim3(256), 0, st, m, sorted, (const int *)newid, dF, out9, rset);
+    launch_fill_i32(set_first, -1, (size_t)m.nsets, st);
     GA_LAUNCH(k_canon_set_first, dim3(FIXED_GRID), dim3(256), 0, st, m, (const int *)rset, dF, set_first);
 }
 
