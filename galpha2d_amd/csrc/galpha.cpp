@@ -660,23 +660,22 @@ static BatchDev upload_plan(galpha_ctx *c, const BatchPlan &b)
     return d;
 }
 
+// what the discrete diagram needs cleared: site map, island marks, far flags (its counters are zero too)
+static void pba_clears(galpha_ctx *c, const BatchPlan &b, IntFills &f)
+{
+    f.add(c->smap.p, b.P, 0x7fffffff);
+    f.add(c->bad.p, (size_t)b.V + 1, 0);
+    f.add(c->setfar.p, (size_t)b.nsets(), 0);
+    f.add(c->far.p, 4 * (size_t)b.blocks[BM_LABEL], 0);
+}
+
 // perm: input index of each real point when they were renumbered (NULL: input order)
 static void run_pba(galpha_ctx *c, const double *d_xy, const BatchDev &bd, int *iters, int *island_sites,
                     const int *perm)
 {
     hipStream_t st = c->stream;
-    launch_fill_i32(c->smap.as<int>(), 0x7fffffff, bd.P, st);
     if (!perm) launch_vset(bd, c->vset.as<int>(), st);   // (else the renumbering has done it)
     launch_splat((const double2 *)d_xy, bd, perm, c->smap.as<int>(), c->pix.as<int>(), c->fpix.as<int>(), st);
-    {
-        IntFills f;   // island marks, and the island counters of the first pass
-        f.add(c->bad.p, (size_t)bd.V + 1, 0);
-        f.add(c->counters.as<int>() + C_ISLAND_SITES, 1, 0);
-        f.add(c->counters.as<int>() + C_FLAG, 1, 0);
-        f.add(c->setfar.p, (size_t)bd.nsets, 0);
-        f.add(c->far.p, 4 * (size_t)bd.blocks[BM_LABEL], 0);
-        launch_fill_multi(f, st);
-    }
     PbaBuffers b{c->smap.as<int>(), c->g.as<short>(), c->hmin.as<short>(), c->far.as<int>(), c->setfar.as<int>(),
                  c->vor.as<int>()};
     int it = 0, isl = 0;
@@ -765,17 +764,7 @@ static Snap remove_frame(galpha_ctx *c, MeshDev &m, hipStream_t st)
 static const double *renumber_points(galpha_ctx *c, const double *d_xy, const BatchDev &bd, const BatchPlan &plan)
 {
     hipStream_t st = c->stream;
-    int n = bd.ntot;
-    size_t nc = (size_t)plan.ncells + 1;
-    c->perm.ensure(4 * (size_t)n + 64);
-    c->xys.ensure(16 * (size_t)n + 64);
-    c->pcell.ensure(4 * (size_t)n + 64);
-    c->lt.ensure(4 * (size_t)n);   // (the missing sites' later)
-    c->ccount.ensure(4 * nc + 64);
-    c->ccursor.ensure(4 * nc + 64);
-    c->scanTmp.ensure(scan_temp_bytes(nc) + 4096);
     launch_vset(bd, c->vset.as<int>(), st);
-    HIPCHK(hipMemsetAsync(c->ccount.p, 0, 4 * nc, st));
     launch_renumber((const double2 *)d_xy, bd, c->pcell.as<int>(), c->lt.as<int>(), c->ccount.as<int>(), c->ccursor.as<int>(),
                     plan.ncells, c->scanTmp.p, c->perm.as<int>(), c->xys.as<double2>(), st);
     return c->xys.as<double>();
@@ -797,18 +786,14 @@ static int run_batch(galpha_ctx *c, const double *d_xy, const BatchPlan &plan)
     if (nsets == 0) return 0;
     int V = plan.V, n = plan.ntot;
     ensure_pba(c, plan);
-    {
-        IntFills f;
-        f.add(c->counters.p, COUNTER_BYTES / sizeof(int), 0);
-        f.add(c->status.p, 4, 0);
-        launch_fill_multi(f, st);
-    }
-    BatchDev bd = upload_plan(c, plan);
-    ev_mark(c, 0, st);
-    d_xy = renumber_points(c, d_xy, bd, plan);
-    run_pba(c, d_xy, bd, &S.pbaIterations, &S.islandSites, c->perm.as<int>());
-    ev_mark(c, 1, st);
-
+    // ---- spatial numbering
+    const size_t nc = (size_t)plan.ncells + 1;
+    c->perm.ensure(4 * (size_t)n + 64);
+    c->xys.ensure(16 * (size_t)n + 64);
+    c->pcell.ensure(4 * (size_t)n + 64);
+    c->ccount.ensure(4 * nc + 64);
+    c->ccursor.ensure(4 * nc + 64);
+    c->scanTmp.ensure(scan_temp_bytes(nc) + 4096);
     // ---- mesh buffers
     // dual triangles <= 2V; each re-inserted point adds 2 slots, each deleted vertex leaves 2 dead
     int cap = 3 * V + 8192;
@@ -841,8 +826,9 @@ static int run_batch(galpha_ctx *c, const double *d_xy, const BatchPlan &plan)
     // only grow, across runs too, so values left by earlier runs never match or beat later ones.
     // The arrays are cleared only when their memory is new (or carved from a shared scratch
     // region) and when the numbers would run out.
+    // One launch clears these and everything else that the run needs cleared.
+    IntFills f;
     {
-        IntFills f;
         const bool arena = galpha_arena_active();
         if (arena || c->op > (1 << 30) || c->tag_p[0] != c->stamp.p || c->tag_p[1] != c->claim.p ||
             c->tag_p[2] != c->lmark.p) {
@@ -857,9 +843,21 @@ static int run_batch(galpha_ctx *c, const double *d_xy, const BatchPlan &plan)
             c->mx_p = c->mx.p;
             c->prio_round = 0;
         }
-        f.add(c->vt.p, (size_t)V, -1);
-        launch_fill_multi(f, st);
     }
+    f.add(c->vt.p, (size_t)V, -1);
+    f.add(c->deg.p, (size_t)V + 1, 0);
+    f.add(c->fill.p, (size_t)V + 1, 0);
+    f.add(c->ccount.p, nc, 0);
+    f.add(c->counters.p, COUNTER_BYTES / sizeof(int), 0);
+    f.add(c->status.p, 4, 0);
+    pba_clears(c, plan, f);
+    launch_fill_multi(f, st);
+    BatchDev bd = upload_plan(c, plan);
+    ev_mark(c, 0, st);
+    d_xy = renumber_points(c, d_xy, bd, plan);
+    run_pba(c, d_xy, bd, &S.pbaIterations, &S.islandSites, c->perm.as<int>());
+    ev_mark(c, 1, st);
+
     auto next_prio_round = [&]() {
         if (++c->prio_round >= (1 << 20)) throw GalphaError("too many removal rounds");
         return c->prio_round;
@@ -892,7 +890,6 @@ static int run_batch(galpha_ctx *c, const double *d_xy, const BatchPlan &plan)
     launch_recon(c->vor.as<int>(), c->pix.as<int>(), bd, m, c->tileCnt.as<int>(), c->tileOff.as<int>(),
                  c->scanTmp.p, st);
     launch_adjacency(m, c->deg.as<int>(), c->off.as<int>(), c->fill.as<int>(), c->fan.as<int2>(), c->scanTmp.p, st);
-    launch_init_positions(m, st);
     ev_mark(c, 2, st);
     // Flip helpers: Lawson passes over the list of triangles to test; a pass with no flip has no candidate
     // left (the highest candidate always wins), so three passes run per host read.
@@ -1679,7 +1676,10 @@ int galphaVoronoi(galpha_ctx *c, const double *xy, int n, int T, int *labels, in
         ensure_pba(c, plan);
         c->xy.ensure(16 * (size_t)n);
         stage_h2d(c->stage, c->xy.p, xy, 16 * (size_t)n, c->stream);
-        HIPCHK(hipMemsetAsync(c->counters.p, 0, COUNTER_BYTES, c->stream));
+        IntFills f;
+        f.add(c->counters.p, COUNTER_BYTES / sizeof(int), 0);
+        pba_clears(c, plan, f);
+        launch_fill_multi(f, c->stream);
         BatchDev bd = upload_plan(c, plan);
         int iters = 0, isl = 0;
         run_pba(c, c->xy.as<double>(), bd, &iters, &isl, nullptr);

@@ -242,11 +242,11 @@ struct CopyParts {
     int n;
 };
 void launch_gather_parts(const CopyParts &g, int *dst, size_t words, hipStream_t st);
-// up to eight device int arrays, each set to one value, in one launch
+// up to 16 device int arrays, each set to one value, in one launch
 struct IntFills {
-    int *p[8];
-    size_t len[8];
-    int v[8];
+    int *p[16];
+    size_t len[16];
+    int v[16];
     int n = 0;
     void add(void *ptr, size_t ints, int value)
     {
@@ -265,10 +265,10 @@ void launch_exclusive_scan(const int *in, int *out, size_t n, void *temp, hipStr
 // mesh.hip
 void launch_recon(const int *vor, const int *pix, const BatchDev &b, MeshDev &m, int *tile_cnt, int *tile_off,
                   void *scan_tmp, hipStream_t st);
+// deg, fill (V + 1 ints) zero and vt -1 on entry
 void launch_adjacency(MeshDev &m, int *deg, int *off, int *fill, int2 *fan, void *scan_tmp, hipStream_t st);
-void launch_init_positions(MeshDev &m, hipStream_t st);
-// bulk shifting: one pass over all triangles (reverted vertices listed in wl_out, mark[] zero on
-// entry), then passes over the stars of the vertices the previous pass listed
+// states and positions of the vertices after the reconstruction, then bulk shifting: one pass over all
+// triangles (reverted vertices listed in wl_out), then passes over the stars of the vertices the previous pass listed
 void launch_shift_bulk(MeshDev &m, unsigned char *moved, int *mark, int *wl_out, int cnt_out_slot,
                        int cnt_next_slot, hipStream_t st);
 void launch_shift_star(MeshDev &m, unsigned char *moved, int *mark, const int *wl_in, int cnt_in_slot, int *wl_out,

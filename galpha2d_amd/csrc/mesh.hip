@@ -418,39 +418,10 @@ __global__ void k_match(const int4 *__restrict__ tv, const int *__restrict__ ntr
 
 void launch_adjacency(MeshDev &m, int *deg, int *off, int *fill, int2 *fan, void *scan_tmp, hipStream_t st)
 {
-    IntFills f;
-    f.add(deg, (size_t)m.V + 1, 0);
-    f.add(fill, (size_t)m.V + 1, 0);
-    launch_fill_multi(f, st);
     GA_LAUNCH(k_deg, dim3(FIXED_GRID), dim3(256), 0, st, m.tv, m.ntri, deg);
     launch_exclusive_scan(deg, off, m.V + 1, scan_tmp, st);
     GA_LAUNCH(k_fanfill, dim3(FIXED_GRID), dim3(256), 0, st, m.tv, m.ntri, off, fill, fan, m.vt);
     GA_LAUNCH(k_match, dim3(FIXED_GRID), dim3(256), 0, st, m.tv, m.ntri, off, fan, m.tn);
-}
-
-// ---- positions / states after reconstruction ------------------------------------------------
-// deg (from the adjacency build, still valid) says which vertices are in the mesh.
-__global__ void k_init_positions(MeshDev m, const int *__restrict__ deg)
-{
-    GRID_STRIDE(v, m.V) {
-        int in = deg[v] > 0;
-        if (v >= m.n) {
-            m.vstate[v] = VS_IN_MESH;
-            m.pos[v] = snapped(m, v);
-        } else if (in) {
-            m.vstate[v] = VS_PENDING;
-            m.pos[v] = snapped(m, v);
-        } else {
-            m.vstate[v] = VS_MISSING;
-            m.pos[v] = m.xy[v];
-            m.vt[v] = -1;
-        }
-    }
-}
-
-void launch_init_positions(MeshDev &m, hipStream_t st)
-{
-    GA_LAUNCH(k_init_positions, dim3(FIXED_GRID), dim3(256), 0, st, m, (const int *)m.deg);
 }
 
 // ---- shifting ----------------------------------------------------------------------------------
@@ -465,9 +436,12 @@ GA_INLINE double2 cand_pos(const MeshDev &m, const unsigned char *moved, int v)
 // triangle does.  Reverting only ever clears moved[], so the first pass looks at every triangle
 // and later passes only at the stars of the vertices reverted by the pass before (a worklist;
 // mark[] lists each vertex once).
-// also zeroes the revert marks, the count of k_shift_bulk's output list and that of the first
-// star pass's, and keeps what the reconstruction left in the slot count and the status word
-__global__ void k_shift_init(MeshDev m, unsigned char *moved, int *mark, int cnt_out_slot, int cnt_next_slot)
+// The first choice, with the states and positions after the reconstruction: deg (from the
+// adjacency build, still valid) says which vertices are in the mesh, and every real one of these is
+// pending.  Also zeroes the revert marks, the count of k_shift_bulk's output list and that of the
+// first star pass's, and keeps what the reconstruction left in the slot count and the status word.
+__global__ void k_shift_init(MeshDev m, const int *__restrict__ deg, unsigned char *moved, int *mark, int cnt_out_slot,
+                             int cnt_next_slot)
 {
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         m.counters[cnt_out_slot] = 0;
@@ -475,8 +449,19 @@ __global__ void k_shift_init(MeshDev m, unsigned char *moved, int *mark, int cnt
         m.counters[C_RECON_SLOTS] = *m.ntri;
         m.counters[C_RECON_STATUS] = *m.status;
     }
-    GRID_STRIDE(v, m.n) moved[v] = (m.vstate[v] == VS_PENDING) ? 1 : 0;
-    GRID_STRIDE(v, m.V) mark[v] = 0;
+    GRID_STRIDE(v, m.V) {
+        mark[v] = 0;
+        if (v >= m.n) {
+            m.vstate[v] = VS_IN_MESH;
+            m.pos[v] = snapped(m, v);
+            continue;
+        }
+        const bool in = deg[v] > 0;
+        moved[v] = in ? 1 : 0;
+        m.vstate[v] = in ? VS_PENDING : VS_MISSING;
+        m.pos[v] = in ? snapped(m, v) : m.xy[v];
+        if (!in) m.vt[v] = -1;
+    }
 }
 
 // test triangle v (vertex ids) with the current choice; revert and list its moved vertices when
@@ -542,7 +527,8 @@ __global__ void k_shift_star(MeshDev m, unsigned char *moved, int *mark, const i
 void launch_shift_bulk(MeshDev &m, unsigned char *moved, int *mark, int *wl_out, int cnt_out_slot,
                        int cnt_next_slot, hipStream_t st)
 {
-    GA_LAUNCH(k_shift_init, dim3(FIXED_GRID), dim3(256), 0, st, m, moved, mark, cnt_out_slot, cnt_next_slot);
+    GA_LAUNCH(k_shift_init, dim3(FIXED_GRID), dim3(256), 0, st, m, (const int *)m.deg, moved, mark, cnt_out_slot,
+              cnt_next_slot);
     GA_LAUNCH(k_shift_bulk, dim3(FIXED_GRID), dim3(256), 0, st, m, moved, mark, wl_out, cnt_out_slot);
 }
 

@@ -152,28 +152,22 @@ __global__ void k_splat(const double2 *__restrict__ xy, BatchDev b, const int *_
     atomicMin(&smap[sd.toff + ((size_t)px << sd.logT) + py], perm ? perm[i] : i);
 }
 
-__global__ void k_splat_own(BatchDev b, const int *__restrict__ perm, const int *__restrict__ pix,
-                            int *__restrict__ smap)
+// The winners' own indices, and the frame sites (global ids ntot .. V-1) at their border pixels (fpix: packed
+// local pixels).
+__global__ void k_splat_own(BatchDev b, const int *__restrict__ perm, const int *__restrict__ fpix,
+                            int *__restrict__ pix, int *__restrict__ smap)
 {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= b.ntot) return;
+    if (i >= b.V || (i < b.ntot && !perm)) return;
     const SetDesc &sd = b.sets[b.vset[i]];
-    int pp = pix[i];
+    const int pp = i < b.ntot ? pix[i] : fpix[i - b.ntot];
     int *cellp = &smap[sd.toff + ((size_t)(pp >> 16) << sd.logT) + (pp & 0xffff)];
-    if (*cellp == perm[i]) *cellp = i;    // one winner per pixel: no other thread writes here
-}
-
-// Frame sites (global ids ntot .. V-1) at their border pixels (fpix: packed local pixels).
-__global__ void k_splat_frame(const int *__restrict__ fpix, BatchDev b, int *__restrict__ smap,
-                              int *__restrict__ pix)
-{
-    int k = blockIdx.x * blockDim.x + threadIdx.x;
-    int f = b.ntot + k;
-    if (f >= b.V) return;
-    const SetDesc &sd = b.sets[b.vset[f]];
-    int pp = fpix[k];
-    pix[f] = pp;
-    smap[sd.toff + ((size_t)(pp >> 16) << sd.logT) + (pp & 0xffff)] = f;
+    if (i >= b.ntot) {
+        pix[i] = pp;
+        *cellp = i;
+    } else if (*cellp == perm[i]) {
+        *cellp = i;    // one winner per pixel: no other thread writes here
+    }
 }
 
 // ---- phase 1: nearest site per column --------------------------------------------------
@@ -836,14 +830,8 @@ void launch_renumber(const double2 *xy, const BatchDev &b, int *cell, int *slot,
 void launch_splat(const double2 *xy, const BatchDev &b, const int *perm, int *smap, int *pix, const int *fpix,
                   hipStream_t st)
 {
-    if (b.ntot > 0) {
-        GA_LAUNCH(k_splat, dim3((b.ntot + 255) / 256), dim3(256), 0, st, xy, b, perm, smap, pix);
-        if (perm)
-            GA_LAUNCH(k_splat_own, dim3((b.ntot + 255) / 256), dim3(256), 0, st, b, perm, (const int *)pix, smap);
-    }
-    int nf = b.V - b.ntot;
-    if (nf > 0)
-        GA_LAUNCH(k_splat_frame, dim3((nf + 255) / 256), dim3(256), 0, st, fpix, b, smap, pix);
+    if (b.ntot > 0) GA_LAUNCH(k_splat, dim3((b.ntot + 255) / 256), dim3(256), 0, st, xy, b, perm, smap, pix);
+    GA_LAUNCH(k_splat_own, dim3((b.V + 255) / 256), dim3(256), 0, st, b, perm, fpix, pix, smap);
 }
 
 void launch_pba(const PbaBuffers &p, const int *pix, const BatchDev &b, hipStream_t st)
