@@ -2,6 +2,7 @@
 // launch of one named kernel (used by bench.py for the roofline figure).  Off by default; the
 // check on every launch is one relaxed load.
 #include <hip/hip_runtime.h>
+#include <algorithm>
 #include <atomic>
 #include <cstring>
 #include <mutex>
@@ -14,13 +15,19 @@ std::mutex g_mu;
 std::string g_name;
 std::vector<hipEvent_t> g_ev;   // pairs
 size_t g_used = 0;
+// k is the probed kernel or an instance of the probed template (name<...>)
+bool probed(const char *k)
+{
+    const size_t n = g_name.size();
+    return g_name.compare(0, n, k, std::min(n, strlen(k))) == 0 && (k[n] == 0 || k[n] == '<');
+}
 }
 
 void ga_probe_begin(const char *k, hipStream_t st)
 {
     if (!g_on.load(std::memory_order_relaxed)) return;
     std::lock_guard<std::mutex> lk(g_mu);
-    if (g_name != k) return;
+    if (!probed(k)) return;
     if (g_used + 2 > g_ev.size()) {
         for (int i = 0; i < 64; i++) {
             hipEvent_t e;
@@ -35,7 +42,7 @@ void ga_probe_end(const char *k, hipStream_t st)
 {
     if (!g_on.load(std::memory_order_relaxed)) return;
     std::lock_guard<std::mutex> lk(g_mu);
-    if (g_name != k) return;
+    if (!probed(k)) return;
     (void)hipEventRecord(g_ev[g_used + 1], st);
     g_used += 2;
 }
