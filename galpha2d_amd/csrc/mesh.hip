@@ -698,8 +698,10 @@ GA_INLINE void del_failed(const MeshDev &m, int v, int msz, F poly)
 }
 
 // one lane, any number d of corners (the polygon in the scratch arena); returns the first slot, -1 when
-// the arena is full
-__device__ __noinline__ int del_serial(const MeshDev &m, int v, int d)
+// the arena is full.  Inlined: a call takes the mesh by reference, so that every lane of the caller first
+// stored its copy of the launch's argument, 36 MB per launch (k_del_apply 155 us of a run of 1,048,576
+// points with the call and 147 registers, 105 without and with 119; 1,024 sets 1,454 and 1,080).
+GA_INLINE int del_serial(const MeshDev &m, int v, int d)
 {
     // scratch: poly[d], plink[d], slots[d]
     int base = atomicAdd(&m.counters[C_SCR], 3 * d);
@@ -777,7 +779,7 @@ GA_INLINE void wave_lds_sync()
 // LDS; the lanes check its corners' maxima and then test all ears at once (the one with the lowest index
 // is cut, and only its two neighbours are tested again).  One lane per vertex, walking the
 // star twice and testing ears one after another from memory, took 37 us per round at 1M points and
-// 40, up to 106, at 12,007 in clusters (long polygons), this 27 and 14, up to 40.
+// 40, up to 106, at 12,007 in clusters (long polygons), this 17 and 10, up to 40.
 template <int BD, int ENT>
 GA_INLINE bool del_apply_body(const MeshDev &m, const unsigned long long *mx, int round, int np)
 {
