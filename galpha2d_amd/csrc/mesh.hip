@@ -47,7 +47,7 @@ GA_INLINE XcdRange xcd_range(int n, int unit, int at)
 #define GRID_STRIDE(i, n) \
     for (auto [i, i##_end, i##_step] = xcd_range(n, (int)blockDim.x, (int)threadIdx.x); i < i##_end; i += i##_step)
 #define FIXED_GRID 2048
-#define TAIL_THREADS 1024    // of the single-workgroup insertion rounds and flip passes
+#define TAIL_THREADS 1024    // of the single-workgroup insertion rounds
 
 GA_INLINE int ic(const int4 &a, int i) { return i == 0 ? a.x : (i == 1 ? a.y : a.z); }
 GA_INLINE void sc(int4 &a, int i, int v)
@@ -1520,8 +1520,12 @@ __global__ void k_flip_commit(MeshDev m, int op, int *list_out, int cnt_out_slot
 // of launches, until a pass flips nothing (counters[C_TAIL_DONE] = 1) or the list outgrows
 // limit or max_passes run out (the host goes on with grid passes).  Pass k uses op op0 + k;
 // counters[C_TAIL_PASSES] = passes run (odd: the lists have swapped).
-__global__ __launch_bounds__(TAIL_THREADS) void k_flip_tail(MeshDev m, int *lA, int sA, int *lB, int sB,
-                                                            int prev_op, int op0, int max_passes, int limit)
+// 512 threads: the exact test needs 174 registers, and 1,024 leave 128 (305 spilled).  All passes of 1,000
+// points 91 -> 59 us, of 12,007 in clusters 171 -> 111; with the exact tests as a step of their own 106 and
+// 202 (1,024 threads), 65 and 126 (512), at 256 threads without it 69 and 122.
+#define FLIP_TAIL_THREADS 512
+__global__ __launch_bounds__(FLIP_TAIL_THREADS) void k_flip_tail(MeshDev m, int *lA, int sA, int *lB, int sB,
+                                                                 int prev_op, int op0, int max_passes, int limit)
 {
     int *lin = lA, *lout = lB, sin = sA, sout = sB;
     int prev = prev_op, pass = 0, done = 0;
@@ -1565,7 +1569,8 @@ __global__ __launch_bounds__(TAIL_THREADS) void k_flip_tail(MeshDev m, int *lA, 
 void launch_flip_tail(MeshDev &m, int *lA, int sA, int *lB, int sB, int prev_op, int op0, int max_passes,
                       int limit, hipStream_t st)
 {
-    GA_LAUNCH(k_flip_tail, dim3(1), dim3(TAIL_THREADS), 0, st, m, lA, sA, lB, sB, prev_op, op0, max_passes, limit);
+    GA_LAUNCH(k_flip_tail, dim3(1), dim3(FLIP_TAIL_THREADS), 0, st, m, lA, sA, lB, sB, prev_op, op0, max_passes,
+              limit);
 }
 
 // Three launches per pass (four with the exact tests split off) and no counter resets of their own: the test clears the output list's
@@ -2559,8 +2564,10 @@ __device__ void cons_commit_one(const MeshDev &m, int c, int K, int *done, const
     for (int i = lane; i < K; i += width) modlist[q + i] = R.slots[i];
 }
 
-__global__ void k_cons_commit_small(MeshDev m, int nc, int *done, const int *cnt, const int *roff, int *work,
-                                    int *modlist, int op)
+// (the bound: without it the compiler keeps to 128 registers, for 1,024 threads, and spills; 96 us per launch
+// for 10,000 constraints at 100,000 points without, 58 with)
+__global__ __launch_bounds__(256) void k_cons_commit_small(MeshDev m, int nc, int *done, const int *cnt,
+                                                           const int *roff, int *work, int *modlist, int op)
 {
     GRID_STRIDE(c, nc) {
         int K = cnt[c];
