@@ -1785,11 +1785,28 @@ __global__ __launch_bounds__(256) void k_hull_edges(MeshDev m, HullDev h, int op
     }
 }
 
-// squared distances to v: true when a is nearer than b
-__device__ __noinline__ bool hull_nearer(double2 v, double2 a, double2 b, int *status)
+// The boundary vertices [b0, b1) of a set, and a power of two that brings the differences of its
+// coordinates to 2^15 at most.  The searches below decide in floating point what can be left out, by products
+// of up to three differences: without it these lose their bits below coordinates of 1e-103, and are
+// infinite above 1e154, where the order of the apexes (t) becomes NaN.  What is still too small (vertices
+// that lie 1e-100 of the set's size and less apart) is not left out.
+struct HullSet {
+    int b0, b1;
+    double s;
+};
+#define HULL_TINY 1e-290   // above what is lost to underflow in scaled coordinates
+__device__ HullSet hull_set(const MeshDev &m, const HullDev &h, int v)
 {
-    const double ax = a.x - v.x, ay = a.y - v.y, bx = b.x - v.x, by = b.y - v.y;
-    const double da = ax * ax + ay * ay, db = bx * bx + by * by, eb = 8.0 * GA_EPS * (da + db);
+    const SetDesc &sd = m.sets[m.vset[v]];
+    const int e = -ilogb(sd.scale);
+    return HullSet{h.bidx[sd.poff], h.bidx[sd.poff + sd.n], ldexp(1.0, e < 1023 ? e : 1023)};
+}
+
+// squared distances to v: true when a is nearer than b
+__device__ __noinline__ bool hull_nearer(double2 v, double2 a, double2 b, double sc, int *status)
+{
+    const double ax = (a.x - v.x) * sc, ay = (a.y - v.y) * sc, bx = (b.x - v.x) * sc, by = (b.y - v.y) * sc;
+    const double da = ax * ax + ay * ay, db = bx * bx + by * by, eb = 8.0 * GA_EPS * (da + db) + HULL_TINY;
     if (da - db < -eb) return true;
     if (da - db > eb) return false;
     // |a - v|^2 - |b - v|^2 exactly
@@ -1813,16 +1830,16 @@ __device__ __noinline__ bool hull_nearer(double2 v, double2 a, double2 b, int *s
     return bi_sign(sum) < 0;
 }
 
-// the boundary vertex of the set [b0, b1) nearest to its position k (one wave; -1: there is no other)
-GA_INLINE int hull_nearest(const MeshDev &m, const HullDev &h, int k, int b0, int b1, int lane)
+// the boundary vertex of the set nearest to its position k (one wave; -1: there is no other)
+GA_INLINE int hull_nearest(const MeshDev &m, const HullDev &h, int k, HullSet set, int lane)
 {
     const double2 P = h.bpos[k];
     int best = -1;
-    for (int j = b0 + lane; j < b1; j += 64)
-        if (j != k && (best < 0 || hull_nearer(P, h.bpos[j], h.bpos[best], m.status))) best = j;
+    for (int j = set.b0 + lane; j < set.b1; j += 64)
+        if (j != k && (best < 0 || hull_nearer(P, h.bpos[j], h.bpos[best], set.s, m.status))) best = j;
     for (int d = 32; d > 0; d >>= 1) {
         const int o = __shfl_xor(best, d, 64);
-        if (o >= 0 && (best < 0 || hull_nearer(P, h.bpos[o], h.bpos[best], m.status))) best = o;
+        if (o >= 0 && (best < 0 || hull_nearer(P, h.bpos[o], h.bpos[best], set.s, m.status))) best = o;
     }
     return best < 0 ? -1 : h.blist[best];
 }
@@ -1833,15 +1850,15 @@ struct HullBest {
     double2 X;
 };
 
-// The wave's best c (the same in all lanes) against the boundary positions 64 g + lane of the set
-// [b0, b1): replaced by a vertex left of p -> q and inside its circle until no lane has one.  The
+// The wave's best c (the same in all lanes) against the boundary positions 64 g + lane of the set:
+// replaced by a vertex left of p -> q and inside its circle until no lane has one.  The
 // next to try is the one that sees the edge under the largest angle (in floating point: it only
 // decides how often the loop runs, mostly once).
-GA_INLINE void hull_chunk(const MeshDev &m, const HullDev &h, double2 P, double2 Q, int p, int q, int g, int b0,
-                          int b1, int lane, HullBest &c)
+GA_INLINE void hull_chunk(const MeshDev &m, const HullDev &h, double2 P, double2 Q, int p, int q, int g, HullSet set,
+                          int lane, HullBest &c)
 {
     const int j = 64 * g + lane;
-    const bool in = j >= b0 && j < b1;
+    const bool in = j >= set.b0 && j < set.b1;
     const double2 X = in ? h.bpos[j] : P;
     const int x = in ? h.blist[j] : p;
     int o = orient_filter(P, Q, X);
@@ -1851,7 +1868,8 @@ GA_INLINE void hull_chunk(const MeshDev &m, const HullDev &h, double2 P, double2
     bool better = o > 0 && x != p && x != q;
     double t = INFINITY;
     if (better) {
-        const double ax = P.x - X.x, ay = P.y - X.y, bx = Q.x - X.x, by = Q.y - X.y;
+        const double ax = (P.x - X.x) * set.s, ay = (P.y - X.y) * set.s;
+        const double bx = (Q.x - X.x) * set.s, by = (Q.y - X.y) * set.s;
         const double cr = ax * by - ay * bx, dot = ax * bx + ay * by;
         t = cr > 0.0 ? dot / cr : (dot < 0.0 ? -INFINITY : INFINITY);
         if (c.v >= 0) better = x != c.v && incircle_at(m, P, Q, c.X, X, p, q, c.v, x) > 0;
@@ -1865,42 +1883,45 @@ GA_INLINE void hull_chunk(const MeshDev &m, const HullDev &h, double2 P, double2
     }
 }
 
-// The apex of p -> q among the boundary vertices [b0, b1) of its set (one wave; -1: none).  First
+// The apex of p -> q among the boundary vertices of its set (one wave; -1: none).  First
 // the vertices numbered next to p and q, which gives a circle near the final one; then the
 // boxes, 64 at a time: a box can hold a better apex only if it reaches left of the edge and into
 // the circle, which leaves one to three of B / 64.  (Every vertex tested, in steps of 64, took
 // 51 us per launch at B = 2,500, one dependent read after another.)  Both box tests keep a margin
-// far above their rounding; a circle too flat for that is not used.
-__device__ int hull_apex(const MeshDev &m, const HullDev &h, int p, int q, int b0, int b1, int lane)
+// far above their rounding; a circle too flat or too small for that is not used.
+__device__ int hull_apex(const MeshDev &m, const HullDev &h, int p, int q, HullSet set, int lane)
 {
+    const double sc = set.s;
+
     const double2 P = m.pos[p], Q = m.pos[q];
     const int gp = h.bidx[p] >> 6, gq = h.bidx[q] >> 6;
     HullBest c{-1, P};
-    hull_chunk(m, h, P, Q, p, q, gp, b0, b1, lane, c);
-    if (gq != gp) hull_chunk(m, h, P, Q, p, q, gq, b0, b1, lane, c);
-    const double ux = Q.x - P.x, uy = Q.y - P.y;
-    const int g1 = (b1 - 1) >> 6;
-    for (int gb = b0 >> 6; gb <= g1; gb += 64) {
+    hull_chunk(m, h, P, Q, p, q, gp, set, lane, c);
+    if (gq != gp) hull_chunk(m, h, P, Q, p, q, gq, set, lane, c);
+    const double ux = (Q.x - P.x) * sc, uy = (Q.y - P.y) * sc;
+    const int g1 = (set.b1 - 1) >> 6;
+    for (int gb = set.b0 >> 6; gb <= g1; gb += 64) {
         const int g = gb + lane;
         const bool in = g <= g1 && g != gp && g != gq;
         const HullBox bx = h.bbox[min(g, g1)];
         // largest cross product (Q - P) x (X - P) over the box
-        const double ex = (uy > 0 ? bx.lx : bx.hx) - P.x, ey = (ux > 0 ? bx.hy : bx.ly) - P.y;
+        const double ex = ((uy > 0 ? bx.lx : bx.hx) - P.x) * sc, ey = ((ux > 0 ? bx.hy : bx.ly) - P.y) * sc;
         const double l = ux * ey, r = uy * ex;
-        const bool left = in && l - r >= -1e-14 * (fabs(l) + fabs(r));
+        const bool left = in && l - r >= -1e-14 * (fabs(l) + fabs(r)) - HULL_TINY;
         for (unsigned long long todo = __ballot(left); todo;) {
             if (c.v >= 0) {
                 // circle of (P, Q, C): centre P + (ox, oy)
-                const double vx = c.X.x - P.x, vy = c.X.y - P.y;
+                const double vx = (c.X.x - P.x) * sc, vy = (c.X.y - P.y) * sc;
                 const double a = ux * vy, b = uy * vx, cr = a - b;
-                if (cr > 1e-6 * (fabs(a) + fabs(b))) {
+                // (cr > 1e-200: the radius is above 1e-101, what the products below lose, times f, below 1e-118)
+                if (cr > 1e-6 * (fabs(a) + fabs(b)) && cr > 1e-200) {
                     const double uu = ux * ux + uy * uy, vv = vx * vx + vy * vy, f = 0.5 / cr;
                     const double ox = f * (vy * uu - uy * vv), oy = f * (ux * vv - vx * uu);
-                    const double dx = fmax(fmax(bx.lx - P.x - ox, P.x + ox - bx.hx), 0.0);
-                    const double dy = fmax(fmax(bx.ly - P.y - oy, P.y + oy - bx.hy), 0.0);
+                    const double dx = fmax(fmax((bx.lx - P.x) * sc - ox, ox - (bx.hx - P.x) * sc), 0.0);
+                    const double dy = fmax(fmax((bx.ly - P.y) * sc - oy, oy - (bx.hy - P.y) * sc), 0.0);
                     const double rad = sqrt(ox * ox + oy * oy);
-                    // the centre's cancellation error, the relative error of f and of the differences
-                    const double reach = rad * (1.0 + 1e-8) + 1e-14 * (fabs(P.x) + fabs(P.y) + rad) +
+                    // the relative error of f and of the differences, the centre's cancellation error
+                    const double reach = rad * (1.0 + 1e-8) +
                                          1e-14 * f * ((fabs(vx) + fabs(vy)) * uu + (fabs(ux) + fabs(uy)) * vv);
                     const bool out = dx * dx + dy * dy > reach * reach;
                     todo &= ~__ballot(out);
@@ -1909,7 +1930,7 @@ __device__ int hull_apex(const MeshDev &m, const HullDev &h, int p, int q, int b
             }
             const int k = __ffsll((long long)todo) - 1;
             todo &= todo - 1;
-            hull_chunk(m, h, P, Q, p, q, gb + k, b0, b1, lane, c);
+            hull_chunk(m, h, P, Q, p, q, gb + k, set, lane, c);
         }
     }
     return c.v;
@@ -1989,23 +2010,19 @@ __global__ __launch_bounds__(256) void k_hull_fill(MeshDev m, HullDev h)
     }
     const int lane = threadIdx.x & 63, nw = (gridDim.x * blockDim.x) >> 6;
     for (int i = (blockIdx.x * blockDim.x + threadIdx.x) >> 6; i < nd + B; i += nw) {
-        int head = -1, slot = -1, b0, b1;
+        int head = -1, slot = -1;
+        HullSet set;
         if (i < nd) {
             const int2 f = h.list[i];
             head = f.x;
             slot = f.y;
             if (lane == 0) h.next[head] = -1;
-            const int v = (int)((h.table[head >> 1] - 1) >> 32);
-            const SetDesc &sd = m.sets[m.vset[v]];
-            b0 = h.bidx[sd.poff];
-            b1 = h.bidx[sd.poff + sd.n];
+            set = hull_set(m, h, (int)((h.table[head >> 1] - 1) >> 32));
         } else {
             const int v = h.blist[i - nd];
             if (h.mark[v] == 3) continue;
-            const SetDesc &sd = m.sets[m.vset[v]];
-            b0 = h.bidx[sd.poff];
-            b1 = h.bidx[sd.poff + sd.n];
-            const int w = hull_nearest(m, h, i - nd, b0, b1, lane);
+            set = hull_set(m, h, v);
+            const int w = hull_nearest(m, h, i - nd, set, lane);
             if (w < 0) continue;
             int e = 0;
             u64 old = 0;
@@ -2036,7 +2053,7 @@ __global__ __launch_bounds__(256) void k_hull_fill(MeshDev m, HullDev h)
             key = __shfl(key, 0, 64);
             const int lo = (int)(key >> 32), hi = (int)(key & 0xffffffffull);
             const int p = it & 1 ? hi : lo, q = it & 1 ? lo : hi;
-            const int c = hull_apex(m, h, p, q, b0, b1, lane);
+            const int c = hull_apex(m, h, p, q, set, lane);
             if (c >= 0) {
                 hull_create(m, h, H, it, p, q, c, lane, &slot, &head);
             } else if (lane == 0) {
