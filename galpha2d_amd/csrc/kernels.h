@@ -169,7 +169,7 @@ struct HullDev {
 #define C_CHANGED 17          // pixels relabelled by an island repair
 #define C_DELETED 18
 #define C_ISLAND_SITES 19
-#define C_HSTART 20
+#define C_HULL_ROOM 20        // triangle slots unused before frame removal
 #define C_FLIPS_TOTAL 21
 #define C_XFLIP 22            // edges left to k_flip_exact
 #define C_INSERT_ROUNDS 23    // rounds run by the last k_insert_tail

@@ -1666,6 +1666,12 @@ void launch_counters_to_host(int *counters, int slot, int n, int fold, int *host
 // was known of it, and no fence orders anything: every link of a new triangle is written by
 // whichever of its two sides comes second (or by both, with one value).
 // Triangles and demands are those of a planar graph on B vertices: at most 3 B edges.
+// Slots: a triangle takes its wave's free slot, that of a dropped frame triangle or a new one.  A wave whose
+// triangle was created by another first has a slot left at the end of a demand: at most 2 nt + B new
+// slots for nt frame triangles.  Where the capacity has not that many (most vertices on the boundary: 200,000
+// points on a curve), hull_tight, all frame triangles' slots are shared and a wave keeps its free slot for its
+// next demand.  The new triangles are nt - nf at most (every set loses its frame vertices from the
+// hull), so nf + room waves need no more than `room` new slots, whatever they do.
 // What bounds it is latency: the dependent reads of an apex and five device-scope atomics of a
 // triangle, 5 to 8 us a step.  The boundary stage, against cutting ears of the boundary cycle in
 // 16-32 rounds (which needed one simple cycle per set, and left flips to do; sets without one lost
@@ -1679,6 +1685,10 @@ GA_INLINE int hull_table(const MeshDev &m, const HullDev &h)
 {
     const long long want = 6ll * hull_b(m, h) + 64;
     return (int)(want < h.room ? want : h.room);
+}
+GA_INLINE bool hull_tight(const MeshDev &m, const HullDev &h)
+{
+    return m.counters[C_HULL_ROOM] < 2ll * m.counters[C_FTRI] + hull_b(m, h);
 }
 typedef unsigned long long u64;
 #define HULL_LISTED 1u
@@ -1726,9 +1736,10 @@ __global__ __launch_bounds__(256) void k_hull_scan(MeshDev m, HullDev h, int op)
 
 // bidx (the exclusive scan of the marks) numbers the boundary vertices in vertex order, so those of
 // a set are consecutive and in spatial order.  Clears the table, places the boundary vertices,
-// marks those with a real edge (mark 3).
+// marks those with a real edge (mark 3), and notes how many slots are unused.
 __global__ void k_hull_place(MeshDev m, HullDev h)
 {
+    if (blockIdx.x == 0 && threadIdx.x == 0) m.counters[C_HULL_ROOM] = m.cap - ntri_used(m);
     const int H = hull_table(m, h), nt = m.counters[C_FTRI];
     GRID_STRIDE(q, nt) {
         const int4 v = m.tv[h.ftri[q]];
@@ -1748,30 +1759,31 @@ __global__ void k_hull_place(MeshDev m, HullDev h)
 
 // The first demands: the real edge of every frame triangle with two real vertices (list: the demand
 // and the triangle's slot), with the real triangle across it.  The other frame triangles die here,
-// their slots go to the pool.  Also the boxes of 64 consecutive boundary vertices each, one wave
+// their slots go to the pool (hull_tight: those of all, and the list holds none).  Also the boxes of 64 consecutive boundary vertices each, one wave
 // per box.
 __global__ __launch_bounds__(256) void k_hull_edges(MeshDev m, HullDev h, int op)
 {
     const int H = hull_table(m, h), nt = m.counters[C_FTRI], B = hull_b(m, h);
+    const bool tight = hull_tight(m, h);
     u64 *own = h.table + H;
     GRID_STRIDE(qq, nt) {
         const int t = h.ftri[qq];
         const int4 v = m.tv[t];
-        const bool one = frame_vertices(m, v) == 1;
+        const bool one = frame_vertices(m, v) == 1, shared = !one || tight;
         const int k = wave_reserve(&m.counters[C_HULL], one);
-        const int kp = wave_reserve(&m.counters[C_HULL_POOL], !one);
-        if (!one) {
+        const int kp = wave_reserve(&m.counters[C_HULL_POOL], shared);
+        if (shared) {
             h.pool[kp] = t;
             m.tv[t] = make_int4(GA_DEAD, GA_DEAD, GA_DEAD, 0);
-            continue;
         }
+        if (!one) continue;
         const int i = v.x >= m.n ? 0 : (v.y >= m.n ? 1 : 2);
         const int p = ic(v, p1(i)), q = ic(v, m1(i)), nb = ic(m.tn[t], i);
         const int e = hull_entry(m, h, H, p, q), d = p < q ? 0 : 1;
         u64 w = (u64)HULL_LISTED << (32 * d);
         if (nb >= 0 && m.stamp[enc_t(nb)] != op) w |= (u64)(hull_value(enc_t(nb), enc_j(nb)) << 1) << (32 * (1 - d));
         atomicOr(&own[e], w);
-        h.list[k] = make_int2(2 * e + d, t);
+        h.list[k] = make_int2(2 * e + d, tight ? -1 : t);
     }
     const int lane = threadIdx.x & 63, nw = (gridDim.x * blockDim.x) >> 6;
     for (int g = (blockIdx.x * blockDim.x + threadIdx.x) >> 6; 64 * g < B; g += nw) {
@@ -1937,9 +1949,9 @@ __device__ int hull_apex(const MeshDev &m, const HullDev &h, int p, int q, HullS
 }
 
 // Creates the triangle (p, q, c) unless another demand did, in *slot when the wave has one (then
-// -1), else in one from the pool or a new one; pushes the far sides that nothing is known of on the
+// -1), else in one from the pool (its share of it, or any: all) or a new one; pushes the far sides that nothing is known of on the
 // wave's stack (next[] links the demands, *head the first).  One wave; lanes 0, 1 and 2 take a side each.
-__device__ void hull_create(const MeshDev &m, const HullDev &h, int H, int it0, int p, int q, int c, int lane,
+__device__ void hull_create(const MeshDev &m, const HullDev &h, int H, int it0, int p, int q, int c, bool all, int lane,
                             int *slot, int *head)
 {
     u64 *own = h.table + H;
@@ -1952,9 +1964,12 @@ __device__ void hull_create(const MeshDev &m, const HullDev &h, int H, int it0, 
     if (lane < 3) it = 2 * hull_entry(m, h, H, su, sv) + (su < sv ? 0 : 1);
     if (T < 0 && lane == 0) {
         // the pool's shares are taken one by one, so that no counter serves all waves
-        const int s = (int)((blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) % HULL_SHARES);
-        const int x = s + HULL_SHARES * atomicAdd(&h.share[s * HULL_SHARE_INTS], 1);
-        T = x < m.counters[C_HULL_POOL] ? h.pool[x] : atomicAdd(m.ntri, 1);
+        int s = (int)((blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) % HULL_SHARES);
+        for (int u = all ? HULL_SHARES : 1; u > 0 && T < 0; u--, s = (s + 1) % HULL_SHARES) {
+            const int x = s + HULL_SHARES * atomicAdd(&h.share[s * HULL_SHARE_INTS], 1);
+            if (x < m.counters[C_HULL_POOL]) T = h.pool[x];
+        }
+        if (T < 0) T = atomicAdd(m.ntri, 1);
     }
     T = __shfl(T, 0, 64);
     if (T >= m.cap) {
@@ -2008,14 +2023,18 @@ __global__ __launch_bounds__(256) void k_hull_fill(MeshDev m, HullDev h)
         if (m.vstate[f] == VS_IN_MESH) m.vstate[f] = VS_REMOVED;
         m.vt[f] = -1;
     }
-    const int lane = threadIdx.x & 63, nw = (gridDim.x * blockDim.x) >> 6;
-    for (int i = (blockIdx.x * blockDim.x + threadIdx.x) >> 6; i < nd + B; i += nw) {
-        int head = -1, slot = -1;
+    const bool tight = hull_tight(m, h);
+    const int lane = threadIdx.x & 63, all = (int)((gridDim.x * blockDim.x) >> 6);
+    const int nw = tight ? min(all, m.V - m.n + m.counters[C_HULL_ROOM]) : all;
+    const int w0 = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
+    int slot = -1;
+    for (int i = w0 < nw ? w0 : nd + B; i < nd + B; i += nw) {
+        int head = -1;
         HullSet set;
         if (i < nd) {
             const int2 f = h.list[i];
             head = f.x;
-            slot = f.y;
+            if (!tight) slot = f.y;
             if (lane == 0) h.next[head] = -1;
             set = hull_set(m, h, (int)((h.table[head >> 1] - 1) >> 32));
         } else {
@@ -2055,15 +2074,18 @@ __global__ __launch_bounds__(256) void k_hull_fill(MeshDev m, HullDev h)
             const int p = it & 1 ? hi : lo, q = it & 1 ? lo : hi;
             const int c = hull_apex(m, h, p, q, set, lane);
             if (c >= 0) {
-                hull_create(m, h, H, it, p, q, c, lane, &slot, &head);
+                hull_create(m, h, H, it, p, q, c, tight, lane, &slot, &head);
             } else if (lane == 0) {
                 const int d = it & 1;
                 const unsigned ov = hull_half(atomicOr(&own[it >> 1], (u64)(HULL_EDGE << 1) << (32 * d)), 1 - d) >> 1;
                 if (ov && ov != HULL_EDGE) set_link(m, (int)((ov - 1) / 3u), (int)((ov - 1) % 3u), -1);
             }
         }
+        if (tight) continue;
         if (slot >= 0 && lane == 0) m.tv[slot] = make_int4(GA_DEAD, GA_DEAD, GA_DEAD, 0);
+        slot = -1;
     }
+    if (slot >= 0 && lane == 0) m.tv[slot] = make_int4(GA_DEAD, GA_DEAD, GA_DEAD, 0);
 }
 
 void launch_hull(MeshDev &m, const HullDev &h, int op, void *scan_tmp, hipStream_t st)
