@@ -139,7 +139,9 @@ __global__ void k_gather_xy(const double2 *__restrict__ xy, const int *__restric
 
 // Map real points to pixels of their set's texture.  pix = (px << 16) | py; the point with the
 // smallest input index (perm[i], or i without a renumbering) wins a pixel; k_splat_own then
-// stores the winner's own index.
+// stores the winner's own index.  Input indices carry SPLAT_INPUT (indices stay below 2^28), so that a
+// thread of k_splat_own never takes another's own index, stored while it runs, for its input index.
+#define SPLAT_INPUT 0x40000000
 __global__ void k_splat(const double2 *__restrict__ xy, BatchDev b, const int *__restrict__ perm,
                         int *__restrict__ smap, int *__restrict__ pix)
 {
@@ -149,7 +151,7 @@ __global__ void k_splat(const double2 *__restrict__ xy, BatchDev b, const int *_
     int px, py;
     point_pixel(sd, xy[i], &px, &py);
     pix[i] = (px << 16) | py;
-    atomicMin(&smap[sd.toff + ((size_t)px << sd.logT) + py], perm ? perm[i] : i);
+    atomicMin(&smap[sd.toff + ((size_t)px << sd.logT) + py], perm ? perm[i] | SPLAT_INPUT : i);
 }
 
 // The winners' own indices, and the frame sites (global ids ntot .. V-1) at their border pixels (fpix: packed
@@ -165,7 +167,7 @@ __global__ void k_splat_own(BatchDev b, const int *__restrict__ perm, const int 
     if (i >= b.ntot) {
         pix[i] = pp;
         *cellp = i;
-    } else if (*cellp == perm[i]) {
+    } else if (*cellp == (perm[i] | SPLAT_INPUT)) {
         *cellp = i;    // one winner per pixel: no other thread writes here
     }
 }
