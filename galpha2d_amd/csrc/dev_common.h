@@ -270,6 +270,27 @@ GA_INLINE int orient_expansion(double2 a, double2 b, double2 c)
     return top > 0.0 ? 1 : (top < 0.0 ? -1 : 0);
 }
 
+// Exact orientation sign where the four differences to c are exact and no product leaves the range in
+// which its error is exact (lattices, points of few bits); 2 elsewhere.  Each product is a rounded
+// value and its exact error, and the rounded values of different products are in their order.
+GA_INLINE int orient_diff(double2 a, double2 b, double2 c)
+{
+    const double u[4] = {a.x, b.y, a.y, b.x}, w[4] = {c.x, c.y, c.y, c.x};
+    double d[4];
+    bool exact = true;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        d[k] = u[k] - w[k];
+        const double bv = d[k] - u[k];
+        exact = exact && u[k] - (d[k] - bv) == 0.0 && w[k] + bv == 0.0;
+    }
+    const double p = d[0] * d[1], q = d[2] * d[3];
+    auto sound = [](double v, double x, double y) { return v == 0.0 ? x == 0.0 || y == 0.0 : fabs(v) > 1e-280 && fabs(v) < 1e300; };
+    if (!exact || !sound(p, d[0], d[1]) || !sound(q, d[2], d[3])) return 2;
+    const double s = p != q ? p - q : fma(d[0], d[1], -p) - fma(d[2], d[3], -q);
+    return s > 0.0 ? 1 : (s < 0.0 ? -1 : 0);
+}
+
 // exact orientation sign (ovf set when the capacity would be exceeded)
 GA_INLINE int orient_exact(double2 a, double2 b, double2 c, int *ovf)
 {

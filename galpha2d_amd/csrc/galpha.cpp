@@ -744,11 +744,12 @@ static Snap remove_frame(galpha_ctx *c, MeshDev &m, hipStream_t st)
     h.next = (int *)m.remap;
     h.pool = m.modB;
     h.share = (int *)(h.bbox + m.n / 64 + 2);
+    h.lines = (unsigned long long *)(h.share + HULL_SHARES * HULL_SHARE_INTS);
     h.room = (int)std::min<size_t>({c->fan.bytes / 16, c->remap.bytes / 8, (size_t)1 << 30});
     {
         IntFills f;
         f.add(h.mark, (size_t)m.n + 1, 0);
-        f.add(h.share, HULL_SHARES * HULL_SHARE_INTS, 0);
+        f.add(h.share, HULL_SHARES * HULL_SHARE_INTS + 2 * HULL_LINES, 0);   // and the lines
         f.add(c->counters.as<int>() + C_FTRI, 3, 0);
         launch_fill_multi(f, st);
     }

@@ -135,11 +135,13 @@ struct HullDev {
     int2 *list;                 // first demands and the slots of their frame triangles (counters[C_HULL])
     int *pool;                  // slots of the other frame triangles (counters[C_HULL_POOL])
     int *share;                 // HULL_SHARES counters: slots taken from each share of the pool
+    unsigned long long *lines;  // [HULL_LINES] hull edges found (p << 32 | q; 0: none yet)
     int *next;                  // [2 H] links of the waves' stacks
     int room;                   // most table entries
 };
 #define HULL_SHARES 32
 #define HULL_SHARE_INTS 32      // ints between the counters
+#define HULL_LINES 32
 
 // vertex states
 #define VS_IN_MESH 1       // in the mesh, position final

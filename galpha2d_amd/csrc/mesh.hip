@@ -1805,13 +1805,14 @@ __global__ __launch_bounds__(256) void k_hull_edges(MeshDev m, HullDev h, int op
 struct HullSet {
     int b0, b1;
     double s;
+    int first;   // vertex that hull_apex tries first (-1: none): the wave's last apex, in a pocket mostly near the next
 };
 #define HULL_TINY 1e-290   // above what is lost to underflow in scaled coordinates
 __device__ HullSet hull_set(const MeshDev &m, const HullDev &h, int v)
 {
     const SetDesc &sd = m.sets[m.vset[v]];
     const int e = -ilogb(sd.scale);
-    return HullSet{h.bidx[sd.poff], h.bidx[sd.poff + sd.n], ldexp(1.0, e < 1023 ? e : 1023)};
+    return HullSet{h.bidx[sd.poff], h.bidx[sd.poff + sd.n], ldexp(1.0, e < 1023 ? e : 1023), -1};
 }
 
 // squared distances to v: true when a is nearer than b
@@ -1875,8 +1876,10 @@ GA_INLINE void hull_chunk(const MeshDev &m, const HullDev &h, double2 P, double2
     const int x = in ? h.blist[j] : p;
     int o = orient_filter(P, Q, X);
     // p, q themselves and points on one axis-parallel line with them are exactly collinear
-    if (o == 0 && x != p && x != q && !(P.x == Q.x && Q.x == X.x) && !(P.y == Q.y && Q.y == X.y))
-        o = orient_dev(m, P, Q, X);
+    if (o == 0 && x != p && x != q && !(P.x == Q.x && Q.x == X.x) && !(P.y == Q.y && Q.y == X.y)) {
+        o = orient_diff(P, Q, X);   // (a search along 20,000 points on a sloped line: half the time)
+        if (o == 2) o = orient_dev(m, P, Q, X);
+    }
     bool better = o > 0 && x != p && x != q;
     double t = INFINITY;
     if (better) {
@@ -1895,7 +1898,26 @@ GA_INLINE void hull_chunk(const MeshDev &m, const HullDev &h, double2 P, double2
     }
 }
 
-// The apex of p -> q among the boundary vertices of its set (one wave; -1: none).  First
+// p -> q lies on the line of a hull edge found before (h.lines: some whose search took more than 16 boxes;
+// lane k tests line k), in its direction: then it is a hull edge as well.  Without that, every edge of a long
+// straight side looks at every box that the side passes through (two sloped sides of 30,000 points each: 127 ms, 2.4
+// with it).
+__device__ bool hull_on_line(const MeshDev &m, const HullDev &h, int p, int q, double2 P, double2 Q, HullSet set, int lane)
+{
+    bool on = false;
+    if (lane < HULL_LINES) {
+        const unsigned long long e = __hip_atomic_load(&h.lines[lane], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const int a = (int)(e >> 32), b = (int)(e & 0xffffffffull);
+        if (a != b && h.bidx[a] >= set.b0 && h.bidx[a] < set.b1) {
+            const double2 A = m.pos[a], B = m.pos[b];
+            on = (A.x < B.x) == (P.x < Q.x) && (A.x > B.x) == (P.x > Q.x) && (A.y < B.y) == (P.y < Q.y) &&
+                 (A.y > B.y) == (P.y > Q.y) && orient_dev(m, A, B, P) == 0 && orient_dev(m, A, B, Q) == 0;
+        }
+    }
+    return __any(on);
+}
+
+// The apex of p -> q among the boundary vertices of its set (one wave; -1: none).  First set.first and
 // the vertices numbered next to p and q, which gives a circle near the final one; then the
 // boxes, 64 at a time: a box can hold a better apex only if it reaches left of the edge and into
 // the circle, which leaves one to three of B / 64.  (Every vertex tested, in steps of 64, took
@@ -1908,19 +1930,31 @@ __device__ int hull_apex(const MeshDev &m, const HullDev &h, int p, int q, HullS
     const double2 P = m.pos[p], Q = m.pos[q];
     const int gp = h.bidx[p] >> 6, gq = h.bidx[q] >> 6;
     HullBest c{-1, P};
+    if (set.first >= 0 && set.first != p && set.first != q) {
+        const double2 X = m.pos[set.first];
+        if (orient_dev(m, P, Q, X) > 0) c = HullBest{set.first, X};
+    }
     hull_chunk(m, h, P, Q, p, q, gp, set, lane, c);
     if (gq != gp) hull_chunk(m, h, P, Q, p, q, gq, set, lane, c);
     const double ux = (Q.x - P.x) * sc, uy = (Q.y - P.y) * sc;
     const int g1 = (set.b1 - 1) >> 6;
+    bool asked = !h.lines;
     for (int gb = set.b0 >> 6; gb <= g1; gb += 64) {
         const int g = gb + lane;
         const bool in = g <= g1 && g != gp && g != gq;
         const HullBox bx = h.bbox[min(g, g1)];
-        // largest cross product (Q - P) x (X - P) over the box
-        const double ex = ((uy > 0 ? bx.lx : bx.hx) - P.x) * sc, ey = ((ux > 0 ? bx.hy : bx.ly) - P.y) * sc;
-        const double l = ux * ey, r = uy * ex;
-        const bool left = in && l - r >= -1e-14 * (fabs(l) + fabs(r)) - HULL_TINY;
-        for (unsigned long long todo = __ballot(left); todo;) {
+        // largest cross product (Q - P) x (X - P) over the box, at its corner (cx, cy); exactly zero when that
+        // lies on an axis-parallel line with p and q
+        const double cx = uy > 0 ? bx.lx : bx.hx, cy = ux > 0 ? bx.hy : bx.ly;
+        const double l = ux * ((cy - P.y) * sc), r = uy * ((cx - P.x) * sc);
+        const bool flat = (P.x == Q.x && cx == P.x) || (P.y == Q.y && cy == P.y);
+        const bool left = in && !flat && l - r >= -1e-14 * (fabs(l) + fabs(r)) - HULL_TINY;
+        unsigned long long todo = __ballot(left);
+        if (!asked && c.v < 0 && __popcll(todo) > 16) {
+            asked = true;
+            if (hull_on_line(m, h, p, q, P, Q, set, lane)) return -1;
+        }
+        while (todo) {
             if (c.v >= 0) {
                 // circle of (P, Q, C): centre P + (ox, oy)
                 const double vx = (c.X.x - P.x) * sc, vy = (c.X.y - P.y) * sc;
@@ -1945,6 +1979,9 @@ __device__ int hull_apex(const MeshDev &m, const HullDev &h, int p, int q, HullS
             hull_chunk(m, h, P, Q, p, q, gb + k, set, lane, c);
         }
     }
+    if (asked && c.v < 0 && h.lines && lane == 0)
+        __hip_atomic_store(&h.lines[p % HULL_LINES], (unsigned long long)p << 32 | (unsigned)q, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
     return c.v;
 }
 
@@ -2027,7 +2064,7 @@ __global__ __launch_bounds__(256) void k_hull_fill(MeshDev m, HullDev h)
     const int lane = threadIdx.x & 63, all = (int)((gridDim.x * blockDim.x) >> 6);
     const int nw = tight ? min(all, m.V - m.n + m.counters[C_HULL_ROOM]) : all;
     const int w0 = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
-    int slot = -1;
+    int slot = -1, last = -1, last_set = -1;   // last: the wave's last apex, in the set of boundary vertices from last_set on
     for (int i = w0 < nw ? w0 : nd + B; i < nd + B; i += nw) {
         int head = -1;
         HullSet set;
@@ -2057,6 +2094,7 @@ __global__ __launch_bounds__(256) void k_hull_fill(MeshDev m, HullDev h)
                     head = 2 * e + d;
                 }
         }
+        if (set.b0 == last_set) set.first = last;
         while (head >= 0) {
             const int it = head;
             int nx = 0, known = 0;
@@ -2074,8 +2112,12 @@ __global__ __launch_bounds__(256) void k_hull_fill(MeshDev m, HullDev h)
             const int p = it & 1 ? hi : lo, q = it & 1 ? lo : hi;
             const int c = hull_apex(m, h, p, q, set, lane);
             if (c >= 0) {
+                set.first = last = c;
+                last_set = set.b0;
                 hull_create(m, h, H, it, p, q, c, tight, lane, &slot, &head);
-            } else if (lane == 0) {
+                continue;
+            }
+            if (lane == 0) {
                 const int d = it & 1;
                 const unsigned ov = hull_half(atomicOr(&own[it >> 1], (u64)(HULL_EDGE << 1) << (32 * d)), 1 - d) >> 1;
                 if (ov && ov != HULL_EDGE) set_link(m, (int)((ov - 1) / 3u), (int)((ov - 1) % 3u), -1);

@@ -25,7 +25,8 @@ static int g_lane;
 static ucontext_t g_main, g_ctx[64];
 static unsigned long long g_val[2][64];
 static int g_phase[64];
-static void meet() { swapcontext(&g_ctx[g_lane], &g_main); }
+static long long g_steps;   // of all lanes
+static void meet() { g_steps++; swapcontext(&g_ctx[g_lane], &g_main); }
 template <class T> static T exchange(T v, int from)
 {
     const int l = g_lane, p = g_phase[l]++ & 1;
@@ -52,6 +53,8 @@ static unsigned long long h_ballot(bool b)
 #define __shfl_xor(v, k, w) exchange(v, g_lane ^ (k))
 #define atomicOr(p, v) (*(p) |= (v))
 #define __ffsll(x) __builtin_ffsll(x)
+#define __popcll(x) __builtin_popcountll(x)
+typedef unsigned long long u64;
 static int orient_dev(const MeshDev &m, double2 a, double2 b, double2 c)
 {
     int ovf = 0;
@@ -59,10 +62,8 @@ static int orient_dev(const MeshDev &m, double2 a, double2 b, double2 c)
     if (ovf) *m.status = 1;
     return s;
 }
-static long long g_incircles;
 static int incircle_at(const MeshDev &m, double2 a, double2 b, double2 c, double2 d, int ia, int ib, int ic, int id)
 {
-    g_incircles++;
     const int s = incircle_filter(a, b, c, d);
     if (s) return s;
     int ovf = 0;
@@ -101,7 +102,7 @@ static void wave(std::function<void(int)> body)
     }
 }
 // argv[1]: n, demands, the set's snap scale, n points, demands (p, q); prints the apexes, then
-// the nearest vertices of the demands' first ends
+// the nearest vertices of the demands' first ends, the status and the number of collectives
 int main(int, char **argv)
 {
     FILE *f = fopen(argv[1], "r");
@@ -122,7 +123,9 @@ int main(int, char **argv)
     sd.n = n;
     MeshDev m{};
     m.n = n; m.pos = pos.data(); m.status = &status; m.sets = &sd; m.vset = zero.data();
+    std::vector<u64> lines(HULL_LINES);
     HullDev h{};
+    h.lines = lines.data();
     h.bidx = ids.data(); h.blist = ids.data(); h.bpos = pos.data(); h.bbox = box.data();
     for (int k = 0; k < nd; k++) {
         int p, q, r[64], w[64];
@@ -130,10 +133,10 @@ int main(int, char **argv)
         wave([&](int lane) { r[lane] = CALL_APEX; });
         wave([&](int lane) { w[lane] = CALL_NEAREST; });
         for (int l = 1; l < 64; l++)
-            if (r[l] != r[0] || w[l] != w[0]) return 2;   // the wave's answer is one
+            if (r[l] != r[0]) return 2;   // the wave's answer is one (of the nearest, lane 0's counts)
         printf("%d %d\n", r[0], w[0]);
     }
-    printf("%d %lld\n", status, g_incircles);
+    printf("%d %lld\n", status, g_steps / 64);
     return 0;
 }
 """
@@ -191,6 +194,12 @@ def _points(kind, n):
         a, r = a / 2, np.ones(n)
     elif kind == "box":
         return _morton(rng.random((n, 2)))
+    elif kind == "sides":   # four straight sides, two of them sloped, and some points inside
+        t = rng.permutation(4096)[:n] / 4096.0
+        k = n // 5
+        side = lambda i, a, b: np.array(a) + t[i * k:(i + 1) * k, None] * (np.array(b) - a)
+        c = [(0.0, 0.0), (1.0, 0.25), (1.0, 1.25), (0.25, 1.25)]
+        return _morton(np.concatenate([side(i, c[i], c[(i + 1) % 4]) for i in range(4)] + [0.25 + 0.5 * rng.random((n - 4 * k, 2))]))
     else:   # near the origin: distances down to 1e-13 of the largest
         r = 10.0 ** (-13 * rng.random(n))
     return _morton(np.stack([r * np.cos(a), r * np.sin(a)], 1))
@@ -209,7 +218,7 @@ def _scale(xy, T=512):
     return float(np.ptp(xy, axis=0).max()) / T
 
 
-@pytest.mark.parametrize("kind", ["ring", "arc", "box", "origin"])
+@pytest.mark.parametrize("kind", ["ring", "arc", "box", "origin", "sides"])
 @pytest.mark.parametrize("e", [-365, 520])
 def test_scaled(search, kind, e):
     xy = _points(kind, 1500)
@@ -222,27 +231,44 @@ def test_scaled(search, kind, e):
 def _apex(xy, p, q):
     """The vertex left of p -> q whose circle through p and q holds no other, in rationals."""
     F = [(Fraction(float(x)), Fraction(float(y))) for x, y in xy]
-    (px, py), (qx, qy), best, at = F[p], F[q], None, -1
+    (px, py), (qx, qy), best, at = F[p], F[q], None, []
     for i, (x, y) in enumerate(F):
         ax, ay, bx, by = px - x, py - y, qx - x, qy - y
         area = ax * by - ay * bx
         if area > 0:
             t = (ax * bx + ay * by) / area   # the cotangent of the angle under which it sees the edge
             if best is None or t < best:
-                best, at = t, i
-    return at
+                best, at = t, [i]
+            elif t == best:
+                at.append(i)   # on one circle with p and q
+    return [-1] if best is None else at
 
 
-@pytest.mark.parametrize("kind", ["ring", "arc", "origin"])
+@pytest.mark.parametrize("kind", ["ring", "arc", "origin", "sides"])
 def test_rational(search, kind):
     xy = _points(kind, 700)
     demands = _demands(xy, 25, 2)
     got, _ = search(xy, demands, _scale(xy))
     for (p, q), (c, w) in zip(demands, got):
-        assert c == _apex(xy, p, q)
+        assert c in _apex(xy, p, q)
         F = [(Fraction(float(x)) - Fraction(float(xy[p][0]))) ** 2 + (Fraction(float(y)) - Fraction(float(xy[p][1]))) ** 2
              for x, y in xy]
         assert w != p and F[w] == min(f for i, f in enumerate(F) if i != p)
+
+
+@pytest.mark.parametrize("slope", [0.0, 0.25])
+def test_straight_side(search, slope):
+    """The hull edges along a straight side: after the first, no search looks along the whole side (190 boxes)."""
+    rng = np.random.default_rng(4)
+    n = 12000
+    t = rng.permutation(16384)[:n] / 16384.0
+    xy = _morton(np.concatenate([np.stack([t, slope * t], 1), [0, 1] + rng.random((500, 2))]))
+    side = np.flatnonzero(xy[:, 1] == slope * xy[:, 0])
+    side = side[np.argsort(xy[side, 0])]
+    k = rng.integers(0, n - 1, 60)
+    got, steps = search(xy, np.stack([side[k + 1], side[k]], 1), _scale(xy))
+    assert (got[:, 0] == -1).all()
+    assert steps < 2 * 190 + 60 * 25
 
 
 @pytest.mark.gpu
