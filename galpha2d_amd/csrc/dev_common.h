@@ -74,6 +74,47 @@ GA_INLINE int incircle_filter(double2 a, double2 b, double2 c, double2 d)
     return 0;
 }
 
+// The same sign in pairs of doubles (sums of a rounded value and an error, 106 bits): 0 when these cannot decide
+// either.  sc: a power of two that brings the differences to 2^15 at most.  With u = 2^-53, differences
+// are exact, a product is off by 8 u^2 of its size, a sum by 4 u^2 of the sizes of its terms, so the determinant
+// by less than 64 u^2 = 2^-100 of perm; the bound is 2^-96 of it.  (perm above 1e-200: what underflows is
+// below 2^-1074 2^50 per product.)
+struct DD {
+    double h, l;
+};
+GA_INLINE DD dd_diff(double a, double b, double sc)
+{
+    const double s = a - b, v = s - a;
+    return DD{s * sc, ((a - (s - v)) - (b + v)) * sc};
+}
+GA_INLINE DD dd_mul(DD a, DD b)
+{
+    const double p = a.h * b.h, e = fma(a.h, b.h, -p) + (a.h * b.l + a.l * b.h), s = p + e;
+    return DD{s, e - (s - p)};
+}
+GA_INLINE DD dd_add(DD a, DD b)
+{
+    const double s = a.h + b.h, v = s - a.h, e = ((a.h - (s - v)) + (b.h - v)) + (a.l + b.l), t = s + e;
+    return DD{t, e - (t - s)};
+}
+GA_INLINE DD dd_sub(DD a, DD b) { return dd_add(a, DD{-b.h, -b.l}); }
+GA_INLINE int incircle_dd(double2 a, double2 b, double2 c, double2 d, double sc)
+{
+    const DD x[3] = {dd_diff(a.x, d.x, sc), dd_diff(b.x, d.x, sc), dd_diff(c.x, d.x, sc)};
+    const DD y[3] = {dd_diff(a.y, d.y, sc), dd_diff(b.y, d.y, sc), dd_diff(c.y, d.y, sc)};
+    DD det{0.0, 0.0};
+    double perm = 0.0;
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        const int i = k == 2 ? 0 : k + 1, j = k == 0 ? 2 : k - 1;
+        const DD lift = dd_add(dd_mul(x[k], x[k]), dd_mul(y[k], y[k])), p = dd_mul(x[i], y[j]), q = dd_mul(x[j], y[i]);
+        det = dd_add(det, dd_mul(lift, dd_sub(p, q)));
+        perm += lift.h * (fabs(p.h) + fabs(q.h));
+    }
+    if (!(perm > 1e-200)) return 0;
+    return det.h > 0x1p-96 * perm ? 1 : (det.h < -0x1p-96 * perm ? -1 : 0);
+}
+
 // ---- exact path: fixed-capacity signed integers -------------------------------------
 // All coordinates that take part in one exact evaluation are written as integers
 // m * 2^(e - s) over the common unit 2^s (s = smallest ulp exponent among them), so the

@@ -62,7 +62,7 @@ static int orient_dev(const MeshDev &m, double2 a, double2 b, double2 c)
     if (ovf) *m.status = 1;
     return s;
 }
-static int incircle_at(const MeshDev &m, double2 a, double2 b, double2 c, double2 d, int ia, int ib, int ic, int id)
+static inline int incircle_at(const MeshDev &m, double2 a, double2 b, double2 c, double2 d, int ia, int ib, int ic, int id)
 {
     const int s = incircle_filter(a, b, c, d);
     if (s) return s;
