@@ -1805,14 +1805,13 @@ __global__ __launch_bounds__(256) void k_hull_edges(MeshDev m, HullDev h, int op
 struct HullSet {
     int b0, b1;
     double s;
-    int first;   // vertex that hull_apex tries first (-1: none): the wave's last apex, in a pocket mostly near the next
 };
 #define HULL_TINY 1e-290   // above what is lost to underflow in scaled coordinates
 __device__ HullSet hull_set(const MeshDev &m, const HullDev &h, int v)
 {
     const SetDesc &sd = m.sets[m.vset[v]];
     const int e = -ilogb(sd.scale);
-    return HullSet{h.bidx[sd.poff], h.bidx[sd.poff + sd.n], ldexp(1.0, e < 1023 ? e : 1023), -1};
+    return HullSet{h.bidx[sd.poff], h.bidx[sd.poff + sd.n], ldexp(1.0, e < 1023 ? e : 1023)};
 }
 
 // squared distances to v: true when a is nearer than b
@@ -1932,7 +1931,7 @@ __device__ bool hull_on_line(const MeshDev &m, const HullDev &h, int p, int q, d
     return __any(on);
 }
 
-// The apex of p -> q among the boundary vertices of its set (one wave; -1: none).  First set.first and
+// The apex of p -> q among the boundary vertices of its set (one wave; -1: none).  First
 // the vertices numbered next to p and q, which gives a circle near the final one; then the
 // boxes, 64 at a time: a box can hold a better apex only if it reaches left of the edge and into
 // the circle, which leaves one to three of B / 64.  (Every vertex tested, in steps of 64, took
@@ -1945,10 +1944,6 @@ __device__ int hull_apex(const MeshDev &m, const HullDev &h, int p, int q, HullS
     const double2 P = m.pos[p], Q = m.pos[q];
     const int gp = h.bidx[p] >> 6, gq = h.bidx[q] >> 6;
     HullBest c{-1, P};
-    if (set.first >= 0 && set.first != p && set.first != q) {
-        const double2 X = m.pos[set.first];
-        if (orient_dev(m, P, Q, X) > 0) c = HullBest{set.first, X};
-    }
     hull_chunk(m, h, P, Q, p, q, gp, set, lane, c);
     if (gq != gp) hull_chunk(m, h, P, Q, p, q, gq, set, lane, c);
     const double ux = (Q.x - P.x) * sc, uy = (Q.y - P.y) * sc;
@@ -2079,7 +2074,7 @@ __global__ __launch_bounds__(256) void k_hull_fill(MeshDev m, HullDev h)
     const int lane = threadIdx.x & 63, all = (int)((gridDim.x * blockDim.x) >> 6);
     const int nw = tight ? min(all, m.V - m.n + m.counters[C_HULL_ROOM]) : all;
     const int w0 = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
-    int slot = -1, last = -1, last_set = -1;   // last: the wave's last apex, in the set of boundary vertices from last_set on
+    int slot = -1;
     for (int i = w0 < nw ? w0 : nd + B; i < nd + B; i += nw) {
         int head = -1;
         HullSet set;
@@ -2109,7 +2104,6 @@ __global__ __launch_bounds__(256) void k_hull_fill(MeshDev m, HullDev h)
                     head = 2 * e + d;
                 }
         }
-        if (set.b0 == last_set) set.first = last;
         while (head >= 0) {
             const int it = head;
             int nx = 0, known = 0;
@@ -2127,8 +2121,6 @@ __global__ __launch_bounds__(256) void k_hull_fill(MeshDev m, HullDev h)
             const int p = it & 1 ? hi : lo, q = it & 1 ? lo : hi;
             const int c = hull_apex(m, h, p, q, set, lane);
             if (c >= 0) {
-                set.first = last = c;
-                last_set = set.b0;
                 hull_create(m, h, H, it, p, q, c, tight, lane, &slot, &head);
                 continue;
             }
