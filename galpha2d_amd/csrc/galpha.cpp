@@ -1158,50 +1158,55 @@ static int run_batch(galpha_ctx *c, const double *d_xy, const BatchPlan &plan)
     c->rot.ensure(4 * (size_t)nslots + 64);
     c->newid.ensure(4 * (size_t)nslots + 64);
     // one key (v0, v1) of 2B bits, input indices below 2^B (a batch's sets are consecutive ranges);
-    // up to B = 24 a 32-bit key (v0, top bits of v1 - v0) whose ties k_canon_newid orders
+    // up to B = 24 a 32-bit key (v0, top bits of v1 - v0) whose ties k_canon_newid orders, unless they
+    // are too many (a vertex with thousands of neighbours numbered close together): then the order is made
+    // again with the whole key
     int kb = 2;
     while ((1LL << kb) < (long long)n) kb++;
     if (2 * kb > 64) throw GalphaError("too many points for the canonical key");
     int *vals = c->vals.as<int>(), *vals2 = c->vals2.as<int>();
-    const unsigned *skey32 = nullptr, *v1s = nullptr;
-    size_t tb = 0;
-    if (kb <= CANON_KEY32_BITS) {
-        unsigned *K = c->keys.as<unsigned>(), *Ko = K + nslots, *V1 = c->keys2.as<unsigned>();
-        launch_canon_keys32(m, K, V1, vals, c->rot.as<int>(), kb, st);
-        const int bits = std::min(32, 2 * kb);
-        sort_pairs_u32(K, vals, Ko, vals2, nslots, 0, bits, nullptr, &tb, st);
-        c->sortTmp.ensure(tb + 256);
-        tb = c->sortTmp.bytes;
-        if (sort_pairs_u32(K, vals, Ko, vals2, nslots, 0, bits, c->sortTmp.p, &tb, st))
-            throw GalphaError("radix sort failed");
-        skey32 = Ko;
-        v1s = V1;
-    } else {
-        unsigned long long *K = c->keys.as<unsigned long long>(), *K2 = c->keys2.as<unsigned long long>();
-        launch_canon_keys(m, K, vals, c->rot.as<int>(), kb, st);
-        sort_pairs_u64(K, vals, K2, vals2, nslots, 0, 2 * kb, nullptr, &tb, st);
-        c->sortTmp.ensure(tb + 256);
-        tb = c->sortTmp.bytes;
-        if (sort_pairs_u64(K, vals, K2, vals2, nslots, 0, 2 * kb, c->sortTmp.p, &tb, st))
-            throw GalphaError("radix sort failed");
-    }
-    int *order = vals2;
-    // the live-triangle count stays on the device (folded statistic) until the final read
     c->out9.ensure(36 * (size_t)nslots + 64);
-    launch_fold_stats(c->counters.as<int>(), st);
-    // (records in the fan buffer, 24 bytes per slot)
-    launch_canon_emit(m, order, skey32, v1s, vals, c->rot.as<int>(), c->newid.as<int>(), c->fan.as<int2>(),
-                      c->counters.as<int>() + C_FOLD + C_RECON_TRIS, c->out9.as<int>(), c->setFirst.as<int>(),
-                      c->keys2.as<int>(), st);   // keys2 (v1s) is free after k_canon_newid: output sets
-    ev_mark(c, 8, st);
     Snap fin;
     std::vector<int> sfv((size_t)nsets + sizeof(fin.v) / 4);   // first triangle of every set, then the counters
-    if (nsets > 1)
-        ctx_read_segments(c, {{c->setFirst.as<int>(), nsets}, {c->counters.as<int>(), (int)(sizeof(fin.v) / 4)}},
-                          sfv.data());
-    else
-        ctx_read_segments(c, {{c->counters.as<int>(), (int)(sizeof(fin.v) / 4)}}, sfv.data() + 1);
-    memcpy(fin.v, sfv.data() + nsets, sizeof(fin.v));
+    for (bool whole = kb > CANON_KEY32_BITS, again = false;; whole = again = true) {
+        const unsigned *skey32 = nullptr, *v1s = nullptr;
+        size_t tb = 0;
+        if (!whole) {
+            unsigned *K = c->keys.as<unsigned>(), *Ko = K + nslots, *V1 = c->keys2.as<unsigned>();
+            launch_canon_keys32(m, K, V1, vals, c->rot.as<int>(), kb, st);
+            const int bits = std::min(32, 2 * kb);
+            sort_pairs_u32(K, vals, Ko, vals2, nslots, 0, bits, nullptr, &tb, st);
+            c->sortTmp.ensure(tb + 256);
+            tb = c->sortTmp.bytes;
+            if (sort_pairs_u32(K, vals, Ko, vals2, nslots, 0, bits, c->sortTmp.p, &tb, st))
+                throw GalphaError("radix sort failed");
+            skey32 = Ko;
+            v1s = V1;
+        } else {
+            unsigned long long *K = c->keys.as<unsigned long long>(), *K2 = c->keys2.as<unsigned long long>();
+            launch_canon_keys(m, K, vals, c->rot.as<int>(), kb, !again, st);
+            sort_pairs_u64(K, vals, K2, vals2, nslots, 0, 2 * kb, nullptr, &tb, st);
+            c->sortTmp.ensure(tb + 256);
+            tb = c->sortTmp.bytes;
+            if (sort_pairs_u64(K, vals, K2, vals2, nslots, 0, 2 * kb, c->sortTmp.p, &tb, st))
+                throw GalphaError("radix sort failed");
+        }
+        int *order = vals2;
+        // the live-triangle count stays on the device (folded statistic) until the final read
+        launch_fold_stats(c->counters.as<int>(), st);
+        // (records in the fan buffer, 24 bytes per slot)
+        launch_canon_emit(m, order, skey32, v1s, vals, c->rot.as<int>(), c->newid.as<int>(), c->fan.as<int2>(),
+                          c->counters.as<int>() + C_FOLD + C_RECON_TRIS, c->out9.as<int>(), c->setFirst.as<int>(),
+                          c->keys2.as<int>(), st);   // keys2 (v1s) is free after k_canon_newid: output sets
+        ev_mark(c, 8, st);
+        if (nsets > 1)
+            ctx_read_segments(c, {{c->setFirst.as<int>(), nsets}, {c->counters.as<int>(), (int)(sizeof(fin.v) / 4)}},
+                              sfv.data());
+        else
+            ctx_read_segments(c, {{c->counters.as<int>(), (int)(sizeof(fin.v) / 4)}}, sfv.data() + 1);
+        memcpy(fin.v, sfv.data() + nsets, sizeof(fin.v));
+        if (whole || !fin.v[C_LONG_RUN]) break;
+    }
     const int *sf = sfv.data();   // (a single set's: 0)
     if (fin.status()) throw GalphaError("canonical output failed (status " + std::to_string(fin.status()) + ")");
     int F = fin.stat(C_RECON_TRIS);

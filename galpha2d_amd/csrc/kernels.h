@@ -191,6 +191,7 @@ struct HullDev {
 #define C_TAIL_DONE 36        // 1 when that tail ended with a pass without flips
 #define C_TAIL_LISTED 37      // triangles listed by flip tails (also counted in C_FLIP_LISTED)
 #define C_STAR 41             // 41..43: list counts of the bulk shifting passes
+#define C_LONG_RUN 44         // a run of equal 32-bit canonical keys was too long to be ordered by counting
 #define FLIP_SPLIT (1 << 20)  // flip lists from this length on, and those behind passes with many exact tests, leave the
                               // exact tests to a launch of their own
 #define TAIL_LIST 2048        // longest flip list the single-workgroup tail takes, and of sets of up to
@@ -321,7 +322,8 @@ void launch_cons_insert(MeshDev &m, const int2 *cv, int nc, int *done, const int
 // frame removal (see mesh.hip); mark, share and the counters C_FTRI .. C_HULL_POOL zero on entry
 void launch_hull(MeshDev &m, const HullDev &h, int op, void *scan_tmp, hipStream_t st);
 // canonical order: key (v0 << B) | v1 of input indices below 2^B, sorted on its low 2B bits
-void launch_canon_keys(MeshDev &m, unsigned long long *keys, int *vals, int *rot, int B, hipStream_t st);
+// (count: the live triangles are to be counted)
+void launch_canon_keys(MeshDev &m, unsigned long long *keys, int *vals, int *rot, int B, bool count, hipStream_t st);
 // canonical keys of 32 bits up to input indices below 2^CANON_KEY32_BITS
 #define CANON_KEY32_BITS 24
 void launch_canon_keys32(MeshDev &m, unsigned *keys, unsigned *v1s, int *vals, int *rot, int B, hipStream_t st);

@@ -2151,7 +2151,7 @@ void launch_hull(MeshDev &m, const HullDev &h, int op, void *scan_tmp, hipStream
 // of a batch are consecutive ranges in set order, so this is also set order.  Every directed edge
 // belongs to one triangle, so (v0, v1) alone is unique: the key is v0 << B | v1 (indices below 2^B),
 // sorted on its low 2B bits.  Dead slots get all ones there, above every live key (v0 <= n - 3).
-__global__ void k_canon_keys(MeshDev m, unsigned long long *keys, int *vals, int *rot, int B)
+__global__ void k_canon_keys(MeshDev m, unsigned long long *keys, int *vals, int *rot, int B, int count)
 {
     int n = ntri_used(m);
     int alive = 0;
@@ -2168,12 +2168,12 @@ __global__ void k_canon_keys(MeshDev m, unsigned long long *keys, int *vals, int
         unsigned long long a = (unsigned)ic(o, r), b = (unsigned)ic(o, (r + 1) % 3);
         keys[t] = (a << B) | b;
     }
-    stat_add_full(m.stats, C_RECON_TRIS, alive);
+    if (count) stat_add_full(m.stats, C_RECON_TRIS, alive);
 }
 
-void launch_canon_keys(MeshDev &m, unsigned long long *keys, int *vals, int *rot, int B, hipStream_t st)
+void launch_canon_keys(MeshDev &m, unsigned long long *keys, int *vals, int *rot, int B, bool count, hipStream_t st)
 {
-    GA_LAUNCH(k_canon_keys, dim3(FIXED_GRID), dim3(256), 0, st, m, keys, vals, rot, B);
+    GA_LAUNCH(k_canon_keys, dim3(FIXED_GRID), dim3(256), 0, st, m, keys, vals, rot, B, count ? 1 : 0);
 }
 
 // 32-bit keys (indices below 2^B, B <= CANON_KEY32_BITS): v0 in the top B bits, then the top
@@ -2217,10 +2217,14 @@ void launch_canon_keys32(MeshDev &m, unsigned *keys, unsigned *v1s, int *vals, i
 
 // newid[slot] = output position << 2 | rotation of the slot's triangle: one gather per neighbour
 // in k_canon_emit.  With 32-bit keys (skey, v1s non-null) every triangle of a run of equal sorted
-// keys counts those with a smaller v1 (runs are mostly short; around one vertex with all others as
-// neighbours they can have 2^15 entries, which counting takes in parallel); out[] gets the final order.
+// keys counts those with a smaller v1; out[] gets the final order.  Runs are mostly short.  Around one vertex
+// with all others as neighbours they have up to 2^(2B - 32) entries (256 at B = 20, 2^16 at 24), and counting is
+// quadratic: a run of more than CANON_RUN entries is left as it is and reported, and the host orders by whole
+// keys instead (4.2M points, one with 400,000 neighbours: canonical stage 179 ms with counting alone, 2.3 now;
+// 1.1M points, one with 1,000 neighbours, where counting is still the cheaper: 0.49 and 0.81).
+#define CANON_RUN 512
 __global__ void k_canon_newid(const int *order, const unsigned *skey, const unsigned *v1s, const int *rot, const int *dF,
-                              int *newid, int *out)
+                              int *newid, int *out, int *long_run)
 {
     int F = *dF;
     GRID_STRIDE(r, F) {
@@ -2231,8 +2235,15 @@ __global__ void k_canon_newid(const int *order, const unsigned *skey, const unsi
             const bool before = r > 0 && skey[r - 1] == key, after = r + 1 < F && skey[r + 1] == key;
             if (before || after) {
                 const unsigned v = v1s[s];
-                for (int j = r - 1; j >= 0 && skey[j] == key; j--) at -= v1s[order[j]] > v;
-                for (int j = r + 1; j < F && skey[j] == key; j++) at += v1s[order[j]] < v;
+                // others of the run that are looked at; none when it is seen to be too long from here
+                const bool far = (r + CANON_RUN < F && skey[r + CANON_RUN] == key) || (r >= CANON_RUN && skey[r - CANON_RUN] == key);
+                int room = far ? 0 : CANON_RUN;
+                for (int j = r - 1; j >= 0 && room > 0 && skey[j] == key; j--, room--) at -= v1s[order[j]] > v;
+                for (int j = r + 1; j < F && room > 0 && skey[j] == key; j++, room--) at += v1s[order[j]] < v;
+                if (room == 0) {   // (for every triangle of the run: the order stays a permutation)
+                    at = r;
+                    if (!before) *long_run = 1;
+                }
             }
             out[at] = s;
         }
@@ -2328,7 +2339,8 @@ __global__ void k_canon_set_first(MeshDev m, const int *rset, const int *dF, int
 void launch_canon_emit(MeshDev &m, const int *order, const unsigned *skey, const unsigned *v1s, int *out, const int *rot,
                        int *newid, int2 *rec, const int *dF, int *out9, int *set_first, int *rset, hipStream_t st)
 {
-    GA_LAUNCH(k_canon_newid, dim3(FIXED_GRID), dim3(256), 0, st, order, skey, v1s, rot, dF, newid, out);
+    GA_LAUNCH(k_canon_newid, dim3(FIXED_GRID), dim3(256), 0, st, order, skey, v1s, rot, dF, newid, out,
+              m.counters + C_LONG_RUN);
     const int *sorted = skey ? out : order;
     if (m.nsets == 1) {   // (its first triangle is triangle 0)
         GA_LAUNCH(k_canon_records, dim3(FIXED_GRID), dim3(256), 0, st, m, (const int *)newid, rec);
