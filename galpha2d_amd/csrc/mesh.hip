@@ -1523,12 +1523,17 @@ __global__ void k_flip_commit(MeshDev m, int op, int *list_out, int cnt_out_slot
 // 512 threads: the exact test needs 174 registers, and 1,024 leave 128 (305 spilled).  All passes of 1,000
 // points 91 -> 59 us, of 12,007 in clusters 171 -> 111; with the exact tests as a step of their own 106 and
 // 202 (1,024 threads), 65 and 126 (512), at 256 threads without it 69 and 122.
+// Small sets (limit above TAIL_LIST) with more than three points of four inserted leave long lists to grid passes as
+// well: their points lie far closer together than the pixels, their exact tests need the big integers, and these
+// come one after another in every wave (2,000 points, all but two within 1e-9 of the set's size: all passes 8.2 ms, 5.7
+// so).
 #define FLIP_TAIL_THREADS 512
 __global__ __launch_bounds__(FLIP_TAIL_THREADS) void k_flip_tail(MeshDev m, int *lA, int sA, int *lB, int sB,
                                                                  int prev_op, int op0, int max_passes, int limit)
 {
     int *lin = lA, *lout = lB, sin = sA, sout = sB;
     int prev = prev_op, pass = 0, done = 0;
+    if (4 * m.counters[C_MISS] > 3 * m.n) limit = min(limit, TAIL_LIST);
     for (; pass < max_passes; pass++) {
         const int n = m.counters[sin];
         if (n > limit) break;
