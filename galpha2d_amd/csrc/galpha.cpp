@@ -1004,7 +1004,7 @@ static int run_batch(galpha_ctx *c, const double *d_xy, const BatchPlan &plan)
         bool shifting = true, deleting = true;
         // grids before the lists' lengths are known: one vertex in 8 pending, one in 4 missing
         int pgrid = round_grid(m.n), dgrid = round_grid(m.n / 2), mgrid = round_grid(m.n / 4);
-        const bool tail = m.n <= SHIFT_TAIL_POINTS;
+        bool tail = m.n <= SHIFT_TAIL_POINTS, greedy = false;   // greedy: the tail left the rounds after the commit
         for (int r = 0;; r++) {
             if (tail && deleting) {
                 const int max_rounds = 64, round0 = c->prio_round + 1;
@@ -1020,7 +1020,11 @@ static int run_batch(galpha_ctx *c, const double *d_xy, const BatchPlan &plan)
                 stars += 4;
                 if (stars > 100000) throw GalphaError("bulk shifting did not converge");
                 launch_shift_commit(m, moved, slot[stars % 3], st);
+                greedy = true;
+            }
+            if (greedy) {
                 for (int k = 0; k < 8; k++) launch_shift_greedy(m, k, m.mark, pgrid, st);
+                greedy = false;
             }
             if (deleting) {
                 // (k_del_prio zeroes C_SCR and C_PLEFT)
@@ -1071,6 +1075,10 @@ static int run_batch(galpha_ctx *c, const double *d_xy, const BatchPlan &plan)
                 throw GalphaError("vertex deletion failed (status " + std::to_string(stt) + ")" + d + "]");
             }
             if (!deleting && !last.v[C_MLEFT]) break;
+            if (tail && last.v[C_PLIST] > SHIFT_TAIL_PENDING) {
+                tail = false;
+                greedy = true;
+            }
             if (r > 10000) throw GalphaError(deleting ? "vertex deletion did not finish" : "missing-site insertion did not finish");
             pgrid = round_grid(8LL * last.v[C_PLIST]);
             dgrid = round_grid(4LL * last.v[C_PLIST]);

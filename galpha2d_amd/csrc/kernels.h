@@ -284,6 +284,7 @@ void launch_delete_round(MeshDev &m, unsigned int *mx, int round, int grid, hipS
 // small sets (see mesh.hip): everything from the bulk passes' first worklist to the deletions, and the
 // insertion rounds, one workgroup each
 #define SHIFT_TAIL_POINTS 8192
+#define SHIFT_TAIL_PENDING 1024
 #define INSERT_TAIL_POINTS 2048
 void launch_shift_tail(MeshDev &m, unsigned char *moved, int *mark, int *wlA, int *wlB, int slot, unsigned int *mx,
                        int round0, int max_rounds, bool more, hipStream_t st);

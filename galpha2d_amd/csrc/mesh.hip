@@ -935,7 +935,9 @@ __global__ __launch_bounds__(256) void k_del_apply(MeshDev m, const unsigned lon
 // deletions in one workgroup, phases separated by barriers.  A launch of a few thousand lanes costs the host
 // about 5 us and the device 2.5, and there are 25 of them (1,000 points: 840 us for the call with them, 770;
 // 5,003 points 762 and 699); from some ten thousand points on the rounds keep more than one CU busy.
-// more: only further deletion rounds (the ones before were not enough).
+// more: only further deletion rounds (the ones before were not enough).  With more than SHIFT_TAIL_PENDING vertices
+// pending the greedy and deletion rounds are left to launches of their own (8,000 points on a spiral, 3,600 of them
+// pending: shifting stage 7.4 ms in one workgroup, 2.9 so).
 #define SHIFT_TAIL_THREADS 512
 __global__ __launch_bounds__(SHIFT_TAIL_THREADS) void k_shift_tail(MeshDev m, unsigned char *moved, int *mark, int *wlA,
                                                                    int *wlB, int slot, unsigned long long *mx, int round0,
@@ -957,6 +959,10 @@ __global__ __launch_bounds__(SHIFT_TAIL_THREADS) void k_shift_tail(MeshDev m, un
     if (!more) shift_commit_body(m, moved);
     __syncthreads();
     const int np = m.counters[C_PLIST];
+    if (np > SHIFT_TAIL_PENDING) {
+        if (threadIdx.x == 0) m.counters[C_PLEFT] = 1;
+        return;
+    }
     bool left = np > 0;
     for (int r = 0; r < 8 && left && !more; r++)
         if (!__syncthreads_or(shift_greedy_body(m, r, mark, np))) break;
@@ -1444,6 +1450,7 @@ __global__ __launch_bounds__(256) void k_flip_exact(MeshDev m, int op)
         m.cand[slot] = c;
     }
 }
+
 
 // Block-uniform loop (block_reserve inside): up to four candidates per thread and step, and one
 // reservation of output-list slots per block and step (a reservation per wave put thousands of

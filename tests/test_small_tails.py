@@ -1,5 +1,5 @@
-"""Small sets that the single-workgroup stages hand over to grid launches: long flip lists of points that nearly all share
-pixels.  Triangles against the oracle, and
+"""Small sets that the single-workgroup stages hand over to grid launches: many vertices left to move or delete (points on a
+spiral), and long flip lists of points that nearly all share pixels.  Triangles against the oracle, and
 the launches that say who did the work."""
 import numpy as np
 import pytest
@@ -9,13 +9,22 @@ from galpha2d_amd import datagen
 pytestmark = pytest.mark.gpu
 
 
+def _spiral(n, seed):
+    t = np.sqrt(np.random.default_rng(seed).random(n)) * 40
+    return np.stack([t * np.cos(t), t * np.sin(t)], 1)
+
+
 def _one_pixel(n, seed):
     p = np.random.default_rng(seed).random((n, 2)) * 1e-9
     p[:2] = [[1.0, 1.0], [-1.0, 0.5]]
     return p
 
 
-CASES = [("one pixel 2,000", "k_flip_test", lambda: _one_pixel(2000, 5), True),
+CASES = [("spiral 2,000", "k_shift_greedy", lambda: _spiral(2000, 1), True),
+         ("spiral 8,000", "k_shift_greedy", lambda: _spiral(8000, 2), True),
+         ("spiral 1,000", "k_shift_greedy", lambda: _spiral(1000, 3), False),
+         ("uniform 8,000", "k_shift_greedy", lambda: datagen.uniform(4, 8000), False),
+         ("one pixel 2,000", "k_flip_test", lambda: _one_pixel(2000, 5), True),
          ("one pixel 300", "k_flip_test", lambda: _one_pixel(300, 6), False),
          ("uniform 2,000", "k_flip_test", lambda: datagen.uniform(7, 2000), False)]
 
