@@ -102,7 +102,7 @@ struct galpha_ctx {
     std::string err;
     // PBA
     DevBuf smap, g, hmin, far, setfar, vor, bad, fpix;
-    DevBuf chg, chgset;   // island repair: relabelled pixels and their sets
+    DevBuf chg;           // island repair: blocks with relabelled pixels
     // mesh
     DevBuf perm, xys, pcell, ccount, ccursor;   // spatial numbering of the real points
     DevBuf cls;                                  // alpha-complex classes (host queries)
@@ -620,6 +620,8 @@ static void ensure_pba(galpha_ctx *c, const BatchPlan &b)
     c->hmin.ensure(P / 8);
     c->far.ensure(P / 256);
     c->setfar.ensure(4 * (size_t)b.nsets() + 16);
+    c->chg.ensure(4 * (size_t)b.blocks[BM_PIX]);
+    c->mlist.ensure(4 * (size_t)b.ntot);   // (free until the shifting: the sites that an island repair removes)
     c->vor.ensure(4 * P);
     c->bad.ensure(4 * (size_t)(b.V + 1));
     c->fpix.ensure(4 * (size_t)(b.V - b.ntot + 1));
@@ -687,11 +689,8 @@ static void run_pba(galpha_ctx *c, const double *d_xy, const BatchDev &bd, int *
         ctx_counters_read(c, cv, 0, C_ISLAND_SITES + 1);
         isl = cv[C_ISLAND_SITES];
         if (cv[C_FLAG] == 0) break;
-        c->mlist.ensure(4 * (size_t)bd.ntot);   // (free until the shifting: the removed sites)
-        c->chg.ensure(4 * bd.P);
-        c->chgset.ensure(4 * bd.P);
         launch_island_repair(b, bd, c->bad.as<int>(), c->pix.as<int>(), cnt + C_ISLAND_SITES, isl, c->mlist.as<int>(),
-                             c->chg.as<unsigned>(), c->chgset.as<int>(), cnt + C_CHANGED, cnt + C_FLAG, st);
+                             c->chg.as<int>(), cnt + C_CHANGED, cnt + C_FLAG, st);
     }
     if (it == 16) throw GalphaError("discrete Voronoi diagram did not settle (island certificate)");
     *iters = it + 1;
@@ -1397,7 +1396,7 @@ galpha_ctx *galphaCreate(int device)
 
 static void release_all(galpha_ctx *c)
 {
-    DevBuf *bufs[] = {&c->smap, &c->g, &c->hmin, &c->far, &c->setfar, &c->chg, &c->chgset, &c->vor, &c->bad, &c->fpix, &c->tv,
+    DevBuf *bufs[] = {&c->smap, &c->g, &c->hmin, &c->far, &c->setfar, &c->chg, &c->vor, &c->bad, &c->fpix, &c->tv,
                       &c->tn, &c->remap, &c->stamp, &c->claim, &c->modA, &c->modB, &c->cand, &c->pos, &c->vt,
                       &c->vstate, &c->pix, &c->deg, &c->off, &c->fill, &c->fan, &c->moved, &c->mark, &c->mx,
                       &c->mlist, &c->loc, &c->lt, &c->scratch, &c->keys, &c->keys2,
@@ -1416,7 +1415,7 @@ static void release_all(galpha_ctx *c)
 // device bytes held by a context (all grown buffers)
 size_t galpha_ctx_device_bytes(galpha_ctx *c)
 {
-    DevBuf *bufs[] = {&c->smap, &c->g, &c->hmin, &c->far, &c->setfar, &c->chg, &c->chgset, &c->vor, &c->bad, &c->fpix, &c->tv,
+    DevBuf *bufs[] = {&c->smap, &c->g, &c->hmin, &c->far, &c->setfar, &c->chg, &c->vor, &c->bad, &c->fpix, &c->tv,
                       &c->tn, &c->remap, &c->stamp, &c->claim, &c->modA, &c->modB, &c->cand, &c->pos, &c->vt,
                       &c->vstate, &c->pix, &c->deg, &c->off, &c->fill, &c->fan, &c->moved, &c->mark, &c->mx,
                       &c->mlist, &c->loc, &c->lt, &c->scratch, &c->keys, &c->keys2,

@@ -168,7 +168,7 @@ struct HullDev {
 #define C_TESTS_INCIRCLE 14
 #define C_TESTS_ORIENT 15
 #define C_RECON_TRIS 16
-#define C_CHANGED 17          // pixels relabelled by an island repair
+#define C_CHANGED 17          // blocks of 1,024 pixels with some that an island repair relabelled
 #define C_DELETED 18
 #define C_ISLAND_SITES 19
 #define C_HULL_ROOM 20        // triangle slots unused before frame removal
@@ -229,7 +229,7 @@ void launch_pba(const PbaBuffers &p, const int *pix, const BatchDev &b, hipStrea
 void launch_islands(const int *vor, const int *pix, const BatchDev &b, int *bad, int *flag, hipStream_t st);
 // repairs the diagram around the sites that the certificate flagged (see pba.hip)
 void launch_island_repair(const PbaBuffers &p, const BatchDev &b, int *bad, const int *pix, int *removed, int first,
-                          int *rlist, unsigned *changed, int *chset, int *nchanged, int *flag, hipStream_t st);
+                          int *rlist, int *changed, int *nchanged, int *flag, hipStream_t st);
 
 // util.hip: up to four segments of device ints copied into one contiguous device array
 struct IntSegments {

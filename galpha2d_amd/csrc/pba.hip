@@ -20,6 +20,7 @@
 // the nearest site that is left, so every label stays an exact nearest site.
 #include "dev_common.h"
 #include "kernels.h"
+#include <algorithm>
 
 #define PBA_EMPTY 0x7fffffff
 
@@ -637,18 +638,16 @@ GA_INLINE void island_fail(int s, int *bad, int *flag)
 // contiguous eighth of the blocks, whose neighbour columns are then in its own L2.  Bound by the
 // reads of the diagram: 136 us at T = 8192 (2.0 TB/s); one pixel per thread, in launch order, took 226 us,
 // and 1,640 us against 754 us on a batch of 1,024 textures (357M pixels).
-__global__ __launch_bounds__(256) void k_islands(const int *__restrict__ vor_all, const int *__restrict__ pix,
-                                                 BatchDev bd, int *__restrict__ bad, int *__restrict__ flag)
+GA_INLINE void island_block(const int *__restrict__ vor_all, const int *__restrict__ pix, const BatchDev &bd, int blk,
+                            int *__restrict__ bad, int *__restrict__ flag)
 {
-    const unsigned nb = gridDim.x, q8 = nb >> 3;   // the last nb % 8 blocks keep their numbers
-    const unsigned blk = blockIdx.x < 8 * q8 ? (blockIdx.x & 7u) * q8 + (blockIdx.x >> 3) : blockIdx.x;
     const int *bm = bd.bmap(BM_PIX);
-    int set = set_of(bm, bd.nsets, (int)blk);
+    int set = set_of(bm, bd.nsets, blk);
     const SetDesc &sd = bd.sets[set];
     int logT = sd.logT;
     int T = 1 << logT;
     const int *vor = vor_all + sd.toff;
-    size_t idx = (size_t)((int)blk - bm[set]) * 1024 + 4 * threadIdx.x;
+    size_t idx = (size_t)(blk - bm[set]) * 1024 + 4 * threadIdx.x;
     const int x = (int)(idx >> logT), y0 = (int)(idx & (T - 1));
     const int4 own = *(const int4 *)(vor + idx);
     const int lab[4] = {own.x, own.y, own.z, own.w};
@@ -679,6 +678,14 @@ __global__ __launch_bounds__(256) void k_islands(const int *__restrict__ vor_all
         if (!ok && dx != 0 && dy != 0) ok = vor[idx + j + dy + ((long long)dx << logT)] == s;
         if (!ok) island_fail(s, bad, flag);
     }
+}
+
+__global__ __launch_bounds__(256) void k_islands(const int *__restrict__ vor_all, const int *__restrict__ pix,
+                                                 BatchDev bd, int *__restrict__ bad, int *__restrict__ flag)
+{
+    const unsigned nb = gridDim.x, q8 = nb >> 3;   // the last nb % 8 blocks keep their numbers
+    const unsigned blk = blockIdx.x < 8 * q8 ? (blockIdx.x & 7u) * q8 + (blockIdx.x >> 3) : blockIdx.x;
+    island_block(vor_all, pix, bd, (int)blk, bad, flag);
 }
 
 // Takes the sites flagged by the certificate out of the site map, and lists them (count in *removed).
@@ -723,13 +730,12 @@ __global__ __launch_bounds__(64) void k_repair_cols(const int *__restrict__ rlis
 // flight.  A repair takes 0.15 ms at T = 2048 and 0.3 ms at T = 8192, where a whole second diagram took
 // 0.4 and 2.2 ms, and a batch of 1,024 sets (10-20% of them repaired, three times) 1.5 instead of 17 ms.
 // Only these pixels need the certificate again (any other keeps its label, and the
-// neighbour that certified it had the same one): they are listed.  Blocks of 1,024 pixels; sets
+// neighbour that certified it had the same one): the blocks of 1,024 pixels that hold some are listed.  Sets
 // without a removed site return at once.
 __global__ __launch_bounds__(256) void k_relabel(int *__restrict__ vor_all, const short *__restrict__ g_all,
                                                  const int *__restrict__ smap_all, const int *__restrict__ bad,
                                                  const int *__restrict__ setbad, BatchDev bd,
-                                                 unsigned *__restrict__ changed, int *__restrict__ chset,
-                                                 int *__restrict__ nchanged)
+                                                 int *__restrict__ changed, int *__restrict__ nchanged)
 {
     const int *bm = bd.bmap(BM_PIX);
     int set = set_of(bm, bd.nsets, blockIdx.x);
@@ -739,11 +745,13 @@ __global__ __launch_bounds__(256) void k_relabel(int *__restrict__ vor_all, cons
     int *vor = vor_all + sd.toff;
     const short *g = g_all + sd.toff;
     const int *smap = smap_all + sd.toff;
+    bool any = false;
     for (int q = 0; q < 4; q++) {
         const size_t idx = (size_t)(blockIdx.x - bm[set]) * 1024 + q * 256 + threadIdx.x;
         const int s = vor[idx];
         const bool act = s >= 0 && bad[s] == BAD_REMOVED;
         if (!__any(act)) continue;
+        any = any || act;
         const int x = (int)(idx >> logT), y = (int)(idx & (T - 1));
         long long best = act ? 0x7fffffffffffffffll : -1;
         int bx = -1, by = 0;
@@ -767,35 +775,18 @@ __global__ __launch_bounds__(256) void k_relabel(int *__restrict__ vor_all, cons
                 }
             }
         }
-        const int c = wave_reserve(nchanged, act);
-        if (!act) continue;
-        vor[idx] = bx < 0 ? -1 : smap[((size_t)bx << logT) + by];
-        changed[c] = (unsigned)idx;
-        chset[c] = set;
+        if (act) vor[idx] = bx < 0 ? -1 : smap[((size_t)bx << logT) + by];
     }
+    if (__syncthreads_or(any) && threadIdx.x == 0) changed[atomicAdd(nchanged, 1)] = (int)blockIdx.x;
 }
 
-// the certificate of the relabelled pixels (set and pixel of each)
-__global__ void k_recheck(const int *__restrict__ vor_all, const int *__restrict__ pix, BatchDev bd,
-                          const unsigned *__restrict__ changed, const int *__restrict__ chset,
-                          const int *__restrict__ nchanged, int *__restrict__ bad, int *__restrict__ flag)
+// the certificate of the listed blocks
+__global__ __launch_bounds__(256) void k_recheck(const int *__restrict__ vor_all, const int *__restrict__ pix, BatchDev bd,
+                                                 const int *__restrict__ changed, const int *__restrict__ nchanged,
+                                                 int *__restrict__ bad, int *__restrict__ flag)
 {
     const int n = *nchanged;
-    for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < n; c += gridDim.x * blockDim.x) {
-        const SetDesc &sd = bd.sets[chset[c]];
-        const size_t idx = changed[c];
-        const int logT = sd.logT, T = 1 << logT;
-        const int *vor = vor_all + sd.toff;
-        const int s = vor[idx];
-        if (s < 0) continue;
-        const int x = (int)(idx >> logT), y = (int)(idx & (T - 1)), sp = pix[s], sx = sp >> 16, sy = sp & 0xffff;
-        const int dx = (sx > x) - (sx < x), dy = (sy > y) - (sy < y);
-        if (dx == 0 && dy == 0) continue;
-        bool ok = dx != 0 && vor[idx + ((long long)dx << logT)] == s;
-        if (!ok && dy != 0) ok = vor[idx + dy] == s;
-        if (!ok && dx != 0 && dy != 0) ok = vor[idx + ((long long)dx << logT) + dy] == s;
-        if (!ok) island_fail(s, bad, flag);
-    }
+    for (int c = blockIdx.x; c < n; c += gridDim.x) island_block(vor_all, pix, bd, changed[c], bad, flag);
 }
 
 // ---- host-side launchers ---------------------------------------------------------------
@@ -866,9 +857,9 @@ void launch_islands(const int *vor, const int *pix, const BatchDev &b, int *bad,
 }
 
 // removes the flagged sites (listed in rlist from position `first`, the number removed before) and
-// repairs the diagram around them, then checks the pixels that changed; zeroes *flag and *nchanged
+// repairs the diagram around them, then checks the blocks that changed (listed in changed); zeroes *flag and *nchanged
 void launch_island_repair(const PbaBuffers &p, const BatchDev &b, int *bad, const int *pix, int *removed, int first,
-                          int *rlist, unsigned *changed, int *chset, int *nchanged, int *flag, hipStream_t st)
+                          int *rlist, int *changed, int *nchanged, int *flag, hipStream_t st)
 {
     // (free after phase 3)
     int *setbad = p.setfar;
@@ -882,7 +873,7 @@ void launch_island_repair(const PbaBuffers &p, const BatchDev &b, int *bad, cons
     GA_LAUNCH(k_repair_cols, dim3(1024), dim3(64), 0, st, (const int *)rlist, first, (const int *)removed, pix, b,
               (const int *)p.smap, p.g);
     GA_LAUNCH(k_relabel, dim3(b.blocks[BM_PIX]), dim3(256), 0, st, p.vor, (const short *)p.g, (const int *)p.smap,
-              (const int *)bad, (const int *)setbad, b, changed, chset, nchanged);
-    GA_LAUNCH(k_recheck, dim3(1024), dim3(256), 0, st, (const int *)p.vor, pix, b, (const unsigned *)changed,
-              (const int *)chset, (const int *)nchanged, bad, flag);
+              (const int *)bad, (const int *)setbad, b, changed, nchanged);
+    GA_LAUNCH(k_recheck, dim3(std::min(b.blocks[BM_PIX], 2048)), dim3(256), 0, st, (const int *)p.vor, pix, b,
+              (const int *)changed, (const int *)nchanged, bad, flag);
 }
