@@ -1022,13 +1022,3 @@ GA_INLINE uint32_t hash32(uint32_t x)
     x ^= x >> 16;
     return x;
 }
-
-// error codes written to the device status word
-#define GA_ERR_EXACT_OVERFLOW 1
-#define GA_ERR_WALK 2
-#define GA_ERR_RECON 4
-#define GA_ERR_SCRATCH 8
-#define GA_ERR_CAPACITY 16
-#define GA_ERR_ISLANDS 32
-#define GA_ERR_PATCH 64
-// GA_ERR_CONS_* (constraint insertion): kernels.h

@@ -1047,7 +1047,7 @@ static int run_batch(galpha_ctx *c, const double *d_xy, const BatchPlan &plan)
             flip_all();
             if (m.n <= INSERT_TAIL_POINTS) S.insertRounds += last.v[C_INSERT_ROUNDS];
             S.reconTris = last.v[C_RECON_SLOTS];
-            if (last.v[C_RECON_SLOTS] > cap) throw GalphaError("triangle capacity exceeded in reconstruction");
+            if (last.v[C_RECON_STATUS] & GA_ERR_CAPACITY) throw GalphaError("triangle capacity exceeded in reconstruction");
             if (last.v[C_RECON_STATUS])
                 throw GalphaError("reconstruction produced an invalid triangle (status " +
                                   std::to_string(last.v[C_RECON_STATUS]) + ")");

@@ -196,7 +196,15 @@ struct HullDev {
                               // exact tests to a launch of their own
 #define TAIL_LIST 2048        // longest flip list the single-workgroup tail takes, and of sets of up to
 #define TAIL_LIST_SMALL 16384 // INSERT_TAIL_POINTS points, whose passes cost less there than their launches
-// status bits of constraint insertion (the other GA_ERR_* bits are in dev_common.h)
+// error codes written to the device status word
+#define GA_ERR_EXACT_OVERFLOW 1
+#define GA_ERR_WALK 2
+#define GA_ERR_RECON 4
+#define GA_ERR_SCRATCH 8
+#define GA_ERR_CAPACITY 16
+#define GA_ERR_ISLANDS 32
+#define GA_ERR_PATCH 64
+// constraint insertion
 #define GA_ERR_CONS_POINT 128     // a point lies inside a constraint segment
 #define GA_ERR_CONS_CROSS 256     // two constraints cross
 #define GA_ERR_CONS_WALK 512      // the walk along a constraint left the mesh
