@@ -1455,8 +1455,8 @@ __attribute__((visibility("hidden"))) galpha_ctx *galpha_noalloc_ctx_new(int dev
 
 // Upper bound of the bytes a single-set DT run of n points on a T x T texture carves: every
 // buffer the run ensures, at its largest size (slots at the capacity 3 V + 8192), the scan and sort
-// temporaries as rocPRIM reports them, and 256-byte rounding.  About 100 V bytes of it are room that
-// no buffer takes: the sizes that fit the scratch are part of the interface.
+// temporaries as rocPRIM reports them, and 256-byte rounding; and room that no buffer takes, since the sizes that
+// fit the scratch are part of the interface.
 __attribute__((visibility("hidden"))) size_t galpha_noalloc_need(int n, int T)
 {
     if (n < 3) return 4096;
@@ -1469,9 +1469,11 @@ __attribute__((visibility("hidden"))) size_t galpha_noalloc_need(int n, int T)
     sort_pairs_u32(nullptr, nullptr, nullptr, nullptr, (int)cap, 0, (int)std::min(32LL, 2 * kb), nullptr, &sort_tmp32, 0);
     sort_tmp = std::max(sort_tmp, sort_tmp32);
     double b = 0;
-    b += 18.0 * P + 516.0 * T + 8.0 * ntiles + 8.0 * nc;          // textures, band ranges, tiles, cells
-    b += (116.0 + 68.0) * cap;                                     // mesh slots, canonical keys + output
-    b += (89.0 + 76.0 + 12.0) * V + 36.0 * n + 4.0 * nf;           // vertex arrays, boundary cycle, plan
+    // site map, labels, column field; its 16-column minima, far flags and repaired blocks; tiles, cells
+    b += (4.0 + 4.0 + 2.0) * P + P / 8.0 + P / 256.0 + P / 256.0 + 8.0 * ntiles + 8.0 * nc;
+    b += (108.0 + 68.0) * cap;                                     // mesh slots, canonical keys + output
+    b += (16.0 + 45.0 + 32.0) * V + 36.0 * n + 4.0 * nf;           // vertex arrays, scratch, point arrays, frame pixels
+    b += 7.8671875 * P + 516.0 * T + 8.0 * cap + 84.0 * V;         // room
     b += (double)COUNTER_BYTES + 4096.0 + 8.0 * 5 * 64;           // counters, status, box partials
     b += (double)scan_temp_bytes((size_t)std::max(ntiles, V + 2)) + (double)scan_temp_bytes((size_t)nc) + 8192.0;
     b += (double)sort_tmp + 256.0 + 96.0 * 256.0 + 65536.0;        // sort temporary, rounding, slack
