@@ -31,6 +31,11 @@ GA_INLINE int m1(int i) { return i == 0 ? 2 : i - 1; }
 #define GA_EPS 1.1102230246251565e-16
 #define GA_CCWERRA ((3.0 + 16.0 * GA_EPS) * GA_EPS)
 #define GA_ICCERRA ((10.0 + 96.0 * GA_EPS) * GA_EPS)
+// The bounds hold while nothing underflows.  Below these sums of magnitudes (differences of about 1e-148 and 1e-72)
+// the filters leave the sign open; above them what underflows, 2^-1074 times lifts of 1e15 at most, is less than a
+// thousandth of the bounds.
+#define GA_CCW_TINY 1e-295
+#define GA_ICC_TINY 1e-288
 
 // returns +1/-1 when certain, 0 when the filter cannot decide
 GA_INLINE int orient_filter(double2 a, double2 b, double2 c)
@@ -49,6 +54,7 @@ GA_INLINE int orient_filter(double2 a, double2 b, double2 c)
         // detleft == 0: det = -detright, exact in sign
         return det > 0 ? 1 : (det < 0 ? -1 : 0);
     }
+    if (detsum < GA_CCW_TINY) return 0;
     double eb = GA_CCWERRA * detsum;
     if (det >= eb && det != 0.0) return 1;
     if (-det >= eb && det != 0.0) return -1;
@@ -68,7 +74,7 @@ GA_INLINE int incircle_filter(double2 a, double2 b, double2 c, double2 d)
     double det = alift * (bdxcdy - cdxbdy) + blift * (cdxady - adxcdy) + clift * (adxbdy - bdxady);
     double perm = (fabs(bdxcdy) + fabs(cdxbdy)) * alift + (fabs(cdxady) + fabs(adxcdy)) * blift
                 + (fabs(adxbdy) + fabs(bdxady)) * clift;
-    double eb = GA_ICCERRA * perm;
+    double eb = perm < GA_ICC_TINY ? perm : GA_ICCERRA * perm;   // (no sum exceeds that of the magnitudes)
     if (det > eb) return 1;
     if (-det > eb) return -1;
     return 0;
