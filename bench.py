@@ -235,9 +235,9 @@ def stress_c3(G, reps=3, seed=3):
                        f"Gaussian clusters (sigma 0.005); seed {seed}; texture {T}x{T}; DT + full alpha",
            "ms": round(med * 1e3, 2), "mpoints_per_s": round(n / med / 1e6, 3), "runs": reps,
            "stage_ms": {k: round(float(np.median(v)), 3) for k, v in stage.items()},
-           "triangles": st["nTris"], "frame_bulk": st["frameBulk"],
+           "triangles": st["nTris"],
            "work": {k: st[k] for k in ("shiftBad", "deleted", "missing", "inserted", "duplicates", "insertRounds",
-                                        "flipPasses", "flips", "flipListed", "earRounds", "alphaClusters",
+                                        "flipPasses", "flips", "flipListed", "alphaClusters",
                                         "alphaMaxCluster")},
            "fallback": {
                "incircle": rate(st["incircleExact"], st["incircleTests"]),
@@ -245,7 +245,7 @@ def stress_c3(G, reps=3, seed=3):
                "alpha_compare": rate(st["alphaExactCompares"], st["nTris"] + st["nEdges"], "entries"),
                "attachment": rate(st["alphaExactAttach"], st["nEdges"], "edges")}}
     if "stageIncircleTests" in st:
-        names = ("shift, insertion and flips", "frame removal and final flips", "constraints and canonical output")
+        names = ("shift, insertion and flips", "frame removal", "constraints and canonical output")
         out["fallback"]["per_stage"] = {
             nm: {"incircle": rate(st["stageIncircleExact"][i], st["stageIncircleTests"][i]),
                  "orient_exact": int(st["stageOrientExact"][i])} for i, nm in enumerate(names)}
@@ -491,7 +491,7 @@ def main():
         "roofline": roof,
         "stage_gbs": stages,
         "work": {k: st[k] for k in ("reconTris", "shiftBad", "deleted", "missing", "inserted", "duplicates",
-                                     "insertRounds", "flipPasses", "flips", "flipListed", "frameBulk", "earRounds",
+                                     "insertRounds", "flipPasses", "flips", "flipListed",
                                      "islandSites", "alphaClusters", "alphaMaxCluster")},
     }
     ctx.close()
