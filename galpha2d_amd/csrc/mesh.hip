@@ -1970,7 +1970,8 @@ __device__ int hull_apex(const MeshDev &m, const HullDev &h, int p, int q, HullS
         const double cx = uy > 0 ? bx.lx : bx.hx, cy = ux > 0 ? bx.hy : bx.ly;
         const double l = ux * ((cy - P.y) * sc), r = uy * ((cx - P.x) * sc);
         const bool flat = (P.x == Q.x && cx == P.x) || (P.y == Q.y && cy == P.y);
-        const bool left = in && !flat && l - r >= -1e-14 * (fabs(l) + fabs(r)) - HULL_TINY;
+        // (a box with vertices of another set may be so large that this is NaN: it stays)
+        const bool left = in && !flat && !(l - r < -1e-14 * (fabs(l) + fabs(r)) - HULL_TINY);
         unsigned long long todo = __ballot(left);
         if (!asked && c.v < 0 && __popcll(todo) > 16) {
             asked = true;

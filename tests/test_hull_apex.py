@@ -101,14 +101,14 @@ static void wave(std::function<void(int)> body)
             }
     }
 }
-// argv[1]: n, demands, the set's snap scale, n points, demands (p, q); prints the apexes, then
+// argv[1]: n, demands, the set's snap scale, the vertices of another set before it, n points, demands (p, q); prints the apexes, then
 // the nearest vertices of the demands' first ends, the status and the number of collectives
 int main(int, char **argv)
 {
     FILE *f = fopen(argv[1], "r");
-    int n, nd, status = 0;
+    int n, nd, other, status = 0;
     SetDesc sd{};
-    if (fscanf(f, "%d %d %la", &n, &nd, &sd.scale) != 3) return 1;
+    if (fscanf(f, "%d %d %la %d", &n, &nd, &sd.scale, &other) != 4) return 1;
     std::vector<double2> pos(n + 1);
     std::vector<int> ids(n + 1), zero(n + 1);
     std::vector<HullBox> box(n / 64 + 1, HullBox{INFINITY, INFINITY, -INFINITY, -INFINITY});
@@ -120,7 +120,8 @@ int main(int, char **argv)
         b.ly = fmin(b.ly, pos[i].y); b.hy = fmax(b.hy, pos[i].y);
     }
     ids[n] = n;
-    sd.n = n;
+    sd.poff = other;
+    sd.n = n - other;
     MeshDev m{};
     m.n = n; m.pos = pos.data(); m.status = &status; m.sets = &sd; m.vset = zero.data();
     std::vector<u64> lines(HULL_LINES);
@@ -166,8 +167,8 @@ def search(tmp_path_factory):
     subprocess.run([HIPCC, "--offload-host-only", "-O2", "-std=c++17", "-ffp-contract=off", "-I", str(d), str(d / "h.cpp"), "-o", str(d / "h")] +
                    calls, check=True, capture_output=True)
 
-    def run(xy, demands, scale):
-        (d / "in").write_text("%d %d %s\n" % (len(xy), len(demands), float(scale).hex()) +
+    def run(xy, demands, scale, other=0):
+        (d / "in").write_text("%d %d %s %d\n" % (len(xy), len(demands), float(scale).hex(), other) +
                               "\n".join(float(x).hex() + " " + float(y).hex() for x, y in xy) + "\n" +
                               "\n".join("%d %d" % tuple(e) for e in demands) + "\n")
         out = subprocess.run([str(d / "h"), str(d / "in")], check=True, capture_output=True, text=True, timeout=30).stdout.split()
@@ -228,6 +229,26 @@ def test_scaled(search, kind, e):
     assert np.array_equal(got, want), (got != want).any(1).sum()
 
 
+@pytest.mark.parametrize("e", [(-500, 500), (500, -500), (-1000, 100)])
+def test_two_sets(search, e):
+    """A box may hold vertices of two sets of a batch, of very different scale."""
+    rng = np.random.default_rng(8)
+    xy = np.stack(np.meshgrid(np.arange(38.0), np.arange(38.0)), -1).reshape(-1, 2) / 64
+    xy = _morton(xy[rng.random(len(xy)) < 0.6])
+    at = {tuple(v): k for k, v in enumerate(xy)}
+    demands = []
+    for k in range(120):   # axis-parallel edges of the lattice, the first box's vertices left of some
+        for d in ((1, 0), (0, 1), (2, 0), (0, 2)):
+            o = at.get((xy[k, 0] + d[0] / 64, xy[k, 1] + d[1] / 64))
+            if o is not None:
+                demands += [(k, o), (o, k)]
+    demands = np.array(demands)
+    want, _ = search(xy, demands, _scale(xy))
+    other = 40
+    got, _ = search(np.concatenate([np.ldexp(xy[:other], e[1]), np.ldexp(xy, e[0])]), demands + other, np.ldexp(_scale(xy), e[0]), other)
+    assert np.array_equal(got[:, 0] - other * (got[:, 0] >= 0), want[:, 0])
+
+
 def _apex(xy, p, q):
     """The vertex left of p -> q whose circle through p and q holds no other, in rationals."""
     F = [(Fraction(float(x)), Fraction(float(y))) for x, y in xy]
@@ -286,4 +307,18 @@ def test_scaled_triangulation(kind, e):
     want = ctx.delaunay(xy, 512)
     assert len(want) > 600
     assert np.array_equal(ctx.delaunay(np.ldexp(xy, e), 512), want)
+    ctx.close()
+
+
+@pytest.mark.gpu
+def test_scaled_batch():
+    """Sets of a batch with scales so far apart that a box of both overflows in either's."""
+    import galpha2d_amd as G
+    print("case: batch of scaled sets", flush=True)
+    grid = np.stack(np.meshgrid(np.arange(20.0), np.arange(20.0)), -1).reshape(-1, 2)
+    sets = [_points("ring", 700)[:650], grid, _points("arc", 500)[:333], grid[:390]]
+    ctx = G.Context(0)
+    want = ctx.batch(sets)
+    for t, u in zip(ctx.batch([np.ldexp(xy, e) for xy, e in zip(sets, (-500, 480, 0, -360))]), want):
+        assert len(u) > 300 and np.array_equal(t, u)
     ctx.close()
